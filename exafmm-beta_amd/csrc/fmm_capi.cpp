@@ -91,7 +91,7 @@ struct fmm_ctx {
   int p2p_nwide = 0;  // P2P targets [0, p2p_nwide) are leaves of >= 16 bodies
   fmm::M2LGroups groups;
   DBuf g_tgt, g_src, g_dx, g_chunk, r_ptr, r_src, r_tgt;
-  DBuf t_tgt, t_ptr, t_slice, t_src, t_lt, g_y, g_ops, c_dx, c_sc;
+  DBuf t_tgt, t_ptr, t_slice, t_src, t_lt, g_ops, c_dx;
   // M2M / L2L as per-level operators on MFMA (regular trees)
   bool xl = false;
   std::vector<int> xl_tptr;  // per child level: first L2L tile
@@ -102,8 +102,7 @@ struct fmm_ctx {
   DBuf per_F, per_T, per_S, per_cur, per_tmp, per_dx, per_kind;
   // mixed precision: per-group (R_s, R_t), cell radii, FP32 multipoles
   bool mixed = false;
-  bool h16 = false;  // FMM_MIXED16: split-FP16 M2L operands (M16 instead of M32)
-  DBuf g_sc, cr, M32, M16;
+  DBuf g_sc, cr, M32;
   DBuf dip;  // dipole partial sums
   DBuf ew_b, ew_t, ew_k, ew_s;  // fmm_ewald: bodies, targets, wave vectors, structure factors
   DBuf op_d, op_i;  // fmm_kernel_*: doubles (bodies, centres, expansions) and ints of one call
@@ -359,6 +358,7 @@ int fmm_create(fmm_ctx **out, const fmm_params *p) {
         std::lock_guard<std::mutex> lk(g_init_mu);
         if (!g_init_done[p->device]) {
           HIPCHK(fmmdev::init_constants());
+          HIPCHK(fmmdev::init_rot_constants());
           HIPCHK(fmmdev::init_scratch(p->device));
           g_init_done[p->device] = true;
         }
@@ -400,6 +400,22 @@ void fmm_destroy(fmm_ctx *c) {
 const char *fmm_last_error(const fmm_ctx *c) { return c ? c->err.c_str() : "null context"; }
 
 namespace {
+// the M2L of these parameters runs on target tiles (offset groups that do not
+// fix the levels, whatever the precision), else on chunks (MIXED: by level)
+bool takes_tiles(const fmm_params &p) {
+  return (p.m2l_mode == FMM_M2L_TILES || p.m2l_mode == FMM_M2L_AUTO) && fmmdev::m2l_rot_supported(p.P);
+}
+bool uniform_levels(const fmm::Tree &t) {  // every radius R0 / 2^level
+  for (int k = 0; k < t.ncell; k++)
+    if (t.R[k] != t.R[0] / (1 << t.level[k])) return false;
+  return true;
+}
+// groups built on the device hold no pair arrays (grp_ptr is {0})
+bool holds_pairs(const fmm::M2LGroups &g) { return g.grp_ptr.size() == (size_t)g.ngroup + 1; }
+int groups_kind_for(const fmm_params &p) {
+  return p.precision != FMM_FP64 && !takes_tiles(p) ? FMM_MIXED : FMM_FP64;
+}
+
 void plan_fill(fmm_plan *pl, int n, const double *x, int ncrit, double theta, int nspawn, int images = 0,
                const double *cycle = nullptr) {
   pl->images = images;
@@ -522,16 +538,13 @@ int fmm_plan_build_device(fmm_ctx *c, fmm_plan **out, int n, const double *x, in
     double t3 = now_ms();
     // the M2L groups and tiles of the context's precision and order, when its
     // M2L takes the tile path (else, or if they do not fit, built at upload)
-    const bool mixed = c->p.precision != FMM_FP64;
-    const bool tiles = c->p.m2l_mode == FMM_M2L_TILES ||
-                       (c->p.m2l_mode == FMM_M2L_AUTO && fmmdev::m2l_tiles_preferred(c->p.P, mixed));
-    if (tiles && (mixed ? fmmdev::m2l_mixed_supported(c->p.P) : fmmdev::m2l_mfma_supported(c->p.P))) {
+    if (takes_tiles(c->p)) {
       bool done = false;
-      HIPCHK(fmmdev::device_groups_tiles(pl->tree, pl->lists, mixed, fmmdev::m2l_tile_targets(c->p.P), 16,
-                                         fmmdev::kM2LItemSlices, pl->groups, pl->tiles, done, c->st,
+      HIPCHK(fmmdev::device_groups_tiles(pl->tree, pl->lists, fmmdev::m2l_tile_targets(c->p.P),
+                                         fmmdev::kM2LSlicePairs, 0, pl->groups, pl->tiles, done, c->st,
                                          pl->dev.get()));
       if (done) {
-        pl->groups_kind = mixed ? FMM_MIXED : FMM_FP64;
+        pl->groups_kind = FMM_FP64;
       } else {
         pl->groups = fmm::M2LGroups();
         pl->tiles = fmm::M2LTiles();
@@ -637,21 +650,21 @@ int fmm_plan_prepare(fmm_plan *pl, const fmm_params *p) {
     return FMM_ERR_ARG;
   if (p->m2l_mode == FMM_M2L_TARGET) return FMM_OK;
   const bool mixed = p->precision != FMM_FP64;
-  const int kind = mixed ? FMM_MIXED : FMM_FP64;  // FMM_MIXED16 groups as FMM_MIXED
+  const int kind = groups_kind_for(*p);
   if (!(mixed ? fmmdev::m2l_mixed_supported(p->P) : fmmdev::m2l_mfma_supported(p->P))) return FMM_OK;
   try {
-    if (pl->groups_kind != kind) {
+    const int TT = fmmdev::m2l_tile_targets(p->P);
+    const bool fit_tiles = takes_tiles(*p) && pl->tiles.TT == TT;
+    if (pl->groups_kind != kind || !(fit_tiles || holds_pairs(pl->groups))) {
       if (plan_to_host(pl) != hipSuccess) return FMM_ERR_DEVICE;
-      pl->groups = fmm::build_m2l_groups(pl->tree, pl->lists, fmmdev::kM2LChunkPairs, mixed,
+      pl->dev.reset();  // lists on the host now, other tiles than the device's below
+      pl->groups = fmm::build_m2l_groups(pl->tree, pl->lists, fmmdev::kM2LChunkPairs, kind == FMM_MIXED,
                                          pl->images > 0 ? pl->cycle : nullptr);
       pl->groups_kind = kind;
       pl->tiles = fmm::M2LTiles();
     }
-    const int TT = fmmdev::m2l_tile_targets(p->P);
-    const bool tiles =
-        p->m2l_mode == FMM_M2L_TILES || (p->m2l_mode == FMM_M2L_AUTO && fmmdev::m2l_tiles_preferred(p->P, mixed));
-    if (tiles && pl->tiles.TT != TT)
-      pl->tiles = fmm::build_m2l_tiles(pl->tree, pl->groups, TT, 16);
+    if (takes_tiles(*p) && pl->tiles.TT != TT)
+      pl->tiles = fmm::build_m2l_tiles(pl->tree, pl->groups, TT, fmmdev::kM2LSlicePairs, 0);
   } catch (const std::bad_alloc &) {
     return FMM_ERR_MEMORY;
   }
@@ -952,11 +965,9 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
     UP(xl_child8, child8) UP(xl_children, children) UP(xl_tiles, tiles) UP(xl_dx, dxs) UP(xl_kinds, kinds)
   }
   c->mixed = c->p.precision == FMM_MIXED || c->p.precision == FMM_MIXED16;
-  c->h16 = c->p.precision == FMM_MIXED16;
   c->use_mfma = c->p.m2l_mode != FMM_M2L_TARGET && L.nm2l > 0 &&
                 (c->mixed ? fmmdev::m2l_mixed_supported(c->p.P) : fmmdev::m2l_mfma_supported(c->p.P));
-  c->use_tiles = c->use_mfma && (c->p.m2l_mode == FMM_M2L_TILES ||
-                                 (c->p.m2l_mode == FMM_M2L_AUTO && fmmdev::m2l_tiles_preferred(c->p.P, c->mixed)));
+  c->use_tiles = c->use_mfma && takes_tiles(c->p);
   c->groups = fmm::M2LGroups();
   c->nchunk = 0;
   c->ntile = 0;
@@ -964,12 +975,12 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
   fmmdev::PlanArrays loc;  // groups and tiles built on the device by this upload
   bool plan_tiles = false;  // tiles taken from the plan
   if (c->use_mfma) {
-    // groups built with the plan on the device carry no chunks (grp_ptr is
-    // {0}): the chunk path builds its own
-    if (pl.groups_kind == (c->mixed ? FMM_MIXED : FMM_FP64) &&
-        (c->use_tiles || pl.groups.grp_ptr.size() == (size_t)pl.groups.ngroup + 1)) {
+    // groups built with the plan on the device hold no pair arrays: they serve
+    // only with the tiles built beside them (of this order's tile size)
+    const bool fit_tiles = c->use_tiles && pl.tiles.TT == fmmdev::m2l_tile_targets(c->p.P);
+    if (pl.groups_kind == groups_kind_for(c->p) && (fit_tiles || holds_pairs(pl.groups))) {
       c->groups = std::move(pl.groups);
-      if (pl.tiles.TT == fmmdev::m2l_tile_targets(c->p.P)) {
+      if (fit_tiles) {
         tiles = std::move(pl.tiles);
         plan_tiles = true;
       }
@@ -980,8 +991,8 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
         // the lists just uploaded (the host build's groups, classes, tiles
         // and slices), their pair arrays left there; irregular trees and
         // offsets out of the key's range fall back to the host build
-        const hipError_t e = fmmdev::device_groups_tiles(t, L, c->mixed, fmmdev::m2l_tile_targets(c->p.P), 16,
-                                                         fmmdev::kM2LItemSlices, c->groups, tiles, done, c->st,
+        const hipError_t e = fmmdev::device_groups_tiles(t, L, fmmdev::m2l_tile_targets(c->p.P),
+                                                         fmmdev::kM2LSlicePairs, 0, c->groups, tiles, done, c->st,
                                                          &loc, c->m2l_src.as<int>());
         if (e != hipSuccess) {
           (void)hipStreamSynchronize(c->st);
@@ -1000,7 +1011,10 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
             HIPCHK(e);
           }
         }
-        c->groups = fmm::build_m2l_groups(t, L, fmmdev::kM2LChunkPairs, c->mixed,
+        // mixed: on a tree whose levels do not share a radius the pairs of
+        // other radii than their group's run per target, as on chunks
+        const bool by_level = c->mixed && (!c->use_tiles || !uniform_levels(t));
+        c->groups = fmm::build_m2l_groups(t, L, fmmdev::kM2LChunkPairs, by_level,
                                           c->p.images > 0 ? c->p.cycle : nullptr);
       }
     }
@@ -1008,12 +1022,9 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
     UP(g_dx, G.dx) UP(r_ptr, G.rest_ptr) UP(r_src, G.rest_src) UP(r_tgt, G.rest_targets)
     if (c->use_tiles) {
       const bool dt = plan_tiles && dev_tiles;  // the plan's tiles, their pair arrays on this device
-      if (tiles.TT == 0) tiles = fmm::build_m2l_tiles(t, G, fmmdev::m2l_tile_targets(c->p.P), 16);
+      if (tiles.TT == 0)
+        tiles = fmm::build_m2l_tiles(t, G, fmmdev::m2l_tile_targets(c->p.P), fmmdev::kM2LSlicePairs, 0);
       c->ntile = (int)(tiles.item.size() / 4);  // work items
-      // the tile kernel holds an item's slice descriptors one per lane
-      for (size_t i = 0; i < tiles.item.size(); i += 4)
-        if (tiles.item[i + 2] - tiles.item[i + 1] > fmmdev::kM2LItemSlices)
-          FMM_FAIL(FMM_ERR_UNSUPPORTED, "M2L tiles: a work item holds more than 64 slices");
       UP(t_tgt, tiles.tgt) UP(t_ptr, tiles.item)
       if (dt) {
         DC(t_slice, pdev->t_slice) DC(t_src, pdev->t_src) DC(t_lt, pdev->t_lt)
@@ -1025,12 +1036,11 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
         UP(t_slice, tiles.slice) UP(t_src, tiles.src) UP(t_lt, tiles.lt)
       }
       UP(c_dx, G.cdx)
-      if (c->mixed) UP(c_sc, G.cscale)
     } else {
       c->nchunk = (int)(G.chunk.size() / 4);
       UP(g_tgt, G.tgt) UP(g_src, G.src) UP(g_chunk, G.chunk)
     }
-    if (c->mixed) {
+    if (c->mixed && !c->use_tiles) {
       UP(g_sc, G.scale) UP(cr, t.R)
     }
   }
@@ -1043,8 +1053,7 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
   if ((rc = ensure(c, c->az, sizeof(double) * n))) return rc;
   if ((rc = ensure(c, c->M, sizeof(double2) * NT * nc))) return rc;
   if ((rc = ensure(c, c->L, sizeof(double2) * NT * nc))) return rc;
-  if (c->mixed && !c->h16 && (rc = ensure(c, c->M32, sizeof(float2) * NT * nc))) return rc;
-  if (c->h16 && (rc = ensure(c, c->M16, fmmdev::m16_record_bytes(c->p.P) * nc))) return rc;
+  if (c->mixed && c->use_mfma && !c->use_tiles && (rc = ensure(c, c->M32, sizeof(float2) * NT * nc))) return rc;
   c->cyc = c->p.images > 0 ? make_double3(c->p.cycle[0], c->p.cycle[1], c->p.cycle[2]) : make_double3(0, 0, 0);
   c->far = c->p.images >= 2 && nc > 0;
   if (c->far) {  // traversePeriodic (include/traversal.h:233-287) as one operator on the root
@@ -1107,14 +1116,10 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
     if ((rc = ensure(c, c->xl_frag, sizeof(double) * fmmdev::xlate_frag_stride(c->p.P) * nop))) return rc;
     HIPCHK(fmmdev::launch_ops_to_frag(c->p.P, c->xl_ops.as<double>(), nop, c->xl_frag.as<double>(), c->st));
   }
-  if (c->use_tiles) {  // harmonics, then the dense operator, of every representative offset, once per plan
+  if (c->use_tiles) {  // the operators of every representative offset, once per plan
     const int nr = c->groups.ncanon;
-    const size_t ny = (size_t)fmmdev::group_harmonics_size(c->p.P) * nr;
-    if ((rc = ensure(c, c->g_y, sizeof(double2) * ny))) return rc;
-    HIPCHK(fmmdev::launch_group_harmonics(c->p.P, c->c_dx.as<double>(), nr, c->g_y.as<double2>(), c->st));
-    if ((rc = ensure(c, c->g_ops, fmmdev::group_ops_bytes(c->p.P, c->mixed, c->h16) * nr))) return rc;
-    HIPCHK(fmmdev::launch_group_ops(c->p.P, c->mixed, c->h16, c->g_y.as<double2>(), c->c_sc.as<double2>(), nr,
-                                    c->g_ops.p, c->st));
+    if ((rc = ensure(c, c->g_ops, fmmdev::rot_ops_bytes(c->p.P) * nr))) return rc;
+    HIPCHK(fmmdev::launch_rot_ops(c->p.P, c->c_dx.as<double>(), nr, c->g_ops.p, c->st));
   }
   double t4 = now_ms();
   pl.tree = fmm::Tree();
@@ -1277,19 +1282,13 @@ int fmm_m2l(fmm_ctx *c) {
   const double3 xper = c->cyc;  // image shifts of the source codes
   if (c->timing) HIPCHK(hipEventRecord(c->kev[0], c->st));
   if (c->use_mfma) {
-    if (c->h16)
-      HIPCHK(fmmdev::launch_m_to_f16(c->p.P, c->M.as<double2>(), c->cr.as<double>(), c->tree.ncell, c->M16.p,
-                                     c->st));
-    else if (c->mixed)
+    if (c->use_tiles) {
+      HIPCHK(fmmdev::launch_m2l_rot(c->p.P, c->ntile, c->t_tgt.as<int>(), c->t_ptr.as<int4>(), c->t_slice.as<int4>(),
+                                    c->t_src.as<int>(), c->t_lt.as<unsigned short>(), c->g_ops.p, c->M.as<double2>(),
+                                    c->L.as<double2>(), c->st));
+    } else if (c->mixed) {
       HIPCHK(fmmdev::launch_m_to_f32(c->p.P, c->M.as<double2>(), c->cr.as<double>(), c->tree.ncell,
                                      c->M32.as<float2>(), c->st));
-    if (c->use_tiles) {
-      HIPCHK(fmmdev::launch_m2l_tile(c->p.P, c->mixed, c->h16, c->ntile, c->t_tgt.as<int>(), c->t_ptr.as<int4>(),
-                                     c->t_slice.as<int4>(), c->t_src.as<int>(), c->t_lt.as<unsigned short>(),
-                                     c->g_ops.p, c->cr.as<double>(),
-                                     c->h16 ? c->M16.p : (c->mixed ? c->M32.p : c->M.p), c->L.as<double2>(),
-                                     c->st));
-    } else if (c->mixed) {
       HIPCHK(fmmdev::launch_m2l_mfma32(c->p.P, c->g_chunk.as<int4>(), c->nchunk, c->g_dx.as<double>(),
                                        c->g_sc.as<double2>(), c->g_tgt.as<int>(), c->g_src.as<int>(),
                                        c->M32.as<float2>(), c->L.as<double2>(), c->st));

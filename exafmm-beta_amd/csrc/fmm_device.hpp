@@ -58,7 +58,6 @@ hipError_t launch_m2l(int P, DevCells C, const int *targets, int ntarget, const 
 // value).  Available for the orders where m2l_mfma_supported(P).
 bool m2l_mfma_supported(int P);
 constexpr int kM2LChunkPairs = 512;  // pairs per M2L chunk (one block)
-constexpr int kM2LItemSlices = 64;   // most slices in one M2L tile work item (one per lane)
 hipError_t launch_m2l_mfma(int P, const int4 *chunks, int nchunk, const double *gdx, const int *ptgt,
                            const int *psrc, const double2 *M, double2 *L, hipStream_t s);
 // L2L into every cell in `cells` from its parent (laplace.h:324-357); accumulates
@@ -66,27 +65,20 @@ hipError_t launch_l2l(int P, DevCells C, const int *cells, int ncell, double2 *L
 // L2P for every body (laplace.h:359-388); accumulates into the targets
 hipError_t launch_l2p(int P, DevBodies B, DevCells C, const int *body_leaf, int n,
                       const double2 *L, hipStream_t s);
-// P2P for every target leaf over its CSR list (laplace.h:150-235); overwrites
-// the targets of each listed leaf
-// target-stationary grouped M2L (tiles of m2l_tile_targets(P) targets, slices
-// of <= 16 pairs of one group, one block per work item of a tile); mix: FP32
-// operands on M32, else FP64 on M.  A tile in one item stores its targets' L,
-// a split tile adds into L (which must start at zero).
+// Target-tile M2L (fmm_rot.hip, 2 <= P <= 12): tiles of m2l_tile_targets(P)
+// targets, slices of at most kM2LSlicePairs pairs of one offset class, one
+// wavefront per work item of a tile.  ops: every class's record
+// (rot_ops_bytes(P) each) from its offset with non-negative components.  A
+// tile in one item stores its targets' L, a split tile adds into L (which
+// must start at zero).
+bool m2l_rot_supported(int P);
 int m2l_tile_targets(int P);
-bool m2l_tiles_preferred(int P, bool mixed);  // AUTO uses tiles (else chunks) at this order
-// h16 (with mix): split-FP16 operands (tables of group_ops_bytes(P, true, true)
-// per group, multipoles from launch_m_to_f16)
-hipError_t launch_m2l_tile(int P, bool mix, bool h16, int nitem, const int *ttgt, const int4 *items,
-                           const int4 *slices, const int *psrc, const unsigned short *plt, const void *ops,
-                           const double *cr, const void *M, double2 *L, hipStream_t s);
-// every group's dense operator as the tile kernel's MFMA A operands (from the
-// group harmonics); group_ops_bytes: bytes per group
-size_t group_ops_bytes(int P, bool mix, bool h16 = false);
-hipError_t launch_group_ops(int P, bool mix, bool h16, const double2 *gY, const double2 *gscale, int ngroup,
-                            void *ops, hipStream_t s);
-// singular harmonics of every group offset (group_harmonics_size(P) complex each)
-int group_harmonics_size(int P);
-hipError_t launch_group_harmonics(int P, const double *gdx, int ngroup, double2 *Y, hipStream_t s);
+constexpr int kM2LSlicePairs = 4;
+size_t rot_ops_bytes(int P);
+hipError_t init_rot_constants();
+hipError_t launch_rot_ops(int P, const double *cdx, int nrep, void *ops, hipStream_t s);
+hipError_t launch_m2l_rot(int P, int nitem, const int *ttgt, const int4 *items, const int4 *slices, const int *psrc,
+                          const unsigned short *plt, const void *ops, const double2 *M, double2 *L, hipStream_t s);
 // M2M / L2L as per-level dense operators on MFMA (8 child offsets per level):
 // ops built once per plan (kind 0 M2M with dX = X_parent - X_child, 1 L2L
 // with dX = X_child - X_parent; xlate_op_stride(P) doubles each)
@@ -115,13 +107,10 @@ hipError_t launch_l2l_mfma(int P, const int4 *tiles, int ntile, const int *child
 // M2L with per-group scales (R_s, R_t) accumulating into the FP64 L; FP32 P2P
 bool m2l_mixed_supported(int P);
 hipError_t launch_m_to_f32(int P, const double2 *M, const double *R, int ncell, float2 *M32, hipStream_t s);
-// split-FP16 multipoles: per cell NT terms (re hi|lo, im hi|lo halves) and
-// its k-block scales, m16_record_bytes(P) per cell
-size_t m16_record_bytes(int P);
-hipError_t launch_m_to_f16(int P, const double2 *M, const double *R, int ncell, void *M16, hipStream_t s);
 hipError_t launch_m2l_mfma32(int P, const int4 *chunks, int nchunk, const double *gdx, const double2 *gscale,
                              const int *ptgt, const int *psrc, const float2 *M32, double2 *L, hipStream_t s);
-// targets[0, nwide) are leaves of at least kP2PWideLeaf bodies (run with four
+// P2P for every target leaf over its CSR list (laplace.h:150-235); overwrites
+// the targets of each listed leaf.  targets[0, nwide) are leaves of at least kP2PWideLeaf bodies (run with four
 // targets per lane), the rest run with one
 constexpr int kP2PWideLeaf = 16;
 hipError_t launch_p2p32(DevBodies B, DevCells C, const int *targets, int ntarget, const int *ptr,
@@ -207,7 +196,7 @@ hipError_t fetch_tiles(const PlanArrays &d, fmm::M2LTiles &T, hipStream_t s);
 // the tiles' slices, pair sources and pair targets are left in keep instead
 // of T (keep->tiles).  dsrc_in: the lists' source column already on the
 // device (stream s), read instead of L.m2l_src.
-hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, bool by_level, int TT, int SW, int seg,
+hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, int TT, int SW, int seg,
                                fmm::M2LGroups &G, fmm::M2LTiles &T, bool &done, hipStream_t s,
                                PlanArrays *keep = nullptr, const int *dsrc_in = nullptr);
 // The octree of n bodies (host array x, AoS) built on the device: the same

@@ -1046,10 +1046,24 @@ void deal_m2l_chunks(M2LGroups &G, int chunk_pairs) {
 
 void split_m2l_tiles(M2LTiles &T, int seg) {
   std::vector<int> it;
+  if (seg <= 0) {
+    // Slices per work item.  A split tile pays an atomic per output value of
+    // every item, a long item leaves wavefront slots (2048) idle at the end.
+    // M2L of 16 / 48 / 64 / 128 / 256 slices: 4096-body cube, P = 8 (4.4k
+    // slices) 0.023 / 0.038 / 0.047 / 0.085 / 0.16 ms; 32768, P = 10 (80k)
+    // 0.196 / 0.118 / 0.132 / 0.170 / 0.297; 131072, P = 12 (560k) 0.40 /
+    // 0.24 / 0.20 / 0.28 / 0.39; 10^6, P = 12 (4.6M) 12.1 / 5.48 / 5.47 /
+    // 5.21 / 5.29
+    const int64_t total = T.ntile > 0 ? T.ptr[T.ntile] : 0;
+    seg = (int)std::max<int64_t>({16, std::min<int64_t>(64, total / 1700), std::min<int64_t>(128, total / 16000)});
+  }
   for (int b = 0; b < T.ntile; b++) {
     const int a = T.ptr[b], e = T.ptr[b + 1];
     const int split = e - a > seg ? 1 : 0;
-    for (int k = a; k < e; k += seg) it.insert(it.end(), {b, k, std::min(e, k + seg), split});
+    // a tile's items have equal lengths, to one slice
+    const int n = (e - a + seg - 1) / seg;
+    for (int k = 0; k < n; k++)
+      it.insert(it.end(), {b, a + (int)((int64_t)(e - a) * k / n), a + (int)((int64_t)(e - a) * (k + 1) / n), split});
   }
   // launch order: block i runs on XCD i % 8.  Runs of kRun consecutive items
   // (neighbouring tiles, sharing source multipoles) go to one XCD, and the
@@ -1074,32 +1088,20 @@ M2LTiles build_m2l_tiles(const Tree &t, const M2LGroups &G, int TT, int SW, int 
   const int64_t np = (int64_t)G.tgt.size();
   T.ptr.assign(1, 0);
   if (np == 0) return T;
-  // targets of grouped pairs, ordered by (level, octant in parent, cell)
+  // targets of grouped pairs, ordered by (level, cell): siblings are adjacent
+  // and, being reflections of each other in their parent, have their offsets
+  // in the same classes
   std::vector<char> has(nc, 0);
   for (int c : G.tgt) has[c] = 1;
   std::vector<int> tg;
   for (int c = 0; c < nc; c++)
     if (has[c]) tg.push_back(c);
-  auto octant = [&](int c) {
-    if (c == 0) return 0;
-    const int p = t.iparent[c];
-    int o = 0;
-    for (int d = 0; d < 3; d++)
-      if (t.X[3 * (size_t)c + d] > t.X[3 * (size_t)p + d]) o |= 1 << d;
-    return o;
-  };
-  std::vector<int64_t> key(tg.size());
-  for (size_t i = 0; i < tg.size(); i++)
-    key[i] = ((int64_t)t.level[tg[i]] << 40) | ((int64_t)octant(tg[i]) << 32) | tg[i];
-  std::vector<int> ord(tg.size());
-  for (size_t i = 0; i < ord.size(); i++) ord[i] = (int)i;
-  std::sort(ord.begin(), ord.end(), [&](int a, int b) { return key[a] < key[b]; });
+  std::stable_sort(tg.begin(), tg.end(), [&](int a, int b) { return t.level[a] < t.level[b]; });
   const int nt = (int)((tg.size() + TT - 1) / TT);
   std::vector<int> tile_of(nc, -1), local(nc, -1);
-  for (size_t i = 0; i < ord.size(); i++) {
-    const int c = tg[ord[i]];
-    tile_of[c] = (int)(i / TT);
-    local[c] = (int)(i % TT);
+  for (size_t i = 0; i < tg.size(); i++) {
+    tile_of[tg[i]] = (int)(i / TT);
+    local[tg[i]] = (int)(i % TT);
   }
   // pairs bucketed by tile; taking the groups in (representative,
   // reflection) order keeps each tile's pairs sorted that way, so a tile
@@ -1171,7 +1173,7 @@ M2LTiles build_m2l_tiles(const Tree &t, const M2LGroups &G, int TT, int SW, int 
   // slice mixes reflections but never repeats a target.
   T.ntile = nt;
   T.tgt.assign((size_t)T.ntile * TT, -1);
-  for (size_t i = 0; i < ord.size(); i++) T.tgt[i] = tg[ord[i]];
+  for (size_t i = 0; i < tg.size(); i++) T.tgt[i] = tg[i];
   std::vector<std::vector<int>> tsl(nt);  // per tile: (representative, first, count) per slice
   const int RT = std::min(R, std::max(nt, 1));
   par(RT, [&](int r) {

@@ -146,16 +146,15 @@ M2LGroups build_m2l_groups(const Tree &t, const Lists &L, int chunk_pairs, bool 
 void list_counts(const Tree &t, const Lists &L, uint64_t *icell, int *nump2p, int *numm2l);
 
 // Target-stationary layout of the grouped M2L pairs: targets are sorted by
-// (level, octant within the parent, cell) -- cells of one octant class share
-// their offsets -- and cut into tiles of TT targets.  A tile's pairs are
-// ordered by representative and cut into slices of at most SW pairs with
-// distinct targets (a slice may mix the representative's reflections), so a
-// block can apply each representative's operator to whole slices and keep the
-// tile's local expansions in LDS until one final store.  Tiles are listed in
-// launch order (dealt to the 8 XCDs in contiguous runs; empty tiles pad).
-// A block runs one work item: at most `seg` consecutive slices of one tile.
-// A tile split over several items adds its results (atomics); a tile in one
-// item stores them.
+// (level, cell) -- siblings are adjacent and, being each other's reflections,
+// share their offset classes -- and cut into tiles of TT targets.  A tile's
+// pairs are ordered by representative and cut into slices of at most SW pairs
+// with distinct targets (a slice may mix the representative's reflections),
+// so that one operator serves whole slices while the tile's local expansions
+// stay in LDS.  A work item is at most `seg` consecutive slices of one tile
+// (seg <= 0: chosen from the number of slices), listed in launch order (dealt
+// to the 8 XCDs in contiguous runs; empty items pad).  A tile split over
+// several items adds its results (atomics); a tile in one item stores them.
 struct M2LTiles {
   int TT = 0, ntile = 0;
   std::vector<int> tgt;        // ntile*TT target cells (-1 pads), launch order
@@ -166,7 +165,7 @@ struct M2LTiles {
                                // reflection bits of its group (bits 8-10)
   std::vector<int> item;       // 4 per work item: tile, first slice, end slice, split (0/1)
 };
-M2LTiles build_m2l_tiles(const Tree &t, const M2LGroups &G, int TT, int SW, int seg = 64);
+M2LTiles build_m2l_tiles(const Tree &t, const M2LGroups &G, int TT, int SW, int seg = 0);
 void split_m2l_tiles(M2LTiles &T, int seg);
 
 // (Re)build G.chunk from the groups: chunks of at most chunk_pairs pairs,

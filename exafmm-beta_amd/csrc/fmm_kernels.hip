@@ -1513,903 +1513,6 @@ __global__ __launch_bounds__(64) void p2p32_kernel(DevBodies B, DevCells C, cons
   }
 }
 
-// ---------------------------------------------------------------- M2L, target-stationary
-// One block per tile of up to TT target cells (host: same level and octant
-// class, so they share most offsets).  The tile's pairs come ordered by
-// representative offset in slices of at most 16 pairs of one representative
-// (any of its reflections; each pair carries its own reflection bits).  For
-// each representative the block loads its operator once (A operands in
-// registers, from the per-plan table), then runs every slice of it: the 16
-// source multipoles, sign-flipped per pair, are gathered into an LDS B tile,
-// one MFMA chain per 16-row block, and the 16x16 results, sign-flipped per
-// pair, are added into the tile's local expansions held in LDS (FP64).  A
-// slice's pairs have distinct targets and a wavefront owns its rows, so the
-// LDS additions need no atomics.  At the end every target's
-// local expansion is stored once; a tile too long for one block is split into
-// work items whose parts are added with FP64 atomics (a few per target instead
-// of one per pair).
-// MIX: FP32 operands and FP32-MFMA on level-scaled multipoles (T' = T R_s^n
-// R_t^j, M32 = M~/R^n); the per-group partial results are accumulated in FP64
-// and scaled by R_t^-j at the store.
-template <int P, bool MIX, bool H16 = false> struct TileCfg {
-  static constexpr int PP = P * P;
-  static constexpr int KP = (PP + 3) / 4 * 4;
-  static constexpr int KT = KP / 4;
-  static constexpr int RB = (PP + 15) / 16;
-  // P = 12: the 9 row blocks of 16 run on 8 wavefronts, two per SIMD; the
-  // 9th block's k-steps are split in quarters over wavefronts 0, 2, 5 and 7
-  // (one per SIMD whether wavefront w runs on SIMD w % 4 or w / 2), whose
-  // partial sums wavefront COMB adds in a fixed order one slice later.  With
-  // 9 wavefronts one SIMD ran 3 of the 9 MFMA chains of every slice (and the
-  // split-FP16 kernel, held to 168 registers by 3 wavefronts per SIMD,
-  // spilled).  H16: quarter q takes the 32-wide k-blocks q, q + 4, ...
-  static constexpr bool SPLIT = RB == 9 && PP % 16 == 0 && (H16 || KT % 4 == 0);
-  static constexpr int NW = SPLIT ? RB - 1 : RB;  // wavefronts per block
-  static constexpr int NTH = 64 * NW;
-  static constexpr int KQ = KT / 4;               // k-steps of one quarter of the 9th block
-  static constexpr int COMB = 3;
-  static __device__ __forceinline__ int quarter(int w) {
-    return w == 0 ? 0 : w == 2 ? 1 : w == 5 ? 2 : w == 7 ? 3 : -1;
-  }
-  static constexpr int YSZ = (2 * P - 1) * (3 * P - 2);
-  // targets per tile (LDS accumulators): 64, and 80 at P >= 11.  At P = 12
-  // (8M cube) 32 / 48 / 64 measured FP64 209 / 191 / 183 ms and mixed 123 /
-  // 116 / 113 ms, and with the 8-wavefront layout 64 / 80: FP64 167 / 161 ms,
-  // mixed 104 / 103 ms: a bigger tile reads each representative's operator
-  // rows for more targets; at P = 10, 48 measured slower than 64
-  static constexpr int TT = P >= 11 ? 80 : 64;
-  // B tile in LDS: lane l's operands of KG consecutive k-steps are adjacent
-  // (16 bytes), so one LDS read feeds KG MFMAs
-  static constexpr int KG = MIX ? 4 : 2;
-  static constexpr int KTG = (KT + KG - 1) / KG;
-  static constexpr int BSZ = KTG * 64 * KG;
-  // B element (k, column c) of the 16x16x4 operand: k-step k / 4, lane 16 (k % 4) + c
-  static __device__ __forceinline__ int bidx(int k, int c) {
-    const int kt = k >> 2, l = ((k & 3) << 4) | c;
-    return (kt / KG) * 64 * KG + l * KG + kt % KG;
-  }
-  static constexpr int PPA = PP | 1;           // accumulator row stride (odd: fewer bank conflicts)
-  // H16 (split-FP16 operands): 32-deep k-blocks of v_mfma_f32_16x16x32_f16;
-  // the B tile holds [k-block][hi, lo][lane][8 halves], lane 16 (k % 32 / 8)
-  // + column, half k % 8 (the lo part 512 halves after the hi part)
-  static constexpr int KB = (PP + 31) / 32;
-  static constexpr int BSZ16 = KB * 2 * 64 * 8;
-  static __device__ __forceinline__ int bidx16(int k, int c) {
-    const int kb = k >> 5, r = k & 31;
-    return ((kb * 2) * 64 + 16 * (r >> 3) + c) * 8 + (r & 7);
-  }
-  // bytes of one representative in the H16 operator table: the hi / lo A
-  // operands [row block][k-block][hi, lo][lane] (16 bytes each), then the
-  // power-of-two scale of every (operator row, k-block) (float, [row][KB])
-  static constexpr size_t OPS16 = (size_t)RB * KB * 2 * 64 * 16 + (size_t)RB * 16 * KB * 4;
-  // uint2 entries of one cell's H16 multipole record: NT terms, then KB
-  // k-block scales (floats, two per entry)
-  static constexpr int MREC16 = nterm(P) + (KB + 1) / 2;
-  static constexpr int NQ16 = (KB + 3) / 4;  // H16 SPLIT: k-blocks of a quarter (at most)
-  static constexpr int NRS = NW + (SPLIT ? 1 : 0);  // H16: row-scale blocks in LDS (the 9th last)
-  // LDS bytes of the tile kernel's arrays, and whether the item's pair table
-  // (source cell and target / reflection of each of at most 64 x 16 pairs,
-  // 6 KB) fits without lowering the blocks per CU that LDS allows.  With the
-  // table the slice loop loads no pair index from global memory: a load
-  // issued after the gather and used early in the next iteration made every
-  // iteration wait for that gather (vector loads complete in order).
-  static constexpr size_t VS = MIX ? 4 : 8;
-  static constexpr size_t LDS0 = (size_t)(TT + 1) * PPA * 8 + (H16 ? 16 : 2 * (BSZ + 16 / VS) * VS) +
-                                 (H16 ? 2 * (BSZ16 + 520) * 2 : 16) + (size_t)(PP + 2 * nterm(P)) * 4 +
-                                 (SPLIT ? 2 * 1024 * VS : VS) + (H16 ? 2 * KB * 16 * 4 + NRS * 16 * KB * 4 : 8);
-  static constexpr size_t PTAB_BYTES = 64 * 16 * 6;
-  static constexpr bool PTAB = 163840 / (LDS0 + PTAB_BYTES + 1024) >= 163840 / (LDS0 + 1024);
-  static constexpr bool ok = P <= 12;
-  // occupancy hint: at P = 10 FP64 two 7-wavefront tiles per CU need 4
-  // wavefronts per SIMD (at most 128 VGPRs); elsewhere LDS sets the limit
-  static constexpr int WPE = (!MIX && P == 10) ? 4 : 1;
-};
-
-int m2l_tile_targets(int P) { return P >= 11 ? 80 : 64; }
-
-// Tiles read each group's operator from the per-plan table once per tile and
-// accumulate in LDS; chunks build it once per 512 pairs but pay one FP64
-// atomic per output value.  Measured on MI355X (M2L kernel): FP64 P = 10, 1M
-// Plummer: tiles 8.8 ms, chunks 11.7 ms; mixed P = 8 / 12, 8M cube: tiles
-// 29.0 / 135.6 ms, chunks 41+ / 187.3 ms; FP64 P = 12, 8M cube: tiles of 64
-// targets 183 ms, chunks 193 ms (tiles of 32: 209 ms).
-bool m2l_tiles_preferred(int P, bool) { return P <= 12; }
-
-// Singular harmonics Yh[a][b] (a < 2P-1, |b| <= a) of every group's offset,
-// YSZ complex values per group, computed once per plan: one wavefront per
-// group, lane b runs the recurrence of column b.
-template <int P>
-__global__ __launch_bounds__(64) void group_harmonics_kernel(const double *__restrict__ gdx, int ngroup,
-                                                             double2 *__restrict__ Y) {
-  constexpr int YC = 3 * P - 2, OFF = 2 * P - 2, YSZ = (2 * P - 1) * (3 * P - 2);
-  const int g = blockIdx.x, cc = threadIdx.x;
-  if (g >= ngroup) return;
-  double2 *y = Y + (size_t)g * YSZ;
-  for (int e = cc; e < YSZ; e += 64) y[e] = make_double2(0.0, 0.0);
-  __syncthreads();
-  if (cc > 2 * P - 2) return;
-  const double dx = gdx[3 * g], dy = gdx[3 * g + 1], dz = gdx[3 * g + 2];
-  const double r2 = dx * dx + dy * dy + dz * dz;
-  const double inv_r = 1.0 / sqrt(r2), inv_r2 = inv_r * inv_r;
-  double2 smm = make_double2(inv_r, 0.0);
-  for (int i = 1; i <= cc; i++) smm = cscale(cmul(smm, make_double2(dx, dy)), -(2 * i - 1) * inv_r2);
-  double2 sp = make_double2(0.0, 0.0), sc = smm;
-  for (int a = cc; a <= 2 * P - 2; a++) {
-    if (cc <= P - 1) y[a * YC + OFF + cc] = cmul_ipow(sc, cc);
-    if (cc > 0) y[a * YC + OFF - cc] = cmul_ipow(cconj(sc), cc);
-    double2 nx = cscale(csub(cscale(sc, (2 * a + 1) * dz), cscale(sp, (double)(a * a - cc * cc))), inv_r2);
-    sp = sc;
-    sc = nx;
-  }
-}
-
-// The dense operator of every offset group, built once per plan and stored as
-// the tile kernel's MFMA A operands: ops[g][w][kt][lane] is the value lane
-// `lane` of wavefront w feeds to k-step kt, i.e. T[16w + lane%16][4kt + lane/16]
-// (zero past P^2).  T[row][col] from the group's harmonics Yh (rows (j,k,io),
-// columns (n,m,ii) of the real expansion vectors):
-//   A = (-1)^(j+k) Yh[j+n][m-k] i^(k-m),  B = (-1)^j Yh[j+n][-m-k] i^(-m-k)  (m > 0)
-//   re = ii ? (Bi - Ai) : (Ar + Br),  im = ii ? (Ar - Br) : (Ai + Bi)
-// and, mixed, T' = T R_s^n R_t^j (FP32 operands of level-scaled multipoles).
-template <int P, bool MIX>
-__global__ __launch_bounds__(64 * ((P * P + 15) / 16)) void group_ops_kernel(const double2 *__restrict__ gY,
-                                                                              const double2 *__restrict__ gscale,
-                                                                              int ngroup, void *__restrict__ opsv) {
-  using Cfg = TileCfg<P, MIX>;
-  using VT = typename std::conditional<MIX, float, double>::type;
-  // one wavefront per 16-row block of the table (the tile kernel may run the
-  // blocks on fewer wavefronts)
-  constexpr int PP = Cfg::PP, KT = Cfg::KT, RB = Cfg::RB, NTH = 64 * RB;
-  constexpr int YC = 3 * P - 2, OFF = 2 * P - 2;
-  __shared__ double2 sYa[Cfg::YSZ], sYb[Cfg::YSZ];
-  __shared__ double sPow[2][P];
-  const int g = blockIdx.x, tid = threadIdx.x, w = tid >> 6, l = tid & 63;
-  if (g >= ngroup) return;
-  for (int e = tid; e < Cfg::YSZ; e += NTH) {
-    const int b = e % YC - OFF;
-    const double2 y = gY[(size_t)g * Cfg::YSZ + e];
-    sYa[e] = cmul_ipow_sel(y, -b);
-    sYb[e] = cmul_ipow_sel(y, b);
-  }
-  if (MIX && tid < 2) {
-    const double2 rs = gscale[g];
-    const double base = tid == 0 ? rs.x : rs.y;
-    double pw = 1.0;
-    for (int n = 0; n < P; n++) {
-      sPow[tid][n] = pw;
-      pw *= base;
-    }
-  }
-  __syncthreads();
-  const int arow = w * 16 + (l & 15);
-  const int adec = c_vdec[arow < PP ? arow : 0];
-  const int aj = adec & 255, ak = (adec >> 8) & 255, aio = adec >> 16;
-  const double sj = ((aj & 1) ? -1.0 : 1.0) * (MIX ? sPow[1][aj] : 1.0);
-  const double sjk = (ak & 1) ? -sj : sj;
-  VT *ops = static_cast<VT *>(opsv) + ((size_t)g * RB + w) * KT * 64 + l;
-  for (int kt = 0; kt < KT; kt++) {
-    const int kk = kt * 4 + (l >> 4);
-    double val = 0.0;
-    if (arow < PP && kk < PP) {
-      const int dk = c_vdec[kk];
-      const int n = dk & 255, m = (dk >> 8) & 255, ii = dk >> 16;
-      const double pw = MIX ? sPow[0][n] : 1.0;
-      const int base = (aj + n) * YC + OFF;
-      const double2 Av = sYa[base + m - ak];
-      const double2 Bv = m ? sYb[base - m - ak] : make_double2(0.0, 0.0);
-      const double sa = sjk * pw, sb = sj * pw;
-      const bool xs = ii == aio;  // real parts for (re, Re M) and (im, Im M)
-      const double a1 = xs ? Av.x : Av.y, b1 = xs ? Bv.x : Bv.y;
-      const double sgnA = (ii && !aio) ? -sa : sa, sgnB = (ii && aio) ? -sb : sb;
-      val = fma(sgnA, a1, sgnB * b1);
-    }
-    ops[kt * 64] = (VT)val;
-  }
-}
-
-// Split-FP16 operator table (H16): each representative's dense operator, as
-// group_ops_kernel builds it with the mixed scaling T' = T R_s^n R_t^j, in
-// the A operands of v_mfma_f32_16x16x32_f16.  Each 32-wide k-block of an
-// operator row is scaled by the power of two that brings its largest entry
-// into [1, 2) and split into hi = fp16(x) and lo = fp16((x - hi) 2^11): the
-// lo half is kept in the normal range (the MFMA flushes FP16 subnormals),
-// so every entry within 2^-14 of its block's largest keeps 22 significant
-// bits.  The (row, k-block) scales back follow the operands (Cfg::OPS16
-// bytes per representative).
-template <int P>
-__global__ __launch_bounds__(64 * ((P * P + 15) / 16)) void group_ops16_kernel(const double2 *__restrict__ gY,
-                                                                                const double2 *__restrict__ gscale,
-                                                                                int ngroup, void *__restrict__ opsv) {
-  using Cfg = TileCfg<P, true, true>;
-  typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-  constexpr int PP = Cfg::PP, RB = Cfg::RB, KB = Cfg::KB, NTH = 64 * RB;
-  constexpr int YC = 3 * P - 2, OFF = 2 * P - 2;
-  __shared__ double2 sYa[Cfg::YSZ], sYb[Cfg::YSZ];
-  __shared__ double sPow[2][P];
-  const int g = blockIdx.x, tid = threadIdx.x, w = tid >> 6, l = tid & 63;
-  if (g >= ngroup) return;
-  for (int e = tid; e < Cfg::YSZ; e += NTH) {
-    const int b = e % YC - OFF;
-    const double2 y = gY[(size_t)g * Cfg::YSZ + e];
-    sYa[e] = cmul_ipow_sel(y, -b);
-    sYb[e] = cmul_ipow_sel(y, b);
-  }
-  if (tid < 2) {
-    const double2 rs = gscale[g];
-    const double base = tid == 0 ? rs.x : rs.y;
-    double pw = 1.0;
-    for (int n = 0; n < P; n++) {
-      sPow[tid][n] = pw;
-      pw *= base;
-    }
-  }
-  __syncthreads();
-  const int arow = w * 16 + (l & 15);
-  const int adec = c_vdec[arow < PP ? arow : 0];
-  const int aj = adec & 255, ak = (adec >> 8) & 255, aio = adec >> 16;
-  const double sj = ((aj & 1) ? -1.0 : 1.0) * sPow[1][aj];
-  const double sjk = (ak & 1) ? -sj : sj;
-  double val[KB][8];
-  double mx[KB];
-#pragma unroll
-  for (int kb = 0; kb < KB; kb++) {
-    mx[kb] = 0.0;
-#pragma unroll
-    for (int h = 0; h < 8; h++) {
-      const int kk = kb * 32 + 8 * (l >> 4) + h;
-      double v = 0.0;
-      if (arow < PP && kk < PP) {
-        const int dk = c_vdec[kk];
-        const int n = dk & 255, m = (dk >> 8) & 255, ii = dk >> 16;
-        const double pw = sPow[0][n];
-        const int base = (aj + n) * YC + OFF;
-        const double2 Av = sYa[base + m - ak];
-        const double2 Bv = m ? sYb[base - m - ak] : make_double2(0.0, 0.0);
-        const double sa = sjk * pw, sb = sj * pw;
-        const bool xs = ii == aio;
-        const double a1 = xs ? Av.x : Av.y, b1 = xs ? Bv.x : Bv.y;
-        const double sgnA = (ii && !aio) ? -sa : sa, sgnB = (ii && aio) ? -sb : sb;
-        v = fma(sgnA, a1, sgnB * b1);
-      }
-      val[kb][h] = v;
-      mx[kb] = fmax(mx[kb], fabs(v));
-    }
-  }
-  half8 *o = reinterpret_cast<half8 *>(static_cast<char *>(opsv) + (size_t)g * Cfg::OPS16) + (size_t)w * KB * 2 * 64 + l;
-  float *rs = reinterpret_cast<float *>(static_cast<char *>(opsv) + (size_t)g * Cfg::OPS16 + (size_t)RB * KB * 2 * 64 * 16);
-#pragma unroll
-  for (int kb = 0; kb < KB; kb++) {
-    // the block's largest entry in this row, over the 4 lanes that hold it
-    double m = fmax(mx[kb], __shfl_xor(mx[kb], 16, 64));
-    m = fmax(m, __shfl_xor(m, 32, 64));
-    int ex = 1;
-    if (m > 0.0) frexp(m, &ex);  // m = f 2^ex, f in [0.5, 1)
-    const double sc = ldexp(1.0, 1 - ex);
-    half8 hi, lo;
-#pragma unroll
-    for (int h = 0; h < 8; h++) {
-      const double x = val[kb][h] * sc;
-      const _Float16 xh = (_Float16)(float)x;
-      hi[h] = xh;
-      lo[h] = (_Float16)(float)((x - (double)xh) * 2048.0);
-    }
-    o[(kb * 2) * 64] = hi;
-    o[(kb * 2 + 1) * 64] = lo;
-    if (l < 16) rs[arow * KB + kb] = (float)ldexp(1.0, ex - 1);
-  }
-}
-
-// Split-FP16 multipoles (H16): per cell the FP32 path's M32 = M~ / R^n; each
-// real component, in the operator's column order (row r of the real vector,
-// k-block r / 32), is scaled by the power of two that brings its k-block's
-// largest component into [1, 2) and split into hi = fp16(x) and lo =
-// fp16((x - hi) 2^11) (kept out of the FP16 subnormals, which the MFMA
-// flushes); (re hi | re lo << 16, im hi | im lo << 16) per term, then the
-// cell's KB scales back (floats, two per record entry).  Components fall
-// off by about 4x per degree, so one scale per cell would flush the high
-// degrees (CPU emulation of the operators at P = 12: worst interaction 9e-5
-// with one scale per cell, 4e-7 with one per k-block).  One wavefront per cell.
-template <int P>
-__global__ __launch_bounds__(64) void m_to_f16_kernel(const double2 *__restrict__ M, const double *__restrict__ R,
-                                                      int ncell, uint2 *__restrict__ M16) {
-  using Cfg = TileCfg<P, true, true>;
-  constexpr int NT = nterm(P), NI = (NT + 63) / 64, KB = Cfg::KB, MREC = Cfg::MREC16;
-  const int c = blockIdx.x, l = threadIdx.x;
-  if (c >= ncell) return;
-  const double inv = 1.0 / R[c];
-  double2 v[NI];
-  int kre[NI], kim[NI];  // k-blocks of the real and imaginary parts (-1: none)
-#pragma unroll
-  for (int i = 0; i < NI; i++) {
-    const int u = l + 64 * i;
-    v[i] = make_double2(0.0, 0.0);
-    kre[i] = kim[i] = -1;
-    if (u < NT) {
-      const int rr = c_urow[u];
-      const int n = c_vdec[rr & 0xffff] & 255;
-      double f = 1.0;
-      for (int k = 0; k < n; k++) f *= inv;
-      const double2 x = M[(size_t)c * NT + u];
-      v[i] = make_double2(x.x * f, x.y * f);
-      kre[i] = (rr & 0xffff) >> 5;
-      if ((rr >> 16) != (rr & 0xffff)) kim[i] = (rr >> 16) >> 5;
-    }
-  }
-  double sc[KB];
-  uint2 *dst = M16 + (size_t)c * MREC;
-  float *scb = reinterpret_cast<float *>(dst + NT);
-#pragma unroll
-  for (int kb = 0; kb < KB; kb++) {
-    double mx = 0.0;
-#pragma unroll
-    for (int i = 0; i < NI; i++) {
-      if (kre[i] == kb) mx = fmax(mx, fabs(v[i].x));
-      if (kim[i] == kb) mx = fmax(mx, fabs(v[i].y));
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
-    int ex = 1;
-    if (mx > 0.0) frexp(mx, &ex);
-    sc[kb] = ldexp(1.0, 1 - ex);
-    if (l == 0) scb[kb] = (float)ldexp(1.0, ex - 1);
-  }
-  auto split = [](double x) {
-    const _Float16 h = (_Float16)(float)x;
-    const _Float16 lo = (_Float16)(float)((x - (double)h) * 2048.0);
-    return (unsigned)__builtin_bit_cast(unsigned short, h) | ((unsigned)__builtin_bit_cast(unsigned short, lo) << 16);
-  };
-  auto scale_of = [&](int kb) {  // sc[kb] for a runtime kb (unrolled select)
-    double r = 1.0;
-#pragma unroll
-    for (int b = 0; b < KB; b++)
-      if (b == kb) r = sc[b];
-    return r;
-  };
-#pragma unroll
-  for (int i = 0; i < NI; i++) {
-    const int u = l + 64 * i;
-    if (u < NT)
-      dst[u] = make_uint2(split(v[i].x * scale_of(kre[i])), kim[i] >= 0 ? split(v[i].y * scale_of(kim[i])) : 0u);
-  }
-}
-
-template <int P, bool MIX, bool H16 = false>
-__global__ __launch_bounds__((TileCfg<P, MIX, H16>::NTH)) __attribute__((amdgpu_waves_per_eu(TileCfg<P, MIX, H16>::WPE))) void m2l_tile_kernel(
-    const int *__restrict__ ttgt, const int4 *__restrict__ items, const int4 *__restrict__ slices,
-    const int *__restrict__ psrc, const unsigned short *__restrict__ plt, const void *__restrict__ opsv,
-    const double *__restrict__ cr, const void *__restrict__ Mv, double *__restrict__ L) {
-  using Cfg = TileCfg<P, MIX, H16>;
-  static_assert(!H16 || MIX, "split-FP16 operands accumulate like the FP32 path");
-  using VT = typename std::conditional<MIX, float, double>::type;
-  using VT2 = typename std::conditional<MIX, float2, double2>::type;
-  // gathered multipole term: (re, im) in VT, or (H16) the halves re hi | lo << 16, im hi | lo << 16
-  using GT = typename std::conditional<H16, uint2, VT2>::type;
-  using ACC = typename std::conditional<MIX, flt4, dbl4>::type;
-  constexpr int NT = nterm(P), PP = Cfg::PP, KP = Cfg::KP, KT = Cfg::KT, NTH = Cfg::NTH, RB = Cfg::RB;
-  constexpr int TT = Cfg::TT, PPA = Cfg::PPA, BSZ = Cfg::BSZ, KG = Cfg::KG, KTG = Cfg::KTG;
-  constexpr int IT = (16 * NT + NTH - 1) / NTH;
-  constexpr int BPAD = 16 / (int)sizeof(VT);  // one spare 16-byte slot per B buffer
-  // sAcc row TT and sB slot BSZ take the writes of padding lanes, so the
-  // loop body needs no divergent branches
-  __shared__ double sAcc[(TT + 1) * PPA];
-  __shared__ __align__(16) VT sB[H16 ? 1 : 2][H16 ? BPAD : BSZ + BPAD];
-  // H16: B tiles of halves; the spare slot's lo part lies 512 halves on
-  constexpr int BSZ16 = Cfg::BSZ16, KB = Cfg::KB;
-  __shared__ __align__(16) unsigned short sB16[H16 ? 2 : 1][H16 ? BSZ16 + 520 : 8];
-  __shared__ int sVdec[PP], sUrow[NT], sUpar[NT];
-  constexpr bool SPLIT = Cfg::SPLIT;
-  constexpr int KQ = Cfg::KQ;
-  // SPLIT: the quarter wavefronts' partial 16x16 results of the 9th row
-  // block, [slice parity][quarter][lane][4]
-  __shared__ __align__(16) VT sP[SPLIT ? 2 : 1][SPLIT ? 4 * 64 * 4 : 1];
-  // H16: a cell's record is its NT terms and then its scale (float bits in .x)
-  const GT *M = static_cast<const GT *>(Mv);
-  constexpr int MREC = H16 ? Cfg::MREC16 : NT;
-  // H16: the KB k-block scales back of each column's source cell, staged
-  // with the slice's B tile ([buffer][k-block][column])
-  __shared__ float sMs[H16 ? 2 : 1][H16 ? KB : 1][16];
-  // H16: each wavefront's operator (row, k-block) scales of the current
-  // representative, [wavefront][row * KB + k-block]
-  __shared__ float sRs[H16 ? Cfg::NRS : 1][H16 ? 16 * KB : 1];
-  // the item's pairs: [slice - s0][column] source cell and target / reflection
-  constexpr bool PTAB = Cfg::PTAB;
-  __shared__ int sPs[PTAB ? 64 * 16 : 1];
-  __shared__ unsigned short sPl[PTAB ? 64 * 16 : 1];
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, c = l & 15;
-  const int4 item = items[blockIdx.x];  // tile, slices [s0, s1) (at most 64), split
-  const int s0 = item.y, s1 = item.z;
-  if (s0 == s1) return;  // empty item (whole block exits before any barrier)
-  if constexpr (PTAB) {
-    for (int e = tid; e < (s1 - s0) * 16; e += NTH) {
-      const int4 d = slices[s0 + (e >> 4)];
-      const int p = d.y + min(e & 15, d.z - 1);
-      sPs[e] = psrc[p];
-      sPl[e] = plt[p];
-    }
-  }
-
-  for (int e = tid; e < (TT + 1) * PPA; e += NTH) sAcc[e] = 0.0;
-  if constexpr (H16) {
-    for (int e = tid; e < (32 * KB - PP) * 16; e += NTH) {
-      const int b = Cfg::bidx16(PP + (e >> 4), e & 15);
-      sB16[0][b] = sB16[0][b + 512] = sB16[1][b] = sB16[1][b + 512] = 0;
-    }
-  } else {
-    for (int e = tid; e < (KP - PP) * 16; e += NTH) {
-      const int b = Cfg::bidx(PP + (e >> 4), e & 15);
-      sB[0][b] = VT(0);
-      sB[1][b] = VT(0);
-    }
-  }
-  for (int e = tid; e < PP; e += NTH) sVdec[e] = c_vdec[e];
-  for (int e = tid; e < NT; e += NTH) {
-    sUrow[e] = c_urow[e];
-    // reflection parities of multipole coefficient e = (n, m): bit 0 m, bit 2 n + m
-    const int dv = c_vdec[c_urow[e] & 0xffff];
-    const int n = dv & 255, m = (dv >> 8) & 255;
-    sUpar[e] = (m & 1) | (((n + m) & 1) << 2);
-  }
-  // the item's slice descriptors, lane k holding slice s0 + k, read back with
-  // readlane (uniform slice index): no memory wait in the loop
-  const int4 dsc = s0 + l < s1 ? slices[s0 + l] : make_int4(0, 0, 0, 0);
-  auto rep_of = [&](int s) { return __builtin_amdgcn_readlane(dsc.x, s - s0); };
-  // Every thread's gather and staging elements e = tid + NTH * it share the
-  // column c = e % 16 = l % 16, so each wavefront loads the source cells and
-  // targets of a slice for itself (lane l: column l % 16).  Lanes past the
-  // slice's count read the slice's last pair as a stand-in and send their
-  // results to the spare row.
-  auto pair_of = [&](int s) {  // this lane's pair of slice s (clamped into the item)
-    const int k = min(s, s1 - 1) - s0;
-    const int fst = __builtin_amdgcn_readlane(dsc.y, k), cnt = __builtin_amdgcn_readlane(dsc.z, k);
-    return fst + min(c, cnt - 1);
-  };
-  // this lane's source cell and target / reflection of slice s
-  auto src_at = [&](int s) {
-    if constexpr (PTAB)
-      return sPs[((min(s, s1 - 1) - s0) << 4) | c];
-    else
-      return psrc[pair_of(s)];
-  };
-  auto lt_at = [&](int s) {
-    if constexpr (PTAB)
-      return (int)sPl[((min(s, s1 - 1) - s0) << 4) | c];
-    else
-      return (int)plt[pair_of(s)];
-  };
-  auto live_col = [&](int s) {
-    return s >= s0 && s < s1 && c < __builtin_amdgcn_readlane(dsc.z, min(max(s, s0), s1 - 1) - s0);
-  };
-  GT pre[IT];
-  // H16: threads 0-15 (term 0 of columns 0-15) also carry their column's
-  // k-block scales to the staging
-  float psc[H16 ? KB : 1];
-  auto gather = [&](int src, GT *out) {
-    const size_t base = (size_t)cell_of(src) * MREC;
-#pragma unroll
-    for (int it = 0; it < IT; it++) out[it] = M[base + min((tid + NTH * it) >> 4, NT - 1)];
-    if constexpr (H16) {
-      if (tid < 16) {
-        const float *sb = reinterpret_cast<const float *>(M + base + NT);
-#pragma unroll
-        for (int kb = 0; kb < KB; kb++) psc[kb] = sb[kb];
-      }
-    }
-  };
-  // A pair's offset is the representative's reflected by its bits refl (x,
-  // y, z): T(refl d) = D T(d) D with D = diag((-1)^(x (m + io) + y io + z (n + m)))
-  // over the components (n, m, io) of the multipole columns and, with (j, k),
-  // of the local rows.  Columns get their signs here, rows in the update.
-  // Each thread's staging targets, packed: B slots of its elements' real
-  // (bits 0-11) and imaginary (bits 12-23) rows, the spare slot for none.
-  // Its column signs as tables over the 8 reflections: element it's real
-  // part flips under reflection r when bit 16 (it % 2) + r of sgn[it / 2]
-  // is set, its imaginary part when bit 16 (it % 2) + 8 + r is.
-  static_assert(BSZ < 4096, "B slots fit 12 bits");
-  static_assert(BSZ16 < 8192, "H16 B slots fit 13 bits");
-  constexpr int SB = H16 ? 13 : 12, SM = (1 << SB) - 1;  // slot bits, mask
-  int stg[IT];
-  unsigned sgn[(IT + 1) / 2];
-  auto flip = [](VT x, unsigned bit) {  // -x when bit (0 or 1) is set
-    if constexpr (MIX)
-      return __uint_as_float(__float_as_uint(x) ^ (bit << 31));
-    else
-      return __longlong_as_double(__double_as_longlong(x) ^ ((long long)bit << 63));
-  };
-  auto stage = [&](int buf, const GT *in, int lt) {
-    const int refl = (lt >> 8) & 7;
-#pragma unroll
-    for (int it = 0; it < IT; it++) {
-      const unsigned t = sgn[it / 2] >> (16 * (it % 2));
-      if constexpr (H16) {  // both halves of a value flip together
-        if (it == 0 && tid < 16) {
-#pragma unroll
-          for (int kb = 0; kb < KB; kb++) sMs[buf][kb][tid] = psc[kb];
-        }
-        unsigned short *Bt = sB16[buf];
-        const unsigned re = in[it].x ^ (((t >> refl) & 1u) * 0x80008000u);
-        const unsigned im = in[it].y ^ (((t >> (8 + refl)) & 1u) * 0x80008000u);
-        const int br = stg[it] & SM, bi = (stg[it] >> SB) & SM;
-        Bt[br] = (unsigned short)re;
-        Bt[br + 512] = (unsigned short)(re >> 16);
-        Bt[bi] = (unsigned short)im;
-        Bt[bi + 512] = (unsigned short)(im >> 16);
-      } else {
-        VT *Bt = sB[buf];
-        Bt[stg[it] & SM] = flip(in[it].x, (t >> refl) & 1);
-        Bt[(stg[it] >> SB) & SM] = flip(in[it].y, (t >> (8 + refl)) & 1);
-      }
-    }
-  };
-  auto parity3 = [](int x) { return (0x96u >> (x & 7)) & 1u; };  // parity of 3 bits
-  __syncthreads();
-#pragma unroll
-  for (int it = 0; it < (IT + 1) / 2; it++) sgn[it] = 0;
-#pragma unroll
-  for (int it = 0; it < IT; it++) {
-    const int e = tid + NTH * it;
-    const bool live = e < 16 * NT;
-    const int u = live ? e >> 4 : 0;
-    const int rr = sUrow[u];
-    const int spare = H16 ? BSZ16 : BSZ;
-    const int bre = live ? (H16 ? Cfg::bidx16(rr & 0xffff, c) : Cfg::bidx(rr & 0xffff, c)) : spare;
-    const int bim = live && (rr >> 16) != (rr & 0xffff)
-                        ? (H16 ? Cfg::bidx16(rr >> 16, c) : Cfg::bidx(rr >> 16, c)) : spare;
-    stg[it] = bre | (bim << SB);
-    const int par = sUpar[u];
-    for (int r = 0; r < 8; r++) {
-      sgn[it / 2] |= parity3(par & r) << (16 * (it % 2) + r);            // Re: x m + z (n + m)
-      sgn[it / 2] |= parity3((par ^ 1 ^ 2) & r) << (16 * (it % 2) + 8 + r);  // Im: x (m + 1) + y + z (n + m)
-    }
-  }
-  // row signs of this lane's 4 result rows (j, k, io) over the 8 reflections:
-  // row v flips under reflection r when bit 4 r + v is set (parities: bit 0
-  // k + io, bit 1 io, bit 2 j + k)
-  auto row_signs = [&](int b) {  // of row block b
-    unsigned sg = 0;
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const int r = b * 16 + (MIX ? 4 * (l >> 4) + v : (l >> 4) + 4 * v);
-      const int dv = sVdec[r < PP ? r : 0];
-      const int jj = dv & 255, kk = (dv >> 8) & 255, io = dv >> 16;
-      const int rp = ((kk + io) & 1) | (io << 1) | (((jj + kk) & 1) << 2);
-      for (int q = 0; q < 8; q++) sg |= parity3(rp & q) << (4 * q + v);
-    }
-    return sg;
-  };
-  const unsigned usgn = row_signs(w);
-  const unsigned usgn9 = SPLIT ? row_signs(RB - 1) : 0u;  // the 9th block (COMB adds it)
-  // add a slice's 16x16 results (D: lane l holds column l % 16 and rows
-  // (f64) l/16 + 4v, (f32) 4(l/16) + v of this wavefront's block) into the
-  // tile's local expansions, rows sign-flipped by the pair's reflection
-  // FULL: every row of this wavefront's block is below P^2 (all but a
-  // partial last block), so the four rows sit at fixed offsets
-  // b: the row block (this wavefront's, or the 9th for COMB), sg its signs
-  auto update = [&](const auto &a, int lt, bool ok, auto full_tag, int b, unsigned sg) {
-    constexpr bool FULL = decltype(full_tag)::value;
-    const int tgt = ok ? lt & 255 : TT, rf = (lt >> 8) & 7;
-    const unsigned m = sg >> (4 * rf);
-    double *row0 = sAcc + tgt * PPA + b * 16 + (MIX ? 4 * (l >> 4) : (l >> 4));
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const int r = b * 16 + (MIX ? 4 * (l >> 4) + v : (l >> 4) + 4 * v);
-      const double x = (double)a[v];
-      const double sx = __longlong_as_double(__double_as_longlong(x) ^ ((long long)((m >> v) & 1) << 63));
-      if constexpr (FULL)
-        row0[MIX ? v : 4 * v] += sx;
-      else
-        sAcc[r < PP ? tgt * PPA + r : TT * PPA] += sx;
-    }
-  };
-  // this wavefront's 16 operator rows: k-step kt in A[kt], loaded from the
-  // representative's table when it changes, right after the last MFMA that
-  // reads the previous one.
-  // FP64 with P^2 = 16 (RB - 1) + 1..4 (P = 10: 100 rows): the last
-  // wavefront's block holds at most 4 operator rows, and it runs them with
-  // v_mfma_f64_4x4x4f64 (4 blocks of 4x4, a quarter of the 16x16x4 cycles):
-  // A lane 16k + 4b + r = T[16w + r][4kt + k] for every block b, B lane
-  // 16k + 4b + c = column 4b + c at k (the 16x16x4 B operand as it is), D
-  // lane 16r + 4b + c = row 16w + r of column 4b + c (the 16x16x4 D element
-  // v = 0 of that lane)
-  constexpr bool R4 = !MIX && PP % 16 != 0 && PP % 16 <= 4;
-  const bool quad = R4 && __builtin_amdgcn_readfirstlane(w) == RB - 1;  // wave-uniform
-  const VT *ops = static_cast<const VT *>(opsv) + (size_t)w * KT * 64 + (quad ? 16 * (l >> 4) + (l & 3) : l);
-  // SPLIT: this wavefront's quarter of the 9th block (q < 0: none; wave-uniform)
-  const int q9 = SPLIT ? Cfg::quarter(__builtin_amdgcn_readfirstlane(w)) : -1;
-  const VT *ops9 = static_cast<const VT *>(opsv) + ((size_t)(RB - 1) * KT + (size_t)max(q9, 0) * KQ) * 64 + l;
-  constexpr size_t GS = (size_t)RB * KT * 64;  // one representative's table
-  // H16: this wavefront's hi / lo A operands of every k-block, and the
-  // scales of its 4 result rows per lane, from the representative's record
-  typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-  const char *ops16 = static_cast<const char *>(opsv);
-  constexpr int RSN = H16 ? (16 * KB + 63) / 64 : 1, NQ16 = Cfg::NQ16;
-  float rsv[RSN], rsv9 = 0.0f;
-  // SPLIT quarter wavefronts also load the 9th block's operands of their
-  // k-blocks q9 + 4 j (A9h, A9l) and those k-blocks' row scales (rsv9:
-  // lane l holds row l % 16 of k-block q9 + 4 (l / 16))
-  auto load16 = [&](int g, half8 *Ah, half8 *Al, half8 *A9h, half8 *A9l) {
-    const half8 *o = reinterpret_cast<const half8 *>(ops16 + (size_t)g * Cfg::OPS16) + (size_t)w * KB * 2 * 64 + l;
-#pragma unroll
-    for (int kb = 0; kb < KB; kb++) {
-      Ah[kb] = o[(kb * 2) * 64];
-      Al[kb] = o[(kb * 2 + 1) * 64];
-    }
-    if constexpr (SPLIT && H16) {
-      if (q9 >= 0) {
-        const half8 *o9 = reinterpret_cast<const half8 *>(ops16 + (size_t)g * Cfg::OPS16) + (size_t)(RB - 1) * KB * 2 * 64 + l;
-#pragma unroll
-        for (int j = 0; j < NQ16; j++) {
-          const int kb = min(q9 + 4 * j, KB - 1);
-          A9h[j] = o9[(kb * 2) * 64];
-          A9l[j] = o9[(kb * 2 + 1) * 64];
-        }
-        const int kb = q9 + 4 * (l >> 4);
-        const float *rs9 = reinterpret_cast<const float *>(ops16 + (size_t)g * Cfg::OPS16 + (size_t)RB * KB * 2 * 64 * 16);
-        rsv9 = (l < 16 * NQ16 && kb < KB) ? rs9[((RB - 1) * 16 + (l & 15)) * KB + kb] : 0.0f;
-      }
-    }
-    // the (row, k-block) scales of this wavefront's 16 rows, into registers;
-    // put_rs moves them to the wavefront's own LDS rows once the MFMAs that
-    // wait for the operands have waited for them too (each wavefront reads
-    // only what it wrote)
-    const float *rs = reinterpret_cast<const float *>(ops16 + (size_t)g * Cfg::OPS16 + (size_t)RB * KB * 2 * 64 * 16);
-#pragma unroll
-    for (int i = 0; i < RSN; i++) {
-      const int e = l + 64 * i;
-      rsv[i] = e < 16 * KB ? rs[w * 16 * KB + e] : 0.0f;
-    }
-  };
-  auto put_rs = [&]() {
-#pragma unroll
-    for (int i = 0; i < RSN; i++) {
-      const int e = l + 64 * i;
-      if (e < 16 * KB) sRs[w][e] = rsv[i];
-    }
-    if constexpr (SPLIT && H16) {
-      const int kb = q9 + 4 * (l >> 4);
-      if (q9 >= 0 && l < 16 * NQ16 && kb < KB) sRs[Cfg::NW][(l & 15) * KB + kb] = rsv9;
-    }
-  };
-  // Software pipeline, one barrier per slice.  Behind the MFMA chain of
-  // slice s run the update of slice s - 1, the staging of slice s + 1 (into
-  // the other B buffer, last read before this iteration's barrier) and the
-  // gather of slice s + 2.  Every value an iteration loads is used at the end
-  // of the next one (ltU: slice s - 1's targets for the update, ltS: slice
-  // s + 1's reflections for the staging, srcG: slice s + 2's sources for the
-  // gather, pre: slice s + 1's multipoles), so no load is waited for early
-  // and no loaded value is copied before use.
-  gather(src_at(s0), pre);
-  stage(s0 & 1, pre, lt_at(s0));
-  gather(src_at(s0 + 1), pre);
-  int ltU = 0, ltS = lt_at(s0 + 1), srcG = src_at(s0 + 2);
-  ACC accp;
-#pragma unroll
-  for (int v = 0; v < 4; v++) accp[v] = VT(0);
-  // The MFMA groups: one 16-byte B read a group ahead, then the group's
-  // MFMAs; the empty asm statements keep the compiler from hoisting later LDS
-  // reads, which would cost registers and so occupancy.
-  // COMB: add the 9th block's result of slice sl, the four quarter sums in a
-  // fixed order (ltU holds slice sl's targets and reflections when called)
-  auto combine9 = [&](int sl) {
-    const VT *src = &sP[SPLIT ? (sl & 1) : 0][l * 4];
-    double a9[4];
-#pragma unroll
-    for (int v = 0; v < 4; v++)
-      a9[v] = (((double)src[v] + (double)src[256 + v]) + (double)src[512 + v]) + (double)src[768 + v];
-    update(a9, ltU, live_col(sl), std::true_type{}, RB - 1, usgn9);
-  };
-  auto run = [&](auto quad_tag, auto full_tag) {
-    constexpr bool Q = decltype(quad_tag)::value;
-    VT A[H16 ? 1 : KT];
-    VT A9[SPLIT && !H16 ? KQ : 1];  // SPLIT quarter wavefronts: their k-steps of the 9th block
-    half8 Ah[H16 ? KB : 1], Al[H16 ? KB : 1];
-    half8 A9h[H16 && SPLIT ? NQ16 : 1], A9l[H16 && SPLIT ? NQ16 : 1];
-    int cur_g = rep_of(s0);
-    bool rs_new = false;  // H16: the operator changed, its row scales are in rsv
-    if constexpr (H16) {
-      load16(cur_g, Ah, Al, A9h, A9l);
-      put_rs();
-    } else {
-#pragma unroll
-      for (int kt = 0; kt < KT; kt++) A[kt] = ops[(size_t)cur_g * GS + kt * 64];
-    }
-    if constexpr (SPLIT && !H16) {
-      if (q9 >= 0) {
-#pragma unroll
-        for (int i = 0; i < KQ; i++) A9[i] = ops9[(size_t)cur_g * GS + i * 64];
-      }
-    }
-    for (int s = s0; s < s1; s++) {
-      __syncthreads();
-      const VT *bp = sB[H16 ? 0 : (s & 1)] + l * KG;  // k-step kt at bp[(kt / KG) * 64 * KG + kt % KG]
-      ACC acc;
-#pragma unroll
-      for (int v = 0; v < 4; v++) acc[v] = VT(0);
-      double d = 0.0;
-      if constexpr (H16) {
-        if (rs_new) {
-          put_rs();
-          rs_new = false;
-        }
-        // per k-block: hi x hi into one accumulator, hi x lo' + lo' x hi into
-        // another (lo' = lo 2^11; the lo x lo term is below the FP32
-        // accumulation), combined as a1 + a2 2^-11 and scaled back by the
-        // operator row's and the source cell's k-block scales (exact powers
-        // of two)
-        const half8 *bq = reinterpret_cast<const half8 *>(sB16[s & 1]) + l;
-        half8 bh = bq[0], bl = bq[64];
-        const float *msc = &sMs[s & 1][0][c];  // [16 kb]: this column's source cell's k-block scales
-        // k-block kb's MFMAs run while the results of kb - 1 are scaled
-        // and added; the scheduling barriers keep the compiler from hoisting
-        // every B read and keeping every k-block's results live (registers
-        // past the budget of 3 wavefronts per SIMD spill, and a spill reload
-        // waits for every vector load before it)
-        flt4 p1, p2;
-        auto comb = [&](const flt4 &x1, const flt4 &x2, int kb) {
-#pragma unroll
-          for (int v = 0; v < 4; v++)
-            acc[v] = fmaf(fmaf(x2[v], 1.0f / 2048.0f, x1[v]), sRs[w][(4 * (l >> 4) + v) * KB + kb] * msc[16 * kb], acc[v]);
-        };
-#pragma unroll
-        for (int kb = 0; kb < KB; kb++) {
-          half8 nh, nl;
-          if (kb + 1 < KB) {
-            nh = bq[((kb + 1) * 2) * 64];
-            nl = bq[((kb + 1) * 2 + 1) * 64];
-          }
-          flt4 a1 = {0.0f, 0.0f, 0.0f, 0.0f}, a2 = {0.0f, 0.0f, 0.0f, 0.0f};
-          a1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah[kb], bh, a1, 0, 0, 0);
-          a2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah[kb], bl, a2, 0, 0, 0);
-          a2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al[kb], bh, a2, 0, 0, 0);
-          if (kb > 0) comb(p1, p2, kb - 1);
-          __builtin_amdgcn_sched_barrier(0);
-          p1 = a1;
-          p2 = a2;
-          if (kb + 1 < KB) {
-            bh = nh;
-            bl = nl;
-          }
-        }
-        comb(p1, p2, KB - 1);
-
-      } else {
-      VT b[KG];
-#pragma unroll
-      for (int u = 0; u < KG; u++) b[u] = bp[u];
-#pragma unroll
-      for (int g = 0; g < KTG; g++) {
-        VT nb[KG];
-        if (g + 1 < KTG) {
-#pragma unroll
-          for (int u = 0; u < KG; u++) nb[u] = bp[(g + 1) * 64 * KG + u];
-        }
-#pragma unroll
-        for (int u = 0; u < KG; u++) {
-          const int kt = g * KG + u;
-          if (kt < KT) {
-            if constexpr (Q)
-              d = __builtin_amdgcn_mfma_f64_4x4x4f64(A[kt], b[u], d, 0, 0, 0);
-            else if constexpr (MIX)
-              acc = __builtin_amdgcn_mfma_f32_16x16x4f32(A[kt], b[u], acc, 0, 0, 0);
-            else
-              acc = __builtin_amdgcn_mfma_f64_16x16x4f64(A[kt], b[u], acc, 0, 0, 0);
-          }
-        }
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int u = 0; u < KG; u++) b[u] = nb[u];
-      }
-      }  // H16 / VT operands
-      if constexpr (SPLIT && H16) {
-        if (q9 >= 0) {  // this wavefront's k-blocks of the 9th block, kept for COMB
-          const half8 *bq = reinterpret_cast<const half8 *>(sB16[s & 1]) + l;
-          const float *msc = &sMs[s & 1][0][c];
-          flt4 a9 = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-          for (int j = 0; j < NQ16; j++) {
-            const int kb = q9 + 4 * j;
-            if (kb < KB) {
-              const half8 bh = bq[(kb * 2) * 64], bl = bq[(kb * 2 + 1) * 64];
-              flt4 a1 = {0.0f, 0.0f, 0.0f, 0.0f}, a2 = {0.0f, 0.0f, 0.0f, 0.0f};
-              a1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(A9h[j], bh, a1, 0, 0, 0);
-              a2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(A9h[j], bl, a2, 0, 0, 0);
-              a2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(A9l[j], bh, a2, 0, 0, 0);
-#pragma unroll
-              for (int v = 0; v < 4; v++)
-                a9[v] = fmaf(fmaf(a2[v], 1.0f / 2048.0f, a1[v]),
-                             sRs[Cfg::NW][(4 * (l >> 4) + v) * KB + kb] * msc[16 * kb], a9[v]);
-            }
-          }
-          VT *dst = &sP[s & 1][(q9 * 64 + l) * 4];
-#pragma unroll
-          for (int v = 0; v < 4; v++) dst[v] = a9[v];
-        }
-      } else if constexpr (SPLIT) {
-        if (q9 >= 0) {  // this wavefront's quarter of the 9th block, kept for COMB
-          ACC a9;
-#pragma unroll
-          for (int v = 0; v < 4; v++) a9[v] = VT(0);
-#pragma unroll
-          for (int i = 0; i < KQ; i++) {
-            const int kt = q9 * KQ + i;
-            if constexpr (MIX)
-              a9 = __builtin_amdgcn_mfma_f32_16x16x4f32(A9[i], bp[(kt / KG) * 64 * KG + kt % KG], a9, 0, 0, 0);
-            else
-              a9 = __builtin_amdgcn_mfma_f64_16x16x4f64(A9[i], bp[(kt / KG) * 64 * KG + kt % KG], a9, 0, 0, 0);
-          }
-          VT *dst = &sP[s & 1][(q9 * 64 + l) * 4];
-#pragma unroll
-          for (int v = 0; v < 4; v++) dst[v] = a9[v];
-        }
-      }
-      // behind the last MFMAs: add the previous slice's results, stage slice
-      // s + 1 (gathered an iteration ago), then issue the loads in the order
-      // they are waited for -- the next operator (if it changes), slice
-      // s + 2's gather, the next iteration's indices
-      update(accp, ltU, live_col(s - 1), full_tag, w, usgn);
-      if constexpr (SPLIT) {
-        if (w == Cfg::COMB && s > s0) combine9(s - 1);
-      }
-      if constexpr (Q) acc[0] = d;  // rows past 16w + 3 are beyond P^2: the update skips them
-      stage((s + 1) & 1, pre, ltS);
-      if (s + 1 < s1) {
-        const int rn = rep_of(s + 1);
-        if (rn != cur_g) {  // uniform: the representative changes
-          cur_g = rn;
-          if constexpr (H16) {
-            load16(rn, Ah, Al, A9h, A9l);
-            rs_new = true;
-          } else {
-#pragma unroll
-            for (int kt = 0; kt < KT; kt++) A[kt] = ops[(size_t)rn * GS + kt * 64];
-          }
-          if constexpr (SPLIT && !H16) {
-            if (q9 >= 0) {
-#pragma unroll
-              for (int i = 0; i < KQ; i++) A9[i] = ops9[(size_t)rn * GS + i * 64];
-            }
-          }
-        }
-      }
-      gather(srcG, pre);
-      srcG = src_at(s + 3);
-      ltS = lt_at(s + 2);
-      ltU = lt_at(s);
-      accp = acc;
-    }
-  };
-  const bool full = __builtin_amdgcn_readfirstlane(w + 1) * 16 <= PP;  // wave-uniform
-  if (R4 && quad)
-    run(std::true_type{}, std::false_type{});
-  else if (full)
-    run(std::false_type{}, std::true_type{});
-  else
-    run(std::false_type{}, std::false_type{});
-  update(accp, ltU, live_col(s1 - 1), std::false_type{}, w, usgn);
-  if constexpr (SPLIT) {
-    __syncthreads();  // the last slice's quarter results are in sP
-    if (w == Cfg::COMB) combine9(s1 - 1);
-  }
-  __syncthreads();
-  const int *tt = ttgt + (size_t)item.x * TT;
-  for (int e = tid; e < TT * PP; e += NTH) {
-    const int tl = e / PP, r = e - tl * PP;
-    const int cell = tt[tl];
-    if (cell < 0) continue;
-    const int dr = sVdec[r];
-    const int j = dr & 255;
-    double v = sAcc[tl * PPA + r];
-    if (MIX) {
-      const double inv = 1.0 / cr[cell];
-      for (int k = 0; k < j; k++) v *= inv;
-    }
-    double *dst = L + (size_t)cell * 2 * NT + j * (j + 1) + 2 * ((dr >> 8) & 255) + (dr >> 16);
-    if (item.w)
-      unsafeAtomicAdd(dst, v);  // the tile's other items add theirs
-    else
-      *dst = v;
-  }
-}
-
 // ---------------------------------------------------------------- periodic far images
 // Traversal::traversePeriodic (include/traversal.h:233-287) translates the
 // root multipole to the root local expansion through images - 1 levels of
@@ -3023,72 +2126,6 @@ template <int P> struct RunM2LMfma32 {
     }
   }
 };
-template <int P> struct RunM2LTile {
-  static hipError_t run(bool mix, bool h16, int nitem, const int *ttgt, const int4 *items, const int4 *slices,
-                        const int *psrc, const unsigned short *plt, const void *ops, const double *cr, const void *M,
-                        double2 *L, hipStream_t s) {
-    if constexpr (TileCfg<P, false>::ok) {
-      constexpr int nth = TileCfg<P, false>::NTH;  // same for both value types
-      if (nitem > 0 && h16)
-        hipLaunchKernelGGL((m2l_tile_kernel<P, true, true>), dim3(nitem), dim3(TileCfg<P, true, true>::NTH), 0, s,
-                           ttgt, items, slices, psrc, plt, ops, cr, M, reinterpret_cast<double *>(L));
-      else if (nitem > 0) {
-        if (mix)
-          hipLaunchKernelGGL((m2l_tile_kernel<P, true>), dim3(nitem), dim3(nth), 0, s, ttgt, items, slices, psrc,
-                             plt, ops, cr, M, reinterpret_cast<double *>(L));
-        else
-          hipLaunchKernelGGL((m2l_tile_kernel<P, false>), dim3(nitem), dim3(nth), 0, s, ttgt, items, slices, psrc,
-                             plt, ops, cr, M, reinterpret_cast<double *>(L));
-      }
-      return hipGetLastError();
-    } else {
-      return hipErrorInvalidValue;
-    }
-  }
-};
-hipError_t launch_m2l_tile(int P, bool mix, bool h16, int nitem, const int *ttgt, const int4 *items,
-                           const int4 *slices, const int *psrc, const unsigned short *plt, const void *ops,
-                           const double *cr, const void *M, double2 *L, hipStream_t s) {
-  return dispatch<RunM2LTile>(P, mix, h16, nitem, ttgt, items, slices, psrc, plt, ops, cr, M, L, s);
-}
-template <int P> struct RunGroupOps {
-  static hipError_t run(bool mix, bool h16, const double2 *gY, const double2 *gscale, int ngroup, void *ops,
-                        hipStream_t s) {
-    if constexpr (TileCfg<P, false>::ok) {
-      constexpr int nth = 64 * TileCfg<P, false>::RB;  // one wavefront per row block
-      if (ngroup > 0 && h16)
-        hipLaunchKernelGGL(group_ops16_kernel<P>, dim3(ngroup), dim3(nth), 0, s, gY, gscale, ngroup, ops);
-      else if (ngroup > 0) {
-        if (mix)
-          hipLaunchKernelGGL((group_ops_kernel<P, true>), dim3(ngroup), dim3(nth), 0, s, gY, gscale, ngroup, ops);
-        else
-          hipLaunchKernelGGL((group_ops_kernel<P, false>), dim3(ngroup), dim3(nth), 0, s, gY, gscale, ngroup, ops);
-      }
-      return hipGetLastError();
-    } else {
-      return hipErrorInvalidValue;
-    }
-  }
-};
-size_t group_ops_bytes(int P, bool mix, bool h16) {
-  const int PP = P * P, KT = (PP + 3) / 4, RB = (PP + 15) / 16, KB = (PP + 31) / 32;
-  if (h16) return (size_t)RB * KB * 2 * 64 * 16 + (size_t)RB * 16 * 4;  // TileCfg::OPS16
-  return (size_t)RB * KT * 64 * (mix ? sizeof(float) : sizeof(double));
-}
-hipError_t launch_group_ops(int P, bool mix, bool h16, const double2 *gY, const double2 *gscale, int ngroup,
-                            void *ops, hipStream_t s) {
-  return dispatch<RunGroupOps>(P, mix, h16, gY, gscale, ngroup, ops, s);
-}
-template <int P> struct RunGroupHarmonics {
-  static hipError_t run(const double *gdx, int ngroup, double2 *Y, hipStream_t s) {
-    if (ngroup > 0) hipLaunchKernelGGL(group_harmonics_kernel<P>, dim3(ngroup), dim3(64), 0, s, gdx, ngroup, Y);
-    return hipGetLastError();
-  }
-};
-int group_harmonics_size(int P) { return (2 * P - 1) * (3 * P - 2); }
-hipError_t launch_group_harmonics(int P, const double *gdx, int ngroup, double2 *Y, hipStream_t s) {
-  return dispatch<RunGroupHarmonics>(P, gdx, ngroup, Y, s);
-}
 template <int P> struct RunXlateOps {
   static hipError_t run(const double *dxs, const int *kinds, int nop, double *ops, int accum, hipStream_t s) {
     if (nop > 0) hipLaunchKernelGGL(xlate_ops_kernel<P>, dim3(nop), dim3(256), 0, s, dxs, kinds, nop, ops, accum);
@@ -3175,20 +2212,6 @@ hipError_t launch_l2l_mfma(int P, const int4 *tiles, int ntile, const int *child
 }
 hipError_t launch_m_to_f32(int P, const double2 *M, const double *R, int ncell, float2 *M32, hipStream_t s) {
   return dispatch<RunMToF32>(P, M, R, ncell, M32, s);
-}
-template <int P> struct RunMToF16 {
-  static hipError_t run(const double2 *M, const double *R, int ncell, void *M16, hipStream_t s) {
-    if (ncell > 0)
-      hipLaunchKernelGGL(m_to_f16_kernel<P>, dim3(ncell), dim3(64), 0, s, M, R, ncell, static_cast<uint2 *>(M16));
-    return hipGetLastError();
-  }
-};
-size_t m16_record_bytes(int P) {
-  const int KB = (P * P + 31) / 32;
-  return sizeof(uint2) * ((size_t)P * (P + 1) / 2 + (KB + 1) / 2);
-}
-hipError_t launch_m_to_f16(int P, const double2 *M, const double *R, int ncell, void *M16, hipStream_t s) {
-  return dispatch<RunMToF16>(P, M, R, ncell, M16, s);
 }
 hipError_t launch_m2l_mfma32(int P, const int4 *chunks, int nchunk, const double *gdx, const double2 *gscale,
                              const int *ptgt, const int *psrc, const float2 *M32, double2 *L, hipStream_t s) {

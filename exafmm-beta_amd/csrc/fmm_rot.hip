@@ -1,0 +1,606 @@
+// fmm_rot.hip -- the target-tile M2L as rotate, shift along z, rotate back.
+//
+// The translation of one offset class as a dense real P^2 x P^2 operator costs
+// 2 P^4 flop a pair (41.5 kflop at P = 12).  Turned so that the offset lies on
+// the z axis it factors (M~, L^ as in fmm_device.hpp, s = sqrt((n-m)!(n+m)!)):
+//   u[n,m]  = s M~[n,m] e^{i m phi}                           (z rotation)
+//   v[n,.]  = Q_n(beta) u[n,.]      Re and Im parts apart     (y rotation)
+//   w[j,m]  = sum_n T_m[j,n] v[n,m] (Re and Im alike)         (shift by r)
+//   L^[j,.] = s e^{-i m phi} (S Q_j S) w[j,.],  S = (-1)^m    (back)
+// with Q_n built from the Wigner matrix d^n(beta) (columns m and -m folded),
+// T_m[j,n] = (-1)^(j+m) (j+n)! / (r^(j+n+1) s(j,m) s(n,m)), and S Q S the
+// inverse rotation: one set of matrices serves both rotations.  All blocks
+// have at most P rows: about 6 P^3 multiply-adds a pair in place of P^4.
+//
+// The blocks run on v_mfma_f64_4x4x4f64 (four independent 4x4 products an
+// instruction; A[r][k] of block b in lane 16k + 4b + r, B[k][c] in lane
+// 16k + 4b + c, D[r][c] in lane 16r + 4b + c, so a result is the next
+// product's B operand).  Block b holds one degree n (rotations) or one order
+// m (shift), columns c are four pairs:
+//   layout 1 (rotations): tile (i, j), lane (r, b, c): n = 4i + b, m = 4j + r
+//   layout 2 (shift):     level k, tile i, lane (r, b, c): m = m0(k) + b,
+//                         n = m0(k) + 4i + r
+// and 4 P^2 doubles go through LDS between them (twice a slice).  When the
+// last row of tiles holds only one or two degrees (P = 9, 10, 5, 6) their Re
+// and Im parts share it (b = part, degree), and the orders of the same size
+// likewise: 57 instead of 84 products a slice at P = 10.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <vector>
+
+#include "fmm_device.hpp"
+
+namespace fmmdev {
+
+namespace {
+
+constexpr int kRotMaxP = 12;
+__host__ __device__ constexpr int tri(int i, int j) { return i * (i + 1) / 2 + j; }
+__host__ __device__ constexpr int sq_sum(int n) { return n * (n + 1) * (2 * n + 1) / 6; }
+constexpr int delta_off(int n) { return n * (4 * n * n - 1) / 3; }  // sum of (2k+1)^2, k < n
+
+template <int P> struct RotCfg {
+  static constexpr int NT = P * (P + 1) / 2;
+  static constexpr int G = (P + 3) / 4;         // tiles of 4 along a degree
+  static constexpr int REM = P - 4 * (G - 1);   // degrees in the last row of tiles
+  static constexpr bool COMB = REM <= 2;        // their Re and Im share the blocks
+  static constexpr int NL = COMB ? G - 1 : G;   // full rows of tiles
+  static constexpr int NF = tri(NL, 0);         // full tiles (of each part)
+  static constexpr int NX = COMB ? G : 0;       // tiles of the shared row
+  // products: rotations of the full rows (Re, Im), of the shared row; shifts
+  static constexpr int NQ = sq_sum(NL), NQX = NX * NX;
+  static constexpr int NFRAG = 3 * NQ + 2 * NQX;
+  static constexpr int QRE = 0, QIM = NQ, QX = 2 * NQ, TF = 2 * NQ + NQX, TX = 3 * NQ + NQX;
+  static constexpr int NCS = NF + NX;           // (s cos m phi, s sin m phi) of every tile
+  static constexpr int NREC = NFRAG + 2 * NCS;  // doubles a lane of one class's record
+  static constexpr int NREC2 = (NREC + 1) / 2;  // stored [NREC2][64 lanes][2]
+  // shift levels: orders m0(k) .. m0(k) + 3 with tiles(k) tiles of degrees
+  static __host__ __device__ constexpr int m0(int k) { return (COMB ? REM : 0) + 4 * k; }
+  static __host__ __device__ constexpr int tiles(int k) { return NL - k; }
+  static __host__ __device__ constexpr int off2(int k) { return NF - tri(NL - k, 0); }     // first tile of level k
+  static __host__ __device__ constexpr int offT(int k) { return NQ - sq_sum(NL - k); }     // its products
+  // exchange buffer (doubles): element (n, m, c) at n AST + 4 m + c; AST = 4 x
+  // odd keeps the four blocks of both layouts on distinct banks
+  static constexpr int AST = 16 * G + 4;
+  static constexpr int ROWS = COMB ? P : 4 * G;
+  static constexpr int PART = COMB ? (ROWS * AST + 7) / 16 * 16 + 8 : 0;  // Im part (Re and Im in turn otherwise)
+  static constexpr int XSZ = COMB ? PART + ROWS * AST : ROWS * AST;
+};
+
+// Delta_n = d^n(pi/2), n < kRotMaxP, (2n+1)^2 each, row-major
+__device__ double g_delta[delta_off(kRotMaxP)];
+
+// The record of every class (offset with non-negative components): the A
+// operands of all products and the z rotation factors, one block a class.
+// W[a][b] = sum_k Delta[k][a] Delta[k][b] Re(i^(b-a) e^{-i k beta}) is d^n(beta)
+// without its cancelling explicit sum; Q = W[a][m] +- (-1)^m W[a][-m].
+template <int P>
+__global__ __launch_bounds__(256) void rot_ops_kernel(const double *__restrict__ cdx, int nrep,
+                                                      double *__restrict__ ops) {
+  using C = RotCfg<P>;
+  __shared__ double ck[2][P], zc[2][P], rp[2 * P], fac[2 * P];
+  const int g = blockIdx.x, tid = threadIdx.x;
+  if (g >= nrep) return;
+  if (tid == 0) {
+    const double dx = cdx[3 * g], dy = cdx[3 * g + 1], dz = cdx[3 * g + 2];
+    const double rho = sqrt(dx * dx + dy * dy), r = sqrt(dx * dx + dy * dy + dz * dz);
+    const double cb = dz / r, sb = rho / r;
+    const double cp = rho > 0.0 ? dx / rho : 1.0, sp = rho > 0.0 ? dy / rho : 0.0;
+    ck[0][0] = zc[0][0] = 1.0;
+    ck[1][0] = zc[1][0] = 0.0;
+    for (int k = 1; k < P; k++) {
+      ck[0][k] = ck[0][k - 1] * cb - ck[1][k - 1] * sb;
+      ck[1][k] = ck[1][k - 1] * cb + ck[0][k - 1] * sb;
+      zc[0][k] = zc[0][k - 1] * cp - zc[1][k - 1] * sp;
+      zc[1][k] = zc[1][k - 1] * cp + zc[0][k - 1] * sp;
+    }
+    rp[0] = 1.0 / r;
+    fac[0] = 1.0;
+    for (int k = 1; k < 2 * P; k++) {
+      rp[k] = rp[k - 1] / r;
+      fac[k] = fac[k - 1] * k;
+    }
+  }
+  __syncthreads();
+  auto scale = [&](int n, int m) { return sqrt(fac[n - m]) * sqrt(fac[n + m]); };
+  auto wigner = [&](int n, int a, int b) {
+    const double *D = g_delta + n * (4 * n * n - 1) / 3 + n;
+    const int w = 2 * n + 1, q = (b - a) & 3;
+    double v = 0.0;
+    for (int k = -n; k <= n; k++) {
+      const int ka = k < 0 ? -k : k;
+      const double t = (q & 1) ? (k < 0 ? -ck[1][ka] : ck[1][ka]) : ck[0][ka];
+      v = fma(D[(k + n) * w + a] * D[(k + n) * w + b], t, v);
+    }
+    return (q & 2) ? -v : v;
+  };
+  auto rot = [&](int n, int a, int m, int part) {  // Q_n[a][m] of the part
+    if (n >= P || a > n || m > n || (part && (a == 0 || m == 0))) return 0.0;
+    const double p = wigner(n, a, m);
+    if (m == 0) return p;
+    const double q = (m & 1) ? -wigner(n, a, -m) : wigner(n, a, -m);
+    return part ? p - q : p + q;
+  };
+  auto shift = [&](int m, int j, int n) {  // T_m[j][n], times the inner S of the back rotation
+    if (j >= P || n >= P || j < m || n < m) return 0.0;
+    const double t = fac[j + n] * rp[j + n] / (scale(j, m) * scale(n, m));
+    return (j & 1) ? -t : t;
+  };
+  double *rec = ops + (size_t)g * C::NREC2 * 128;
+  for (int e = tid; e < C::NREC2 * 128; e += 256) {
+    const int f = e >> 6, lane = e & 63;
+    const int k = lane >> 4, b = (lane >> 2) & 3, r = lane & 3;
+    double v = 0.0;
+    if (f < C::QX) {  // full rows
+      const int part = f >= C::QIM;
+      int h = f - (part ? C::QIM : 0), i = 0;
+      while (h >= (i + 1) * (i + 1)) {
+        h -= (i + 1) * (i + 1);
+        i++;
+      }
+      v = rot(4 * i + b, 4 * (h / (i + 1)) + r, 4 * (h % (i + 1)) + k, part);
+    } else if (f < C::TF) {  // shared row
+      const int h = f - C::QX;
+      v = rot(4 * (C::G - 1) + (b & 1), 4 * (h / C::G) + r, 4 * (h % C::G) + k, b >> 1);
+    } else if (f < C::TX) {  // shift levels
+      int h = f - C::TF, lev = 0;
+      while (h >= C::tiles(lev) * C::tiles(lev)) {
+        h -= C::tiles(lev) * C::tiles(lev);
+        lev++;
+      }
+      const int t = C::tiles(lev), mm = C::m0(lev);
+      v = shift(mm + b, mm + 4 * (h / t) + r, mm + 4 * (h % t) + k);
+    } else if (f < C::NFRAG) {  // shared orders m < REM
+      const int h = f - C::TX, m = b & 1;
+      v = m < C::REM ? shift(m, 4 * (h / C::G) + r, 4 * (h % C::G) + k) : 0.0;
+    } else if (f < C::NREC) {  // z rotation factors, lane (r = lane / 16, b, c)
+      const int h = (f - C::NFRAG) >> 1, sn = (f - C::NFRAG) & 1, rr = lane >> 4;
+      int n, m;
+      bool neg = false;
+      if (h < C::NF) {
+        int i = 0, j = h;
+        while (j > i) {
+          j -= i + 1;
+          i++;
+        }
+        n = 4 * i + b;
+        m = 4 * j + rr;
+      } else {  // own factor cos, partner factor -sin (Re) or +sin (Im)
+        n = 4 * (C::G - 1) + (b & 1);
+        m = 4 * (h - C::NF) + rr;
+        neg = !(b >> 1);
+      }
+      if (n < P && m <= n) v = (neg && sn ? -1.0 : 1.0) * scale(n, m) * zc[sn][m];
+    }
+    rec[(size_t)(f >> 1) * 128 + lane * 2 + (f & 1)] = v;
+  }
+}
+
+// v of lane l ^ 8 (the other part of a shared-row lane)
+__device__ __forceinline__ double partner(double v) {
+  const long long x = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)x, 0x128, 0xf, 0xf, true);  // row_ror:8
+  const int hi = __builtin_amdgcn_mov_dpp((int)(x >> 32), 0x128, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double flip(double v, unsigned mask) {
+  return __longlong_as_double(__double_as_longlong(v) ^ ((long long)mask << 32));
+}
+__device__ __forceinline__ double mm(double a, double b, double c) {
+  return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+}
+// the exchange buffer is written and read by one wavefront, whose LDS
+// operations complete in order: the compiler only must not reorder them
+__device__ __forceinline__ void lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// One wavefront per work item: the slices (<= 4 pairs of one class with
+// distinct targets) of a tile of TT targets, whose local expansions are held
+// in LDS (times (-1)^m: the outer S of the back rotation) and stored, or
+// added atomically when the tile is split over items, at the end.  The class's
+// record stays in registers while consecutive slices share it.  No barriers:
+// a wavefront owns its tile and its exchange buffer.
+//
+// Bound: issue.  A slice at P = 12 issues 84 products (16 cycles each) and
+// about 110 other vector instructions, which do not overlap FP64 products on
+// a SIMD; the rest is latency of the LDS round trips, hidden by the other
+// part's products and by the second wavefront of the SIMD (registers: the
+// record alone takes 108 at P = 12).  Measured on MI355X against one dense
+// operator per class on v_mfma_f64_16x16x4 (same lists), M2L in ms: 8M cube,
+// P = 12: 155 -> 47; 1M Plummer, P = 10: 6.7 -> 2.9; 10^6 cube, P = 8: 3.7 ->
+// 2.1, P = 4: 1.10 -> 0.66; also against FP32 (P = 12 10.4 ms, P = 8 2.65) and
+// split-FP16 (8.4, 2.27) dense operators on that cube (5.2, 2.1 here).
+// TT: what LDS leaves room for with 8 wavefronts a CU (P >= 9), 16 below.
+template <int P, int TT>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void m2l_rot_kernel(
+    const int *__restrict__ ttgt, const int4 *__restrict__ items, const int4 *__restrict__ slices,
+    const int *__restrict__ psrc, const unsigned short *__restrict__ plt, const double2 *__restrict__ ops,
+    const double2 *__restrict__ M, double *__restrict__ L) {
+  using C = RotCfg<P>;
+  constexpr int NT = C::NT, G = C::G, NL = C::NL, NF = C::NF, NX = C::NX, AST = C::AST, PART = C::PART;
+  __shared__ double2 sAcc[TT * NT];
+  __shared__ double sX[C::XSZ];
+  const int l = threadIdx.x, r = l >> 4, b = (l >> 2) & 3, c = l & 3;
+  const int4 item = items[blockIdx.x];
+  const int s0 = item.y, s1 = item.z;
+  if (s0 >= s1) return;
+  for (int e = l; e < TT * NT; e += 64) sAcc[e] = make_double2(0.0, 0.0);
+  for (int e = l; e < C::XSZ; e += 64) sX[e] = 0.0;
+  // offsets (terms) of this lane's element of tile (i, 0) in a cell's
+  // expansion; lanes past the order or above the diagonal read a stand-in
+  // inside the cell (their operator columns are zero)
+  int row[G];
+#pragma unroll
+  for (int i = 0; i < G; i++) {
+    const int n = min(4 * i + (C::COMB && i == G - 1 ? b & 1 : b), P - 1);
+    row[i] = n * (n + 1) / 2 + r;
+  }
+  const int last = min(row[G - 1] + 4 * (G - 1), NT - 1);  // tile (G-1, G-1)
+  auto term = [&](int i, int j) { return i == G - 1 && j == G - 1 ? last : row[i] + 4 * j; };
+  auto valid = [&](int i, int j) {  // this lane's element of tile (i, j) exists
+    const int n = 4 * i + (C::COMB && i == G - 1 ? b & 1 : b);
+    return n < P && 4 * j + r <= n;
+  };
+  // exchange addresses
+  const int w1 = b * AST + 4 * r + c, w2 = r * AST + 4 * b + c;
+  const int x1 = min(b & 1, C::REM - 1) * AST + (b >> 1) * PART + 4 * r + c, x2 = r * AST + (b >> 1) * PART + 4 * (b & 1) + c;
+  const int x2l = min(4 * (G - 1) + r, C::ROWS - 1) * AST + (b >> 1) * PART + 4 * (b & 1) + c;
+  // a slice's pairs: lanes past its count read its last pair as a stand-in
+  auto desc = [&](int s) { return slices[min(s, s1 - 1)]; };
+  auto pair_of = [&](const int4 &d) { return d.y + min(c, d.z - 1); };
+  double2 pf[NF > 0 ? NF : 1];
+  double px[NX > 0 ? NX : 1];
+  auto gather = [&](int src) {
+    const double2 *m = M + (size_t)(src & ((1 << 26) - 1)) * NT;
+#pragma unroll
+    for (int i = 0; i < NL; i++)
+#pragma unroll
+      for (int j = 0; j <= i; j++) pf[tri(i, j)] = m[term(i, j)];
+#pragma unroll
+    for (int j = 0; j < NX; j++) px[j] = reinterpret_cast<const double *>(m + term(G - 1, j))[b >> 1];
+  };
+  double A[C::NFRAG];
+  double2 cs[C::NCS];
+  auto load_class = [&](int g) {
+    const double2 *rec = ops + (size_t)g * C::NREC2 * 64 + l;
+#pragma unroll
+    for (int f = 0; f < C::NREC2; f++) {
+      const double2 v = rec[(size_t)f * 64];
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const int u = 2 * f + h;
+        const double x = h ? v.y : v.x;
+        if (u < C::NFRAG)
+          A[u] = x;
+        else if (u < C::NREC) {
+          if ((u - C::NFRAG) & 1)
+            cs[(u - C::NFRAG) / 2].y = x;
+          else
+            cs[(u - C::NFRAG) / 2].x = x;
+        }
+      }
+    }
+  };
+  // products of one part: rotation of the full rows, of the shared row, shift
+  auto rot_part = [&](int q, double *v) {
+    double o[NF > 0 ? NF : 1];
+#pragma unroll
+    for (int t = 0; t < NF; t++) o[t] = 0.0;
+#pragma unroll
+    for (int i = 0; i < NL; i++)
+#pragma unroll
+      for (int ji = 0; ji <= i; ji++)
+#pragma unroll
+        for (int jo = 0; jo <= i; jo++)
+          o[tri(i, jo)] = mm(A[q + sq_sum(i) + jo * (i + 1) + ji], v[tri(i, ji)], o[tri(i, jo)]);
+#pragma unroll
+    for (int t = 0; t < NF; t++) v[t] = o[t];
+  };
+  auto mul_shared = [&](int q, double *v) {
+    double o[NX > 0 ? NX : 1];
+#pragma unroll
+    for (int t = 0; t < NX; t++) o[t] = 0.0;
+#pragma unroll
+    for (int ji = 0; ji < NX; ji++)
+#pragma unroll
+      for (int jo = 0; jo < NX; jo++) o[jo] = mm(A[q + jo * G + ji], v[ji], o[jo]);
+#pragma unroll
+    for (int t = 0; t < NX; t++) v[t] = o[t];
+  };
+  auto shift_part = [&](double *v) {
+    double o[NF > 0 ? NF : 1];
+#pragma unroll
+    for (int t = 0; t < NF; t++) o[t] = 0.0;
+#pragma unroll
+    for (int k = 0; k < NL; k++)
+#pragma unroll
+      for (int ii = 0; ii < C::tiles(k); ii++)
+#pragma unroll
+        for (int io = 0; io < C::tiles(k); io++)
+          o[C::off2(k) + io] = mm(A[C::TF + C::offT(k) + io * C::tiles(k) + ii], v[C::off2(k) + ii], o[C::off2(k) + io]);
+#pragma unroll
+    for (int t = 0; t < NF; t++) v[t] = o[t];
+  };
+  // exchange buffer, layout 1 and 2 of one part, and of the shared tiles
+  auto put1 = [&](const double *v, int off) {
+#pragma unroll
+    for (int i = 0; i < NL; i++)
+#pragma unroll
+      for (int j = 0; j <= i; j++) sX[w1 + off + 4 * i * AST + 16 * j] = v[tri(i, j)];
+  };
+  auto get1 = [&](double *v, int off) {
+#pragma unroll
+    for (int i = 0; i < NL; i++)
+#pragma unroll
+      for (int j = 0; j <= i; j++) v[tri(i, j)] = sX[w1 + off + 4 * i * AST + 16 * j];
+  };
+  auto put2 = [&](const double *v, int off) {
+#pragma unroll
+    for (int k = 0; k < NL; k++)
+#pragma unroll
+      for (int i = 0; i < C::tiles(k); i++) sX[w2 + off + (C::m0(k) + 4 * i) * AST + 4 * C::m0(k)] = v[C::off2(k) + i];
+  };
+  auto get2 = [&](double *v, int off) {
+#pragma unroll
+    for (int k = 0; k < NL; k++)
+#pragma unroll
+      for (int i = 0; i < C::tiles(k); i++) v[C::off2(k) + i] = sX[w2 + off + (C::m0(k) + 4 * i) * AST + 4 * C::m0(k)];
+  };
+  auto put1x = [&](const double *v) {
+#pragma unroll
+    for (int j = 0; j < NX; j++)
+      if ((b & 1) < C::REM) sX[x1 + 4 * (G - 1) * AST + 16 * j] = v[j];
+  };
+  auto get1x = [&](double *v) {
+#pragma unroll
+    for (int j = 0; j < NX; j++) v[j] = sX[x1 + 4 * (G - 1) * AST + 16 * j];
+  };
+  auto put2x = [&](const double *v) {
+#pragma unroll
+    for (int i = 0; i < NX; i++)
+      if ((i < G - 1 || 4 * i + r < P) && (b & 1) < C::REM) sX[x2 + 4 * i * AST] = v[i];
+  };
+  auto get2x = [&](double *v) {
+#pragma unroll
+    for (int i = 0; i < NX; i++) v[i] = sX[i == G - 1 ? x2l : x2 + 4 * i * AST];
+  };
+  // pipeline: slice s computes, s + 1's multipoles load, s + 2's pair indices
+  // load, s + 3's descriptor loads
+  int4 d = desc(s0), d1 = desc(s0 + 1), d2 = desc(s0 + 2);
+  load_class(d.x);
+  gather(psrc[pair_of(d)]);
+  int lt = plt[pair_of(d)], lt1 = plt[pair_of(d1)], src1 = psrc[pair_of(d1)];
+  for (int s = s0; s < s1; s++) {
+    const int4 d3 = desc(s + 3);
+    // the pair's offset is its class's reflected (bits x, y, z): the operator
+    // changes by the sign (-1)^(x m + z (n + m)) on both sides, and phi -> -phi
+    // when one of x and y is reflected
+    const int rf = lt >> 8;
+    const unsigned mc = (unsigned)((rf & r) ^ ((rf >> 2) & (b ^ r))) << 31;
+    const unsigned ms = mc ^ ((unsigned)(rf ^ (rf >> 1)) << 31);
+    double2 z[C::NCS];
+#pragma unroll
+    for (int t = 0; t < C::NCS; t++) z[t] = make_double2(flip(cs[t].x, mc), flip(cs[t].y, ms));
+    double re[NF > 0 ? NF : 1], im[NF > 0 ? NF : 1], xv[NX > 0 ? NX : 1];
+#pragma unroll
+    for (int t = 0; t < NF; t++) {
+      re[t] = fma(z[t].x, pf[t].x, -z[t].y * pf[t].y);
+      im[t] = fma(z[t].x, pf[t].y, z[t].y * pf[t].x);
+    }
+#pragma unroll
+    for (int t = 0; t < NX; t++) xv[t] = fma(z[NF + t].x, px[t], z[NF + t].y * partner(px[t]));
+    gather(src1);
+    const int p2 = pair_of(d2);
+    src1 = psrc[p2];
+    const int lt2 = plt[p2];
+    if constexpr (C::COMB) {
+      mul_shared(C::QX, xv);
+      rot_part(C::QRE, re);
+      put1x(xv);
+      put1(re, 0);
+      rot_part(C::QIM, im);
+      lds_order();
+      get2(re, 0);
+      put1(im, PART);
+      lds_order();
+      get2x(xv);
+      get2(im, PART);
+      lds_order();
+      shift_part(re);
+      put2(re, 0);
+      mul_shared(C::TX, xv);
+      put2x(xv);
+      shift_part(im);
+      lds_order();
+      get1(re, 0);
+      put2(im, PART);
+      lds_order();
+      get1x(xv);
+      get1(im, PART);
+      lds_order();
+    } else {
+      rot_part(C::QRE, re);
+      put1(re, 0);
+      lds_order();
+      get2(re, 0);
+      lds_order();
+      rot_part(C::QIM, im);
+      put1(im, 0);
+      lds_order();
+      get2(im, 0);
+      lds_order();
+      shift_part(re);
+      put2(re, 0);
+      lds_order();
+      get1(re, 0);
+      lds_order();
+      shift_part(im);
+      put2(im, 0);
+      lds_order();
+      get1(im, 0);
+      lds_order();
+    }
+    // the targets' local expansions are read while the back rotation runs
+    const bool live = c < d.z;
+    double2 *acc = sAcc + (lt & 255) * NT;
+    double2 av[NF > 0 ? NF : 1];
+    double ax[NX > 0 ? NX : 1];
+#pragma unroll
+    for (int i = 0; i < NL; i++)
+#pragma unroll
+      for (int j = 0; j <= i; j++) av[tri(i, j)] = acc[term(i, j)];
+#pragma unroll
+    for (int j = 0; j < NX; j++) ax[j] = reinterpret_cast<const double *>(acc + term(G - 1, j))[b >> 1];
+    rot_part(C::QRE, re);
+    if constexpr (C::COMB) mul_shared(C::QX, xv);
+    rot_part(C::QIM, im);
+    if (d1.x != d.x) load_class(d1.x);
+    // z rotation back, added
+#pragma unroll
+    for (int t = 0; t < NF; t++) {
+      av[t].x = fma(z[t].x, re[t], fma(z[t].y, im[t], av[t].x));
+      av[t].y = fma(z[t].x, im[t], fma(-z[t].y, re[t], av[t].y));
+    }
+#pragma unroll
+    for (int j = 0; j < NX; j++) ax[j] = fma(z[NF + j].x, xv[j], fma(-z[NF + j].y, partner(xv[j]), ax[j]));
+    if (live) {
+#pragma unroll
+      for (int i = 0; i < NL; i++)
+#pragma unroll
+        for (int j = 0; j < i; j++)
+          if (4 * i + 3 < P || valid(i, j)) acc[row[i] + 4 * j] = av[tri(i, j)];
+#pragma unroll
+      for (int i = 0; i < NL; i++)
+        if (4 * i + 3 < P ? r <= b : valid(i, i)) acc[row[i] + 4 * i] = av[tri(i, i)];
+#pragma unroll
+      for (int j = 0; j < NX; j++)
+        if (valid(G - 1, j)) reinterpret_cast<double *>(acc + row[G - 1] + 4 * j)[b >> 1] = ax[j];
+    }
+    lds_order();
+    d = d1;
+    d1 = d2;
+    d2 = d3;
+    lt = lt1;
+    lt1 = lt2;
+  }
+  // store (or add) the tile's local expansions
+  for (int t0 = 0; t0 < TT; t0 += 4) {
+    const int t = t0 + c;
+    const int cell = t < TT ? ttgt[(size_t)item.x * TT + t] : -1;
+    if (cell < 0) continue;
+    double *Lc = L + (size_t)cell * NT * 2;
+#pragma unroll
+    for (int i = 0; i < G; i++)
+#pragma unroll
+      for (int j = 0; j <= i; j++) {
+        const int u = row[i] + 4 * j;
+        if (!valid(i, j) || (C::COMB && i == G - 1 && (b >> 1))) continue;
+        double2 v = sAcc[t * NT + u];
+        if (r & 1) v = make_double2(-v.x, -v.y);
+        if (item.w) {
+          unsafeAtomicAdd(Lc + 2 * u, v.x);
+          unsafeAtomicAdd(Lc + 2 * u + 1, v.y);
+        } else {
+          reinterpret_cast<double2 *>(Lc)[u] = v;
+        }
+      }
+  }
+}
+
+template <int P> constexpr int rot_tt() { return P >= 9 ? 12 : 16; }
+
+template <template <int> class F, typename... A> hipError_t rot_dispatch(int P, A... a) {
+  switch (P) {
+    case 2: return F<2>::run(a...);
+    case 3: return F<3>::run(a...);
+    case 4: return F<4>::run(a...);
+    case 5: return F<5>::run(a...);
+    case 6: return F<6>::run(a...);
+    case 7: return F<7>::run(a...);
+    case 8: return F<8>::run(a...);
+    case 9: return F<9>::run(a...);
+    case 10: return F<10>::run(a...);
+    case 11: return F<11>::run(a...);
+    case 12: return F<12>::run(a...);
+    default: return hipErrorInvalidValue;
+  }
+}
+template <int P> struct RotBytes {
+  static hipError_t run(size_t *b, int *tt) {
+    *b = sizeof(double) * 128 * RotCfg<P>::NREC2;
+    *tt = rot_tt<P>();
+    return hipSuccess;
+  }
+};
+template <int P> struct RunRotOps {
+  static hipError_t run(const double *cdx, int nrep, void *ops, hipStream_t s) {
+    hipLaunchKernelGGL((rot_ops_kernel<P>), dim3(nrep), dim3(256), 0, s, cdx, nrep, static_cast<double *>(ops));
+    return hipGetLastError();
+  }
+};
+template <int P> struct RunM2LRot {
+  static hipError_t run(int nitem, const int *ttgt, const int4 *items, const int4 *slices, const int *psrc,
+                        const unsigned short *plt, const void *ops, const double2 *M, double2 *L, hipStream_t s) {
+    hipLaunchKernelGGL((m2l_rot_kernel<P, rot_tt<P>()>), dim3(nitem), dim3(64), 0, s, ttgt, items, slices, psrc, plt,
+                       static_cast<const double2 *>(ops), M, reinterpret_cast<double *>(L));
+    return hipGetLastError();
+  }
+};
+
+}  // namespace
+
+hipError_t init_rot_constants() {
+  // d^n(pi/2)[a][b] = 2^-n sqrt((n+a)!(n-a)! / ((n+b)!(n-b)!)) x an integer sum
+  std::vector<double> h(delta_off(kRotMaxP));
+  auto binom = [](int n, int k) {
+    long long v = 1;
+    for (int i = 1; i <= k; i++) v = v * (n - k + i) / i;
+    return v;
+  };
+  long double f[2 * kRotMaxP];
+  f[0] = 1.0L;
+  for (int i = 1; i < 2 * kRotMaxP; i++) f[i] = f[i - 1] * i;
+  for (int n = 0; n < kRotMaxP; n++)
+    for (int a = -n; a <= n; a++)
+      for (int b = -n; b <= n; b++) {
+        long long t = 0;
+        for (int k = std::max(0, b - a); k <= std::min(n + b, n - a); k++) {
+          const long long v = binom(n + b, k) * binom(n - b, n - a - k);
+          t += (a - b + k) & 1 ? -v : v;
+        }
+        h[delta_off(n) + (a + n) * (2 * n + 1) + b + n] =
+            (double)(std::ldexp((long double)t, -n) * sqrtl(f[n + a] * f[n - a] / (f[n + b] * f[n - b])));
+      }
+  return hipMemcpyToSymbol(HIP_SYMBOL(g_delta), h.data(), h.size() * sizeof(double));
+}
+
+bool m2l_rot_supported(int P) { return P >= 2 && P <= kRotMaxP; }
+
+size_t rot_ops_bytes(int P) {
+  size_t b = 0;
+  int tt = 0;
+  (void)rot_dispatch<RotBytes>(P, &b, &tt);
+  return b;
+}
+
+int m2l_tile_targets(int P) {
+  size_t b = 0;
+  int tt = 0;
+  (void)rot_dispatch<RotBytes>(P, &b, &tt);
+  return tt;
+}
+
+hipError_t launch_rot_ops(int P, const double *cdx, int nrep, void *ops, hipStream_t s) {
+  return nrep > 0 ? rot_dispatch<RunRotOps>(P, cdx, nrep, ops, s) : hipSuccess;
+}
+
+hipError_t launch_m2l_rot(int P, int nitem, const int *ttgt, const int4 *items, const int4 *slices, const int *psrc,
+                          const unsigned short *plt, const void *ops, const double2 *M, double2 *L, hipStream_t s) {
+  return nitem > 0 ? rot_dispatch<RunM2LRot>(P, nitem, ttgt, items, slices, psrc, plt, ops, M, L, s) : hipSuccess;
+}
+
+}  // namespace fmmdev

@@ -78,7 +78,7 @@ int64_t footprint(const fmm_params &p, const fmm_stats &s) {
   const int64_t nt = (int64_t)p.P * (p.P + 1) / 2;
   int64_t b = (int64_t)s.n * (8 * 8 + 4);
   b += (int64_t)s.ncell * (2 * nt * 16 + (p.precision != FMM_FP64 ? nt * 8 + 16 : 0) + 80);
-  b += s.m2l_pairs * (4 + 8) + s.p2p_pairs * 4 + s.m2l_pairs / 32 * 16;
+  b += s.m2l_pairs * (4 + 8) + s.p2p_pairs * 4 + s.m2l_pairs / 3 * 16;  // about 3.6 pairs a slice
   return b;
 }
 
@@ -106,10 +106,12 @@ void builder_loop(fmm_server *s) {
     fmm_plan *pl = nullptr;
     int rc = bc ? fmm_plan_build_device(bc, &pl, r->n, r->x.data(), s->p.ncrit, s->p.theta, s->p.nspawn)
                 : fmm_plan_build(&pl, r->n, r->x.data(), s->p.ncrit, s->p.theta, s->p.nspawn);
-    // M2L groups for the slots' contexts; free-space tiles are left to the
-    // upload, which builds them on the device (for a batch of several
-    // requests the merged forest is grouped on the host there)
-    if (rc == FMM_OK && !(s->p.m2l_mode == FMM_M2L_TILES && s->p.images == 0)) rc = fmm_plan_prepare(pl, &s->p);
+    // M2L groups for the slots' contexts; the tiles of a request that runs
+    // alone are left to the upload, which builds them on the device (a batch
+    // of several takes its requests' groups and tiles, so that a request's
+    // M2L is the same alone and in a batch)
+    if (rc == FMM_OK && !(s->p.m2l_mode == FMM_M2L_TILES && s->cfg.batch_requests == 1))
+      rc = fmm_plan_prepare(pl, &s->p);
     fmm_stats st{};
     if (rc == FMM_OK) fmm_plan_stats(pl, &st);
     std::lock_guard<std::mutex> lk(s->mu);
@@ -294,18 +296,10 @@ int fmm_server_create(fmm_server **out, const fmm_params *p, const fmm_server_co
   fmm_server *s = new (std::nothrow) fmm_server();
   if (!s) return FMM_ERR_MEMORY;
   s->p = *p;
-  // AUTO, one request per batch: target tiles.  The builders then plan only
-  // the tree and lists; a slot's upload builds the groups and tiles on the
-  // device (grouped chunks are built on the host by the builders, about half
-  // of a request's planning).  At 1000 req/s offered, 2^12-2^18-body
-  // requests: tiles 715 req/s, chunks 580 req/s (8 and 5 slots).  Batches of
-  // several requests: grouped chunks, as a merged forest's tiles are grouped
-  // on the host, where mixed precision groups by level across systems of
-  // different radii and runs the pairs left over on the per-target kernel
-  // (results then depend on the batch, about 1e-8).  Split-FP16 runs on
-  // tiles only.
-  if (s->p.m2l_mode == FMM_M2L_AUTO && s->p.precision != FMM_MIXED16)
-    s->p.m2l_mode = c.batch_requests == 1 ? FMM_M2L_TILES : FMM_M2L_GROUPED;
+  // AUTO: target tiles.  With one request per batch the builders plan only
+  // the tree and lists and a slot's upload builds the groups and tiles on the
+  // device, else the builders build them and the batch's are concatenated.
+  if (s->p.m2l_mode == FMM_M2L_AUTO) s->p.m2l_mode = FMM_M2L_TILES;
   s->cfg = c;
   s->t0 = clock_ms();
   for (int i = 0; i < c.host_threads; i++) s->builders.emplace_back(builder_loop, s);

@@ -6,18 +6,17 @@
 // fmm::build_tree or fmmdev::device_tree):
 //
 //  * every M2L pair's offset, in units of its finer cell's size, reduced by
-//    common factors of two (the host's lattice key), with (by level) the two
-//    levels, packed into one 64-bit key; a hash table on the device gives
+//    common factors of two (the host's lattice key), packed into one 64-bit key; a hash table on the device gives
 //    each pair its key's slot;
 //  * on the host, over the distinct keys only (thousands): group numbers in
 //    key order, offsets, reflection classes and their representatives --
 //    the host's numbering is first-appearance order, which only permutes the
 //    groups and classes;
-//  * tiles: the targets sorted by (level, octant in the parent, cell), TT per
-//    tile -- the host's order, so the same tiles; each tile's pairs sorted by
-//    (class, target) and every (tile, class) run of m pairs dealt into S =
-//    max(ceil(m / 16), most pairs of one target) slices of distinct targets,
-//    pair i of the run to slice i mod S, as the host does.
+//  * tiles: the targets sorted by (level, cell), TT per tile -- the host's
+//    order, so the same tiles; each tile's pairs sorted by (class, target) and
+//    every (tile, class) run of m pairs dealt into S = max(ceil(m / SW), most
+//    pairs of one target) slices of distinct targets, pair i of the run to
+//    slice i mod S, as the host does.
 //
 // Keys that do not fit (an offset component of 2^13 or more after the
 // reduction, an offset off the lattice) make the whole plan fall back to
@@ -87,7 +86,7 @@ __global__ void pair_target_kernel(int ncell, const int *__restrict__ ptr, int *
 // every pair's key (host: build_m2l_groups), inserted into the hash table;
 // slot[p] its slot, *bad set when a key does not fit
 __global__ void pair_key_kernel(int64_t np, const int *__restrict__ ptgt, const int *__restrict__ psrc,
-                                const double *__restrict__ X, const int *__restrict__ level, double R0, int by_level,
+                                const double *__restrict__ X, const int *__restrict__ level, double R0,
                                 unsigned long long *__restrict__ table, int *__restrict__ slot,
                                 int *__restrict__ bad) {
 #pragma clang fp contract(off)
@@ -120,8 +119,7 @@ __global__ void pair_key_kernel(int64_t np, const int *__restrict__ ptgt, const 
     slot[p] = -1;
     return;
   }
-  const unsigned long long lv = by_level ? ((unsigned long long)lt << 5 | (unsigned long long)ls) : 0ull;
-  const unsigned long long key = (((unsigned long long)e << 10 | lv) << (3 * kKBits)) |
+  const unsigned long long key = ((unsigned long long)e << (3 * kKBits)) |
                                  ((unsigned long long)(k[0] + kKOff) << (2 * kKBits)) |
                                  ((unsigned long long)(k[1] + kKOff) << kKBits) | (unsigned long long)(k[2] + kKOff);
   const unsigned long long mask = (1ull << kHashBits) - 1;
@@ -161,20 +159,13 @@ __global__ void slot_group_kernel(int ng, const int *__restrict__ gslot, int *__
   if (g < ng) slot2grp[gslot[g]] = g;
 }
 
-// the octant of every target cell in its parent; sort keys (level, octant, cell)
+// the target cells with their sort keys (level, cell): siblings are adjacent
 __global__ void target_key_kernel(int ncell, const int *__restrict__ ptr, const int *__restrict__ level,
-                                  const int *__restrict__ iparent, const double *__restrict__ X,
                                   unsigned long long *__restrict__ key, int *__restrict__ cell, int *__restrict__ cnt) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= ncell || ptr[c + 1] == ptr[c]) return;
-  int o = 0;
-  if (c > 0) {
-    const int p = iparent[c];
-    for (int d = 0; d < 3; d++)
-      if (X[3 * (size_t)c + d] > X[3 * (size_t)p + d]) o |= 1 << d;
-  }
   const int i = atomicAdd(cnt, 1);
-  key[i] = ((unsigned long long)level[c] << 40) | ((unsigned long long)o << 32) | (unsigned)c;
+  key[i] = ((unsigned long long)level[c] << 32) | (unsigned)c;
   cell[i] = c;
 }
 
@@ -274,7 +265,7 @@ __global__ void slice_desc_kernel(int nseg, const unsigned long long *__restrict
 
 }  // namespace
 
-hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, bool by_level, int TT, int SW, int seg,
+hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, int TT, int SW, int seg,
                                fmm::M2LGroups &G, fmm::M2LTiles &T, bool &done, hipStream_t s,
                                PlanArrays *keep, const int *dsrc_in) {
   done = false;
@@ -291,10 +282,9 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, bool by_
   for (int c = 0; c < nc; c++)  // regular tree: every radius R0 / 2^level
     if (t.R[c] != t.R[0] / (1 << t.level[c])) return hipSuccess;
   const double R0 = t.R[0];
-  DBufT dX(s), dlev(s), dpar(s), dptr(s), dsrc(s), dtgt(s), dtab(s), dslot(s), dbad(s);
+  DBufT dX(s), dlev(s), dptr(s), dsrc(s), dtgt(s), dtab(s), dslot(s), dbad(s);
   TCHK(dX.need(sizeof(double) * 3 * (size_t)nc));
   TCHK(dlev.need(4 * (size_t)nc));
-  TCHK(dpar.need(4 * (size_t)nc));
   TCHK(dptr.need(4 * ((size_t)nc + 1)));
   // the pair sources: given on the device, or the lists' device column when
   // the plan keeps one, else uploaded from L
@@ -304,7 +294,6 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, bool by_
   TCHK(dtgt.need(4 * (size_t)np));
   TCHK(hipMemcpyAsync(dX.p, t.X.data(), sizeof(double) * 3 * (size_t)nc, hipMemcpyHostToDevice, s));
   TCHK(hipMemcpyAsync(dlev.p, t.level.data(), 4 * (size_t)nc, hipMemcpyHostToDevice, s));
-  TCHK(hipMemcpyAsync(dpar.p, t.iparent.data(), 4 * (size_t)nc, hipMemcpyHostToDevice, s));
   TCHK(hipMemcpyAsync(dptr.p, L.m2l_ptr.data(), 4 * ((size_t)nc + 1), hipMemcpyHostToDevice, s));
   if (!dev_src) TCHK(hipMemcpyAsync(dsrc.p, L.m2l_src.data(), 4 * (size_t)np, hipMemcpyHostToDevice, s));
   const unsigned nbc = (unsigned)((nc + 255) / 256), nbp = (unsigned)((np + 255) / 256);
@@ -318,7 +307,7 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, bool by_
   TCHK(hipMemsetAsync(dtab.p, 0xff, 8 * tsize, s));
   TCHK(hipMemsetAsync(dbad.p, 0, 4, s));
   pair_key_kernel<<<nbp, 256, 0, s>>>(np, dtgt.as<int>(), psrc, dX.as<double>(), dlev.as<int>(), R0,
-                                       by_level ? 1 : 0, dtab.as<unsigned long long>(), dslot.as<int>(),
+                                       dtab.as<unsigned long long>(), dslot.as<int>(),
                                        dbad.as<int>());
   TCHK(hipGetLastError());
   // the filled slots come back (key, slot), not the whole table
@@ -361,13 +350,12 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, bool by_
   for (int g = 0; g < ng; g++) {
     const unsigned long long key = keys[g].first;
     gslot[g] = keys[g].second;
-    const int e = (int)(key >> (3 * kKBits + 10));
-    const unsigned long long lv = (key >> (3 * kKBits)) & 1023;
+    const int e = (int)(key >> (3 * kKBits));
     long long k[3];
     for (int d = 0; d < 3; d++) k[d] = (long long)((key >> (kKBits * (2 - d))) & kmask) - kKOff;
     const double u = R0 / std::ldexp(1.0, e);
     unsigned char r = 0;
-    unsigned long long ck = (unsigned long long)e << 10 | lv;
+    unsigned long long ck = (unsigned long long)e;
     for (int d = 0; d < 3; d++) {
       G.dx[3 * (size_t)g + d] = (double)k[d] * u;
       if (k[d] < 0) r |= (unsigned char)(1 << d);
@@ -385,25 +373,13 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, bool by_
         cls[x.first] = id;
         const int g = x.second;
         for (int d = 0; d < 3; d++) G.cdx.push_back(std::fabs(G.dx[3 * (size_t)g + d]));
-        if (by_level) {
-          const unsigned long long lv = (x.first >> (3 * kKBits)) & 1023;
-          G.cscale.insert(G.cscale.end(), {R0 / (1 << (int)(lv & 31)), R0 / (1 << (int)(lv >> 5))});
-        }
       }
     for (int g = 0; g < ng; g++) gcanon[g] = cls[gcls[g].first];
   }
   G.ncanon = (int)cls.size();
   G.canon = gcanon;
   G.refl.assign(grefl.begin(), grefl.end());
-  if (by_level) {
-    G.scale.resize(2 * (size_t)ng);
-    for (int g = 0; g < ng; g++) {
-      const unsigned long long lv = (keys[g].first >> (3 * kKBits)) & 1023;
-      G.scale[2 * (size_t)g] = R0 / (1 << (int)(lv & 31));      // R_s
-      G.scale[2 * (size_t)g + 1] = R0 / (1 << (int)(lv >> 5));  // R_t
-    }
-  }
-  // tiles: targets in (level, octant, cell) order
+  // tiles: targets in (level, cell) order
   DBufT dtk(s), dtk2(s), dtc(s), dtc2(s), dcnt(s), dtof(s), dloc(s), tmp(s);
   TCHK(dtk.need(8 * (size_t)nc));
   TCHK(dtk2.need(8 * (size_t)nc));
@@ -413,18 +389,18 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, bool by_
   TCHK(dtof.need(4 * (size_t)nc));
   TCHK(dloc.need(4 * (size_t)nc));
   TCHK(hipMemsetAsync(dcnt.p, 0, 4, s));
-  target_key_kernel<<<nbc, 256, 0, s>>>(nc, dptr.as<int>(), dlev.as<int>(), dpar.as<int>(), dX.as<double>(),
-                                        dtk.as<unsigned long long>(), dtc.as<int>(), dcnt.as<int>());
+  target_key_kernel<<<nbc, 256, 0, s>>>(nc, dptr.as<int>(), dlev.as<int>(), dtk.as<unsigned long long>(),
+                                        dtc.as<int>(), dcnt.as<int>());
   TCHK(hipGetLastError());
   int ntg = 0;
   TCHK(hipMemcpyAsync(&ntg, dcnt.p, 4, hipMemcpyDeviceToHost, s));
   TCHK(hipStreamSynchronize(s));
   size_t tb = 0;
   TCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, dtk.as<unsigned long long>(), dtk2.as<unsigned long long>(),
-                                          dtc.as<int>(), dtc2.as<int>(), ntg, 0, 48, s));
+                                          dtc.as<int>(), dtc2.as<int>(), ntg, 0, 40, s));
   TCHK(tmp.need(tb));
   TCHK(hipcub::DeviceRadixSort::SortPairs(tmp.p, tb, dtk.as<unsigned long long>(), dtk2.as<unsigned long long>(),
-                                          dtc.as<int>(), dtc2.as<int>(), ntg, 0, 48, s));
+                                          dtc.as<int>(), dtc2.as<int>(), ntg, 0, 40, s));
   tile_of_kernel<<<(unsigned)((ntg + 255) / 256), 256, 0, s>>>(ntg, dtc2.as<int>(), TT, dtof.as<int>(),
                                                                 dloc.as<int>());
   TCHK(hipGetLastError());

@@ -32,30 +32,27 @@ typedef enum {
 } fmm_status;
 
 /* FP64: every phase in FP64 (parity with the reference to 1e-10).
- * MIXED: P2P and M2L in FP32 (P2P with FP32 partial sums of at most 32 terms
- * added into FP64 accumulators; M2L as grouped FP32 MFMA translations whose
- * results are added into FP64 local expansions); P2M, M2M, L2L, L2P, the
+ * MIXED: P2P in FP32 (FP32 partial sums of at most 32 terms added into FP64
+ * accumulators).  The M2L on target tiles is the FP64 one (about 6 P^3
+ * multiply-adds a pair, faster than dense FP32 or split-FP16 operators);
+ * m2l_mode GROUPED runs it in FP32 (grouped FP32 MFMA translations whose
+ * results are added into FP64 local expansions).  P2M, M2M, L2L, L2P, the
  * harmonics of every translation and all accumulation across lists stay FP64.
- * Needs P <= 12 and m2l_mode AUTO or GROUPED.
- * MIXED16: MIXED with the M2L on split-FP16 operands: every operator row
- * (scaled by a power of two) and every cell's multipole (likewise) are held
- * as hi + lo halves, applied with v_mfma_f32_16x16x32_f16 as hi x hi + hi x lo
- * + lo x hi into FP32 accumulators (22 significant bits of every value within
- * 2^-14 of its row's or cell's largest); accumulation across lists in FP64
- * as for MIXED.  Needs P <= 12 and m2l_mode AUTO or TILES. */
+ * Needs P <= 12 and an m2l_mode other than TARGET.
+ * MIXED16: as MIXED; needs P <= 12 and m2l_mode AUTO or TILES. */
 typedef enum { FMM_FP64 = 0, FMM_MIXED = 1, FMM_MIXED16 = 2 } fmm_precision;
 
-/* M2L execution.  Pairs are grouped by offset (one dense operator per group,
- * applied on MFMA) in two layouts.  Target tiles: a block owns a tile of
- * target cells and sums all their groups in LDS before one store (a tile too
- * long for one block is split and its parts are added atomically).  Chunks:
- * one block per chunk of <= 512 pairs of one group, results added with FP64
- * atomics.  AUTO (P <= 12) uses tiles (measured faster at every order and
- * precision: the chunks' atomics cost more than the tiles' operator reads); GROUPED
- * always uses chunks, TILES always tiles; all repeat to rounding.  The m2l_path
- * of fmm_stats reports TILES or GROUPED for the layout taken.  TARGET: one wavefront per
- * target cell on vector ALUs (fixed summation order, bitwise repeatable; any
- * P).  Pairs whose offset does not fit a group run per target in every mode. */
+/* M2L execution.  Pairs are grouped by offset in two layouts.  Target tiles:
+ * a wavefront owns a few target cells and sums their pairs in LDS, each pair
+ * translated by rotating its offset onto the z axis, shifting and rotating
+ * back (a long tile is split and its parts are added atomically).  Chunks:
+ * one block per chunk of <= 512 pairs of one group, which share one dense
+ * operator, results added with FP64 atomics.  AUTO (P <= 12) uses tiles
+ * (measured faster); GROUPED always uses chunks, TILES always tiles; all
+ * repeat to rounding.  The m2l_path of fmm_stats reports TILES or GROUPED for
+ * the layout taken.  TARGET: one wavefront per target cell on vector ALUs
+ * (fixed summation order, bitwise repeatable; any P).  Pairs whose offset
+ * does not fit a group run per target in every mode. */
 typedef enum { FMM_M2L_AUTO = 0, FMM_M2L_TARGET = 1, FMM_M2L_GROUPED = 2, FMM_M2L_TILES = 3 } fmm_m2l_mode;
 
 /* The knobs of exafmm-beta's Kernel / Traversal / BuildTree constructors and
@@ -209,8 +206,10 @@ int fmm_plan_from_tree(fmm_plan **out, int n, const double *x, int ncell, const 
                        int why_len);
 
 /* Precompute the plan's M2L offset groups for a context of this precision
- * (FMM_FP64: by offset; FMM_MIXED: by offset and the two levels), so that a
- * context given the plan does no grouping work itself.  Host only. */
+ * (FMM_FP64: by offset, as target tiles take them in every precision;
+ * FMM_MIXED: by offset and the two levels, as GROUPED takes them in mixed
+ * precision), so that a context given the plan does no grouping work itself.
+ * Host only. */
 int fmm_plan_build_groups(fmm_plan *pl, int precision);
 
 /* Everything a context with parameters p needs from the host for its M2L
@@ -348,12 +347,10 @@ int fmm_get_lists(fmm_ctx *c, int *m2l_ptr, int *m2l_src, int *p2p_ptr, int *p2p
  * slots overlap on the GPU.  By default a batch holds one request: a batch of
  * several is merged, then grouped on the host, which measured slower than
  * more slots working at once.  With m2l_mode AUTO the loop's M2L runs on
- * target tiles when batches hold one request (a slot's upload builds their
- * groups on the device; the builders plan tree and lists only), and as
- * grouped chunks when they may hold several.  A system's result does not
- * depend on its batch beyond the order of FP64 atomic additions into its
- * local expansions (for mixed precision on explicit FMM_M2L_TILES with
- * batches of several requests it does, at about 1e-8). */
+ * target tiles: when batches hold one request a slot's upload builds their
+ * groups on the device and the builders plan tree and lists only, else the
+ * builders build them too.  A system's result does not depend on its batch
+ * beyond the order of FP64 atomic additions into its local expansions. */
 typedef struct fmm_server fmm_server;
 
 typedef struct {

@@ -1,0 +1,76 @@
+"""The target-tile M2L (rotate, shift, rotate back) at the sizes where its
+layout changes: every order it takes (P = 2..12: one to three tiles of four
+degrees, with and without a shared last row), tiles stored whole and split
+over work items, reflections (the lattice holds offsets along every axis) and
+periodic images.
+Against the per-target kernel, which evaluates each pair's harmonics directly,
+on the same multipoles: both are FP64 sums of the same terms, a few hundred
+per coefficient with condition numbers below 1e2, so they agree to 1e-12."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _F():
+    import exafmm_amd
+    return exafmm_amd
+
+
+def _locals(F, x, q, mode, **kw):
+    with F.FMM(m2l_mode=mode, nspawn=1000, **kw) as f:
+        f.set_bodies(x, q)
+        f.upward()
+        f.m2l()
+        f.synchronize()
+        return f.expansions()[1], f.stats()
+
+
+def _check(F, x, q, **kw):
+    t, st = _locals(F, x, q, F.M2L_TILES, **kw)
+    r, _ = _locals(F, x, q, F.M2L_TARGET, **kw)
+    assert st["m2l_path"] == F.M2L_TILES and st["m2l_pairs"] > 0 and st["m2l_ungrouped"] == 0
+    assert np.all(np.isfinite(t.view(np.float64)))
+    # per degree: the coefficients of different degrees differ by many orders
+    P = kw["P"]
+    for n in range(P):
+        u = slice(n * (n + 1) // 2, (n + 1) * (n + 2) // 2)
+        assert np.linalg.norm(t[:, u] - r[:, u]) <= 1e-12 * np.linalg.norm(r[:, u]), n
+
+
+@pytest.mark.parametrize("P", range(2, 13))
+@pytest.mark.parametrize("dist,n,ncrit", [("cube1", 200, 8), ("plummer1", 3001, 16)])
+def test_every_order_matches_per_target(P, dist, n, ncrit):
+    F = _F()
+    x, q = F.make_bodies(n, dist, P)
+    _check(F, x, q, P=P, theta=0.5, ncrit=ncrit)
+
+
+@pytest.mark.parametrize("P", [5, 8, 9, 10, 12])
+def test_periodic_images_match_per_target(P):
+    F = _F()
+    rng = np.random.default_rng(P)
+    x = rng.random((1500, 3)) - 0.5
+    q = rng.random(1500) - 0.5
+    _check(F, x, q, P=P, theta=0.4, ncrit=32, images=1, cycle=1.0)
+
+
+def test_device_plan_of_another_order():
+    """a device-built plan holds the tiles of its context's order; a context
+    of another order builds its own"""
+    F = _F()
+    x, q = F.make_bodies(5000, "cube1", 1)
+    with F.FMM(P=10) as a, F.FMM(P=8) as b:
+        plan = F.Plan(x, lists_on=a)
+        b.set_bodies_plan(plan, q)
+        b.evaluate()
+        t = b.targets()
+        plan.prepare(P=8)
+        b.set_bodies_plan(plan, q)
+        b.evaluate()
+        t2 = b.targets()
+        b.set_bodies(x, q)
+        b.evaluate()
+        r = b.targets()
+    for v in (t, t2):
+        assert np.all(np.linalg.norm(v - r, axis=0) <= 1e-12 * np.linalg.norm(r, axis=0))
