@@ -92,14 +92,13 @@ struct fmm_ctx {
   fmm::M2LGroups groups;
   DBuf g_tgt, g_src, g_dx, g_chunk, r_ptr, r_src, r_tgt;
   DBuf t_tgt, t_ptr, t_slice, t_src, t_lt, g_ops, c_dx;
-  // M2M / L2L as per-level operators on MFMA (regular trees)
+  // M2M / L2L by rotation, one record per child level (regular trees)
   bool xl = false;
-  std::vector<int> xl_tptr;  // per child level: first L2L tile
-  DBuf xl_child8, xl_children, xl_tiles, xl_ops, xl_frag, xl_dx, xl_kinds;
+  DBuf xl_child8, xl_kids, xl_dx, xl_m2m, xl_l2l;  // children by octant; L2L {child, parent | octant}; records
   // periodic images: shift unit per image, far-image operator F (images >= 2)
   double3 cyc = {0.0, 0.0, 0.0};
   bool far = false;
-  DBuf per_F, per_T, per_S, per_cur, per_tmp, per_dx, per_kind;
+  DBuf per_F, per_T, per_S, per_cur, per_tmp, per_dx;
   // mixed precision: per-group (R_s, R_t), cell radii, FP32 multipoles
   bool mixed = false;
   DBuf g_sc, cr, M32;
@@ -403,7 +402,7 @@ namespace {
 // the M2L of these parameters runs on target tiles (offset groups that do not
 // fix the levels, whatever the precision), else on chunks (MIXED: by level)
 bool takes_tiles(const fmm_params &p) {
-  return (p.m2l_mode == FMM_M2L_TILES || p.m2l_mode == FMM_M2L_AUTO) && fmmdev::m2l_rot_supported(p.P);
+  return (p.m2l_mode == FMM_M2L_TILES || p.m2l_mode == FMM_M2L_AUTO) && fmmdev::rot_supported(p.P);
 }
 bool uniform_levels(const fmm::Tree &t) {  // every radius R0 / 2^level
   for (int k = 0; k < t.ncell; k++)
@@ -906,7 +905,7 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
   UP(p2p_ptr, L.p2p_ptr) UP(p2p_tgt, p2p_order)
   // M2M / L2L operators: every level's radius uniform and every child at
   // X_parent + R_child (+-1, +-1, +-1) (up to rounding of the centres)
-  c->xl = fmmdev::xlate_mfma_supported(c->p.P) && nc > 1;
+  c->xl = fmmdev::rot_supported(c->p.P) && nc > 1;
   std::vector<double> lrad(t.depth + 1, -1.0);
   for (int k = 0; k < nc && c->xl; k++) {
     const int l = t.level[k];
@@ -930,39 +929,16 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
       const int pc = internal[i];
       for (int k = t.ichild[pc]; k < t.ichild[pc] + t.nchild[pc]; k++) child8[8 * i + octant(k)] = k;
     }
-    // L2L tiles: each level's children grouped by octant, 16 per tile
-    std::vector<int> children, tiles;
-    c->xl_tptr.assign(t.depth + 2, 0);
-    for (int l = 1; l <= t.depth; l++) {
-      c->xl_tptr[l] = (int)(tiles.size() / 4);
-      for (int o = 0; o < 8; o++) {
-        const int first = (int)children.size();
-        for (int k = t.level_ptr[l]; k < t.level_ptr[l + 1]; k++) {
-          const int cell = t.level_cells[k];
-          if (octant(cell) == o) children.push_back(cell);
-        }
-        for (int b = first; b < (int)children.size(); b += 16)
-          tiles.insert(tiles.end(), {o, b, std::min(16, (int)children.size() - b), 0});
-      }
+    // L2L: every level's cells (level order) with their parent and octant
+    std::vector<int> kids(2 * (size_t)nc, 0);
+    for (int i = t.level_ptr[1]; i < nc; i++) {
+      const int k = t.level_cells[i];
+      kids[2 * (size_t)i] = k;
+      kids[2 * (size_t)i + 1] = t.iparent[k] | octant(k) << 27;
     }
-    c->xl_tptr[t.depth + 1] = (int)(tiles.size() / 4);
-    // operators: M2M for parent levels 0..depth-1, L2L for child levels 1..depth
-    const int nop = 16 * (t.depth + 1);
-    std::vector<double> dxs(3 * (size_t)nop, 0.0);
-    std::vector<int> kinds(nop, 0);
-    for (int l = 0; l <= t.depth; l++)
-      for (int o = 0; o < 8; o++) {
-        const int m = l * 8 + o, q = 8 * (t.depth + 1) + l * 8 + o;
-        kinds[q] = 1;
-        for (int d = 0; d < 3; d++) {
-          const double s = (o >> d) & 1 ? 1.0 : -1.0;
-          if (l < t.depth && lrad[l + 1] > 0) dxs[3 * (size_t)m + d] = -s * lrad[l + 1];  // X_parent - X_child
-          if (lrad[l] > 0) dxs[3 * (size_t)q + d] = s * lrad[l];                         // X_child - X_parent
-        }
-        if (l == t.depth || lrad[l + 1] < 0) dxs[3 * (size_t)m] = 1.0;  // unused operator: any finite offset
-        if (l == 0) dxs[3 * (size_t)q] = 1.0;
-      }
-    UP(xl_child8, child8) UP(xl_children, children) UP(xl_tiles, tiles) UP(xl_dx, dxs) UP(xl_kinds, kinds)
+    std::vector<double> dxs;  // child levels 1 .. depth
+    for (int l = 1; l <= t.depth; l++) dxs.insert(dxs.end(), 3, lrad[l]);
+    UP(xl_child8, child8) UP(xl_kids, kids) UP(xl_dx, dxs)
   }
   c->mixed = c->p.precision == FMM_MIXED || c->p.precision == FMM_MIXED16;
   c->use_mfma = c->p.m2l_mode != FMM_M2L_TARGET && L.nm2l > 0 &&
@@ -1064,12 +1040,10 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
         (rc = ensure(c, c->per_cur, mb)) || (rc = ensure(c, c->per_tmp, mb)))
       return rc;
     const int nmax = (nb * nb * nb - 1) * nb * nb * nb;
-    if ((rc = ensure(c, c->per_dx, sizeof(double) * 3 * nmax)) || (rc = ensure(c, c->per_kind, sizeof(int) * nmax)))
-      return rc;
+    if ((rc = ensure(c, c->per_dx, sizeof(double) * 3 * nmax))) return rc;
     HIPCHK(hipMemsetAsync(c->per_F.p, 0, mb, c->st));
     HIPCHK(hipMemsetAsync(c->per_cur.p, 0, mb, c->st));
     HIPCHK(fmmdev::launch_add_identity(c->per_cur.as<double>(), PP, c->st));
-    HIPCHK(hipMemsetAsync(c->per_kind.p, 0, sizeof(int) * nmax, c->st));  // kind 0: M2M
     double cyc[3] = {c->p.cycle[0], c->p.cycle[1], c->p.cycle[2]};
     std::vector<double> dl, ds;
     for (int lev = 0; lev < c->p.images - 1; lev++) {
@@ -1098,8 +1072,7 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
       HIPCHK(hipStreamSynchronize(c->st));  // dl is reused below
       HIPCHK(hipMemcpyAsync(c->per_dx.p, ds.data(), sizeof(double) * ds.size(), hipMemcpyHostToDevice, c->st));
       HIPCHK(hipMemsetAsync(c->per_S.p, 0, mb, c->st));
-      HIPCHK(fmmdev::launch_xlate_ops(P, c->per_dx.as<double>(), c->per_kind.as<int>(), ns, c->per_S.as<double>(), 1,
-                                      c->st));
+      HIPCHK(fmmdev::launch_m2m_op_accum(P, c->per_dx.as<double>(), ns, c->per_S.as<double>(), c->st));
       HIPCHK(fmmdev::launch_add_identity(c->per_S.as<double>(), PP, c->st));
       HIPCHK(fmmdev::launch_matmul(c->per_S.as<double>(), c->per_cur.as<double>(), c->per_tmp.as<double>(), PP, 0,
                                    c->st));
@@ -1108,18 +1081,16 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
       for (int d = 0; d < 3; d++) cyc[d] *= nb;
     }
   }
-  if (c->xl) {  // the per-level M2M / L2L operators, once per plan
-    const int nop = 16 * (t.depth + 1);
-    if ((rc = ensure(c, c->xl_ops, sizeof(double) * fmmdev::xlate_op_stride(c->p.P) * nop))) return rc;
-    HIPCHK(fmmdev::launch_xlate_ops(c->p.P, c->xl_dx.as<double>(), c->xl_kinds.as<int>(), nop,
-                                    c->xl_ops.as<double>(), 0, c->st));
-    if ((rc = ensure(c, c->xl_frag, sizeof(double) * fmmdev::xlate_frag_stride(c->p.P) * nop))) return rc;
-    HIPCHK(fmmdev::launch_ops_to_frag(c->p.P, c->xl_ops.as<double>(), nop, c->xl_frag.as<double>(), c->st));
+  if (c->xl) {  // the per-level M2M / L2L records, once per plan
+    const size_t b = fmmdev::rot_ops_bytes(c->p.P) * t.depth;
+    if ((rc = ensure(c, c->xl_m2m, b)) || (rc = ensure(c, c->xl_l2l, b))) return rc;
+    HIPCHK(fmmdev::launch_rot_ops(c->p.P, 1, c->xl_dx.as<double>(), t.depth, c->xl_m2m.p, c->st));
+    HIPCHK(fmmdev::launch_rot_ops(c->p.P, 2, c->xl_dx.as<double>(), t.depth, c->xl_l2l.p, c->st));
   }
   if (c->use_tiles) {  // the operators of every representative offset, once per plan
     const int nr = c->groups.ncanon;
     if ((rc = ensure(c, c->g_ops, fmmdev::rot_ops_bytes(c->p.P) * nr))) return rc;
-    HIPCHK(fmmdev::launch_rot_ops(c->p.P, c->c_dx.as<double>(), nr, c->g_ops.p, c->st));
+    HIPCHK(fmmdev::launch_rot_ops(c->p.P, 0, c->c_dx.as<double>(), nr, c->g_ops.p, c->st));
   }
   double t4 = now_ms();
   pl.tree = fmm::Tree();
@@ -1237,12 +1208,12 @@ int fmm_upward(fmm_ctx *c) {
   auto C = dev_cells(c);
   HIPCHK(fmmdev::launch_p2m(P, dev_bodies(c), C, c->leaves.as<int>(), (int)c->tree.leaves.size(),
                             c->M.as<double2>(), c->st));
-  const size_t os = fmmdev::xlate_frag_stride(P);
+  const size_t rb = fmmdev::rot_ops_bytes(P);
   for (int l = c->tree.depth; l >= 0; l--) {
     const int b = c->internal_ptr[l], e = c->internal_ptr[l + 1];
     if (e > b && c->xl)
-      HIPCHK(fmmdev::launch_m2m_mfma(P, c->internal.as<int>() + b, c->xl_child8.as<int>() + 8 * (size_t)b, e - b,
-                                     c->xl_frag.as<double>() + os * 8 * l, c->M.as<double2>(), c->st));
+      HIPCHK(fmmdev::launch_m2m_rot(P, c->internal.as<int>() + b, c->xl_child8.as<int>() + 8 * (size_t)b, e - b,
+                                    c->xl_m2m.as<char>() + rb * l, c->M.as<double2>(), c->st));
     else if (e > b)
       HIPCHK(fmmdev::launch_m2m(P, C, c->internal.as<int>() + b, e - b, c->M.as<double2>(), c->st));
   }
@@ -1321,15 +1292,12 @@ int fmm_downward(fmm_ctx *c) {
   if (c->tree.ncell == 0) return FMM_OK;
   const int P = c->p.P;
   auto C = dev_cells(c);
-  const size_t os = fmmdev::xlate_frag_stride(P);
+  const size_t rb = fmmdev::rot_ops_bytes(P);
   for (int l = 1; l <= c->tree.depth; l++) {
     const int b = c->level_ptr[l], e = c->level_ptr[l + 1];
     if (c->xl) {
-      const int t0 = c->xl_tptr[l], t1 = c->xl_tptr[l + 1];
-      if (t1 > t0)
-        HIPCHK(fmmdev::launch_l2l_mfma(P, c->xl_tiles.as<int4>() + t0, t1 - t0, c->xl_children.as<int>(),
-                                       c->iparent.as<int>(), c->xl_frag.as<double>() + os * (8 * (c->tree.depth + 1) + 8 * l),
-                                       c->L.as<double2>(), c->st));
+      HIPCHK(fmmdev::launch_l2l_rot(P, c->xl_kids.as<int2>() + b, e - b, c->xl_l2l.as<char>() + rb * (l - 1),
+                                    c->L.as<double2>(), c->st));
     } else if (e > b) {
       HIPCHK(fmmdev::launch_l2l(P, C, c->level_cells.as<int>() + b, e - b, c->L.as<double2>(), c->st));
     }

@@ -71,38 +71,28 @@ hipError_t launch_l2p(int P, DevBodies B, DevCells C, const int *body_leaf, int 
 // (rot_ops_bytes(P) each) from its offset with non-negative components.  A
 // tile in one item stores its targets' L, a split tile adds into L (which
 // must start at zero).
-bool m2l_rot_supported(int P);
+bool rot_supported(int P);
 int m2l_tile_targets(int P);
 constexpr int kM2LSlicePairs = 4;
 size_t rot_ops_bytes(int P);
 hipError_t init_rot_constants();
-hipError_t launch_rot_ops(int P, const double *cdx, int nrep, void *ops, hipStream_t s);
+hipError_t launch_rot_ops(int P, int kind, const double *cdx, int nrep, void *ops, hipStream_t s);
 hipError_t launch_m2l_rot(int P, int nitem, const int *ttgt, const int4 *items, const int4 *slices, const int *psrc,
                           const unsigned short *plt, const void *ops, const double2 *M, double2 *L, hipStream_t s);
-// M2M / L2L as per-level dense operators on MFMA (8 child offsets per level):
-// ops built once per plan (kind 0 M2M with dX = X_parent - X_child, 1 L2L
-// with dX = X_child - X_parent; xlate_op_stride(P) doubles each)
-bool xlate_mfma_supported(int P);
-int xlate_op_stride(int P);
-// the operators in MFMA A-operand order (what m2m_mfma / l2l_mfma read);
-// xlate_frag_stride(P) doubles each
-int xlate_frag_stride(int P);
-hipError_t launch_ops_to_frag(int P, const double *ops, int nop, double *frag, hipStream_t s);
-// accum != 0: sum of all operators into ops (row stride P^2, no padding)
-hipError_t launch_xlate_ops(int P, const double *dxs, const int *kinds, int nop, double *ops, int accum,
-                            hipStream_t s);
+// M2M and L2L of one level the same way, on one record of the level's child
+// offset (h, h, h) (launch_rot_ops kind 1 M2M, 2 L2L; kind 0 M2L).  child8[8 i +
+// octant]: children of parents[i] (-1: none); kids[k] = {child, parent | octant << 27}
+hipError_t launch_m2m_rot(int P, const int *parents, const int *child8, int np, const void *rec, double2 *M,
+                          hipStream_t s);
+hipError_t launch_l2l_rot(int P, const int2 *kids, int nk, const void *rec, double2 *L, hipStream_t s);
+// S += sum of the M2M operators of the n offsets dxs (dense P^2 x P^2, X_parent - X_child)
+hipError_t launch_m2m_op_accum(int P, const double *dxs, int n, double *S, hipStream_t s);
 // periodic far images: T += sum of the M2L operators of the n offsets dxs
 // (P^2 x P^2, row-major), dense products, and L(root) += F v(M(root))
 hipError_t launch_m2l_op_accum(int P, const double *dxs, int n, double *T, hipStream_t s);
 hipError_t launch_matmul(const double *A, const double *B, double *C, int n, int acc, hipStream_t s);
 hipError_t launch_add_identity(double *A, int n, hipStream_t s);
 hipError_t launch_periodic_far(int P, const double *F, const double2 *M, double2 *L, hipStream_t s);
-// parents of one level in tiles of 16; child8[i*8 + octant] (-1: none)
-hipError_t launch_m2m_mfma(int P, const int *parents, const int *child8, int np, const double *ops8, double2 *M,
-                           hipStream_t s);
-// tiles {octant, first, count <= 16} of one level's children grouped by octant
-hipError_t launch_l2l_mfma(int P, const int4 *tiles, int ntile, const int *children, const int *iparent,
-                           const double *ops8, double2 *L, hipStream_t s);
 // mixed precision (FP32 list phases): M32 = M~ / R^n per cell; grouped FP32-MFMA
 // M2L with per-group scales (R_s, R_t) accumulating into the FP64 L; FP32 P2P
 bool m2l_mixed_supported(int P);

@@ -284,63 +284,19 @@ __global__ __launch_bounds__(64) void l2l_kernel(DevCells C, const int *__restri
   }
 }
 
-// ---------------------------------------------------------------- M2M / L2L on MFMA
-// Children sit at X_parent + R_child (+-1, +-1, +-1), so a level has only 8
-// translations each way.  Each is built once per plan as a dense real
-// P^2 x P^2 operator on the expansion vectors (rows n^2 + (m ? 2m-1 : 0), +1
-// for imaginary parts) by applying the scalar M2M / L2L of this file to unit
-// vectors, then applied with v_mfma_f64_16x16x4: M2M to tiles of 16 parents
-// (the 8 octants accumulate in registers, the parent's multipole is stored
-// once), L2L to tiles of 16 children of one octant (added to their locals).
-template <int P> struct XlCfg {
-  static constexpr int PP = P * P;
-  static constexpr int KP = (PP + 3) / 4 * 4;
-  static constexpr int KT = KP / 4;
-  static constexpr int RB = (PP + 15) / 16;
-  static constexpr int NTH = 64 * RB;
-  static constexpr bool ok = P <= 12;
-};
-
-bool xlate_mfma_supported(int P) { return P >= 2 && P <= 12; }
-int xlate_op_stride(int P) { return P * P * ((P * P + 3) / 4 * 4); }  // doubles per operator
-// doubles per operator in MFMA A-operand order: [wavefront][k-step][lane]
-int xlate_frag_stride(int P) { return (P * P + 15) / 16 * ((P * P + 3) / 4) * 64; }
-
-// frag[op][w][kt][lane] = ops[op][16w + lane%16][4kt + lane/16] (0 past P^2):
-// a wavefront loads its A operand of k-step kt as 64 consecutive doubles
+// S += the dense real P^2 x P^2 M2M operators (rows n^2 + (m ? 2m-1 : 0), +1
+// for imaginary parts) of the offsets dxs, one block each: the supercell
+// copies of the periodic images, whose offsets are not a level's
 template <int P>
-__global__ __launch_bounds__(256) void ops_to_frag_kernel(const double *__restrict__ ops, int nop,
-                                                          double *__restrict__ frag) {
-  using Cfg = XlCfg<P>;
-  constexpr int PP = Cfg::PP, KP = Cfg::KP, KT = Cfg::KT, RB = Cfg::RB;
-  constexpr int FS = RB * KT * 64;
-  const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (e >= (size_t)nop * FS) return;
-  const int op = (int)(e / FS), r = (int)(e % FS);
-  const int w = r / (KT * 64), kt = (r / 64) % KT, l = r % 64;
-  const int row = w * 16 + (l & 15), col = kt * 4 + (l >> 4);
-  frag[e] = (row < PP && col < PP) ? ops[(size_t)op * PP * KP + (size_t)row * KP + col] : 0.0;
-}
-
-// operator `op` of kind 0 (M2M, dX = X_parent - X_child) or 1 (L2L, dX =
-// X_child - X_parent); ops[op][row][col], col padded to KP (zeros)
-// accum: every operator is added (atomically) into ops[0] with row stride PP
-// instead (a sum of translations, e.g. the supercell M2M of the periodic images)
-template <int P>
-__global__ __launch_bounds__(256) void xlate_ops_kernel(const double *__restrict__ dxs, const int *__restrict__ kinds,
-                                                        int nop, double *__restrict__ ops, int accum) {
-  constexpr int NT = nterm(P), PP = P * P, KP0 = (PP + 3) / 4 * 4;
-  const int KP = accum ? PP : KP0;
+__global__ __launch_bounds__(256) void m2m_op_accum_kernel(const double *__restrict__ dxs, int n,
+                                                           double *__restrict__ S) {
+  constexpr int NT = nterm(P), PP = P * P;
   __shared__ double2 T[P * P];
   const int op = blockIdx.x, tid = threadIdx.x;
-  if (op >= nop) return;
+  if (op >= n) return;
   const double dx = dxs[3 * op], dy = dxs[3 * op + 1], dz = dxs[3 * op + 2];
   if (tid < P) regular_column<P>(dx, dy, dz, tid, T);
   __syncthreads();
-  const int kind = kinds[op];
-  double *A = accum ? ops : ops + (size_t)op * PP * KP;
-  if (KP > PP)
-    for (int e = tid; e < PP * (KP - PP); e += 256) A[(e / (KP - PP)) * KP + PP + e % (KP - PP)] = 0.0;
   for (int e = tid; e < PP * NT; e += 256) {
     const int col = e / NT, u = e - col * NT;
     const int dc = c_vdec[col];
@@ -350,199 +306,21 @@ __global__ __launch_bounds__(256) void xlate_ops_kernel(const double *__restrict
     auto in = [&](int idx) { return idx == uin ? v : make_double2(0.0, 0.0); };
     int j, k;
     tdecode(u, j, k);
-    double2 a = make_double2(0.0, 0.0);
-    if (kind == 0) {  // the scalar M2M of m2m_kernel with a unit child multipole
-      for (int n = 0; n <= j; n++) {
-        const double sn = sgn(n);
-        for (int m = -n; m <= min(k - 1, n); m++)
-          if (j - n >= k - m) {
-            const double2 Rc = (m >= 0) ? cconj(T[n * P + m]) : T[n * P - m];
-            const double f = (m >= 0) ? sn : sn * sgn(m);
-            a = cmac(a, cscale(Rc, f), in(tidx(j - n, k - m)));
-          }
-        for (int m = k; m <= n; m++)
-          if (j - n >= m - k) a = cmac(a, cscale(cconj(T[n * P + m]), sgn(k + n + m)), cconj(in(tidx(j - n, m - k))));
-      }
-    } else {  // the scalar L2L of l2l_kernel with a unit parent local expansion
-      const double sk = sgn(k);
-      for (int n = j; n < P; n++) {
-        for (int m = j + k - n; m < 0; m++)
-          a = cmac(a, cscale(cconj(in(tidx(n, -m))), sk), cconj(T[(n - j) * P + (k - m)]));
-        for (int m = 0; m <= n; m++) {
-          const int d = m - k;
-          if (n - j >= abs(d)) {
-            const double2 Rx = (d >= 0) ? T[(n - j) * P + d] : cconj(T[(n - j) * P - d]);
-            a = cmac(a, cscale(in(tidx(n, m)), (d >= 0) ? 1.0 : sgn(d)), Rx);
-          }
+    double2 a = make_double2(0.0, 0.0);  // the scalar M2M of m2m_kernel with a unit child multipole
+    for (int n = 0; n <= j; n++) {
+      const double sn = sgn(n);
+      for (int m = -n; m <= min(k - 1, n); m++)
+        if (j - n >= k - m) {
+          const double2 Rc = (m >= 0) ? cconj(T[n * P + m]) : T[n * P - m];
+          const double f = (m >= 0) ? sn : sn * sgn(m);
+          a = cmac(a, cscale(Rc, f), in(tidx(j - n, k - m)));
         }
-      }
+      for (int m = k; m <= n; m++)
+        if (j - n >= m - k) a = cmac(a, cscale(cconj(T[n * P + m]), sgn(k + n + m)), cconj(in(tidx(j - n, m - k))));
     }
     const int row = j * j + (k ? 2 * k - 1 : 0);
-    if (accum) {
-      unsafeAtomicAdd(A + row * KP + col, a.x);
-      if (k) unsafeAtomicAdd(A + (row + 1) * KP + col, a.y);
-    } else {
-      A[row * KP + col] = a.x;
-      if (k) A[(row + 1) * KP + col] = a.y;
-    }
-  }
-}
-
-// M2M for tiles of 16 parents of one level: child8[i][o] = child of parent i
-// in octant o (-1: none); ops8 = the level's 8 M2M operators as fragments
-// (ops_to_frag_kernel).  Overwrites the
-// parents' multipoles.  The next octant's operator rows and children's
-// multipoles are loaded during the current octant's MFMAs.
-template <int P>
-__global__ __launch_bounds__(64 * ((P * P + 15) / 16)) void m2m_mfma_kernel(const int *__restrict__ parents,
-                                                                           const int *__restrict__ child8, int np,
-                                                                           const double *__restrict__ ops8,
-                                                                           double2 *__restrict__ M) {
-  using Cfg = XlCfg<P>;
-  constexpr int NT = nterm(P), PP = Cfg::PP, KP = Cfg::KP, KT = Cfg::KT, NTH = Cfg::NTH;
-  constexpr int IT = (16 * NT + NTH - 1) / NTH;
-  __shared__ double sB[2][KP * 16];
-  __shared__ double sO[Cfg::RB][16 * 17];
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
-  const int i0 = blockIdx.x * 16;
-  for (int e = tid; e < (KP - PP) * 16; e += NTH) {
-    sB[0][PP * 16 + e] = 0.0;
-    sB[1][PP * 16 + e] = 0.0;
-  }
-  const int arow = w * 16 + (l & 15);
-  constexpr int FS = Cfg::RB * KT * 64;  // one operator's fragments
-  const double *opr = ops8 + (size_t)w * KT * 64 + l;
-  double A[KT], An[KT];
-  double2 pre[IT];
-  auto load_a = [&](int o, double *dst) {
-#pragma unroll
-    for (int kt = 0; kt < KT; kt++) dst[kt] = opr[(size_t)o * FS + kt * 64];
-  };
-  // the children of this thread's parents in all 8 octants, loaded up front
-  int ch8[IT][8];
-#pragma unroll
-  for (int it = 0; it < IT; it++) {
-    const int e = tid + NTH * it;
-    const int i = i0 + (e & 15);
-#pragma unroll
-    for (int o = 0; o < 8; o++) ch8[it][o] = (e < 16 * NT && i < np) ? child8[(size_t)i * 8 + o] : -1;
-  }
-  auto gather = [&](int o) {
-#pragma unroll
-    for (int it = 0; it < IT; it++) {
-      const int e = tid + NTH * it;
-      const int u = min(e >> 4, NT - 1);
-      int ch = -1;
-#pragma unroll
-      for (int k = 0; k < 8; k++) ch = k == o ? ch8[it][k] : ch;
-      pre[it] = ch >= 0 ? M[(size_t)ch * NT + u] : make_double2(0.0, 0.0);
-    }
-  };
-  load_a(0, A);
-  gather(0);
-  dbl4 acc = {0.0, 0.0, 0.0, 0.0};
-  for (int o = 0; o < 8; o++) {
-    double *Bt = sB[o & 1];  // last read by octant o - 2, before the barrier of octant o - 1
-#pragma unroll
-    for (int it = 0; it < IT; it++) {
-      const int e = tid + NTH * it;
-      if (e < 16 * NT) {
-        const int c = e & 15, u = e >> 4;
-        const int rr = c_urow[u];
-        Bt[(rr & 0xffff) * 16 + c] = pre[it].x;
-        if ((rr >> 16) != (rr & 0xffff)) Bt[(rr >> 16) * 16 + c] = pre[it].y;
-      }
-    }
-    __syncthreads();
-    if (o < 7) {  // in flight during this octant's MFMAs
-      load_a(o + 1, An);
-      gather(o + 1);
-    }
-    const double *bp = Bt + (l >> 4) * 16 + (l & 15);
-#pragma unroll
-    for (int kt = 0; kt < KT; kt++) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(A[kt], bp[kt * 64], acc, 0, 0, 0);
-    if (o < 7) {
-#pragma unroll
-      for (int kt = 0; kt < KT; kt++) A[kt] = An[kt];
-    }
-  }
-  // D: lane l, element v -> row l/16 + 4v, column l%16; store through LDS so
-  // a lane writes rows of one parent
-  double *O = sO[w];
-#pragma unroll
-  for (int v = 0; v < 4; v++) O[(l & 15) * 17 + (l >> 4) + 4 * v] = acc[v];
-  __syncthreads();
-  if (arow < PP) {
-    const int dr = c_vdec[arow];
-    const int n = dr & 255;
-    const int off = n * (n + 1) + 2 * ((dr >> 8) & 255) + (dr >> 16);
-#pragma unroll
-    for (int cq = 0; cq < 4; cq++) {
-      const int c = cq * 4 + (l >> 4);
-      const int i = i0 + c;
-      if (i < np) {
-        double *dst = reinterpret_cast<double *>(M + (size_t)parents[i] * NT);
-        dst[off] = O[c * 17 + (l & 15)];
-        if (((dr >> 8) & 255) == 0) dst[off + 1] = 0.0;  // Im M[n,0]
-      }
-    }
-  }
-}
-
-// L2L for tiles of 16 children of one octant: tiles[t] = {octant, first, count}
-// into `children`; ops8 = the child level's 8 L2L operators as fragments.  Adds into the
-// children's local expansions.
-template <int P>
-__global__ __launch_bounds__(64 * ((P * P + 15) / 16)) void l2l_mfma_kernel(const int4 *__restrict__ tiles,
-                                                                           const int *__restrict__ children,
-                                                                           const int *__restrict__ iparent,
-                                                                           const double *__restrict__ ops8,
-                                                                           double2 *__restrict__ L) {
-  using Cfg = XlCfg<P>;
-  constexpr int NT = nterm(P), PP = Cfg::PP, KP = Cfg::KP, KT = Cfg::KT, NTH = Cfg::NTH;
-  constexpr int IT = (16 * NT + NTH - 1) / NTH;
-  __shared__ double sB[KP * 16];
-  __shared__ double sO[Cfg::RB][16 * 17];
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
-  const int4 tl = tiles[blockIdx.x];
-  for (int e = tid; e < (KP - PP) * 16; e += NTH) sB[PP * 16 + e] = 0.0;
-  const int arow = w * 16 + (l & 15);
-  double A[KT];
-  const double *op = ops8 + ((size_t)tl.x * Cfg::RB + w) * KT * 64 + l;  // operator fragments
-#pragma unroll
-  for (int kt = 0; kt < KT; kt++) A[kt] = op[kt * 64];
-#pragma unroll
-  for (int it = 0; it < IT; it++) {
-    const int e = tid + NTH * it;
-    if (e < 16 * NT) {
-      const int c = e & 15, u = e >> 4;
-      const double2 v = c < tl.z ? L[(size_t)iparent[children[tl.y + c]] * NT + u] : make_double2(0.0, 0.0);
-      const int rr = c_urow[u];
-      sB[(rr & 0xffff) * 16 + c] = v.x;
-      if ((rr >> 16) != (rr & 0xffff)) sB[(rr >> 16) * 16 + c] = v.y;
-    }
-  }
-  __syncthreads();
-  dbl4 acc = {0.0, 0.0, 0.0, 0.0};
-  const double *bp = sB + (l >> 4) * 16 + (l & 15);
-#pragma unroll
-  for (int kt = 0; kt < KT; kt++) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(A[kt], bp[kt * 64], acc, 0, 0, 0);
-  double *O = sO[w];
-#pragma unroll
-  for (int v = 0; v < 4; v++) O[(l & 15) * 17 + (l >> 4) + 4 * v] = acc[v];
-  __syncthreads();
-  if (arow < PP) {
-    const int dr = c_vdec[arow];
-    const int n = dr & 255;
-    const int off = n * (n + 1) + 2 * ((dr >> 8) & 255) + (dr >> 16);
-#pragma unroll
-    for (int cq = 0; cq < 4; cq++) {
-      const int c = cq * 4 + (l >> 4);
-      if (c < tl.z) {
-        double *dst = reinterpret_cast<double *>(L + (size_t)children[tl.y + c] * NT);
-        dst[off] += O[c * 17 + (l & 15)];
-      }
-    }
+    unsafeAtomicAdd(S + row * PP + col, a.x);
+    if (k) unsafeAtomicAdd(S + (row + 1) * PP + col, a.y);
   }
 }
 
@@ -2126,12 +1904,15 @@ template <int P> struct RunM2LMfma32 {
     }
   }
 };
-template <int P> struct RunXlateOps {
-  static hipError_t run(const double *dxs, const int *kinds, int nop, double *ops, int accum, hipStream_t s) {
-    if (nop > 0) hipLaunchKernelGGL(xlate_ops_kernel<P>, dim3(nop), dim3(256), 0, s, dxs, kinds, nop, ops, accum);
+template <int P> struct RunM2MOpAccum {
+  static hipError_t run(const double *dxs, int n, double *S, hipStream_t s) {
+    if (n > 0) hipLaunchKernelGGL(m2m_op_accum_kernel<P>, dim3(n), dim3(256), 0, s, dxs, n, S);
     return hipGetLastError();
   }
 };
+hipError_t launch_m2m_op_accum(int P, const double *dxs, int n, double *S, hipStream_t s) {
+  return dispatch<RunM2MOpAccum>(P, dxs, n, S, s);
+}
 template <int P> struct RunM2LOpAccum {
   static hipError_t run(const double *dxs, int n, double *T, hipStream_t s) {
     if (n > 0) hipLaunchKernelGGL(m2l_op_accum_kernel<P>, dim3(n), dim3(256), 0, s, dxs, n, T);
@@ -2157,58 +1938,6 @@ hipError_t launch_add_identity(double *A, int n, hipStream_t s) {
 }
 hipError_t launch_periodic_far(int P, const double *F, const double2 *M, double2 *L, hipStream_t s) {
   return dispatch<RunPeriodicFar>(P, F, M, L, s);
-}
-template <int P> struct RunM2MMfma {
-  static hipError_t run(const int *parents, const int *child8, int np, const double *ops8, double2 *M, hipStream_t s) {
-    if constexpr (XlCfg<P>::ok) {
-      if (np > 0)
-        hipLaunchKernelGGL(m2m_mfma_kernel<P>, dim3((np + 15) / 16), dim3(XlCfg<P>::NTH), 0, s, parents, child8, np,
-                           ops8, M);
-      return hipGetLastError();
-    } else {
-      return hipErrorInvalidValue;
-    }
-  }
-};
-template <int P> struct RunL2LMfma {
-  static hipError_t run(const int4 *tiles, int ntile, const int *children, const int *iparent, const double *ops8,
-                        double2 *L, hipStream_t s) {
-    if constexpr (XlCfg<P>::ok) {
-      if (ntile > 0)
-        hipLaunchKernelGGL(l2l_mfma_kernel<P>, dim3(ntile), dim3(XlCfg<P>::NTH), 0, s, tiles, children, iparent,
-                           ops8, L);
-      return hipGetLastError();
-    } else {
-      return hipErrorInvalidValue;
-    }
-  }
-};
-hipError_t launch_xlate_ops(int P, const double *dxs, const int *kinds, int nop, double *ops, int accum,
-                            hipStream_t s) {
-  return dispatch<RunXlateOps>(P, dxs, kinds, nop, ops, accum, s);
-}
-template <int P> struct RunOpsToFrag {
-  static hipError_t run(const double *ops, int nop, double *frag, hipStream_t s) {
-    if constexpr (XlCfg<P>::ok) {
-      const size_t n = (size_t)nop * XlCfg<P>::RB * XlCfg<P>::KT * 64;
-      if (n > 0) hipLaunchKernelGGL(ops_to_frag_kernel<P>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ops,
-                                    nop, frag);
-      return hipGetLastError();
-    } else {
-      return hipErrorInvalidValue;
-    }
-  }
-};
-hipError_t launch_ops_to_frag(int P, const double *ops, int nop, double *frag, hipStream_t s) {
-  return dispatch<RunOpsToFrag>(P, ops, nop, frag, s);
-}
-hipError_t launch_m2m_mfma(int P, const int *parents, const int *child8, int np, const double *ops8, double2 *M,
-                           hipStream_t s) {
-  return dispatch<RunM2MMfma>(P, parents, child8, np, ops8, M, s);
-}
-hipError_t launch_l2l_mfma(int P, const int4 *tiles, int ntile, const int *children, const int *iparent,
-                           const double *ops8, double2 *L, hipStream_t s) {
-  return dispatch<RunL2LMfma>(P, tiles, ntile, children, iparent, ops8, L, s);
 }
 hipError_t launch_m_to_f32(int P, const double2 *M, const double *R, int ncell, float2 *M32, hipStream_t s) {
   return dispatch<RunMToF32>(P, M, R, ncell, M32, s);

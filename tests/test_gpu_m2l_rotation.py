@@ -6,6 +6,8 @@ periodic images.
 Against the per-target kernel, which evaluates each pair's harmonics directly,
 on the same multipoles: both are FP64 sums of the same terms, a few hundred
 per coefficient with condition numbers below 1e2, so they agree to 1e-12."""
+import math
+
 import numpy as np
 import pytest
 
@@ -74,3 +76,55 @@ def test_device_plan_of_another_order():
         r = b.targets()
     for v in (t, t2):
         assert np.all(np.linalg.norm(v - r, axis=0) <= 1e-12 * np.linalg.norm(r, axis=0))
+
+
+def _multipoles(x, q, t, P):
+    """every cell's multipole from its bodies (extended precision)"""
+    LD, CL = np.longdouble, np.clongdouble
+    M = np.zeros((len(t["R"]), P * (P + 1) // 2), CL)
+    xs, qs = x[t["perm"]].astype(LD), q[t["perm"]].astype(LD)
+    for c, (b, n) in enumerate(zip(t["ibody"], t["nbody"])):
+        dx, dy, dz = (xs[b:b + n] - t["X"][c].astype(LD)).T
+        r2 = dx * dx + dy * dy + dz * dz
+        rmm = np.ones(n, CL)
+        for m in range(P):
+            if m > 0:
+                rmm = rmm * (dx + 1j * dy) * (-LD(1) / (2 * m))
+            r0, r1 = np.zeros(n, CL), rmm
+            for k in range(m, P):
+                if k > m:
+                    r0, r1 = r1, (r1 * (2 * k - 1) * dz - r0 * r2) / LD(k * k - m * m)
+                s = np.sqrt(LD(math.factorial(k - m)) * LD(math.factorial(k + m)))
+                M[c, k * (k + 1) // 2 + m] = (qs[b:b + n] * np.conj(r1)).sum() * s
+    return M
+
+
+@pytest.mark.parametrize("P", range(2, 13))
+@pytest.mark.parametrize("n,ncrit", [(90, 8), (2999, 16)])
+def test_m2m_l2l_every_order(P, n, ncrit):
+    """M2M and L2L by rotation: multipoles of every cell against its bodies'
+    (a cell's own P2M; the scalar M2M kernel itself is 1.1e-12 from them at
+    P = 12), local expansions against the scalar L2L, which the same tree given
+    by the caller takes with one radius a part in 1e12 off.  FP64 sums chained
+    over at most 6 levels: 1e-12 per degree."""
+    F = _F()
+    x, q = F.make_bodies(n, "plummer1", P)
+    out = []
+    with F.FMM(P=P, theta=0.5, ncrit=ncrit, m2l_mode=F.M2L_TARGET) as f:
+        f.set_bodies(x, q)
+        t = f.tree()
+        for scale in (1.0, 1.0 + 1e-12):
+            R = t["R"].copy()
+            R[-1] *= scale
+            f.set_tree(x[t["perm"]], q[t["perm"]], {**t, "R": R})
+            f.upward()
+            f.m2l()
+            f.downward()
+            f.synchronize()
+            out.append((f.expansions(), f.lists()))
+    assert all(np.array_equal(a, b) for a, b in zip(out[0][1], out[1][1]))
+    M = _multipoles(x, q, t, P)
+    for a, b in ((out[0][0][0], M), (out[0][0][1], out[1][0][1])):
+        for k in range(P):
+            u = slice(k * (k + 1) // 2, (k + 1) * (k + 2) // 2)
+            assert np.linalg.norm(a[:, u] - b[:, u]) <= 1e-12 * np.linalg.norm(b[:, u]), k
