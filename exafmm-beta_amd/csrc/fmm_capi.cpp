@@ -104,6 +104,7 @@ struct fmm_ctx {
   DBuf g_sc, cr, M32;
   DBuf dip;  // dipole partial sums
   DBuf ew_b, ew_t, ew_k, ew_s;  // fmm_ewald: bodies, targets, wave vectors, structure factors
+  DBuf dir_t, dir_p, dir_o;  // fmm_direct: targets, partial sums, result
   DBuf op_d, op_i;  // fmm_kernel_*: doubles (bodies, centres, expansions) and ints of one call
   // pinned host staging of the upload's large copies (grow-only, hipHostMalloc)
   void *pin = nullptr;
@@ -247,12 +248,6 @@ hipError_t plan_to_host(const fmm_plan *pl) {
   if (e == hipSuccess && m->tiles.TT > 0) e = fmmdev::fetch_tiles(*pl->dev, m->tiles, nullptr);
   if (cur != pl->dev->device) (void)hipSetDevice(cur);
   return e;
-}
-
-void release(DBuf &b) {
-  if (b.p) (void)hipFree(b.p);
-  b.p = nullptr;
-  b.cap = 0;
 }
 
 // drop the captured solve (its nodes point at the device buffers as they were)
@@ -1407,16 +1402,15 @@ int fmm_direct(fmm_ctx *c, int nt, const double *xt, double *trg) {
   std::vector<double> h(3 * (size_t)nt);
   for (int i = 0; i < nt; i++)
     for (int d = 0; d < 3; d++) h[(size_t)d * nt + i] = xt[3 * (size_t)i + d];
-  DBuf tb, ob;
   auto done = [&](int r) {
     (void)hipStreamSynchronize(c->st);
-    release(tb);
-    release(ob);
     return r;
   };
-  if ((rc = upload(c, tb, h.data(), h.size()))) return done(rc);
-  if ((rc = ensure(c, ob, sizeof(double) * 4 * nt))) return done(rc);
-  const double *tx = tb.as<double>();
+  const int runs = fmmdev::direct_runs(c->n, nt);
+  if ((rc = upload(c, c->dir_t, h.data(), h.size()))) return done(rc);
+  if ((rc = ensure(c, c->dir_o, sizeof(double) * 4 * nt))) return done(rc);
+  if (runs > 1 && (rc = ensure(c, c->dir_p, sizeof(double) * 4 * nt * (size_t)runs))) return done(rc);
+  const double *tx = c->dir_t.as<double>();
   // Traversal::direct (include/traversal.h:355-377): images sum the sources
   // over the cube of shifts |i| <= sum_(l < images) neighbor^l
   int prange = 0;
@@ -1425,14 +1419,15 @@ int fmm_direct(fmm_ctx *c, int nt, const double *xt, double *trg) {
     for (int l = 0, pw = 1; l < c->p.images; l++, pw *= neighbor) prange += pw;
   }
   hipError_t e = fmmdev::launch_direct(dev_bodies(c), c->n, tx, tx + nt, tx + 2 * (size_t)nt, nt,
-                                       ob.as<double>(), c->p.eps2, prange, c->cyc, c->st);
+                                       c->dir_p.as<double>(), c->dir_o.as<double>(), c->p.eps2, prange, c->cyc,
+                                       c->st);
   if (e != hipSuccess) {
     c->err = std::string("direct kernel launch failed: ") + hipGetErrorString(e);
     return done(FMM_ERR_DEVICE);
   }
   std::vector<double> o(4 * (size_t)nt);
   e = hipStreamSynchronize(c->st);
-  if (e == hipSuccess) e = hipMemcpy(o.data(), ob.p, o.size() * sizeof(double), hipMemcpyDeviceToHost);
+  if (e == hipSuccess) e = hipMemcpy(o.data(), c->dir_o.p, o.size() * sizeof(double), hipMemcpyDeviceToHost);
   if (e != hipSuccess) {
     c->err = std::string("fmm_direct: ") + hipGetErrorString(e);
     return done(FMM_ERR_DEVICE);

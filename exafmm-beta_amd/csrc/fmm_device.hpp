@@ -210,7 +210,9 @@ hipError_t device_lists(int ncell, const double *X, const double *R, const int *
                         PlanArrays *keep = nullptr);
 hipError_t launch_ewald_scratch(int device, EwBodies B, int n, int ksize, double3 cyc, double alpha, double sigma,
                                 double cutoff, hipStream_t s);
+// part: 4 nt direct_runs(n, nt) doubles (not read when that is one run), out: [4][nt]
+int direct_runs(int n, int nt);
 hipError_t launch_direct(DevBodies B, int n, const double *tx, const double *ty, const double *tz, int nt,
-                         double *out, double eps2, int prange, double3 cyc, hipStream_t s);
+                         double *part, double *out, double eps2, int prange, double3 cyc, hipStream_t s);
 
 }  // namespace fmmdev

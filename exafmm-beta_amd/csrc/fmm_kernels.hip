@@ -1382,57 +1382,93 @@ __global__ __launch_bounds__(256) void periodic_far_kernel(const double *__restr
 }
 
 // ---------------------------------------------------------------- direct
-// Verification sum: one thread per target, sources staged through LDS.  Uses
-// IEEE sqrt and division (not the P2P rsqrt path) so it checks the P2P kernel
-// independently.  out is [4][nt] (pot, ax, ay, az).
+// Verification sum.  Uses IEEE sqrt and division (not the P2P rsqrt path) so it
+// checks the P2P kernel independently.  A block holds 64 targets and a run of
+// `chunk` sources, staged 256 at a time through LDS, a quarter of them (of the
+// images, where there are any) to each of its 4 wavefronts; the quarters are
+// added in order through LDS and the runs by direct_sum_kernel (part: [run][pot, ax, ay, az][nt]; one run writes
+// the result itself).  Bound: FP64 VALU (about 45 instructions a pair).
+// Accuracy checks sum a thousand targets over all bodies: with one thread per
+// target over every source, 1000 targets of 2^20 bodies ran on 4 blocks.
+// Measured there: 190 -> 1.7 ms a call.
 __global__ __launch_bounds__(256) void direct_kernel(DevBodies B, int n, const double *__restrict__ tx,
                                                      const double *__restrict__ ty,
-                                                     const double *__restrict__ tz, int nt,
-                                                     double *__restrict__ out, double eps2, int prange,
+                                                     const double *__restrict__ tz, int nt, int chunk,
+                                                     double *__restrict__ part, double eps2, int prange,
                                                      double3 cyc) {
-  __shared__ double sx[256], sy[256], sz[256], sq[256];
-  const int i = blockIdx.x * 256 + threadIdx.x;
+  __shared__ double4 sb[256];
+  __shared__ double sr[4][4][64];  // [wavefront][component][target]
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int i = blockIdx.x * 64 + l;
   const bool act = i < nt;
   const double xi = act ? tx[i] : 0.0, yi = act ? ty[i] : 0.0, zi = act ? tz[i] : 0.0;
+  const long long first = (long long)blockIdx.y * chunk;
+  const int j0 = (int)min((long long)n, first), j1 = (int)min((long long)n, first + chunk);
   double pot = 0.0, ax = 0.0, ay = 0.0, az = 0.0;
-  for (int j0 = 0; j0 < n; j0 += 256) {
-    const int j = j0 + threadIdx.x;
-    if (j < n) {
-      sx[threadIdx.x] = B.x[j];
-      sy[threadIdx.x] = B.y[j];
-      sz[threadIdx.x] = B.z[j];
-      sq[threadIdx.x] = B.q[j];
+  for (int base = j0; base < j1; base += 256) {
+    const int j = base + threadIdx.x;
+    if (j < j1) sb[threadIdx.x] = make_double4(B.x[j], B.y[j], B.z[j], B.q[j]);
+    __syncthreads();
+    const int cnt = min(256, j1 - base);
+    auto add = [&](double px, double py, double pz, int k0, int k1) {
+      for (int k = k0; k < k1; k++) {
+        const double4 s4 = sb[k];
+        const double dx = px - s4.x, dy = py - s4.y, dz = pz - s4.z;
+        const double r2 = dx * dx + dy * dy + dz * dz + eps2;
+        if (r2 != 0.0) {
+          const double inv2 = 1.0 / r2;
+          const double qr = s4.w * sqrt(inv2);
+          const double q3 = inv2 * qr;
+          pot += qr;
+          ax -= dx * q3;
+          ay -= dy * q3;
+          az -= dz * q3;
+        }
+      }
+    };
+    if (prange == 0) {
+      add(xi, yi, zi, 64 * w, min(64 * w + 64, cnt));
+    } else {
+      // periodic images (Traversal::direct, include/traversal.h:355-377): sources
+      // shifted by (ix, iy, iz) * cycle, |ix|, |iy|, |iz| <= prange, dealt to the
+      // wavefronts; an image's sources stay together (a neutral system's terms
+      // cancel image by image: quarters of them summed apart lost two digits)
+      const int m = 2 * prange + 1;
+      for (long long e = w; e < (long long)m * m * m; e += 4) {
+        const int ix = (int)(e / ((long long)m * m)) - prange, iy = (int)(e / m % m) - prange, iz = (int)(e % m) - prange;
+        add(xi - ix * cyc.x, yi - iy * cyc.y, zi - iz * cyc.z, 0, cnt);
+      }
     }
     __syncthreads();
-    const int cnt = min(256, n - j0);
-    // periodic images (Traversal::direct, include/traversal.h:355-377): sources
-    // shifted by (ix, iy, iz) * cycle, |ix|, |iy|, |iz| <= prange
-    for (int ix = -prange; ix <= prange; ix++)
-      for (int iy = -prange; iy <= prange; iy++)
-        for (int iz = -prange; iz <= prange; iz++) {
-          const double px = xi - ix * cyc.x, py = yi - iy * cyc.y, pz = zi - iz * cyc.z;
-          for (int k = 0; k < cnt; k++) {
-            const double dx = px - sx[k], dy = py - sy[k], dz = pz - sz[k];
-            const double r2 = dx * dx + dy * dy + dz * dz + eps2;
-            if (r2 != 0.0) {
-              const double inv2 = 1.0 / r2;
-              const double qr = sq[k] * sqrt(inv2);
-              const double q3 = inv2 * qr;
-              pot += qr;
-              ax -= dx * q3;
-              ay -= dy * q3;
-              az -= dz * q3;
-            }
-          }
-        }
-    __syncthreads();
   }
-  if (act) {
-    out[i] = pot;
-    out[nt + i] = ax;
-    out[2 * (size_t)nt + i] = ay;
-    out[3 * (size_t)nt + i] = az;
-  }
+  sr[w][0][l] = pot;
+  sr[w][1][l] = ax;
+  sr[w][2][l] = ay;
+  sr[w][3][l] = az;
+  __syncthreads();
+  // wavefront w adds component w
+  if (act)
+    part[((size_t)blockIdx.y * 4 + w) * nt + i] = ((sr[0][w][l] + sr[1][w][l]) + sr[2][w][l]) + sr[3][w][l];
+}
+
+__global__ __launch_bounds__(256) void direct_sum_kernel(const double *__restrict__ part, int runs, int n4,
+                                                         double *__restrict__ out) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  double v = 0.0;
+  for (int r = 0; r < runs; r++) v += part[(size_t)r * n4 + i];
+  out[i] = v;
+}
+
+// sources per run: about 2048 blocks (8 a CU) in all, whole staging buffers
+static int direct_chunk(int n, int nt) {
+  const long long groups = (nt + 63) / 64, runs = std::max(1LL, 2048 / std::max(1LL, groups));
+  const long long c = ((n + runs - 1) / runs + 255) / 256 * 256;
+  return (int)std::max(256LL, std::min(c, 1LL << 30));
+}
+int direct_runs(int n, int nt) {
+  const int c = direct_chunk(n, nt);
+  return n <= 0 ? 1 : (n - 1) / c + 1;
 }
 
 // UpDownPass::getDipole(bodies, X0 = 0) (include/up_down_pass.h:77-86): per-block
@@ -1608,12 +1644,32 @@ __global__ __launch_bounds__(256) void ewald_dft_kernel(EwBodies B, int n, const
   }
 }
 
+// The per-body sums below run kEwT bodies a block, every body's terms dealt to
+// kEwS lanes (slices) and their partial sums added in slice order through LDS:
+// with a thread per body, 24573 bodies filled 96 of the 256 CUs with one
+// wavefront per SIMD (that system, 1500 wave vectors: 12.3 -> 3.9 ms a call).
+constexpr int kEwT = 16, kEwS = 256 / kEwT;
+__device__ __forceinline__ double4 ew_reduce(double4 v, double4 *sr) {  // the total in slice 0's lanes
+  __syncthreads();
+  sr[threadIdx.x] = v;
+  __syncthreads();
+  if (threadIdx.x < kEwT)
+    for (int k = 1; k < kEwS; k++) {
+      const double4 u = sr[threadIdx.x + kEwT * k];
+      v.x += u.x;
+      v.y += u.y;
+      v.z += u.z;
+      v.w += u.w;
+    }
+  return v;
+}
+
 __global__ __launch_bounds__(256) void ewald_idft_kernel(EwBodies B, int n, const int *__restrict__ kv,
                                                          const double2 *__restrict__ S, int nw, double3 cyc,
                                                          double3 scale) {
   __shared__ double4 sw[256];  // kx, ky, kz scaled; re
   __shared__ double si[256];   // im
-  const int i = blockIdx.x * 256 + threadIdx.x;
+  const int i = blockIdx.x * kEwT + threadIdx.x % kEwT, slice = threadIdx.x / kEwT;
   const bool act = i < n;
   const double3 xi = act ? ew_pos(B, i, cyc) : make_double3(0.0, 0.0, 0.0);
   double p = 0.0, gx = 0.0, gy = 0.0, gz = 0.0;
@@ -1625,7 +1681,7 @@ __global__ __launch_bounds__(256) void ewald_idft_kernel(EwBodies B, int n, cons
     }
     __syncthreads();
     const int cnt = min(256, nw - w0);
-    for (int k = 0; k < cnt; k++) {
+    for (int k = slice; k < cnt; k += kEwS) {
       const double4 kw = sw[k];
       double sn, cs;
       sincos(kw.x * xi.x + kw.y * xi.y + kw.z * xi.z, &sn, &cs);
@@ -1638,16 +1694,17 @@ __global__ __launch_bounds__(256) void ewald_idft_kernel(EwBodies B, int n, cons
     }
     __syncthreads();
   }
-  if (act) ew_add(B, i, p, gx, gy, gz);
+  const double4 v = ew_reduce(make_double4(p, gx, gy, gz), sw);
+  if (act && slice == 0) ew_add(B, i, v.x, v.y, v.z, v.w);
 }
 
 // Real part (ewald.h:90-110) over every pair within the cutoff at its minimum
 // image (the sum ewald.h's cell search aims at), and the self term
-// (ewald.h:156-160).
+// (ewald.h:156-160).  Bound: FP64 VALU (erfc and exp).
 __global__ __launch_bounds__(256) void ewald_real_kernel(EwBodies B, int n, double3 cyc, double alpha,
                                                          double cutoff2) {
   __shared__ double4 sb[256];
-  const int i = blockIdx.x * 256 + threadIdx.x;
+  const int i = blockIdx.x * kEwT + threadIdx.x % kEwT, slice = threadIdx.x / kEwT;
   const bool act = i < n;
   const double3 xi = act ? ew_pos(B, i, cyc) : make_double3(0.0, 0.0, 0.0);
   double p = 0.0, gx = 0.0, gy = 0.0, gz = 0.0;
@@ -1660,7 +1717,7 @@ __global__ __launch_bounds__(256) void ewald_real_kernel(EwBodies B, int n, doub
     }
     __syncthreads();
     const int cnt = min(256, n - j0);
-    for (int k = 0; k < cnt; k++) {
+    for (int k = slice; k < cnt; k += kEwS) {
       const double4 s4 = sb[k];
       double dx = xi.x - s4.x, dy = xi.y - s4.y, dz = xi.z - s4.z;
       // vec.h:217-230 wrap of the separation
@@ -1684,7 +1741,8 @@ __global__ __launch_bounds__(256) void ewald_real_kernel(EwBodies B, int n, doub
     }
     __syncthreads();
   }
-  if (act) ew_add(B, i, p - M_2_SQRTPI * B.q[i] * alpha, gx, gy, gz);
+  const double4 v = ew_reduce(make_double4(p, gx, gy, gz), sb);
+  if (act && slice == 0) ew_add(B, i, v.x - M_2_SQRTPI * B.q[i] * alpha, v.y, v.z, v.w);
 }
 
 hipError_t launch_ewald(EwBodies B, int n, int ksize, int *kv, double2 *S, double3 cyc, double alpha,
@@ -1700,11 +1758,11 @@ hipError_t launch_ewald(EwBodies B, int n, int ksize, int *kv, double2 *S, doubl
     hipLaunchKernelGGL(ewald_dft_kernel, dim3(nw), dim3(256), 0, s, B, n, kv, nw, cyc, scale, coef, coef2, S);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(ewald_idft_kernel, dim3((n + 255) / 256), dim3(256), 0, s, B, n, kv, S, nw, cyc, scale);
+    hipLaunchKernelGGL(ewald_idft_kernel, dim3((n + kEwT - 1) / kEwT), dim3(256), 0, s, B, n, kv, S, nw, cyc, scale);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(ewald_real_kernel, dim3((n + 255) / 256), dim3(256), 0, s, B, n, cyc, alpha,
+  hipLaunchKernelGGL(ewald_real_kernel, dim3((n + kEwT - 1) / kEwT), dim3(256), 0, s, B, n, cyc, alpha,
                      cutoff * cutoff);
   return hipGetLastError();
 }
@@ -1740,10 +1798,14 @@ hipError_t launch_ewald_scratch(int device, EwBodies B, int n, int ksize, double
 }
 
 hipError_t launch_direct(DevBodies B, int n, const double *tx, const double *ty, const double *tz,
-                         int nt, double *out, double eps2, int prange, double3 cyc, hipStream_t s) {
-  if (nt > 0)
-    hipLaunchKernelGGL(direct_kernel, dim3((nt + 255) / 256), dim3(256), 0, s, B, n, tx, ty, tz, nt, out,
-                       eps2, prange, cyc);
+                         int nt, double *part, double *out, double eps2, int prange, double3 cyc, hipStream_t s) {
+  if (nt <= 0) return hipSuccess;
+  const int runs = direct_runs(n, nt);
+  hipLaunchKernelGGL(direct_kernel, dim3((nt + 63) / 64, runs), dim3(256), 0, s, B, n, tx, ty, tz, nt,
+                     direct_chunk(n, nt), runs > 1 ? part : out, eps2, prange, cyc);
+  if (runs > 1)
+    hipLaunchKernelGGL(direct_sum_kernel, dim3((unsigned)(((size_t)nt * 4 + 255) / 256)), dim3(256), 0, s, part, runs,
+                       4 * nt, out);
   return hipGetLastError();
 }
 
