@@ -109,6 +109,8 @@ struct fmm_ctx {
   // pinned host staging of the upload's large copies (grow-only, hipHostMalloc)
   void *pin = nullptr;
   size_t pin_cap = 0;
+  DBuf trg;               // targets as the caller takes them (n x 4)
+  hipEvent_t dl_ev[8] = {};  // one per thread of download_staged
 };
 
 struct fmm_plan {
@@ -176,6 +178,33 @@ int dcopy(fmm_ctx *c, DBuf &b, const fmmdev::DevArray &a) {
   return FMM_OK;
 }
 
+// f(0) .. f(n - 1), each on a host thread of its own (on this one where none
+// could be started)
+template <typename F>
+void on_threads(int n, F f) {
+  std::vector<std::thread> th;
+  int started = 1;
+  try {
+    for (; started < n; started++) th.emplace_back(f, started);
+  } catch (const std::exception &) {
+  }
+  if (n > 0) f(0);
+  for (int t = started; t < n; t++) f(t);
+  for (auto &h : th) h.join();
+}
+
+// grow the context's pinned staging
+int pin_at_least(fmm_ctx *c, size_t bytes) {
+  if (bytes <= c->pin_cap) return FMM_OK;
+  HIPCHK(hipStreamSynchronize(c->st));  // its copies use the old one
+  if (c->pin) HIPCHK(hipHostFree(c->pin));
+  c->pin = nullptr;
+  c->pin_cap = 0;
+  HIPCHK(hipHostMalloc(&c->pin, bytes, hipHostMallocDefault));
+  c->pin_cap = bytes;
+  return FMM_OK;
+}
+
 // host arrays (pointer, bytes) to device buffers through the context's pinned
 // staging: the arrays are packed into it by host threads (large sizes), then
 // copied by DMA from pinned memory, which runs several times the rate of a
@@ -186,11 +215,8 @@ int upload_staged(fmm_ctx *c, std::initializer_list<std::tuple<DBuf *, const voi
   size_t total = 0;
   for (const auto &pt : parts) total += (std::get<2>(pt) + 255) / 256 * 256;
   if (total > c->pin_cap) {
-    if (c->pin) HIPCHK(hipHostFree(c->pin));
-    c->pin = nullptr;
-    c->pin_cap = 0;
-    HIPCHK(hipHostMalloc(&c->pin, total + total / 4, hipHostMallocDefault));
-    c->pin_cap = total + total / 4;
+    const int rc = pin_at_least(c, total + total / 4);
+    if (rc) return rc;
   }
   // pack: runs of about 16 MB per host thread
   std::vector<std::tuple<char *, const char *, size_t>> runs;
@@ -203,16 +229,9 @@ int upload_staged(fmm_ctx *c, std::initializer_list<std::tuple<DBuf *, const voi
     off += (b + 255) / 256 * 256;
   }
   const int nth = (int)std::min<size_t>(runs.size(), 8);
-  if (nth > 1) {
-    std::vector<std::thread> th;
-    for (int t = 0; t < nth; t++)
-      th.emplace_back([&, t] {
-        for (size_t r = t; r < runs.size(); r += nth) std::memcpy(std::get<0>(runs[r]), std::get<1>(runs[r]), std::get<2>(runs[r]));
-      });
-    for (auto &h : th) h.join();
-  } else {
-    for (auto &r : runs) std::memcpy(std::get<0>(r), std::get<1>(r), std::get<2>(r));
-  }
+  on_threads(nth, [&](int t) {
+    for (size_t r = t; r < runs.size(); r += nth) std::memcpy(std::get<0>(runs[r]), std::get<1>(runs[r]), std::get<2>(runs[r]));
+  });
   off = 0;
   for (const auto &pt : parts) {
     const size_t b = std::get<2>(pt);
@@ -221,6 +240,34 @@ int upload_staged(fmm_ctx *c, std::initializer_list<std::tuple<DBuf *, const voi
     if (b) HIPCHK(hipMemcpyAsync(std::get<0>(pt)->p, static_cast<char *>(c->pin) + off, b, hipMemcpyHostToDevice, c->st));
     off += (b + 255) / 256 * 256;
   }
+  return FMM_OK;
+}
+
+// device to host memory through the pinned staging, after the stream's work:
+// each of up to 8 host threads takes chunks in turn through a slot of its own
+// (copies of one slot and the host writes of the others overlap; the writes
+// also fault in the caller's pages).  The targets of 2^23 bodies (256 MB into
+// fresh pages): 7.3 ms; four pageable copies and a host loop took 131 ms.
+int download_staged(fmm_ctx *c, void *dst, const void *src, size_t bytes) {
+  const size_t chunk = (size_t)2 << 20;
+  const size_t n = (bytes + chunk - 1) / chunk;
+  const int nth = (int)std::min<size_t>(n, 8);
+  int rc = pin_at_least(c, std::min(bytes, nth * chunk));
+  if (rc) return rc;
+  hipError_t err[8] = {};
+  on_threads(nth, [&](int t) {
+    hipError_t e = hipSetDevice(c->p.device);
+    char *slot = static_cast<char *>(c->pin) + t * chunk;
+    for (size_t k = t; k < n && e == hipSuccess; k += nth) {
+      const size_t o = k * chunk, b = std::min(bytes - o, chunk);
+      e = hipMemcpyAsync(slot, static_cast<const char *>(src) + o, b, hipMemcpyDeviceToHost, c->st);
+      if (e == hipSuccess) e = hipEventRecord(c->dl_ev[t], c->st);
+      if (e == hipSuccess) e = hipEventSynchronize(c->dl_ev[t]);
+      if (e == hipSuccess) std::memcpy(static_cast<char *>(dst) + o, slot, b);
+    }
+    err[t] = e;
+  });
+  for (int t = 0; t < nth; t++) HIPCHK(err[t]);
   return FMM_OK;
 }
 
@@ -361,6 +408,7 @@ int fmm_create(fmm_ctx **out, const fmm_params *p) {
       HIPCHK(hipStreamCreateWithFlags(&c->st2, hipStreamNonBlocking));
       for (auto &e : c->ev) HIPCHK(hipEventCreate(&e));
       for (auto &e : c->kev) HIPCHK(hipEventCreate(&e));
+      for (auto &e : c->dl_ev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
       HIPCHK(hipEventCreateWithFlags(&c->fork, hipEventDisableTiming));
       HIPCHK(hipEventCreateWithFlags(&c->join, hipEventDisableTiming));
       return FMM_OK;
@@ -378,6 +426,8 @@ void fmm_destroy(fmm_ctx *c) {
   for (auto &e : c->ev)
     if (e) (void)hipEventDestroy(e);
   for (auto &e : c->kev)
+    if (e) (void)hipEventDestroy(e);
+  for (auto &e : c->dl_ev)
     if (e) (void)hipEventDestroy(e);
   if (c->st2) (void)hipStreamSynchronize(c->st2);
   if (c->fork) (void)hipEventDestroy(c->fork);
@@ -1022,6 +1072,7 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
   if ((rc = ensure(c, c->ax, sizeof(double) * n))) return rc;
   if ((rc = ensure(c, c->ay, sizeof(double) * n))) return rc;
   if ((rc = ensure(c, c->az, sizeof(double) * n))) return rc;
+  if ((rc = ensure(c, c->trg, sizeof(double) * 4 * (size_t)n))) return rc;
   if ((rc = ensure(c, c->M, sizeof(double2) * NT * nc))) return rc;
   if ((rc = ensure(c, c->L, sizeof(double2) * NT * nc))) return rc;
   if (c->mixed && c->use_mfma && !c->use_tiles && (rc = ensure(c, c->M32, sizeof(float2) * NT * nc))) return rc;
@@ -1186,12 +1237,11 @@ int fmm_set_charges(fmm_ctx *c, const double *q) {
   int rc = check_ready(c);
   if (rc) return rc;
   if (!q && c->n > 0) FMM_FAIL(FMM_ERR_ARG, "fmm_set_charges: NULL q");
-  std::vector<double> hq(c->n);
-  for (int i = 0; i < c->n; i++) hq[i] = q[c->tree.perm[i]];
-  const void *before = c->q.p;
-  if ((rc = upload(c, c->q, hq.data(), hq.size()))) return rc;
-  if (c->q.p != before) graph_reset(c);  // a captured solve reads the charges in place
-  HIPCHK(hipStreamSynchronize(c->st));
+  if (c->n == 0) return FMM_OK;
+  // staged as given, taken into tree order on the device (in the solve's own
+  // charge buffer, which a captured solve reads in place)
+  if ((rc = upload_staged(c, {{&c->qin, q, sizeof(double) * (size_t)c->n}}))) return rc;
+  HIPCHK(fmmdev::launch_gather_charges(c->n, c->perm.as<int>(), c->qin.as<double>(), c->q.as<double>(), c->st));
   return FMM_OK;
 }
 
@@ -1548,21 +1598,10 @@ int fmm_get_targets(fmm_ctx *c, double *trg, int input_order) {
   int rc = check_ready(c);
   if (rc) return rc;
   if (!trg && c->n > 0) FMM_FAIL(FMM_ERR_ARG, "fmm_get_targets: NULL trg");
-  const int n = c->n;
-  std::vector<double> h(4 * (size_t)n);
-  if (n > 0) {  // on the context's stream: other contexts' work is not waited for
-    const size_t b = sizeof(double) * n;
-    HIPCHK(hipMemcpyAsync(h.data(), c->pot.p, b, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipMemcpyAsync(h.data() + n, c->ax.p, b, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipMemcpyAsync(h.data() + 2 * (size_t)n, c->ay.p, b, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipMemcpyAsync(h.data() + 3 * (size_t)n, c->az.p, b, hipMemcpyDeviceToHost, c->st));
-  }
-  HIPCHK(hipStreamSynchronize(c->st));
-  for (int i = 0; i < n; i++) {
-    const size_t o = input_order ? (size_t)c->tree.perm[i] : (size_t)i;
-    for (int k = 0; k < 4; k++) trg[4 * o + k] = h[(size_t)k * n + i];
-  }
-  return FMM_OK;
+  if (c->n == 0) return FMM_OK;
+  HIPCHK(fmmdev::launch_pack_targets(c->n, input_order ? c->perm.as<int>() : nullptr, dev_bodies(c),
+                                     c->trg.as<double>(), c->st));
+  return download_staged(c, trg, c->trg.p, sizeof(double) * 4 * (size_t)c->n);
 }
 
 int fmm_get_expansions(fmm_ctx *c, double *M, double *L) {

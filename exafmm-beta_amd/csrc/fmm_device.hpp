@@ -36,6 +36,10 @@ hipError_t launch_zero(double *p, size_t n, hipStream_t s);
 // and qin
 hipError_t launch_gather_bodies(int n, const int *perm, const double *xin, const double *qin, double *x, double *y,
                                 double *z, double *q, hipStream_t s);
+// q[i] = qin[perm[i]]; trg[4 o .. 4 o + 3] = body i's potential and gradient, o =
+// perm[i] (i when perm is null)
+hipError_t launch_gather_charges(int n, const int *perm, const double *qin, double *q, hipStream_t s);
+hipError_t launch_pack_targets(int n, const int *perm, DevBodies B, double *trg, hipStream_t s);
 // body_leaf[i] = the leaf holding body i (tree order)
 hipError_t launch_body_leaf(int nleaf, const int *leaves, const int *ibody, const int *nbody, int *body_leaf,
                             hipStream_t s);

@@ -1844,6 +1844,32 @@ hipError_t launch_gather_bodies(int n, const int *perm, const double *xin, const
   return hipGetLastError();
 }
 
+__global__ void gather_charges_kernel(int n, const int *__restrict__ perm, const double *__restrict__ qin,
+                                      double *__restrict__ q) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) q[i] = qin[perm[i]];
+}
+hipError_t launch_gather_charges(int n, const int *perm, const double *qin, double *q, hipStream_t s) {
+  if (n > 0) hipLaunchKernelGGL(gather_charges_kernel, dim3((n - 1) / 256 + 1), dim3(256), 0, s, n, perm, qin, q);
+  return hipGetLastError();
+}
+
+// targets in the caller's order and layout: the random 32-byte writes go to
+// device memory, and the host only copies
+__global__ void pack_targets_kernel(int n, const int *__restrict__ perm, DevBodies B, double2 *__restrict__ trg) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const size_t o = perm ? perm[i] : i;
+  trg[2 * o] = make_double2(B.pot[i], B.ax[i]);
+  trg[2 * o + 1] = make_double2(B.ay[i], B.az[i]);
+}
+hipError_t launch_pack_targets(int n, const int *perm, DevBodies B, double *trg, hipStream_t s) {
+  if (n > 0)
+    hipLaunchKernelGGL(pack_targets_kernel, dim3((n - 1) / 256 + 1), dim3(256), 0, s, n, perm, B,
+                       reinterpret_cast<double2 *>(trg));
+  return hipGetLastError();
+}
+
 // every body's leaf: one thread per leaf over its bodies
 __global__ void body_leaf_kernel(int nleaf, const int *__restrict__ leaves, const int *__restrict__ ibody,
                                  const int *__restrict__ nbody, int *__restrict__ body_leaf) {
