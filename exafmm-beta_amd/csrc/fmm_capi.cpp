@@ -98,7 +98,7 @@ struct fmm_ctx {
   // periodic images: shift unit per image, far-image operator F (images >= 2)
   double3 cyc = {0.0, 0.0, 0.0};
   bool far = false;
-  DBuf per_F, per_T, per_S, per_cur, per_tmp, per_dx;
+  DBuf per_F, per_T, per_S, per_cur, per_tmp, per_sums;
   // mixed precision: per-group (R_s, R_t), cell radii, FP32 multipoles
   bool mixed = false;
   DBuf g_sc, cr, M32;
@@ -1007,14 +1007,15 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
       }
     } else {
       bool done = false;
-      if (c->use_tiles && c->p.images == 0 && L.nm2l > 0) {
-        // free space on tiles: the groups and tiles built on the device from
+      if (c->use_tiles && L.nm2l > 0) {
+        // tiles: the groups and tiles built on the device from
         // the lists just uploaded (the host build's groups, classes, tiles
         // and slices), their pair arrays left there; irregular trees and
         // offsets out of the key's range fall back to the host build
         const hipError_t e = fmmdev::device_groups_tiles(t, L, fmmdev::m2l_tile_targets(c->p.P),
                                                          fmmdev::kM2LSlicePairs, 0, c->groups, tiles, done, c->st,
-                                                         &loc, c->m2l_src.as<int>());
+                                                         &loc, c->m2l_src.as<int>(),
+                                                         c->p.images > 0 ? c->p.cycle : nullptr);
         if (e != hipSuccess) {
           (void)hipStreamSynchronize(c->st);
           HIPCHK(e);
@@ -1083,48 +1084,24 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
     const int prange = (int)(0.5 / c->p.theta + 1), nb = 2 * prange + 1;
     const size_t mb = sizeof(double) * PP * PP;
     if ((rc = ensure(c, c->per_F, mb)) || (rc = ensure(c, c->per_T, mb)) || (rc = ensure(c, c->per_S, mb)) ||
-        (rc = ensure(c, c->per_cur, mb)) || (rc = ensure(c, c->per_tmp, mb)))
+        (rc = ensure(c, c->per_cur, mb)) || (rc = ensure(c, c->per_tmp, mb)) ||
+        (rc = ensure(c, c->per_sums, fmmdev::far_sums_bytes(P))))
       return rc;
-    const int nmax = (nb * nb * nb - 1) * nb * nb * nb;
-    if ((rc = ensure(c, c->per_dx, sizeof(double) * 3 * nmax))) return rc;
-    HIPCHK(hipMemsetAsync(c->per_F.p, 0, mb, c->st));
-    HIPCHK(hipMemsetAsync(c->per_cur.p, 0, mb, c->st));
-    HIPCHK(fmmdev::launch_add_identity(c->per_cur.as<double>(), PP, c->st));
-    double cyc[3] = {c->p.cycle[0], c->p.cycle[1], c->p.cycle[2]};
-    std::vector<double> dl, ds;
-    for (int lev = 0; lev < c->p.images - 1; lev++) {
-      dl.clear();
-      ds.clear();
-      for (int ix = -prange; ix <= prange; ix++)
-        for (int iy = -prange; iy <= prange; iy++)
-          for (int iz = -prange; iz <= prange; iz++) {
-            if (ix == 0 && iy == 0 && iz == 0) continue;
-            // M2L(root, supercell) with Xperiodic = (i*nb + c) * cycle: dX = -Xperiodic
-            for (int cx = -prange; cx <= prange; cx++)
-              for (int cy = -prange; cy <= prange; cy++)
-                for (int cz = -prange; cz <= prange; cz++)
-                  dl.insert(dl.end(), {-(ix * nb + cx) * cyc[0], -(iy * nb + cy) * cyc[1], -(iz * nb + cz) * cyc[2]});
-            // supercell copy at X + i * cycle; M2M dX = X_parent - X_child
-            ds.insert(ds.end(), {-ix * cyc[0], -iy * cyc[1], -iz * cyc[2]});
-          }
-      const int nl = (int)(dl.size() / 3), ns = (int)(ds.size() / 3);
-      // T_l, then F += T_l cur
-      HIPCHK(hipMemcpyAsync(c->per_dx.p, dl.data(), sizeof(double) * dl.size(), hipMemcpyHostToDevice, c->st));
-      HIPCHK(hipMemsetAsync(c->per_T.p, 0, mb, c->st));
-      HIPCHK(fmmdev::launch_m2l_op_accum(P, c->per_dx.as<double>(), nl, c->per_T.as<double>(), c->st));
-      HIPCHK(fmmdev::launch_matmul(c->per_T.as<double>(), c->per_cur.as<double>(), c->per_F.as<double>(), PP, 1,
-                                   c->st));
-      // S_l = I + sum of the supercell M2M operators, cur = S_l cur
-      HIPCHK(hipStreamSynchronize(c->st));  // dl is reused below
-      HIPCHK(hipMemcpyAsync(c->per_dx.p, ds.data(), sizeof(double) * ds.size(), hipMemcpyHostToDevice, c->st));
-      HIPCHK(hipMemsetAsync(c->per_S.p, 0, mb, c->st));
-      HIPCHK(fmmdev::launch_m2m_op_accum(P, c->per_dx.as<double>(), ns, c->per_S.as<double>(), c->st));
-      HIPCHK(fmmdev::launch_add_identity(c->per_S.as<double>(), PP, c->st));
-      HIPCHK(fmmdev::launch_matmul(c->per_S.as<double>(), c->per_cur.as<double>(), c->per_tmp.as<double>(), PP, 0,
-                                   c->st));
-      std::swap(c->per_cur, c->per_tmp);
-      HIPCHK(hipStreamSynchronize(c->st));  // ds dies at the next iteration
-      for (int d = 0; d < 3; d++) cyc[d] *= nb;
+    double3 cyc = make_double3(c->p.cycle[0], c->p.cycle[1], c->p.cycle[2]);
+    for (int lev = 0; lev < c->p.images - 1; lev++) {  // F += T cur, cur = S cur (cur = I at first)
+      const bool more = lev + 2 < c->p.images;
+      HIPCHK(fmmdev::launch_far_ops(P, prange, cyc, c->per_sums.p, (lev ? c->per_T : c->per_F).as<double>(),
+                                    more ? (lev ? c->per_S : c->per_cur).as<double>() : nullptr, c->st));
+      if (lev) {
+        HIPCHK(fmmdev::launch_matmul(c->per_T.as<double>(), c->per_cur.as<double>(), c->per_F.as<double>(), PP, 1,
+                                     c->st));
+        if (more) {
+          HIPCHK(fmmdev::launch_matmul(c->per_S.as<double>(), c->per_cur.as<double>(), c->per_tmp.as<double>(), PP, 0,
+                                       c->st));
+          std::swap(c->per_cur, c->per_tmp);
+        }
+      }
+      cyc = make_double3(cyc.x * nb, cyc.y * nb, cyc.z * nb);
     }
   }
   if (c->xl) {  // the per-level M2M / L2L records, once per plan

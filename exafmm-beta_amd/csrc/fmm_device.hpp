@@ -89,13 +89,12 @@ hipError_t launch_m2l_rot(int P, int nitem, const int *ttgt, const int4 *items, 
 hipError_t launch_m2m_rot(int P, const int *parents, const int *child8, int np, const void *rec, double2 *M,
                           hipStream_t s);
 hipError_t launch_l2l_rot(int P, const int2 *kids, int nk, const void *rec, double2 *L, hipStream_t s);
-// S += sum of the M2M operators of the n offsets dxs (dense P^2 x P^2, X_parent - X_child)
-hipError_t launch_m2m_op_accum(int P, const double *dxs, int n, double *S, hipStream_t s);
-// periodic far images: T += sum of the M2L operators of the n offsets dxs
-// (P^2 x P^2, row-major), dense products, and L(root) += F v(M(root))
-hipError_t launch_m2l_op_accum(int P, const double *dxs, int n, double *T, hipStream_t s);
+// periodic far images, one level of supercells of period cyc: T = sum of its
+// M2L operators, S = I + its M2M operators (dense P^2 x P^2, row-major; S may be
+// null); sums: far_sums_bytes(P) of scratch
+size_t far_sums_bytes(int P);
+hipError_t launch_far_ops(int P, int prange, double3 cyc, void *sums, double *T, double *S, hipStream_t s);
 hipError_t launch_matmul(const double *A, const double *B, double *C, int n, int acc, hipStream_t s);
-hipError_t launch_add_identity(double *A, int n, hipStream_t s);
 hipError_t launch_periodic_far(int P, const double *F, const double2 *M, double2 *L, hipStream_t s);
 // mixed precision (FP32 list phases): M32 = M~ / R^n per cell; grouped FP32-MFMA
 // M2L with per-group scales (R_s, R_t) accumulating into the FP64 L; FP32 P2P
@@ -180,7 +179,7 @@ struct PlanArrays {
 // Copy the device-held parts into the host structures (synchronous on s).
 hipError_t fetch_lists(const PlanArrays &d, fmm::Lists &L, hipStream_t s);
 hipError_t fetch_tiles(const PlanArrays &d, fmm::M2LTiles &T, hipStream_t s);
-// The M2L groups and tiles of a regular free-space tree built on the device
+// The M2L groups and tiles of a regular tree (cycle: of periodic lists) built on the device
 // (fmm_tiles.hip): the same partition into groups and classes as
 // fmm::build_m2l_groups (numbered in key order), the same tiles, slices and
 // work items as fmm::build_m2l_tiles; done = false (no error) when the plan
@@ -192,7 +191,8 @@ hipError_t fetch_tiles(const PlanArrays &d, fmm::M2LTiles &T, hipStream_t s);
 // device (stream s), read instead of L.m2l_src.
 hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, int TT, int SW, int seg,
                                fmm::M2LGroups &G, fmm::M2LTiles &T, bool &done, hipStream_t s,
-                               PlanArrays *keep = nullptr, const int *dsrc_in = nullptr);
+                               PlanArrays *keep = nullptr, const int *dsrc_in = nullptr,
+                               const double *cycle = nullptr);
 // The octree of n bodies (host array x, AoS) built on the device: the same
 // cells, numbering and body order as fmm::build_tree for the root box (X0,
 // R0) (fmm_traverse.hip); outputs are host arrays.  dx_in: the same bodies

@@ -284,46 +284,6 @@ __global__ __launch_bounds__(64) void l2l_kernel(DevCells C, const int *__restri
   }
 }
 
-// S += the dense real P^2 x P^2 M2M operators (rows n^2 + (m ? 2m-1 : 0), +1
-// for imaginary parts) of the offsets dxs, one block each: the supercell
-// copies of the periodic images, whose offsets are not a level's
-template <int P>
-__global__ __launch_bounds__(256) void m2m_op_accum_kernel(const double *__restrict__ dxs, int n,
-                                                           double *__restrict__ S) {
-  constexpr int NT = nterm(P), PP = P * P;
-  __shared__ double2 T[P * P];
-  const int op = blockIdx.x, tid = threadIdx.x;
-  if (op >= n) return;
-  const double dx = dxs[3 * op], dy = dxs[3 * op + 1], dz = dxs[3 * op + 2];
-  if (tid < P) regular_column<P>(dx, dy, dz, tid, T);
-  __syncthreads();
-  for (int e = tid; e < PP * NT; e += 256) {
-    const int col = e / NT, u = e - col * NT;
-    const int dc = c_vdec[col];
-    const int ia = dc & 255, ib = (dc >> 8) & 255;
-    const int uin = tidx(ia, ib);
-    const double2 v = (dc >> 16) ? make_double2(0.0, 1.0) : make_double2(1.0, 0.0);
-    auto in = [&](int idx) { return idx == uin ? v : make_double2(0.0, 0.0); };
-    int j, k;
-    tdecode(u, j, k);
-    double2 a = make_double2(0.0, 0.0);  // the scalar M2M of m2m_kernel with a unit child multipole
-    for (int n = 0; n <= j; n++) {
-      const double sn = sgn(n);
-      for (int m = -n; m <= min(k - 1, n); m++)
-        if (j - n >= k - m) {
-          const double2 Rc = (m >= 0) ? cconj(T[n * P + m]) : T[n * P - m];
-          const double f = (m >= 0) ? sn : sn * sgn(m);
-          a = cmac(a, cscale(Rc, f), in(tidx(j - n, k - m)));
-        }
-      for (int m = k; m <= n; m++)
-        if (j - n >= m - k) a = cmac(a, cscale(cconj(T[n * P + m]), sgn(k + n + m)), cconj(in(tidx(j - n, m - k))));
-    }
-    const int row = j * j + (k ? 2 * k - 1 : 0);
-    unsafeAtomicAdd(S + row * PP + col, a.x);
-    if (k) unsafeAtomicAdd(S + (row + 1) * PP + col, a.y);
-  }
-}
-
 // ---------------------------------------------------------------- L2P
 // One thread per body: regular harmonics of (x_b - X_leaf) streamed column by
 // column; the potential and the degree-1 coefficients of the local expansion
@@ -1301,32 +1261,100 @@ __global__ __launch_bounds__(64) void p2p32_kernel(DevBodies B, DevCells C, cons
 //   S_l = I + sum of the level's supercell M2M operators,
 // and applied each evaluation with one matrix-vector product.
 
-// Tsum += sum over the offsets of the M2L operator (rows/cols as in the
-// grouped M2L: v(L^) = T v(M~)); one block per offset
+// Both operators are linear in the harmonics of their offset, so a level needs
+// only the harmonics' sums over its offsets (M2L: w cycle for the integer w of
+// the cube |w| <= prange nb + prange without |w| <= prange; M2M: |i| <= prange
+// without 0; nb = 2 prange + 1) and one operator of each: summing the 15500
+// operators themselves (prange = 2) took 1.1 ms a level at P = 10.  Blocks 0 ..
+// kFarBlocks - 1: part[block][a][b] = sums of the singular harmonics; block
+// kFarBlocks: rsum[n P + m] = sums of the regular ones.  Fixed order.
+constexpr int kFarBlocks = 48;
 template <int P>
-__global__ __launch_bounds__(256) void m2l_op_accum_kernel(const double *__restrict__ dxs, int n,
-                                                           double *__restrict__ Tsum) {
-  constexpr int PP = P * P, YC = 3 * P - 2, OFF = 2 * P - 2, YSZ = (2 * P - 1) * (3 * P - 2);
-  __shared__ double2 sY[YSZ];
-  const int o = blockIdx.x, tid = threadIdx.x;
-  if (o >= n) return;
-  const double dx = dxs[3 * o], dy = dxs[3 * o + 1], dz = dxs[3 * o + 2];
-  const double r2 = dx * dx + dy * dy + dz * dz;
-  const double inv_r = 1.0 / sqrt(r2), inv_r2 = inv_r * inv_r;
-  for (int cc = tid; cc <= 2 * P - 2; cc += 256) {
-    double2 smm = make_double2(inv_r, 0.0);
-    for (int i = 1; i <= cc; i++) smm = cscale(cmul(smm, make_double2(dx, dy)), -(2 * i - 1) * inv_r2);
-    double2 sp = make_double2(0.0, 0.0), sc = smm;
-    for (int a = cc; a <= 2 * P - 2; a++) {
-      if (cc <= P - 1) sY[a * YC + OFF + cc] = cmul_ipow(sc, cc);
-      if (cc > 0) sY[a * YC + OFF - cc] = cmul_ipow(cconj(sc), cc);
-      double2 nx = cscale(csub(cscale(sc, (2 * a + 1) * dz), cscale(sp, (double)(a * a - cc * cc))), inv_r2);
-      sp = sc;
-      sc = nx;
+__global__ __launch_bounds__(256) void far_sums_kernel(int prange, double3 cyc, double2 *__restrict__ part,
+                                                       double2 *__restrict__ rsum) {
+  constexpr int NC = 2 * P - 1;
+  __shared__ double2 sum[NC * NC];
+  const int tid = threadIdx.x, nb = 2 * prange + 1;
+  double2 acc[NC];
+#pragma unroll
+  for (int a = 0; a < NC; a++) acc[a] = make_double2(0.0, 0.0);
+  for (int e = tid; e < NC * NC; e += 256) sum[e] = make_double2(0.0, 0.0);
+  const bool reg = blockIdx.x == kFarBlocks;
+  const int ncol = reg ? P : NC, SL = 256 / ncol;
+  const int col = tid % ncol, slot = tid / ncol;
+  if (slot < SL) {
+    const int side = reg ? nb : nb * nb, half = side / 2;
+    const int first = reg ? slot : blockIdx.x * SL + slot, step = reg ? SL : kFarBlocks * SL;
+    for (int e = first; e < side * side * side; e += step) {
+      const int wx = e / (side * side) - half, wy = e / side % side - half, wz = e % side - half;
+      if (max(abs(wx), max(abs(wy), abs(wz))) <= (reg ? 0 : prange)) continue;
+      const double dx = -wx * cyc.x, dy = -wy * cyc.y, dz = -wz * cyc.z;
+      const double r2 = dx * dx + dy * dy + dz * dz;
+      double2 c0 = make_double2(0.0, 0.0), c1;
+      if (reg) {
+        c1 = make_double2(1.0, 0.0);
+        for (int i = 1; i <= col; i++) c1 = cscale(cmul(c1, make_double2(dx, dy)), -0.5 * c_rcp[i]);
+#pragma unroll
+        for (int n = 0; n < P; n++)
+          if (n >= col) {
+            if (n > col) {
+              const double2 cn = cscale(csub(cscale(c1, (2 * n - 1) * dz), cscale(c0, r2)), c_rcp[n * n - col * col]);
+              c0 = c1;
+              c1 = cn;
+            }
+            acc[n] = cadd(acc[n], c1);
+          }
+      } else {
+        const double inv_r = 1.0 / sqrt(r2), inv_r2 = inv_r * inv_r;
+        c1 = make_double2(inv_r, 0.0);
+        for (int i = 1; i <= col; i++) c1 = cscale(cmul(c1, make_double2(dx, dy)), -(2 * i - 1) * inv_r2);
+#pragma unroll
+        for (int a = 0; a < NC; a++)
+          if (a >= col) {
+            acc[a] = cadd(acc[a], c1);
+            const double2 cn =
+                cscale(csub(cscale(c1, (2 * a + 1) * dz), cscale(c0, (double)(a * a - col * col))), inv_r2);
+            c0 = c1;
+            c1 = cn;
+          }
+      }
     }
   }
+  for (int k = 0; k < SL; k++) {
+    __syncthreads();
+    if (slot == k)
+#pragma unroll
+      for (int a = 0; a < NC; a++) sum[a * NC + col] = cadd(sum[a * NC + col], acc[a]);
+  }
   __syncthreads();
-  for (int e = tid; e < PP * PP; e += 256) {
+  if (reg)
+    for (int e = tid; e < P * P; e += 256) rsum[e] = sum[(e / P) * NC + e % P];
+  else
+    for (int e = tid; e < NC * NC; e += 256) part[(size_t)blockIdx.x * NC * NC + e] = sum[e];
+}
+
+// The level's operators from the sums (row-major P^2 x P^2, rows and columns
+// n^2 + (m ? 2m-1 : 0), +1 for imaginary parts): blocks 0 .. nt - 1 T (v(L^) =
+// T v(M~)), the rest S = I + the supercell M2M operators.
+template <int P>
+__global__ __launch_bounds__(256) void far_ops_kernel(const double2 *__restrict__ part,
+                                                      const double2 *__restrict__ rsum, int nt,
+                                                      double *__restrict__ T, double *__restrict__ S) {
+  constexpr int PP = P * P, NT = nterm(P), NC = 2 * P - 1, YC = 3 * P - 2, OFF = 2 * P - 2;
+  __shared__ double2 sY[NC * YC];
+  const int tid = threadIdx.x;
+  if ((int)blockIdx.x < nt) {
+    for (int e = tid; e < NC * NC; e += 256) {
+      const int a = e / NC, cc = e - a * NC;
+      if (cc > a) continue;
+      double2 v = make_double2(0.0, 0.0);
+      for (int k = 0; k < kFarBlocks; k++) v = cadd(v, part[(size_t)k * NC * NC + e]);
+      if (cc <= P - 1) sY[a * YC + OFF + cc] = cmul_ipow(v, cc);
+      if (cc > 0) sY[a * YC + OFF - cc] = cmul_ipow(cconj(v), cc);
+    }
+    __syncthreads();
+    const int e = blockIdx.x * 256 + tid;
+    if (e >= PP * PP) return;
     const int row = e / PP, col = e - row * PP;
     const int di = c_vdec[row], dk = c_vdec[col];
     const int j = di & 255, k = (di >> 8) & 255, io = di >> 16;
@@ -1337,8 +1365,36 @@ __global__ __launch_bounds__(256) void m2l_op_accum_kernel(const double *__restr
     if (m == 0) Bv = make_double2(0.0, 0.0);
     const double re = ii ? (Bv.y - Av.y) : (Av.x + Bv.x);
     const double im = ii ? (Av.x - Bv.x) : (Av.y + Bv.y);
-    unsafeAtomicAdd(Tsum + e, io ? im : re);
+    T[e] = io ? im : re;
+    return;
   }
+  for (int e = tid; e < PP; e += 256) sY[e] = rsum[e];
+  __syncthreads();
+  const int e = (blockIdx.x - nt) * 256 + tid;
+  if (e >= PP * NT) return;
+  const int col = e / NT, u = e - col * NT;
+  const int dc = c_vdec[col];
+  const int ia = dc & 255, ib = (dc >> 8) & 255;
+  const double2 v = (dc >> 16) ? make_double2(0.0, 1.0) : make_double2(1.0, 0.0);
+  int j, k;
+  tdecode(u, j, k);
+  // the scalar M2M of m2m_kernel with a unit child multipole at (ia, ib): its
+  // terms (n, m) with (j - n, |k - m|) = (ia, ib)
+  double2 a = make_double2(0.0, 0.0);
+  const int n = j - ia;
+  if (n >= 0) {
+    const double sn = sgn(n);
+    const int m = k - ib;  // k - m = ib >= 0, m <= k - 1 or (ib = 0) m = k
+    if (ib > 0 && m >= -n && m <= n) {
+      const double2 Rc = (m >= 0) ? cconj(sY[n * P + m]) : sY[n * P - m];
+      a = cmac(a, cscale(Rc, (m >= 0) ? sn : sn * sgn(m)), v);
+    }
+    const int m2 = k + ib;  // m - k = ib >= 0
+    if (m2 <= n) a = cmac(a, cscale(cconj(sY[n * P + m2]), sgn(k + n + m2)), cconj(v));
+  }
+  const int row = j * j + (k ? 2 * k - 1 : 0);
+  S[row * PP + col] = a.x + (row == col ? 1.0 : 0.0);
+  if (k) S[(row + 1) * PP + col] = a.y + (row + 1 == col ? 1.0 : 0.0);
 }
 
 // C = A B (+ C when acc), n x n, row-major with leading dimension n
@@ -1350,11 +1406,6 @@ __global__ __launch_bounds__(256) void matmul_kernel(const double *__restrict__ 
   double s = acc ? C[e] : 0.0;
   for (int k = 0; k < n; k++) s = fma(A[i * n + k], B[k * n + j], s);
   C[e] = s;
-}
-
-__global__ __launch_bounds__(256) void add_identity_kernel(double *__restrict__ A, int n) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) A[i * n + i] += 1.0;
 }
 
 // L^(root) += F v(M~(root))
@@ -1992,36 +2043,29 @@ template <int P> struct RunM2LMfma32 {
     }
   }
 };
-template <int P> struct RunM2MOpAccum {
-  static hipError_t run(const double *dxs, int n, double *S, hipStream_t s) {
-    if (n > 0) hipLaunchKernelGGL(m2m_op_accum_kernel<P>, dim3(n), dim3(256), 0, s, dxs, n, S);
+template <int P> struct RunFarOps {
+  static hipError_t run(int prange, double3 cyc, double2 *sums, double *T, double *S, hipStream_t s) {
+    constexpr int NC = 2 * P - 1, PP = P * P, nt = (PP * PP + 255) / 256, ns = (PP * nterm(P) + 255) / 256;
+    double2 *rsum = sums + (size_t)kFarBlocks * NC * NC;
+    hipLaunchKernelGGL(far_sums_kernel<P>, dim3(kFarBlocks + (S ? 1 : 0)), dim3(256), 0, s, prange, cyc, sums, rsum);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(far_ops_kernel<P>, dim3(nt + (S ? ns : 0)), dim3(256), 0, s, sums, rsum, nt, T, S);
     return hipGetLastError();
   }
 };
-hipError_t launch_m2m_op_accum(int P, const double *dxs, int n, double *S, hipStream_t s) {
-  return dispatch<RunM2MOpAccum>(P, dxs, n, S, s);
+size_t far_sums_bytes(int P) { return sizeof(double2) * ((size_t)kFarBlocks * (2 * P - 1) * (2 * P - 1) + P * P); }
+hipError_t launch_far_ops(int P, int prange, double3 cyc, void *sums, double *T, double *S, hipStream_t s) {
+  return dispatch<RunFarOps>(P, prange, cyc, static_cast<double2 *>(sums), T, S, s);
 }
-template <int P> struct RunM2LOpAccum {
-  static hipError_t run(const double *dxs, int n, double *T, hipStream_t s) {
-    if (n > 0) hipLaunchKernelGGL(m2l_op_accum_kernel<P>, dim3(n), dim3(256), 0, s, dxs, n, T);
-    return hipGetLastError();
-  }
-};
 template <int P> struct RunPeriodicFar {
   static hipError_t run(const double *F, const double2 *M, double2 *L, hipStream_t s) {
     hipLaunchKernelGGL(periodic_far_kernel<P>, dim3(1), dim3(256), 0, s, F, M, L);
     return hipGetLastError();
   }
 };
-hipError_t launch_m2l_op_accum(int P, const double *dxs, int n, double *T, hipStream_t s) {
-  return dispatch<RunM2LOpAccum>(P, dxs, n, T, s);
-}
 hipError_t launch_matmul(const double *A, const double *B, double *C, int n, int acc, hipStream_t s) {
   hipLaunchKernelGGL(matmul_kernel, dim3((n * n + 255) / 256), dim3(256), 0, s, A, B, C, n, acc);
-  return hipGetLastError();
-}
-hipError_t launch_add_identity(double *A, int n, hipStream_t s) {
-  hipLaunchKernelGGL(add_identity_kernel, dim3((n + 255) / 256), dim3(256), 0, s, A, n);
   return hipGetLastError();
 }
 hipError_t launch_periodic_far(int P, const double *F, const double2 *M, double2 *L, hipStream_t s) {

@@ -1,8 +1,7 @@
 // fmm_tiles.hip -- the M2L offset groups and target tiles built on the device.
 //
 // The same partition as fmm::build_m2l_groups and the same tiles, slices and
-// work items as fmm::build_m2l_tiles (fmm_host.cpp), for free-space trees
-// whose cells all have the radius of their level (trees built by
+// work items as fmm::build_m2l_tiles (fmm_host.cpp), for trees whose cells all have the radius of their level (trees built by
 // fmm::build_tree or fmmdev::device_tree):
 //
 //  * every M2L pair's offset, in units of its finer cell's size, reduced by
@@ -18,16 +17,16 @@
 //    pairs of one target) slices of distinct targets, pair i of the run to
 //    slice i mod S, as the host does.
 //
-// Keys that do not fit (an offset component of 2^13 or more after the
-// reduction, an offset off the lattice) make the whole plan fall back to
-// the host; so do periodic images.
+// Periodic lists: the image is part of the key, and the reflection class is
+// that of the whole translation vector.  Keys that do not fit (an offset
+// component of 2^13 or more after the reduction, an offset off the lattice)
+// make the whole plan fall back to the host.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
-#include <map>
 #include <utility>
 #include <vector>
 
@@ -40,6 +39,7 @@ namespace {
 
 constexpr unsigned long long kEmptyKey = ~0ull;
 constexpr int kKBits = 14, kKOff = 1 << (kKBits - 1);  // offset components in [-2^13, 2^13)
+constexpr int kImgBits = 5;  // periodic image 0..26
 constexpr int kHashBits = 20;
 
 struct DBufT {  // device scratch from the plan builders' per-stream cache
@@ -92,7 +92,7 @@ __global__ void pair_key_kernel(int64_t np, const int *__restrict__ ptgt, const 
 #pragma clang fp contract(off)
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= np) return;
-  const int c = ptgt[p], sc = psrc[p];
+  const int c = ptgt[p], sc = psrc[p] & fmm::kCellMask;
   const int lt = level[c], ls = level[sc];
   int e = lt > ls ? lt : ls;
   const double scale = ldexp(1.0, e) / R0;
@@ -112,14 +112,15 @@ __global__ void pair_key_kernel(int64_t np, const int *__restrict__ ptgt, const 
       e--;
     }
     for (int d = 0; d < 3; d++)
-      if (k[d] < -kKOff || k[d] >= kKOff) ok = false;
+      if (k[d] <= -kKOff || k[d] >= kKOff) ok = false;
   }
   if (!ok) {
     atomicOr(bad, 1);
     slot[p] = -1;
     return;
   }
-  const unsigned long long key = ((unsigned long long)e << (3 * kKBits)) |
+  const unsigned long long img = (unsigned long long)(psrc[p] >> fmm::kImageShift);
+  const unsigned long long key = ((unsigned long long)e << (3 * kKBits + kImgBits)) | (img << (3 * kKBits)) |
                                  ((unsigned long long)(k[0] + kKOff) << (2 * kKBits)) |
                                  ((unsigned long long)(k[1] + kKOff) << kKBits) | (unsigned long long)(k[2] + kKOff);
   const unsigned long long mask = (1ull << kHashBits) - 1;
@@ -267,7 +268,7 @@ __global__ void slice_desc_kernel(int nseg, const unsigned long long *__restrict
 
 hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, int TT, int SW, int seg,
                                fmm::M2LGroups &G, fmm::M2LTiles &T, bool &done, hipStream_t s,
-                               PlanArrays *keep, const int *dsrc_in) {
+                               PlanArrays *keep, const int *dsrc_in, const double *cycle) {
   done = false;
   if (keep) {
     keep->tiles = false;
@@ -344,39 +345,46 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, int TT, 
   G.dx.resize(3 * (size_t)ng);
   G.rest_ptr.assign((size_t)nc + 1, 0);
   G.grp_ptr.assign(1, 0);
-  std::map<unsigned long long, int> cls;  // representative key -> class
   std::vector<std::pair<unsigned long long, int>> gcls(ng);
   const unsigned long long kmask = (1ull << kKBits) - 1;
   for (int g = 0; g < ng; g++) {
     const unsigned long long key = keys[g].first;
     gslot[g] = keys[g].second;
-    const int e = (int)(key >> (3 * kKBits));
+    const int e = (int)(key >> (3 * kKBits + kImgBits));
+    const int img = (int)((key >> (3 * kKBits)) & ((1u << kImgBits) - 1));
     long long k[3];
     for (int d = 0; d < 3; d++) k[d] = (long long)((key >> (kKBits * (2 - d))) & kmask) - kKOff;
     const double u = R0 / std::ldexp(1.0, e);
+    double sh[3] = {0, 0, 0};
+    if (cycle) fmm::image_shift(img, cycle, sh);
+    // reflected in every axis where the translation vector (offset minus image
+    // shift) is negative: the lattice offset and the image's shift are negated
     unsigned char r = 0;
-    unsigned long long ck = (unsigned long long)e;
+    int ic[3] = {img / 9 - 1, img / 3 % 3 - 1, img % 3 - 1};
     for (int d = 0; d < 3; d++) {
-      G.dx[3 * (size_t)g + d] = (double)k[d] * u;
-      if (k[d] < 0) r |= (unsigned char)(1 << d);
-      ck = ck << kKBits | (unsigned long long)(std::llabs(k[d]) + kKOff);
+      const double tv = (double)k[d] * u - sh[d];
+      G.dx[3 * (size_t)g + d] = tv;
+      if (cycle ? tv < 0.0 : k[d] < 0) {
+        r |= (unsigned char)(1 << d);
+        k[d] = -k[d];
+        ic[d] = -ic[d];
+      }
     }
+    unsigned long long ck = (unsigned long long)e << kImgBits;
+    if (cycle) ck |= (unsigned long long)((ic[0] + 1) * 9 + (ic[1] + 1) * 3 + ic[2] + 1);
+    for (int d = 0; d < 3; d++) ck = ck << kKBits | (unsigned long long)(k[d] + kKOff);
     grefl[g] = r;
     gcls[g] = {ck, g};
   }
-  {
-    std::vector<std::pair<unsigned long long, int>> sorted(gcls);
-    std::sort(sorted.begin(), sorted.end());
-    for (const auto &x : sorted)
-      if (!cls.count(x.first)) {
-        const int id = (int)cls.size();
-        cls[x.first] = id;
-        const int g = x.second;
-        for (int d = 0; d < 3; d++) G.cdx.push_back(std::fabs(G.dx[3 * (size_t)g + d]));
-      }
-    for (int g = 0; g < ng; g++) gcanon[g] = cls[gcls[g].first];
+  std::sort(gcls.begin(), gcls.end());  // by representative key: classes in that order
+  for (int i = 0; i < ng; i++) {
+    const int g = gcls[i].second;
+    if (i == 0 || gcls[i].first != gcls[i - 1].first) {
+      for (int d = 0; d < 3; d++) G.cdx.push_back(std::fabs(G.dx[3 * (size_t)g + d]));
+      G.ncanon++;
+    }
+    gcanon[g] = G.ncanon - 1;
   }
-  G.ncanon = (int)cls.size();
   G.canon = gcanon;
   G.refl.assign(grefl.begin(), grefl.end());
   // tiles: targets in (level, cell) order

@@ -128,3 +128,17 @@ def test_m2m_l2l_every_order(P, n, ncrit):
         for k in range(P):
             u = slice(k * (k + 1) // 2, (k + 1) * (k + 2) // 2)
             assert np.linalg.norm(a[:, u] - b[:, u]) <= 1e-12 * np.linalg.norm(b[:, u]), k
+
+
+@pytest.mark.parametrize("cycle", [1.0, (1.0, 1.5, 2.0)])
+def test_periodic_groups_on_the_device(cycle):
+    """the offset classes of periodic lists, built on the device: every image,
+    a rectangular cycle, the far images' operator added at images = 2"""
+    F = _F()
+    rng = np.random.default_rng(5)
+    c = np.broadcast_to(np.asarray(cycle), (3,))
+    x = (rng.random((2003, 3)) - 0.5) * c
+    q = rng.random(2003) - 0.5
+    q -= q.mean()
+    _check(F, x, q, P=7, theta=0.5, ncrit=20, images=1, cycle=cycle)
+    _check(F, x, q, P=10, theta=0.4, ncrit=50, images=2, cycle=cycle)
