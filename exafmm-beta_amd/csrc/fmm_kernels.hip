@@ -737,6 +737,13 @@ __device__ __forceinline__ double rsqrt_f64(double r2) {
 // slots (slot f belongs to the entry e with off[e] <= f < off[e + 1], found by
 // a 6-step binary search over the offsets in LDS).  The FP64 kernel leaves
 // the leaf's own entry out (count 0) for its masked pass after the list.
+// LDS arrays of one wavefront: its operations complete in order, the compiler
+// only must not reorder them
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 struct P2PWindow {
   int off[65];
   int ib[64];
@@ -758,7 +765,7 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
 // image shift) counts no bodies and sets *self.
 __device__ __forceinline__ int p2p_window(P2PWindow &W, DevCells C, const int *__restrict__ src, int c, int w0,
                                           int k1, double3 xper, bool skip_own, bool *self) {
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
   const int e = w0 + lane;
   int cnt = 0, ib = 0;
   double3 sh = make_double3(0.0, 0.0, 0.0);
@@ -793,7 +800,9 @@ __device__ __forceinline__ int p2p_entry(const P2PWindow &W, int f) {
   return lo;
 }
 
-// One wavefront per target leaf.  Each lane holds K target bodies (t,
+// W wavefronts per target leaf (one where the leaves fill the GPU), each
+// with its own staging: the list's chunks of CH bodies are dealt to them in
+// turn and their sums added in order at the end.  Each lane holds K target bodies (t,
 // t + nk, ... of the leaf's nk = ceil(nt / K) groups), so one LDS read of a
 // source feeds K interactions, and the leaf's target groups take
 // S = 64 / nk slices of the sources.
@@ -808,20 +817,21 @@ __device__ __forceinline__ int p2p_entry(const P2PWindow &W, int f) {
 // solve 9.84 / 9.57 / 9.50 / 9.49 ms; 8M uniform cube (10.5 bodies per leaf),
 // all leaves with K = 4: P2P 4% (FP64) and 20% (FP32) slower than K = 1 (a
 // fifth of the lanes' targets empty, occupancy lost to registers).
-template <int K>
-__global__ __launch_bounds__(64) void p2p_kernel(DevBodies B, DevCells C, const int *__restrict__ targets,
+template <int K, int W>
+__global__ __launch_bounds__(64 * W) void p2p_kernel(DevBodies B, DevCells C, const int *__restrict__ targets,
                                                  int ntarget, const int *__restrict__ ptr,
                                                  const int *__restrict__ src, double3 xper, double eps2,
                                                  int mask_all) {
   constexpr int CH = 256;
   static_assert(64 * K <= CH, "the partial sums reuse the staging buffer");
-  __shared__ double4 sb[CH];
-  __shared__ P2PWindow W;
-  double4 *sred = sb;
+  __shared__ double4 sball[W][CH];
+  __shared__ P2PWindow win[W];
+  const int lane = threadIdx.x & 63, wave = W > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  double4 *sb = sball[wave];
+  P2PWindow &Q = win[wave];
   const int c = targets[blockIdx.x];
   const int ib = C.ibody[c], ni = C.nbody[c];
   const int k0 = ptr[c], k1 = ptr[c + 1];
-  const int lane = threadIdx.x;
   for (int tb = 0; tb < ni; tb += 64 * K) {
     const int nt = min(ni - tb, 64 * K);
     const int nk = (nt + K - 1) / K;
@@ -858,47 +868,53 @@ __global__ __launch_bounds__(64) void p2p_kernel(DevBodies B, DevCells C, const 
       }
     };
     bool self = false;  // the leaf's own entry was met (and left for the masked pass)
+    int turn = 0;       // of the chunks, over the wavefronts
     for (int w0 = k0; w0 < k1; w0 += 64) {
-      const int total = p2p_window(W, C, src, c, w0, k1, xper, true, &self);
-      __syncthreads();
-      for (int base = 0; base < total; base += CH) {
+      wave_lds_order();  // the last window's readers
+      const int total = p2p_window(Q, C, src, c, w0, k1, xper, true, &self);
+      wave_lds_order();
+      for (int base = 0; base < total; base += CH, turn++) {
+        if (W > 1 && turn % W != wave) continue;
         const int cnt = min(CH, total - base);
         for (int u = lane; u < cnt; u += 64) {
-          const int f = base + u, e = p2p_entry(W, f);
-          const int j = W.ib[e] + (f - W.off[e]);
-          sb[u] = make_double4(B.x[j] + W.sx[e], B.y[j] + W.sy[e], B.z[j] + W.sz[e], B.q[j]);
+          const int f = base + u, e = p2p_entry(Q, f);
+          const int j = Q.ib[e] + (f - Q.off[e]);
+          sb[u] = make_double4(B.x[j] + Q.sx[e], B.y[j] + Q.sy[e], B.z[j] + Q.sz[e], B.q[j]);
         }
-        __syncthreads();
+        wave_lds_order();
         if (mask_all)
           accumulate(cnt, true);
         else
           accumulate(cnt, false);
-        __syncthreads();
+        wave_lds_order();
       }
     }
-    for (int j0 = 0; self && j0 < ni; j0 += CH) {  // the own leaf, masked
+    for (int j0 = 0; self && j0 < ni; j0 += CH, turn++) {  // the own leaf, masked
+      if (W > 1 && turn % W != wave) continue;
       const int cnt = min(ni - j0, CH);
       for (int u = lane; u < cnt; u += 64) {
         const int j = ib + j0 + u;
         sb[u] = make_double4(B.x[j], B.y[j], B.z[j], B.q[j]);
       }
-      __syncthreads();
+      wave_lds_order();
       accumulate(cnt, true);
-      __syncthreads();
+      wave_lds_order();
     }
 #pragma unroll
-    for (int h = 0; h < K; h++) sred[64 * h + lane] = make_double4(ap[h], ax[h], ay[h], az[h]);
+    for (int h = 0; h < K; h++) sb[64 * h + lane] = make_double4(ap[h], ax[h], ay[h], az[h]);
     __syncthreads();
-    for (int t = lane; t < nt; t += 64) {  // target t = tg + h nk: its S slices, in order
+    for (int t = threadIdx.x; t < nt; t += 64 * W) {  // target t = tg + h nk: its wavefronts and slices, in order
       const int h = t / nk, tg = t - h * nk;
-      double4 acc = sred[64 * h + tg];
-      for (int k = 1; k < S; k++) {
-        const double4 v = sred[64 * h + tg + k * nk];
-        acc.x += v.x;
-        acc.y += v.y;
-        acc.z += v.z;
-        acc.w += v.w;
-      }
+      double4 acc = make_double4(0.0, 0.0, 0.0, 0.0);
+#pragma unroll
+      for (int w = 0; w < W; w++)
+        for (int k = 0; k < S; k++) {
+          const double4 v = sball[w][64 * h + tg + k * nk];
+          acc.x += v.x;
+          acc.y += v.y;
+          acc.z += v.z;
+          acc.w += v.w;
+        }
       const int bi = ib + tb + t;
       B.pot[bi] = acc.x;
       B.ax[bi] = acc.y;
@@ -1150,21 +1166,22 @@ __global__ __launch_bounds__(Mfma32Cfg<P>::NTH) void m2l_mfma32_kernel(
 // accumulators (cascaded summation: the FP32 rounding of a partial covers 32
 // terms, never the whole list).
 // Each lane holds K target bodies, as in p2p_kernel.
-template <int K>
-__global__ __launch_bounds__(64) void p2p32_kernel(DevBodies B, DevCells C, const int *__restrict__ targets,
+template <int K, int W>
+__global__ __launch_bounds__(64 * W) void p2p32_kernel(DevBodies B, DevCells C, const int *__restrict__ targets,
                                                    int ntarget, const int *__restrict__ ptr,
                                                    const int *__restrict__ src, double3 xper, double eps2) {
   constexpr int CH = 256, RUN = 32;
   constexpr int NRED = 64 * K > CH / 2 ? 64 * K : CH / 2;  // holds the CH FP32 staging slots too
-  __shared__ double4 sred[NRED];  // the FP32 staging buffer lives in the same bytes
-  __shared__ P2PWindow W;
-  float4 *sb = reinterpret_cast<float4 *>(sred);
+  __shared__ double4 sball[W][NRED];  // the FP32 staging buffer lives in the same bytes
+  __shared__ P2PWindow win[W];
+  const int lane = threadIdx.x & 63, wave = W > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  float4 *sb = reinterpret_cast<float4 *>(sball[wave]);
+  P2PWindow &Q = win[wave];
   const int c = targets[blockIdx.x];
   const int ib = C.ibody[c], ni = C.nbody[c];
   const int k0 = ptr[c], k1 = ptr[c + 1];
   const double Xc = C.cx[c], Yc = C.cy[c], Zc = C.cz[c];
   const float e2 = (float)eps2;
-  const int lane = threadIdx.x;
   for (int tb = 0; tb < ni; tb += 64 * K) {
     const int nt = min(ni - tb, 64 * K);
     const int nk = (nt + K - 1) / K;
@@ -1182,19 +1199,22 @@ __global__ __launch_bounds__(64) void p2p32_kernel(DevBodies B, DevCells C, cons
       tz[h] = (float)(B.z[bi] - Zc);
       ap[h] = ax[h] = ay[h] = az[h] = 0.0;
     }
+    int turn = 0;  // of the chunks, over the wavefronts (a chunk's FP32 partial sums do not depend on W)
     for (int w0 = k0; w0 < k1; w0 += 64) {
       bool unused = false;
-      const int total = p2p_window(W, C, src, c, w0, k1, xper, false, &unused);
-      __syncthreads();
-      for (int base = 0; base < total; base += CH) {
+      wave_lds_order();  // the last window's readers
+      const int total = p2p_window(Q, C, src, c, w0, k1, xper, false, &unused);
+      wave_lds_order();
+      for (int base = 0; base < total; base += CH, turn++) {
+        if (W > 1 && turn % W != wave) continue;
         const int cnt = min(CH, total - base);
         for (int u = lane; u < cnt; u += 64) {
-          const int f = base + u, e = p2p_entry(W, f);
-          const int j = W.ib[e] + (f - W.off[e]);
-          sb[u] = make_float4((float)(B.x[j] + W.sx[e] - Xc), (float)(B.y[j] + W.sy[e] - Yc),
-                              (float)(B.z[j] + W.sz[e] - Zc), (float)B.q[j]);
+          const int f = base + u, e = p2p_entry(Q, f);
+          const int j = Q.ib[e] + (f - Q.off[e]);
+          sb[u] = make_float4((float)(B.x[j] + Q.sx[e] - Xc), (float)(B.y[j] + Q.sy[e] - Yc),
+                              (float)(B.z[j] + Q.sz[e] - Zc), (float)B.q[j]);
         }
-        __syncthreads();
+        wave_lds_order();
         if (active) {
           for (int j0 = sl; j0 < cnt; j0 += RUN * S) {
             const int jend = min(cnt, j0 + RUN * S);
@@ -1225,22 +1245,24 @@ __global__ __launch_bounds__(64) void p2p32_kernel(DevBodies B, DevCells C, cons
             }
           }
         }
-        __syncthreads();
+        wave_lds_order();
       }
     }
 #pragma unroll
-    for (int h = 0; h < K; h++) sred[64 * h + lane] = make_double4(ap[h], ax[h], ay[h], az[h]);
+    for (int h = 0; h < K; h++) sball[wave][64 * h + lane] = make_double4(ap[h], ax[h], ay[h], az[h]);
     __syncthreads();
-    for (int t = lane; t < nt; t += 64) {  // target t = tg + h nk: its S slices, in order
+    for (int t = threadIdx.x; t < nt; t += 64 * W) {  // target t = tg + h nk: its wavefronts and slices, in order
       const int h = t / nk, tg = t - h * nk;
-      double4 acc = sred[64 * h + tg];
-      for (int k = 1; k < S; k++) {
-        const double4 v = sred[64 * h + tg + k * nk];
-        acc.x += v.x;
-        acc.y += v.y;
-        acc.z += v.z;
-        acc.w += v.w;
-      }
+      double4 acc = make_double4(0.0, 0.0, 0.0, 0.0);
+#pragma unroll
+      for (int w = 0; w < W; w++)
+        for (int k = 0; k < S; k++) {
+          const double4 v = sball[w][64 * h + tg + k * nk];
+          acc.x += v.x;
+          acc.y += v.y;
+          acc.z += v.z;
+          acc.w += v.w;
+        }
       const int bi = ib + tb + t;
       B.pot[bi] = acc.x;
       B.ax[bi] = acc.y;
@@ -2078,27 +2100,49 @@ hipError_t launch_m2l_mfma32(int P, const int4 *chunks, int nchunk, const double
                              const int *ptgt, const int *psrc, const float2 *M32, double2 *L, hipStream_t s) {
   return dispatch<RunM2LMfma32>(P, chunks, nchunk, gdx, gscale, ptgt, psrc, M32, L, s);
 }
+// Wavefronts per leaf: four while the leaves fill the GPU's wavefront slots
+// (about 15 of this kernel a CU) less than about three times over, as the
+// longest lists then set the time.  Solve of 1 / 4 wavefronts a leaf, P = 8:
+// 239 leaves 0.262 / 0.146 ms, 3037 0.705 / 0.550, 4118 (ragged) 2.05 / 0.74,
+// 7229 0.685 / 0.665, 10047 0.854 / 0.826, 13003 1.080 / 1.093, 13248 0.687 /
+// 0.759, 21300 1.611 / 1.697; a mixed-precision solve of 3037 0.526 / 0.420
+template <template <int, int> class F, typename... A> static hipError_t p2p_dispatch(int ntarget, int nwide, A... a) {
+  nwide = std::min(std::max(nwide, 0), ntarget);
+  const bool four = ntarget < 12000;
+  if (nwide > 0) {
+    if (four) F<4, 4>::run(0, nwide, a...);
+    else F<4, 1>::run(0, nwide, a...);
+  }
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  if (ntarget > nwide) {
+    if (four) F<1, 4>::run(nwide, ntarget - nwide, a...);
+    else F<1, 1>::run(nwide, ntarget - nwide, a...);
+  }
+  return hipGetLastError();
+}
+template <int K, int W> struct RunP2P {
+  static void run(int first, int n, DevBodies B, DevCells C, const int *targets, const int *ptr, const int *src,
+                  double3 xper, double eps2, int mask_all, hipStream_t s) {
+    hipLaunchKernelGGL((p2p_kernel<K, W>), dim3(n), dim3(64 * W), 0, s, B, C, targets + first, n, ptr, src, xper, eps2,
+                       mask_all);
+  }
+};
+template <int K, int W> struct RunP2P32 {
+  static void run(int first, int n, DevBodies B, DevCells C, const int *targets, const int *ptr, const int *src,
+                  double3 xper, double eps2, hipStream_t s) {
+    hipLaunchKernelGGL((p2p32_kernel<K, W>), dim3(n), dim3(64 * W), 0, s, B, C, targets + first, n, ptr, src, xper,
+                       eps2);
+  }
+};
 hipError_t launch_p2p32(DevBodies B, DevCells C, const int *targets, int ntarget, const int *ptr,
                         const int *src, double3 xper, double eps2, int /*mask_all: every pair is masked*/,
                         int nwide, hipStream_t s) {
-  nwide = std::min(std::max(nwide, 0), ntarget);
-  if (nwide > 0)
-    hipLaunchKernelGGL(p2p32_kernel<4>, dim3(nwide), dim3(64), 0, s, B, C, targets, nwide, ptr, src, xper, eps2);
-  if (ntarget > nwide)
-    hipLaunchKernelGGL(p2p32_kernel<1>, dim3(ntarget - nwide), dim3(64), 0, s, B, C, targets + nwide,
-                       ntarget - nwide, ptr, src, xper, eps2);
-  return hipGetLastError();
+  return p2p_dispatch<RunP2P32>(ntarget, nwide, B, C, targets, ptr, src, xper, eps2, s);
 }
 hipError_t launch_p2p(DevBodies B, DevCells C, const int *targets, int ntarget, const int *ptr,
                       const int *src, double3 xper, double eps2, int mask_all, int nwide, hipStream_t s) {
-  nwide = std::min(std::max(nwide, 0), ntarget);
-  if (nwide > 0)
-    hipLaunchKernelGGL(p2p_kernel<4>, dim3(nwide), dim3(64), 0, s, B, C, targets, nwide, ptr, src, xper, eps2,
-                       mask_all);
-  if (ntarget > nwide)
-    hipLaunchKernelGGL(p2p_kernel<1>, dim3(ntarget - nwide), dim3(64), 0, s, B, C, targets + nwide,
-                       ntarget - nwide, ptr, src, xper, eps2, mask_all);
-  return hipGetLastError();
+  return p2p_dispatch<RunP2P>(ntarget, nwide, B, C, targets, ptr, src, xper, eps2, mask_all, s);
 }
 
 }  // namespace fmmdev
