@@ -127,57 +127,107 @@ __device__ void regular_column(double dx, double dy, double dz, int m, double2 *
 }
 
 // ---------------------------------------------------------------- P2M
-// One wavefront per leaf; lane = (slot, m) with S = 64/P body slots: each lane
-// walks the bodies b = slot, slot + S, ... of the leaf and builds the
-// m-column of their multipole; the slots' partial columns are then summed in
-// slot order through LDS (deterministic).
-template <int P>
+// H = ceil(P / 2) lanes share a leaf: lane h runs the columns m = h and m' =
+// P - 1 - h of the regular harmonics one after the other, P + 1 steps in all,
+// so that every lane has the same number of steps and step t adds into the
+// register acc[t] whatever its (n, m); the recurrence's constants sit in
+// registers.  With S > 1 the bodies of a leaf are dealt to S such groups whose
+// sums are added in order through LDS; a wavefront takes 64 / (H S) leaves.
+// Bound: FP64 VALU (about 180 instructions a body and lane) and the serial
+// steps of each body.  A lane per (body slot, m) left half its steps masked off
+// and loaded a constant from memory in every step: 8M cube, P = 12, 4.9 -> 0.6
+// ms beside P2P; 1M Plummer, P = 10, 1.5 -> 0.15 ms.
+template <int P, int S>
 __global__ __launch_bounds__(64) void p2m_kernel(DevBodies B, DevCells C, const int *__restrict__ leaves,
                                                  int nleaf, double2 *__restrict__ M) {
-  constexpr int NT = nterm(P);
-  constexpr int S = 64 / P;
-  __shared__ double2 sRed[S][P][P];  // [slot][m][n]
-  const int li = blockIdx.x;
-  if (li >= nleaf) return;
-  const int slot = threadIdx.x / P, m = threadIdx.x % P;
-  const int c = leaves[li];
+  constexpr int NT = nterm(P), H = (P + 1) / 2, LW = 64 / (H * S);
+  __shared__ double2 sRed[S > 1 ? 64 * (P + 1) : 1];
+  const int lane = threadIdx.x;
+  const int h = lane % H, slot = lane / H % S, lf = lane / (H * S);
+  const int li = blockIdx.x * LW + lf;
+  const bool act = lf < LW && li < nleaf;
+  const int c = act ? leaves[li] : 0;
   const double Xc = C.cx[c], Yc = C.cy[c], Zc = C.cz[c];
-  const int b0 = C.ibody[c], nb = C.nbody[c];
-  if (slot < S) {
-    double2 acc[P];
+  const int b1 = act ? C.ibody[c] + C.nbody[c] : 0;
+  int b = act ? C.ibody[c] + slot : 0;
+  const int m1 = h, m2 = P - 1 - h, n1 = P - m1;  // steps of the first column
+  // step t: degree n of its column m; r_n = (2n-1)/(n^2-m^2) z r_(n-1) - r^2/(n^2-m^2) r_(n-2),
+  // started (k1 = k2 = 0 here) at n = m
+  double k1[P + 1], k2[P + 1];
 #pragma unroll
-    for (int n = 0; n < P; n++) acc[n] = make_double2(0.0, 0.0);
-    for (int b = b0 + slot; b < b0 + nb; b += S) {
-      const double dx = B.x[b] - Xc, dy = B.y[b] - Yc, dz = B.z[b] - Zc, q = B.q[b];
-      const double r2 = dx * dx + dy * dy + dz * dz;
-      double2 rmm = make_double2(1.0, 0.0);
-      for (int i = 1; i <= m; i++) rmm = cscale(cmul(rmm, make_double2(dx, dy)), -0.5 * c_rcp[i]);
-      double2 r0 = make_double2(0.0, 0.0), r1 = make_double2(0.0, 0.0);
-#pragma unroll
-      for (int n = 0; n < P; n++) {
-        if (n >= m) {
-          double2 rn = (n == m) ? rmm
-                                : cscale(csub(cscale(r1, (2 * n - 1) * dz), cscale(r0, r2)),
-                                         c_rcp[n * n - m * m]);
-          acc[n].x = fma(q, rn.x, acc[n].x);
-          acc[n].y = fma(-q, rn.y, acc[n].y);
-          r0 = r1;
-          r1 = rn;
-        }
-      }
-    }
-#pragma unroll
-    for (int n = 0; n < P; n++) sRed[slot][m][n] = acc[n];
+  for (int t = 0; t <= P; t++) {
+    const bool second = t >= n1;
+    const int m = second ? m2 : m1, n = m + (second ? t - n1 : t);
+    const double inv = n > m ? 1.0 / (double)(n * n - m * m) : 0.0;
+    k1[t] = (2 * n - 1) * inv;
+    k2[t] = inv;
   }
-  __syncthreads();
+  // (-1/2)^m / m! of the two columns
+  double f1 = 1.0, f2 = 1.0;
+  for (int i = 1; i <= m2; i++) {
+    f2 *= -0.5 / i;
+    if (i <= m1) f1 = f2;
+  }
+  double2 acc[P + 1];
+#pragma unroll
+  for (int t = 0; t <= P; t++) acc[t] = make_double2(0.0, 0.0);
+  double bx = 0.0, by = 0.0, bz = 0.0, bq = 0.0;
+  if (b < b1) {
+    bx = B.x[b];
+    by = B.y[b];
+    bz = B.z[b];
+    bq = B.q[b];
+  }
+  while (b < b1) {
+    const double dx = bx - Xc, dy = by - Yc, dz = bz - Zc, q = bq;
+    b += S;
+    if (b < b1) {  // the next body loads during this one's recurrences
+      bx = B.x[b];
+      by = B.y[b];
+      bz = B.z[b];
+      bq = B.q[b];
+    }
+    const double r2 = dx * dx + dy * dy + dz * dz;
+    // q (x + i y)^m of both columns from the squares
+    double2 z = make_double2(dx, dy), p1 = make_double2(q * f1, 0.0), p2 = make_double2(q * f2, 0.0);
+#pragma unroll
+    for (int bit = 0; (1 << bit) < P; bit++) {
+      if (bit > 0) z = make_double2(z.x * z.x - z.y * z.y, 2.0 * z.x * z.y);
+      const double2 w1 = cmul(p1, z), w2 = cmul(p2, z);
+      if ((m1 >> bit) & 1) p1 = w1;
+      if ((m2 >> bit) & 1) p2 = w2;
+    }
+    double2 r0 = make_double2(0.0, 0.0), r1 = p1;
+#pragma unroll
+    for (int t = 0; t <= P; t++) {
+      if (t > 0) {
+        const double u = k1[t] * dz, v = k2[t] * r2;
+        double2 rn = make_double2(u * r1.x - v * r0.x, u * r1.y - v * r0.y);
+        const bool start = t == n1;
+        r0 = start ? make_double2(0.0, 0.0) : r1;
+        r1 = start ? p2 : rn;
+      }
+      acc[t].x += r1.x;
+      acc[t].y -= r1.y;
+    }
+  }
+  if constexpr (S > 1) {
+#pragma unroll
+    for (int t = 0; t <= P; t++) sRed[t * 64 + lane] = acc[t];
+    __syncthreads();
+    if (slot == 0) {
+#pragma unroll
+      for (int t = 0; t <= P; t++)
+        for (int k = 1; k < S; k++) acc[t] = cadd(acc[t], sRed[t * 64 + lane + H * k]);
+    }
+  }
+  if (!act || slot > 0) return;
   double2 *Mc = M + (size_t)c * NT;
-  for (int u = threadIdx.x; u < NT; u += 64) {
-    int n = 0;
-    while ((n + 1) * (n + 2) / 2 <= u) n++;
-    const int mm = u - n * (n + 1) / 2;
-    double2 a = sRed[0][mm][n];
-    for (int k = 1; k < S; k++) a = make_double2(a.x + sRed[k][mm][n].x, a.y + sRed[k][mm][n].y);
-    Mc[u] = a;
+#pragma unroll
+  for (int t = 0; t <= P; t++) {
+    const bool second = t >= n1;
+    const int m = second ? m2 : m1, n = m + (second ? t - n1 : t);
+    if (!second || m2 != m1) Mc[n * (n + 1) / 2 + m] = acc[t];
   }
 }
 
@@ -1975,8 +2025,21 @@ static hipError_t dispatch(int P, A... a) {
 }
 
 template <int P> struct RunP2M {
+  template <int S> static void go(DevBodies B, DevCells C, const int *leaves, int nleaf, double2 *M, hipStream_t s) {
+    constexpr int LW = 64 / ((P + 1) / 2 * S);
+    hipLaunchKernelGGL((p2m_kernel<P, S>), dim3((nleaf + LW - 1) / LW), dim3(64), 0, s, B, C, leaves, nleaf, M);
+  }
   static hipError_t run(DevBodies B, DevCells C, const int *leaves, int nleaf, double2 *M, hipStream_t s) {
-    if (nleaf > 0) hipLaunchKernelGGL(p2m_kernel<P>, dim3(nleaf), dim3(64), 0, s, B, C, leaves, nleaf, M);
+    constexpr int SM = 64 / ((P + 1) / 2);  // one leaf a wavefront
+    if (nleaf <= 0) return hipSuccess;
+    // few leaves: a leaf's bodies over the whole wavefront, else over two groups
+    // of lanes.  Upward pass with SM / 2 / 1 groups: 253 leaves, P = 8, 29 / 38 /
+    // 46 us; 3229, P = 8, 52 / 55 / 66; 13003, P = 10, 101 / 101 / 116; 56095, P =
+    // 10, 244 / 177 / 195; 797144, P = 12, 3032 / 1530 / 1487
+    if (nleaf < 8192)
+      go<SM>(B, C, leaves, nleaf, M, s);
+    else
+      go<2>(B, C, leaves, nleaf, M, s);
     return hipGetLastError();
   }
 };
