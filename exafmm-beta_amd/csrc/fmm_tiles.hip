@@ -7,10 +7,10 @@
 //  * every M2L pair's offset, in units of its finer cell's size, reduced by
 //    common factors of two (the host's lattice key), packed into one 64-bit key; a hash table on the device gives
 //    each pair its key's slot;
-//  * on the host, over the distinct keys only (thousands): group numbers in
-//    key order, offsets, reflection classes and their representatives --
-//    the host's numbering is first-appearance order, which only permutes the
-//    groups and classes;
+//  * over the distinct keys only (thousands): group numbers in key order,
+//    reflection classes and their representatives' offsets -- the host's
+//    numbering is first-appearance order, which only permutes the groups and
+//    classes;
 //  * tiles: the targets sorted by (level, cell), TT per tile -- the host's
 //    order, so the same tiles; each tile's pairs sorted by (class, target) and
 //    every (tile, class) run of m pairs dealt into S = max(ceil(m / SW), most
@@ -76,11 +76,14 @@ __device__ __forceinline__ unsigned long long mix64(unsigned long long k) {
   return k;
 }
 
-// the target cell of every pair
-__global__ void pair_target_kernel(int ncell, const int *__restrict__ ptr, int *__restrict__ ptgt) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+// the target cell of every pair; a wavefront a cell, its lanes the cell's
+// pairs (a thread a cell wrote one pair after the other: 30 us at 14k cells
+// of some 30 pairs, 4 us now)
+__global__ void __launch_bounds__(256) pair_target_kernel(int ncell, const int *__restrict__ ptr,
+                                                          int *__restrict__ ptgt) {
+  const int c = blockIdx.x * 4 + threadIdx.x / 64;
   if (c >= ncell) return;
-  for (int p = ptr[c]; p < ptr[c + 1]; p++) ptgt[p] = c;
+  for (int p = ptr[c] + threadIdx.x % 64; p < ptr[c + 1]; p += 64) ptgt[p] = c;
 }
 
 // every pair's key (host: build_m2l_groups), inserted into the hash table;
@@ -141,33 +144,102 @@ __global__ void pair_key_kernel(int64_t np, const int *__restrict__ ptgt, const 
   slot[p] = -1;
 }
 
-// the filled slots of the hash table (any order: the host sorts them)
-__global__ void table_compact_kernel(int tsize, const unsigned long long *__restrict__ table,
-                                     unsigned long long *__restrict__ okey, int *__restrict__ oslot,
-                                     int *__restrict__ count) {
-  const int h = blockIdx.x * blockDim.x + threadIdx.x;
-  if (h >= tsize) return;
-  const unsigned long long k = table[h];
-  if (k == kEmptyKey) return;
-  const int at = atomicAdd(count, 1);
-  okey[at] = k;
-  oslot[at] = h;
+// The filled slots of the hash table (any order: they are sorted next). Bound
+// by the additions to the one counter, about 8 ns each, so a block counts its
+// kCompact * 256 slots in LDS and adds once: 104 us at 13k keys when every
+// wavefront that held a key added for itself, 7 us now.
+constexpr int kCompact = 16;
+__global__ void __launch_bounds__(256) table_compact_kernel(int tsize, const unsigned long long *__restrict__ table,
+                                                            unsigned long long *__restrict__ okey,
+                                                            int *__restrict__ oslot, int *__restrict__ count) {
+  __shared__ int nblk, base;
+  if (threadIdx.x == 0) nblk = 0;
+  __syncthreads();
+  const int h0 = blockIdx.x * (256 * kCompact) + threadIdx.x;
+  unsigned long long k[kCompact];
+  int at[kCompact];
+#pragma unroll
+  for (int i = 0; i < kCompact; i++) {
+    const int h = h0 + 256 * i;
+    k[i] = h < tsize ? table[h] : kEmptyKey;
+  }
+#pragma unroll
+  for (int i = 0; i < kCompact; i++) at[i] = k[i] != kEmptyKey ? atomicAdd(&nblk, 1) : 0;
+  __syncthreads();
+  if (threadIdx.x == 0) base = nblk ? atomicAdd(count, nblk) : 0;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kCompact; i++)
+    if (k[i] != kEmptyKey) {
+      okey[base + at[i]] = k[i];
+      oslot[base + at[i]] = h0 + 256 * i;
+    }
 }
 
-// slot2grp[gslot[g]] = g: the group of every filled slot
-__global__ void slot_group_kernel(int ng, const int *__restrict__ gslot, int *__restrict__ slot2grp) {
+// group g (keys in order) of slot gslot[g]: slot2grp, its reflections and the
+// key of its class: the offset and image of the translation vector (offset
+// minus image shift) reflected into non-negative components
+__global__ void group_class_kernel(int ng, const unsigned long long *__restrict__ gkey, const int *__restrict__ gslot,
+                                   double R0, double3 cycle, int periodic, int *__restrict__ slot2grp,
+                                   unsigned char *__restrict__ grefl, unsigned long long *__restrict__ ckey,
+                                   int *__restrict__ gid, double *__restrict__ adx) {
+#pragma clang fp contract(off)
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g < ng) slot2grp[gslot[g]] = g;
+  if (g >= ng) return;
+  slot2grp[gslot[g]] = g;
+  const unsigned long long key = gkey[g], kmask = (1ull << kKBits) - 1;
+  const int e = (int)(key >> (3 * kKBits + kImgBits));
+  const int img = (int)((key >> (3 * kKBits)) & ((1u << kImgBits) - 1));
+  const double u = R0 / ldexp(1.0, e);
+  const double cyc[3] = {cycle.x, cycle.y, cycle.z};
+  int ic[3] = {img / 9 - 1, img / 3 % 3 - 1, img % 3 - 1};
+  unsigned char r = 0;
+  unsigned long long ck = (unsigned long long)e << kImgBits;
+  long long k[3];
+  for (int d = 0; d < 3; d++) {
+    k[d] = (long long)((key >> (kKBits * (2 - d))) & kmask) - kKOff;
+    const double sh = periodic ? ic[d] * cyc[d] : 0.0;
+    const double tv = (double)k[d] * u - sh;
+    adx[3 * (size_t)g + d] = fabs(tv);
+    if (periodic ? tv < 0.0 : k[d] < 0) {
+      r |= (unsigned char)(1 << d);
+      k[d] = -k[d];
+      ic[d] = -ic[d];
+    }
+  }
+  if (periodic) ck |= (unsigned long long)((ic[0] + 1) * 9 + (ic[1] + 1) * 3 + ic[2] + 1);
+  for (int d = 0; d < 3; d++) ck = ck << kKBits | (unsigned long long)(k[d] + kKOff);
+  grefl[g] = r;
+  ckey[g] = ck;
+  gid[g] = g;
 }
 
-// the target cells with their sort keys (level, cell): siblings are adjacent
+// class keys in order: 1 where a class starts
+__global__ void class_flag_kernel(int ng, const unsigned long long *__restrict__ ckey, int *__restrict__ flag) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < ng) flag[i] = i == 0 || ckey[i] != ckey[i - 1];
+}
+
+// every group's class (cid: inclusive sum of the flags), every class's offset
+__global__ void class_number_kernel(int ng, const unsigned long long *__restrict__ ckey, const int *__restrict__ cid,
+                                    const int *__restrict__ gid, const double *__restrict__ adx,
+                                    int *__restrict__ gcanon, double *__restrict__ cdx) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= ng) return;
+  const int g = gid[i], c = cid[i] - 1;
+  gcanon[g] = c;
+  if (i == 0 || ckey[i] != ckey[i - 1])
+    for (int d = 0; d < 3; d++) cdx[3 * (size_t)c + d] = adx[3 * (size_t)g + d];
+}
+
+// the cells' sort keys: (level, cell) of a target -- siblings are adjacent --
+// and behind them the cells without pairs
 __global__ void target_key_kernel(int ncell, const int *__restrict__ ptr, const int *__restrict__ level,
-                                  unsigned long long *__restrict__ key, int *__restrict__ cell, int *__restrict__ cnt) {
+                                  unsigned long long *__restrict__ key, int *__restrict__ cell) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncell || ptr[c + 1] == ptr[c]) return;
-  const int i = atomicAdd(cnt, 1);
-  key[i] = ((unsigned long long)level[c] << 32) | (unsigned)c;
-  cell[i] = c;
+  if (c >= ncell) return;
+  key[c] = ptr[c + 1] == ptr[c] ? 1ull << 39 : ((unsigned long long)level[c] << 32) | (unsigned)c;
+  cell[c] = c;
 }
 
 __global__ void tile_of_kernel(int nt, const int *__restrict__ cells, int TT, int *__restrict__ tile_of,
@@ -280,8 +352,11 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, int TT, 
   const int nc = t.ncell;
   const int64_t np = L.nm2l;
   if (nc == 0 || np == 0 || np > 0x7fffffff || TT > 255) return hipSuccess;
-  for (int c = 0; c < nc; c++)  // regular tree: every radius R0 / 2^level
-    if (t.R[c] != t.R[0] / (1 << t.level[c])) return hipSuccess;
+  int ntg = 0;  // cells with pairs
+  for (int c = 0; c < nc; c++) {
+    if (t.R[c] != t.R[0] / (1 << t.level[c])) return hipSuccess;  // regular tree: every radius R0 / 2^level
+    ntg += L.m2l_ptr[c + 1] > L.m2l_ptr[c];
+  }
   const double R0 = t.R[0];
   DBufT dX(s), dlev(s), dptr(s), dsrc(s), dtgt(s), dtab(s), dslot(s), dbad(s);
   TCHK(dX.need(sizeof(double) * 3 * (size_t)nc));
@@ -298,7 +373,7 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, int TT, 
   TCHK(hipMemcpyAsync(dptr.p, L.m2l_ptr.data(), 4 * ((size_t)nc + 1), hipMemcpyHostToDevice, s));
   if (!dev_src) TCHK(hipMemcpyAsync(dsrc.p, L.m2l_src.data(), 4 * (size_t)np, hipMemcpyHostToDevice, s));
   const unsigned nbc = (unsigned)((nc + 255) / 256), nbp = (unsigned)((np + 255) / 256);
-  pair_target_kernel<<<nbc, 256, 0, s>>>(nc, dptr.as<int>(), dtgt.as<int>());
+  pair_target_kernel<<<(unsigned)((nc + 3) / 4), 256, 0, s>>>(nc, dptr.as<int>(), dtgt.as<int>());
   TCHK(hipGetLastError());
   // keys and the hash table
   const size_t tsize = (size_t)1 << kHashBits;
@@ -312,103 +387,74 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, int TT, 
                                        dbad.as<int>());
   TCHK(hipGetLastError());
   // the filled slots come back (key, slot), not the whole table
-  DBufT dck(s), dcs(s), dcn(s);
-  TCHK(dck.need(8 * tsize));
-  TCHK(dcs.need(4 * tsize));
+  DBufT dfk(s), dfs(s), dcn(s);
+  TCHK(dfk.need(8 * tsize));
+  TCHK(dfs.need(4 * tsize));
   TCHK(dcn.need(4));
   TCHK(hipMemsetAsync(dcn.p, 0, 4, s));
-  table_compact_kernel<<<(unsigned)((tsize + 255) / 256), 256, 0, s>>>((int)tsize, dtab.as<unsigned long long>(),
-                                                                        dck.as<unsigned long long>(), dcs.as<int>(),
-                                                                        dcn.as<int>());
+  table_compact_kernel<<<(unsigned)((tsize + 256 * kCompact - 1) / (256 * kCompact)), 256, 0, s>>>(
+      (int)tsize, dtab.as<unsigned long long>(), dfk.as<unsigned long long>(), dfs.as<int>(), dcn.as<int>());
   TCHK(hipGetLastError());
   int bad = 0, nfill = 0;
   TCHK(hipMemcpyAsync(&bad, dbad.p, 4, hipMemcpyDeviceToHost, s));
   TCHK(hipMemcpyAsync(&nfill, dcn.p, 4, hipMemcpyDeviceToHost, s));
   TCHK(hipStreamSynchronize(s));
   if (bad) return hipSuccess;  // the host groups this plan
-  std::vector<unsigned long long> fk(nfill);
-  std::vector<int> fs(nfill);
-  if (nfill) {
-    TCHK(hipMemcpyAsync(fk.data(), dck.p, 8 * (size_t)nfill, hipMemcpyDeviceToHost, s));
-    TCHK(hipMemcpyAsync(fs.data(), dcs.p, 4 * (size_t)nfill, hipMemcpyDeviceToHost, s));
-    TCHK(hipStreamSynchronize(s));
-  }
-  // groups in key order, classes in representative-key order (host)
-  std::vector<std::pair<unsigned long long, int>> keys(nfill);
-  for (int f = 0; f < nfill; f++) keys[f] = {fk[f], fs[f]};
-  std::sort(keys.begin(), keys.end());
-  const int ng = (int)keys.size();
-  std::vector<int> gslot(ng), gcanon(ng);
-  std::vector<unsigned char> grefl(ng);
+  // groups in key order, classes in the order of their representatives' keys
+  const int ng = nfill;
+  const unsigned nbg = (unsigned)((ng + 255) / 256);
+  DBufT dgk(s), dgs(s), ds2g(s), dgc(s), dgr(s), dck(s), dck2(s), dgi(s), dgi2(s), dadx(s), dcf(s), dcid(s), dcdx(s),
+      tmp(s);
+  TCHK(dgk.need(8 * (size_t)ng));
+  TCHK(dgs.need(4 * (size_t)ng));
+  TCHK(ds2g.need(4 * tsize));
+  TCHK(dgc.need(4 * (size_t)ng));
+  TCHK(dgr.need((size_t)ng));
+  for (DBufT *d : {&dck, &dck2}) TCHK(d->need(8 * (size_t)ng));
+  for (DBufT *d : {&dgi, &dgi2, &dcf, &dcid}) TCHK(d->need(4 * (size_t)ng));
+  for (DBufT *d : {&dadx, &dcdx}) TCHK(d->need(24 * (size_t)ng));
+  constexpr int kKeyBits = 3 * kKBits + kImgBits + 6;
+  auto sort_u64 = [&](const DBufT &k, const DBufT &ko, const DBufT &v, const DBufT &vo, int n, int bits) -> hipError_t {
+    size_t bytes = 0;
+    TCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, k.as<unsigned long long>(), ko.as<unsigned long long>(),
+                                            v.as<int>(), vo.as<int>(), n, 0, bits, s));
+    TCHK(tmp.need(bytes));
+    return hipcub::DeviceRadixSort::SortPairs(tmp.p, bytes, k.as<unsigned long long>(), ko.as<unsigned long long>(),
+                                              v.as<int>(), vo.as<int>(), n, 0, bits, s);
+  };
+  TCHK(sort_u64(dfk, dgk, dfs, dgs, ng, kKeyBits));
+  group_class_kernel<<<nbg, 256, 0, s>>>(ng, dgk.as<unsigned long long>(), dgs.as<int>(), R0,
+                                         cycle ? make_double3(cycle[0], cycle[1], cycle[2]) : make_double3(0, 0, 0),
+                                         cycle ? 1 : 0, ds2g.as<int>(), dgr.as<unsigned char>(),
+                                         dck.as<unsigned long long>(), dgi.as<int>(), dadx.as<double>());
+  TCHK(hipGetLastError());
+  TCHK(sort_u64(dck, dck2, dgi, dgi2, ng, kKeyBits));
+  class_flag_kernel<<<nbg, 256, 0, s>>>(ng, dck2.as<unsigned long long>(), dcf.as<int>());
+  TCHK(hipGetLastError());
+  size_t tbc = 0;
+  TCHK(hipcub::DeviceScan::InclusiveSum(nullptr, tbc, dcf.as<int>(), dcid.as<int>(), ng, s));
+  TCHK(tmp.need(tbc));
+  TCHK(hipcub::DeviceScan::InclusiveSum(tmp.p, tbc, dcf.as<int>(), dcid.as<int>(), ng, s));
+  class_number_kernel<<<nbg, 256, 0, s>>>(ng, dck2.as<unsigned long long>(), dcid.as<int>(), dgi2.as<int>(),
+                                          dadx.as<double>(), dgc.as<int>(), dcdx.as<double>());
+  TCHK(hipGetLastError());
+  // the tile path reads the counts and the classes' offsets only
   G = fmm::M2LGroups();
   G.ngroup = ng;
-  G.dx.resize(3 * (size_t)ng);
   G.rest_ptr.assign((size_t)nc + 1, 0);
   G.grp_ptr.assign(1, 0);
-  std::vector<std::pair<unsigned long long, int>> gcls(ng);
-  const unsigned long long kmask = (1ull << kKBits) - 1;
-  for (int g = 0; g < ng; g++) {
-    const unsigned long long key = keys[g].first;
-    gslot[g] = keys[g].second;
-    const int e = (int)(key >> (3 * kKBits + kImgBits));
-    const int img = (int)((key >> (3 * kKBits)) & ((1u << kImgBits) - 1));
-    long long k[3];
-    for (int d = 0; d < 3; d++) k[d] = (long long)((key >> (kKBits * (2 - d))) & kmask) - kKOff;
-    const double u = R0 / std::ldexp(1.0, e);
-    double sh[3] = {0, 0, 0};
-    if (cycle) fmm::image_shift(img, cycle, sh);
-    // reflected in every axis where the translation vector (offset minus image
-    // shift) is negative: the lattice offset and the image's shift are negated
-    unsigned char r = 0;
-    int ic[3] = {img / 9 - 1, img / 3 % 3 - 1, img % 3 - 1};
-    for (int d = 0; d < 3; d++) {
-      const double tv = (double)k[d] * u - sh[d];
-      G.dx[3 * (size_t)g + d] = tv;
-      if (cycle ? tv < 0.0 : k[d] < 0) {
-        r |= (unsigned char)(1 << d);
-        k[d] = -k[d];
-        ic[d] = -ic[d];
-      }
-    }
-    unsigned long long ck = (unsigned long long)e << kImgBits;
-    if (cycle) ck |= (unsigned long long)((ic[0] + 1) * 9 + (ic[1] + 1) * 3 + ic[2] + 1);
-    for (int d = 0; d < 3; d++) ck = ck << kKBits | (unsigned long long)(k[d] + kKOff);
-    grefl[g] = r;
-    gcls[g] = {ck, g};
-  }
-  std::sort(gcls.begin(), gcls.end());  // by representative key: classes in that order
-  for (int i = 0; i < ng; i++) {
-    const int g = gcls[i].second;
-    if (i == 0 || gcls[i].first != gcls[i - 1].first) {
-      for (int d = 0; d < 3; d++) G.cdx.push_back(std::fabs(G.dx[3 * (size_t)g + d]));
-      G.ncanon++;
-    }
-    gcanon[g] = G.ncanon - 1;
-  }
-  G.canon = gcanon;
-  G.refl.assign(grefl.begin(), grefl.end());
   // tiles: targets in (level, cell) order
-  DBufT dtk(s), dtk2(s), dtc(s), dtc2(s), dcnt(s), dtof(s), dloc(s), tmp(s);
+  DBufT dtk(s), dtk2(s), dtc(s), dtc2(s), dtof(s), dloc(s);
   TCHK(dtk.need(8 * (size_t)nc));
   TCHK(dtk2.need(8 * (size_t)nc));
   TCHK(dtc.need(4 * (size_t)nc));
   TCHK(dtc2.need(4 * (size_t)nc));
-  TCHK(dcnt.need(4));
   TCHK(dtof.need(4 * (size_t)nc));
   TCHK(dloc.need(4 * (size_t)nc));
-  TCHK(hipMemsetAsync(dcnt.p, 0, 4, s));
   target_key_kernel<<<nbc, 256, 0, s>>>(nc, dptr.as<int>(), dlev.as<int>(), dtk.as<unsigned long long>(),
-                                        dtc.as<int>(), dcnt.as<int>());
+                                        dtc.as<int>());
   TCHK(hipGetLastError());
-  int ntg = 0;
-  TCHK(hipMemcpyAsync(&ntg, dcnt.p, 4, hipMemcpyDeviceToHost, s));
-  TCHK(hipStreamSynchronize(s));
-  size_t tb = 0;
-  TCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, dtk.as<unsigned long long>(), dtk2.as<unsigned long long>(),
-                                          dtc.as<int>(), dtc2.as<int>(), ntg, 0, 40, s));
-  TCHK(tmp.need(tb));
-  TCHK(hipcub::DeviceRadixSort::SortPairs(tmp.p, tb, dtk.as<unsigned long long>(), dtk2.as<unsigned long long>(),
-                                          dtc.as<int>(), dtc2.as<int>(), ntg, 0, 40, s));
+  TCHK(sort_u64(dtk, dtk2, dtc, dtc2, nc, 40));
   tile_of_kernel<<<(unsigned)((ntg + 255) / 256), 256, 0, s>>>(ntg, dtc2.as<int>(), TT, dtof.as<int>(),
                                                                 dloc.as<int>());
   TCHK(hipGetLastError());
@@ -416,21 +462,8 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, int TT, 
   T.TT = TT;
   T.ntile = (ntg + TT - 1) / TT;
   T.tgt.assign((size_t)T.ntile * TT, -1);
-  TCHK(hipMemcpyAsync(T.tgt.data(), dtc2.p, 4 * (size_t)ntg, hipMemcpyDeviceToHost, s));
   // pairs sorted by (tile, class, target)
-  DBufT ds2g(s), dgc(s), dgr(s), dpk(s), dpk2(s), dpv(s), dpv2(s);
-  TCHK(ds2g.need(4 * tsize));
-  TCHK(dgc.need(4 * (size_t)ng));
-  TCHK(dgr.need((size_t)ng));
-  {  // every filled slot's group, scattered on the device
-    DBufT dgs(s);
-    TCHK(dgs.need(4 * (size_t)ng));
-    TCHK(hipMemcpyAsync(dgs.p, gslot.data(), 4 * (size_t)ng, hipMemcpyHostToDevice, s));
-    slot_group_kernel<<<(unsigned)((ng + 255) / 256), 256, 0, s>>>(ng, dgs.as<int>(), ds2g.as<int>());
-    TCHK(hipGetLastError());
-  }
-  TCHK(hipMemcpyAsync(dgc.p, gcanon.data(), 4 * (size_t)ng, hipMemcpyHostToDevice, s));
-  TCHK(hipMemcpyAsync(dgr.p, grefl.data(), (size_t)ng, hipMemcpyHostToDevice, s));
+  DBufT dpk(s), dpk2(s), dpv(s), dpv2(s);
   TCHK(dpk.need(8 * (size_t)np));
   TCHK(dpk2.need(8 * (size_t)np));
   TCHK(dpv.need(4 * (size_t)np));
@@ -441,12 +474,7 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, int TT, 
   TCHK(hipGetLastError());
   int tbits = 1;
   while ((1 << tbits) < T.ntile) tbits++;
-  size_t tb2 = 0;
-  TCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, tb2, dpk.as<unsigned long long>(), dpk2.as<unsigned long long>(),
-                                          dpv.as<int>(), dpv2.as<int>(), (int)np, 0, 40 + tbits, s));
-  TCHK(tmp.need(tb2));
-  TCHK(hipcub::DeviceRadixSort::SortPairs(tmp.p, tb2, dpk.as<unsigned long long>(), dpk2.as<unsigned long long>(),
-                                          dpv.as<int>(), dpv2.as<int>(), (int)np, 0, 40 + tbits, s));
+  TCHK(sort_u64(dpk, dpk2, dpv, dpv2, (int)np, 40 + tbits));
   // segments (tile, class) and runs (target)
   DBufT dsegf(s), dsegid(s), druns(s), drs(s);
   TCHK(dsegf.need(4 * (size_t)np));
@@ -463,6 +491,7 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, int TT, 
   TCHK(hipcub::DeviceScan::InclusiveScan(tmp.p, ts2, druns.as<int>(), drs.as<int>(), hipcub::Max(), (int)np, s));
   int nseg = 0;
   TCHK(hipMemcpyAsync(&nseg, dsegid.as<int>() + (np - 1), 4, hipMemcpyDeviceToHost, s));
+  TCHK(hipMemcpyAsync(&G.ncanon, dcid.as<int>() + (ng - 1), 4, hipMemcpyDeviceToHost, s));
   TCHK(hipStreamSynchronize(s));
   DBufT dss(s), dsl(s), dsm(s), dns(s), dsb(s);
   for (DBufT *b : {&dss, &dsl, &dsm, &dns, &dsb}) TCHK(b->need(4 * ((size_t)nseg + 1)));
@@ -511,6 +540,9 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, int TT, 
   slice_desc_kernel<<<nbs, 256, 0, s>>>(nseg, dpk2.as<unsigned long long>(), dss.as<int>(), dsl.as<int>(),
                                         dns.as<int>(), dsb.as<int>(), osd, dtp.as<int>());
   TCHK(hipGetLastError());
+  G.cdx.resize(3 * (size_t)G.ncanon);
+  TCHK(hipMemcpyAsync(G.cdx.data(), dcdx.p, 24 * (size_t)G.ncanon, hipMemcpyDeviceToHost, s));
+  TCHK(hipMemcpyAsync(T.tgt.data(), dtc2.p, 4 * (size_t)ntg, hipMemcpyDeviceToHost, s));
   T.ptr.resize((size_t)T.ntile + 1);
   TCHK(hipMemcpyAsync(T.ptr.data(), dtp.p, 4 * (size_t)T.ntile, hipMemcpyDeviceToHost, s));
   if (keep) {

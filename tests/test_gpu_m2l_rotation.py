@@ -142,3 +142,18 @@ def test_periodic_groups_on_the_device(cycle):
     q -= q.mean()
     _check(F, x, q, P=7, theta=0.5, ncrit=20, images=1, cycle=cycle)
     _check(F, x, q, P=10, theta=0.4, ncrit=50, images=2, cycle=cycle)
+
+
+@pytest.mark.parametrize("n,theta,ncrit", [(24, 0.5, 1), (500, 0.5, 8), (20000, 0.3, 64)])
+def test_group_numbering(n, theta, ncrit):
+    """Groups and classes numbered on the device, from a few to thousands of
+    distinct offsets over a table of 2^20 slots: as many as the host finds."""
+    F = _F()
+    x, q = F.make_bodies(n, "plummer1", n)
+    _check(F, x, q, P=4, theta=theta, ncrit=ncrit)
+    st = {}
+    for mode in (F.M2L_TILES, F.M2L_GROUPED):
+        with F.FMM(P=4, theta=theta, ncrit=ncrit, m2l_mode=mode) as f:
+            f.set_bodies(x, q)
+            st[mode] = f.stats()["m2l_groups"]
+    assert st[F.M2L_TILES] == st[F.M2L_GROUPED] > 1
