@@ -59,8 +59,8 @@ struct fmm_ctx {
   fmm_params p{};
   std::string err;
   hipStream_t st = nullptr;
-  hipEvent_t ev[5] = {};
-  hipEvent_t kev[4] = {};  // M2L kernel begin/end, P2P kernel begin/end
+  hipEvent_t ev[4] = {};
+  hipEvent_t kev[2] = {};  // P2P kernels' begin, end
   // fmm_evaluate runs P2P on a second stream (default priority), beside the
   // upward pass and M2L: fork after the previous work, join before L2P
   hipStream_t st2 = nullptr;
@@ -1252,18 +1252,14 @@ int fmm_upward(fmm_ctx *c) {
 namespace {
 // P2P (targets overwritten) on stream s
 int p2p_on(fmm_ctx *c, hipStream_t s) {
-  if (c->n > 0) {
-    HIPCHK(fmmdev::launch_zero(c->pot.as<double>(), c->n, s));
-    HIPCHK(fmmdev::launch_zero(c->ax.as<double>(), c->n, s));
-    HIPCHK(fmmdev::launch_zero(c->ay.as<double>(), c->n, s));
-    HIPCHK(fmmdev::launch_zero(c->az.as<double>(), c->n, s));
-  }
+  HIPCHK(fmmdev::launch_zero_targets(c->pot.as<double>(), c->ax.as<double>(), c->ay.as<double>(), c->az.as<double>(),
+                                     (size_t)c->n, s));
   const double3 xper = c->cyc;  // image shifts of the source codes
-  if (c->timing) HIPCHK(hipEventRecord(c->kev[2], s));
+  if (c->timing) HIPCHK(hipEventRecord(c->kev[0], s));
   HIPCHK((c->mixed ? fmmdev::launch_p2p32 : fmmdev::launch_p2p)(
       dev_bodies(c), dev_cells(c), c->p2p_tgt.as<int>(), (int)c->lists.p2p_targets.size(),
       c->p2p_ptr.as<int>(), c->p2p_src.as<int>(), xper, c->p.eps2, c->tree.adopted ? 1 : 0, c->p2p_nwide, s));
-  if (c->timing) HIPCHK(hipEventRecord(c->kev[3], s));
+  if (c->timing) HIPCHK(hipEventRecord(c->kev[1], s));
   return FMM_OK;
 }
 }  // namespace
@@ -1274,13 +1270,14 @@ int fmm_p2p(fmm_ctx *c) {
   return p2p_on(c, c->st);
 }
 
-int fmm_m2l(fmm_ctx *c) {
-  int rc = check_ready(c);
-  if (rc) return rc;
-  if (c->tree.ncell == 0) return FMM_OK;
+namespace {
+int zero_locals(fmm_ctx *c) {
   HIPCHK(fmmdev::launch_zero(c->L.as<double>(), 2 * (size_t)nterm(c) * c->tree.ncell, c->st));
+  return FMM_OK;
+}
+// the M2L of every pair, added to the local expansions
+int m2l_added(fmm_ctx *c) {
   const double3 xper = c->cyc;  // image shifts of the source codes
-  if (c->timing) HIPCHK(hipEventRecord(c->kev[0], c->st));
   if (c->use_mfma) {
     if (c->use_tiles) {
       HIPCHK(fmmdev::launch_m2l_rot(c->p.P, c->ntile, c->t_tgt.as<int>(), c->t_ptr.as<int4>(), c->t_slice.as<int4>(),
@@ -1311,8 +1308,16 @@ int fmm_m2l(fmm_ctx *c) {
   }
   if (c->far)
     HIPCHK(fmmdev::launch_periodic_far(c->p.P, c->per_F.as<double>(), c->M.as<double2>(), c->L.as<double2>(), c->st));
-  if (c->timing) HIPCHK(hipEventRecord(c->kev[1], c->st));
   return FMM_OK;
+}
+}  // namespace
+
+int fmm_m2l(fmm_ctx *c) {
+  int rc = check_ready(c);
+  if (rc) return rc;
+  if (c->tree.ncell == 0) return FMM_OK;
+  if ((rc = zero_locals(c))) return rc;
+  return m2l_added(c);
 }
 
 int fmm_downward(fmm_ctx *c) {
@@ -1338,11 +1343,12 @@ int fmm_downward(fmm_ctx *c) {
 
 namespace {
 // The solve's launch sequence on the context's two streams: P2P needs the
-// bodies only, so it runs on the second stream beside the upward pass and M2L
-// (vector ALUs beside the matrix cores), and L2P, which adds into the same
-// targets, waits for it (forking after the upward pass instead, so that P2P
-// runs beside M2L, was measured no faster: M2L's LDS leaves no room for P2P
-// blocks on a CU).  With c->timing the phase events are recorded too.
+// bodies only, so it runs on the second stream beside the upward pass, and
+// L2P, which adds into the same targets, waits for it.  The local expansions
+// are cleared beside it too, before the upward pass rather than between it and
+// M2L.  With c->timing the phase events are recorded: begin, upward, M2L and
+// downward done, and the P2P kernels' begin and end (a recorded event holds
+// its stream for some microseconds, so there are no more than these).
 int solve_sequence(fmm_ctx *c) {
   int rc;
   if (c->timing) HIPCHK(hipEventRecord(c->ev[0], c->st));
@@ -1350,14 +1356,14 @@ int solve_sequence(fmm_ctx *c) {
   HIPCHK(hipStreamWaitEvent(c->st2, c->fork, 0));
   if ((rc = p2p_on(c, c->st2))) return rc;
   HIPCHK(hipEventRecord(c->join, c->st2));
+  if ((rc = zero_locals(c))) return rc;
   if ((rc = fmm_upward(c))) return rc;
   if (c->timing) HIPCHK(hipEventRecord(c->ev[1], c->st));
+  if (c->tree.ncell > 0 && (rc = m2l_added(c))) return rc;
   if (c->timing) HIPCHK(hipEventRecord(c->ev[2], c->st));
-  if ((rc = fmm_m2l(c))) return rc;
-  if (c->timing) HIPCHK(hipEventRecord(c->ev[3], c->st));
   HIPCHK(hipStreamWaitEvent(c->st, c->join, 0));
   if ((rc = fmm_downward(c))) return rc;
-  if (c->timing) HIPCHK(hipEventRecord(c->ev[4], c->st));
+  if (c->timing) HIPCHK(hipEventRecord(c->ev[3], c->st));
   return FMM_OK;
 }
 }  // namespace
@@ -1369,21 +1375,18 @@ int fmm_evaluate(fmm_ctx *c) {
   rc = [&]() -> int {
   int rc2 = solve_sequence(c);
   if (rc2) return rc2;
-  HIPCHK(hipEventSynchronize(c->ev[4]));
-  float ms[4];
-  for (int i = 0; i < 4; i++) HIPCHK(hipEventElapsedTime(&ms[i], c->ev[i], c->ev[i + 1]));
+  HIPCHK(hipEventSynchronize(c->ev[3]));
+  float ms[3];
+  for (int i = 0; i < 3; i++) HIPCHK(hipEventElapsedTime(&ms[i], c->ev[i], c->ev[i + 1]));
   float tot;
-  HIPCHK(hipEventElapsedTime(&tot, c->ev[0], c->ev[4]));
+  HIPCHK(hipEventElapsedTime(&tot, c->ev[0], c->ev[3]));
   c->stats.dev_upward_ms = ms[0];
-  c->stats.dev_m2l_ms = ms[2];
-  c->stats.dev_downward_ms = ms[3];  // includes any wait for P2P
+  c->stats.dev_m2l_ms = ms[1];
+  c->stats.dev_downward_ms = ms[2];  // includes any wait for P2P
   c->stats.dev_total_ms = tot;
-  float km = 0.f, kp = 0.f;
-  if (c->tree.ncell > 0) {
-    HIPCHK(hipEventElapsedTime(&km, c->kev[0], c->kev[1]));
-    HIPCHK(hipEventElapsedTime(&kp, c->kev[2], c->kev[3]));
-  }
-  c->stats.dev_m2l_kernel_ms = km;
+  float kp = 0.f;
+  if (c->tree.ncell > 0) HIPCHK(hipEventElapsedTime(&kp, c->kev[0], c->kev[1]));
+  c->stats.dev_m2l_kernel_ms = c->tree.ncell > 0 ? ms[1] : 0.f;
   c->stats.dev_p2p_kernel_ms = kp;
   c->stats.dev_p2p_ms = kp;  // beside the upward pass and M2L
   return FMM_OK;
@@ -1418,10 +1421,10 @@ int fmm_evaluate_graph(fmm_ctx *c) {
   }
   HIPCHK(hipEventRecord(c->ev[0], c->st));
   HIPCHK(hipGraphLaunch(c->gexec, c->st));
-  HIPCHK(hipEventRecord(c->ev[4], c->st));
-  HIPCHK(hipEventSynchronize(c->ev[4]));
+  HIPCHK(hipEventRecord(c->ev[3], c->st));
+  HIPCHK(hipEventSynchronize(c->ev[3]));
   float tot;
-  HIPCHK(hipEventElapsedTime(&tot, c->ev[0], c->ev[4]));
+  HIPCHK(hipEventElapsedTime(&tot, c->ev[0], c->ev[3]));
   c->stats.dev_upward_ms = c->stats.dev_m2l_ms = c->stats.dev_downward_ms = 0.0;
   c->stats.dev_p2p_ms = c->stats.dev_m2l_kernel_ms = c->stats.dev_p2p_kernel_ms = 0.0;
   c->stats.dev_total_ms = tot;

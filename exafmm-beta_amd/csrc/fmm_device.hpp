@@ -32,6 +32,8 @@ constexpr int kMaxP = 20;
 
 // p[0, n) = 0 with a kernel (no memset node when the stream is being captured)
 hipError_t launch_zero(double *p, size_t n, hipStream_t s);
+// p, x, y, z[0, n) = 0 likewise
+hipError_t launch_zero_targets(double *p, double *x, double *y, double *z, size_t n, hipStream_t s);
 // bodies into tree order: x/y/z/q[i] from input body perm[i] of xin (AoS)
 // and qin
 hipError_t launch_gather_bodies(int n, const int *perm, const double *xin, const double *qin, double *x, double *y,

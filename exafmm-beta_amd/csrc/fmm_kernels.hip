@@ -2003,6 +2003,21 @@ hipError_t launch_zero(double *p, size_t n, hipStream_t s) {
   return hipGetLastError();
 }
 
+// a solve's four target arrays in one launch (four of them led a solve of 4096
+// bodies by 12 of its 210 us)
+__global__ __launch_bounds__(256) void zero_targets_kernel(double *__restrict__ p, double *__restrict__ x,
+                                                           double *__restrict__ y, double *__restrict__ z, size_t n) {
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256)
+    p[i] = x[i] = y[i] = z[i] = 0.0;
+}
+
+hipError_t launch_zero_targets(double *p, double *x, double *y, double *z, size_t n, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  const size_t blocks = std::min<size_t>((n + 255) / 256, 8192);
+  hipLaunchKernelGGL(zero_targets_kernel, dim3((unsigned)blocks), dim3(256), 0, s, p, x, y, z, n);
+  return hipGetLastError();
+}
+
 // bodies into tree order (SoA): body i of the tree is input body perm[i]
 __global__ void gather_bodies_kernel(int n, const int *__restrict__ perm, const double *__restrict__ xin,
                                      const double *__restrict__ qin, double *__restrict__ x,
