@@ -467,8 +467,9 @@ int groups_kind_for(const fmm_params &p) {
   return p.precision != FMM_FP64 && !takes_tiles(p) ? FMM_MIXED : FMM_FP64;
 }
 
+// lists: the interaction lists of pl->tree, if not walked on the host
 void plan_fill(fmm_plan *pl, int n, const double *x, int ncrit, double theta, int nspawn, int images = 0,
-               const double *cycle = nullptr) {
+               const double *cycle = nullptr, const std::function<bool(fmm_plan &)> &lists = nullptr) {
   pl->images = images;
   if (images > 0)
     for (int d = 0; d < 3; d++) pl->cycle[d] = cycle[d];
@@ -479,7 +480,7 @@ void plan_fill(fmm_plan *pl, int n, const double *x, int ncrit, double theta, in
   pl->tree = fmm::build_tree(n, x, ncrit, pl->xmin, pl->xmax);
   double t2 = now_ms();
   const double xper[3] = {0, 0, 0};
-  pl->lists = fmm::build_lists(pl->tree, theta, nspawn, xper, images, pl->cycle);
+  if (!lists || !lists(*pl)) pl->lists = fmm::build_lists(pl->tree, theta, nspawn, xper, images, pl->cycle);
   double t3 = now_ms();
   pl->t_bounds = t1 - t0;
   pl->t_tree = t2 - t1;
@@ -508,7 +509,9 @@ void plan_stats(const fmm_plan *pl, fmm_stats &s) {
 
 // x_on_device: x is already in c->xin (fmm_set_bodies_device: the plan was
 // just built from it there)
-int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, bool x_on_device = false);
+// lists_on_device: the lists' source columns are already in c->m2l_src, c->p2p_src
+int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, bool x_on_device = false,
+                bool lists_on_device = false);
 }  // namespace
 
 int fmm_make_bodies(int n, const char *dist, int seed, double *x, double *q) {
@@ -833,12 +836,41 @@ int fmm_set_bodies(fmm_ctx *c, int n, const double *x, const double *q) {
   if (n < 0 || (n > 0 && (!x || !q))) FMM_FAIL(FMM_ERR_ARG, "fmm_set_bodies: bad n or NULL array");
   if (!c->st) FMM_FAIL(FMM_ERR_STATE, "context was not created successfully");
   fmm_plan pl;
+  bool on_device = false;  // lists
+  hipError_t e = hipSetDevice(c->p.device);
+  if (e != hipSuccess) HIPCHK(e);
+  // The device walk takes 0.4 ms at least (its rounds' launches and sizes read
+  // back), the host one grows with the pairs: 521 cells 0.68 ms on the host,
+  // 0.82 on the device, 1031 cells 1.48 and 0.98, 3679 cells 3.9 and 1.1,
+  // 97810 cells 43 and 4.0; with periodic images (27 roots) 81 cells 0.18 and
+  // 0.39, 585 cells 1.2 and 0.53, 4830 cells 7.6 and 0.95.
+  const int least = c->p.images > 0 ? 200 : 600;
+  const auto lists = [&](fmm_plan &p) {
+    if (p.tree.ncell < least) return false;
+    c->have_bodies = false;  // the columns of the bodies before are overwritten
+    graph_reset(c);
+    e = fmmdev::device_visit_lists(
+        p.tree, c->p.theta, c->p.nspawn, c->p.images, c->p.cycle, p.lists,
+        [&](bool p2p, int64_t k) -> int * {
+          DBuf &b = p2p ? c->p2p_src : c->m2l_src;
+          return ensure(c, b, sizeof(int) * (size_t)k) == FMM_OK ? b.as<int>() : nullptr;
+        },
+        on_device, c->st);
+    if (e != hipSuccess) (void)hipStreamSynchronize(c->st);
+    if (e == hipErrorOutOfMemory) {  // no room beside the solve's buffers: the host walks
+      (void)hipGetLastError();
+      e = hipSuccess;
+      on_device = false;
+    }
+    return on_device || e != hipSuccess;
+  };
   try {
-    plan_fill(&pl, n, x, c->p.ncrit, c->p.theta, c->p.nspawn, c->p.images, c->p.cycle);
+    plan_fill(&pl, n, x, c->p.ncrit, c->p.theta, c->p.nspawn, c->p.images, c->p.cycle, lists);
   } catch (const std::bad_alloc &) {
     FMM_FAIL(FMM_ERR_MEMORY, "host allocation failed while building the tree");
   }
-  return upload_plan(c, std::move(pl), x, q);
+  HIPCHK(e);
+  return upload_plan(c, std::move(pl), x, q, false, on_device);
 }
 
 int fmm_set_bodies_device(fmm_ctx *c, int n, const double *x, const double *q) {
@@ -868,7 +900,7 @@ int fmm_set_bodies_plan(fmm_ctx *c, const fmm_plan *pl, const double *x, const d
 }
 
 namespace {
-int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, bool x_on_device) {
+int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, bool x_on_device, bool lists_on_device) {
   HIPCHK(hipSetDevice(c->p.device));
   graph_reset(c);
   c->have_bodies = false;
@@ -945,7 +977,7 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
   UP(m2l_ptr, L.m2l_ptr) UP(m2l_tgt, L.m2l_targets)
   if (dev_lists) {
     DC(m2l_src, pdev->m2l_src) DC(p2p_src, pdev->p2p_src)
-  } else {
+  } else if (!lists_on_device) {
     UP(m2l_src, L.m2l_src) UP(p2p_src, L.p2p_src)
   }
   // P2P targets, leaves of >= 16 bodies first (the kernel's targets per lane
@@ -1039,6 +1071,17 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
             (void)hipStreamSynchronize(c->st);
             HIPCHK(e);
           }
+        }
+        if (lists_on_device) {
+          c->lists.m2l_src.resize(L.nm2l);
+          c->lists.p2p_src.resize(L.np2p);
+          hipError_t e = hipMemcpyAsync(c->lists.m2l_src.data(), c->m2l_src.p, sizeof(int) * (size_t)L.nm2l,
+                                        hipMemcpyDeviceToHost, c->st);
+          if (e == hipSuccess)
+            e = hipMemcpyAsync(c->lists.p2p_src.data(), c->p2p_src.p, sizeof(int) * (size_t)L.np2p,
+                               hipMemcpyDeviceToHost, c->st);
+          const hipError_t e2 = hipStreamSynchronize(c->st);
+          HIPCHK(e != hipSuccess ? e : e2);
         }
         // mixed: on a tree whose levels do not share a radius the pairs of
         // other radii than their group's run per target, as on chunks

@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <functional>
 #include <vector>
 
 #include "fmm_host.hpp"
@@ -214,6 +215,13 @@ hipError_t device_lists(int ncell, const double *X, const double *R, const int *
                         std::vector<int> &m2l_ptr, std::vector<int> &m2l_src, std::vector<int> &p2p_ptr,
                         std::vector<int> &p2p_src, int64_t &body_pairs, hipStream_t s,
                         PlanArrays *keep = nullptr);
+// The interaction lists of a tree with the host walker's order
+// (fmm::build_lists of the root with itself), the source columns copied to
+// the device arrays that dst gives for their lengths (m2l_src and p2p_src are
+// left empty); done = false (no error) when the host has to walk the tree.
+hipError_t device_visit_lists(const fmm::Tree &t, double theta, int nspawn, int images, const double *cycle,
+                              fmm::Lists &L, const std::function<int *(bool p2p, int64_t n)> &dst, bool &done,
+                              hipStream_t s);
 hipError_t launch_ewald_scratch(int device, EwBodies B, int n, int ksize, double3 cyc, double alpha, double sigma,
                                 double cutoff, hipStream_t s);
 // part: 4 nt direct_runs(n, nt) doubles (not read when that is one run), out: [4][nt]

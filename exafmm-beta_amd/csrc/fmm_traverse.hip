@@ -9,11 +9,15 @@
 // found are exactly those of the recursive walk; only their order differs,
 // and the lists are sorted by (target, source) at the end.  The acceptance
 // test rounds exactly like the host walker's: no contraction into FMAs.
+// device_visit_lists keeps the recursive walk's order instead: see there.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
 #include <cstdint>
+#include <cstring>
+#include <deque>
+#include <functional>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -551,6 +555,302 @@ hipError_t device_lists(int ncell, const double *X, const double *R, const int *
   TCHK(pairs_to_csr(M.as<int2>(), nm, ncell, m2l_ptr, m2l_src, s, keep ? &keep->m2l_src : nullptr));
   TCHK(pairs_to_csr(Pp.as<int2>(), np, ncell, p2p_ptr, p2p_src, s, keep ? &keep->p2p_src : nullptr));
   if (keep) keep->lists = true;
+  return hipSuccess;
+}
+
+// ---- the lists in the recursive walk's order ----
+//
+// The rounds keep the visiting order: a round's pairs stand in it, and a
+// split pair writes its children, in the order the recursion takes them, to
+// the slots that an exclusive sum over the round gives it.  A pair's place
+// among all emitted pairs is its parent's plus the emitted pairs below its
+// earlier siblings: emitted pairs are counted bottom-up (a round's counts are
+// differences of the next round's running sum), places handed out top-down,
+// and one stable radix sort of the pairs so placed by (list, target) gives
+// both lists, every target's sources in visiting order as the host's.
+// Periodic images are 27 roots in image order, as the host walks them.
+// Bound by latency: per round three launches and one size read back by the
+// host, and as many launches again on the way back.
+namespace {
+struct VisitOrder {
+  unsigned char o[8][8][64];  // [na - 1][nb - 1][k] = 8 a + b of the k-th child pair
+};
+// TraverseRange::operator() (traversal.h:196-229) over the children a, b
+constexpr void visit_range(unsigned char *o, int &k, int ib, int ie, int jb, int je) {
+  if (ie - ib == 1 || je - jb == 1) {
+    for (int i = ib; i < ie; i++)
+      for (int j = jb; j < je; j++) o[k++] = (unsigned char)(8 * i + j);
+  } else {
+    const int im = ib + (ie - ib) / 2, jm = jb + (je - jb) / 2;
+    visit_range(o, k, ib, im, jb, jm);
+    visit_range(o, k, im, ie, jm, je);
+    visit_range(o, k, ib, im, jm, je);
+    visit_range(o, k, im, ie, jb, jm);
+  }
+}
+constexpr VisitOrder visit_order() {
+  VisitOrder v{};
+  for (int na = 1; na <= 8; na++)
+    for (int nb = 1; nb <= 8; nb++) {
+      int k = 0;
+      visit_range(v.o[na - 1][nb - 1], k, 0, na, 0, nb);
+    }
+  return v;
+}
+__device__ constexpr VisitOrder kVisit = visit_order();
+
+struct Shifts {
+  double s[27][3];
+};
+
+__device__ __forceinline__ int visit_kind(const TravCells &t, int2 pr, double theta, const Shifts &sh, int nspawn,
+                                          int &na, int &nb, int &sa, int &sb) {
+  const int img = pr.y >> fmm::kImageShift;
+  int kind;
+  classify(t, pr.x, pr.y & fmm::kCellMask, theta, sh.s[img][0], sh.s[img][1], sh.s[img][2], nspawn, kind, na, nb, sa,
+           sb);
+  return kind;
+}
+
+// kind[i] and the number of children cn[i] of every pair of a round; cn[nf] = 0
+__global__ __launch_bounds__(256) void visit_count_kernel(const int2 *__restrict__ F, int nf, TravCells t, double theta,
+                                                          Shifts sh, int nspawn, unsigned char *__restrict__ kind,
+                                                          int *__restrict__ cn) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i > nf) return;
+  int na = 0, nb = 0, sa, sb;
+  if (i < nf) kind[i] = (unsigned char)visit_kind(t, F[i], theta, sh, nspawn, na, nb, sa, sb);
+  cn[i] = na * nb;
+}
+
+// the next round: the children of every split pair from slot co[i] on, a
+// wavefront's lanes a pair's children
+__global__ __launch_bounds__(256) void visit_expand_kernel(const int2 *__restrict__ F, int nf, TravCells t,
+                                                           double theta, Shifts sh, int nspawn,
+                                                           const unsigned char *__restrict__ kind,
+                                                           const int *__restrict__ co, int2 *__restrict__ next,
+                                                           int *__restrict__ par) {
+  const int i0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 64, lane = threadIdx.x & 63;
+  int na = 0, nb = 0, sa = 0, sb = 0, at = 0;
+  const int i = i0 + lane;
+  if (i < nf && kind[i] == kNext) {
+    visit_kind(t, F[i], theta, sh, nspawn, na, nb, sa, sb);
+    sb |= F[i].y & ~fmm::kCellMask;
+    at = co[i];
+  }
+  for (unsigned long long m = __ballot(na > 0); m; m &= m - 1) {
+    const int l = __ffsll((long long)m) - 1;
+    const int a = __shfl(na, l), b = __shfl(nb, l), ca = __shfl(sa, l), cb = __shfl(sb, l), o = __shfl(at, l);
+    if (lane < a * b) {
+      const int k = kVisit.o[a - 1][b - 1][lane];
+      next[o + lane] = make_int2(ca + (k >> 3), cb + (k & 7));
+      par[o + lane] = i0 + l;
+    }
+  }
+}
+
+// emitted pairs at or below every pair of a round; sub[nf] = 0
+__global__ __launch_bounds__(256) void visit_below_kernel(int nf, const unsigned char *__restrict__ kind,
+                                                          const int *__restrict__ co, const int *__restrict__ nsum,
+                                                          int *__restrict__ sub) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i > nf) return;
+  sub[i] = i == nf ? 0 : kind[i] == kNext ? nsum[co[i + 1]] - nsum[co[i]] : 1;
+}
+
+// the places of a round's pairs among the emitted ones, the emitted ones
+// written there, and the body pairs of the P2P ones added up
+__global__ __launch_bounds__(256) void visit_place_kernel(const int2 *__restrict__ F, int nf,
+                                                          const unsigned char *__restrict__ kind,
+                                                          const int *__restrict__ sum, const int *__restrict__ par,
+                                                          const int *__restrict__ pplace, const int *__restrict__ pco,
+                                                          const int *__restrict__ nbody, int tbits,
+                                                          int *__restrict__ place, unsigned *__restrict__ key,
+                                                          int *__restrict__ src, unsigned long long *__restrict__ bp) {
+  __shared__ unsigned long long part[4];
+  unsigned long long v = 0;
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < nf) {
+    int at = sum[i];
+    if (par) {
+      const int p = par[i];
+      at += pplace[p] - sum[pco[p]];
+    }
+    place[i] = at;
+    const int kd = kind[i];
+    if (kd != kNext) {
+      const int2 pr = F[i];
+      key[at] = (unsigned)kd << tbits | (unsigned)pr.x;
+      src[at] = pr.y;
+      if (kd == kP2P) v = (unsigned long long)nbody[pr.x] * (unsigned long long)nbody[pr.y & fmm::kCellMask];
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const unsigned long long tot = part[0] + part[1] + part[2] + part[3];
+    if (tot) atomicAdd(bp, tot);
+  }
+}
+
+// ptr[c] of both lists (M2L: [0, ncell], P2P behind it) in the sorted keys
+__global__ void visit_ptr_kernel(int ncell, int n, const unsigned *__restrict__ key, int tbits, int *__restrict__ ptr) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= 2 * (ncell + 1)) return;
+  const bool p2p = i > ncell;
+  auto below = [&](unsigned k) {  // keys < k
+    int lo = 0, hi = n;
+    while (lo < hi) {
+      const int m = (lo + hi) >> 1;
+      if (key[m] < k)
+        lo = m + 1;
+      else
+        hi = m;
+    }
+    return lo;
+  };
+  const unsigned list = (unsigned)kP2P << tbits;
+  ptr[i] = p2p ? below(list + (unsigned)(i - ncell - 1)) - below(list) : below((unsigned)i);
+}
+}  // namespace
+
+hipError_t device_visit_lists(const fmm::Tree &t, double theta, int nspawn, int images, const double *cycle,
+                              fmm::Lists &L, const std::function<int *(bool p2p, int64_t n)> &dst, bool &done,
+                              hipStream_t s) {
+  done = false;
+  const int nc = t.ncell;
+  if (nc == 0) return hipSuccess;
+  // the cells in one copy: X, R, then nchild, ichild, nbody
+  std::vector<double> h((size_t)nc * 4 + ((size_t)nc * 3 + 1) / 2);
+  std::memcpy(h.data(), t.X.data(), sizeof(double) * 3 * (size_t)nc);
+  std::memcpy(h.data() + 3 * (size_t)nc, t.R.data(), sizeof(double) * (size_t)nc);
+  int *hi = reinterpret_cast<int *>(h.data() + 4 * (size_t)nc);
+  for (int c = 0; c < nc; c++) {
+    if (t.nchild[c] > 8) return hipSuccess;
+    hi[c] = t.nchild[c];
+    hi[nc + c] = t.ichild[c];
+    hi[2 * (size_t)nc + c] = t.nbody[c];
+  }
+  Buf dcell(s), tmp(s), dbp(s), key(s), key2(s), src(s), src2(s), dptr(s);
+  TCHK(dcell.need(8 * h.size()));
+  TCHK(hipMemcpyAsync(dcell.p, h.data(), 8 * h.size(), hipMemcpyHostToDevice, s));
+  const double *dX = dcell.as<double>();
+  const int *di = reinterpret_cast<const int *>(dX + 4 * (size_t)nc);
+  const TravCells cells{dX, dX + 3 * (size_t)nc, di, di + nc, di + 2 * (size_t)nc};
+  Shifts sh{};
+  const int nimg = images > 0 ? 27 : 1;
+  for (int m = 0; images > 0 && m < nimg; m++) fmm::image_shift(m, cycle, sh.s[m]);
+  struct Round {
+    Buf F, par, kind, co, sum, place;
+    int n = 0;
+    explicit Round(hipStream_t st) : F(st), par(st), kind(st), co(st), sum(st), place(st) {}
+  };
+  std::deque<Round> R;
+  auto scan = [&](const Buf &in, Buf &out, int n) -> hipError_t {
+    size_t tb = 0;
+    TCHK(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, in.as<int>(), out.as<int>(), n, s));
+    TCHK(tmp.need(tb));
+    return hipcub::DeviceScan::ExclusiveSum(tmp.p, tb, in.as<int>(), out.as<int>(), n, s);
+  };
+  int2 root[27];
+  for (int m = 0; m < nimg; m++) root[m] = make_int2(0, m << fmm::kImageShift);
+  R.emplace_back(s);
+  R.back().n = nimg;
+  TCHK(R.back().F.need(sizeof(int2) * nimg));
+  TCHK(hipMemcpyAsync(R.back().F.p, root, sizeof(int2) * nimg, hipMemcpyHostToDevice, s));
+  Buf cn(s);
+  int64_t total = 0;
+  for (;;) {
+    Round &r = R.back();
+    const size_t n = (size_t)r.n;
+    const unsigned nb = (unsigned)(n / 256 + 1);
+    total += r.n;
+    if (total > 0x3fffffff) return hipSuccess;  // beyond the 32-bit sums: the host walks this tree
+    TCHK(r.kind.need(n));
+    TCHK(cn.need(4 * (n + 1)));
+    TCHK(r.co.need(4 * (n + 1)));
+    visit_count_kernel<<<nb, 256, 0, s>>>(r.F.as<int2>(), r.n, cells, theta, sh, nspawn, r.kind.as<unsigned char>(),
+                                          cn.as<int>());
+    TCHK(hipGetLastError());
+    TCHK(scan(cn, r.co, r.n + 1));
+    int nn = 0;
+    TCHK(hipMemcpyAsync(&nn, r.co.as<int>() + n, 4, hipMemcpyDeviceToHost, s));
+    TCHK(hipStreamSynchronize(s));
+    if (nn < 0) return hipSuccess;
+    if (nn == 0) break;
+    R.emplace_back(s);
+    Round &q = R.back();
+    q.n = nn;
+    TCHK(q.F.need(sizeof(int2) * (size_t)nn));
+    TCHK(q.par.need(4 * (size_t)nn));
+    visit_expand_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(
+        r.F.as<int2>(), r.n, cells, theta, sh, nspawn, r.kind.as<unsigned char>(), r.co.as<int>(), q.F.as<int2>(),
+        q.par.as<int>());
+    TCHK(hipGetLastError());
+  }
+  // emitted pairs below, bottom-up (cn: this round's counts)
+  for (size_t k = R.size(); k-- > 0;) {
+    Round &r = R[k];
+    TCHK(cn.need(4 * ((size_t)r.n + 1)));
+    TCHK(r.sum.need(4 * ((size_t)r.n + 1)));
+    visit_below_kernel<<<(unsigned)(r.n / 256 + 1), 256, 0, s>>>(
+        r.n, r.kind.as<unsigned char>(), r.co.as<int>(), k + 1 < R.size() ? R[k + 1].sum.as<int>() : nullptr,
+        cn.as<int>());
+    TCHK(hipGetLastError());
+    TCHK(scan(cn, r.sum, r.n + 1));
+  }
+  int ne = 0;  // emitted pairs
+  TCHK(hipMemcpyAsync(&ne, R[0].sum.as<int>() + R[0].n, 4, hipMemcpyDeviceToHost, s));
+  TCHK(dbp.need(8));
+  TCHK(hipMemsetAsync(dbp.p, 0, 8, s));
+  TCHK(hipStreamSynchronize(s));
+  int tbits = 1;
+  while ((1ll << tbits) < nc) tbits++;
+  for (Buf *b : {&key, &key2, &src, &src2}) TCHK(b->need(4 * (size_t)ne));
+  for (size_t k = 0; k < R.size(); k++) {
+    Round &r = R[k];
+    TCHK(r.place.need(4 * (size_t)r.n));
+    visit_place_kernel<<<(unsigned)((r.n + 255) / 256), 256, 0, s>>>(
+        r.F.as<int2>(), r.n, r.kind.as<unsigned char>(), r.sum.as<int>(), k ? r.par.as<int>() : nullptr,
+        k ? R[k - 1].place.as<int>() : nullptr, k ? R[k - 1].co.as<int>() : nullptr, cells.nbody, tbits,
+        r.place.as<int>(), key.as<unsigned>(), src.as<int>(), dbp.as<unsigned long long>());
+    TCHK(hipGetLastError());
+  }
+  size_t tb = 0;
+  TCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, key.as<unsigned>(), key2.as<unsigned>(), src.as<int>(),
+                                          src2.as<int>(), ne, 0, tbits + 1, s));
+  TCHK(tmp.need(tb));
+  TCHK(hipcub::DeviceRadixSort::SortPairs(tmp.p, tb, key.as<unsigned>(), key2.as<unsigned>(), src.as<int>(),
+                                          src2.as<int>(), ne, 0, tbits + 1, s));
+  const size_t np = 2 * ((size_t)nc + 1);
+  TCHK(dptr.need(4 * np));
+  visit_ptr_kernel<<<(unsigned)((np + 255) / 256), 256, 0, s>>>(nc, ne, key2.as<unsigned>(), tbits, dptr.as<int>());
+  TCHK(hipGetLastError());
+  std::vector<int> ptr(np);
+  unsigned long long bp = 0;
+  TCHK(hipMemcpyAsync(ptr.data(), dptr.p, 4 * np, hipMemcpyDeviceToHost, s));
+  TCHK(hipMemcpyAsync(&bp, dbp.p, 8, hipMemcpyDeviceToHost, s));
+  TCHK(hipStreamSynchronize(s));
+  L = fmm::Lists();
+  L.m2l_ptr.assign(ptr.begin(), ptr.begin() + nc + 1);
+  L.p2p_ptr.assign(ptr.begin() + nc + 1, ptr.end());
+  L.nm2l = L.m2l_ptr[nc];
+  L.np2p = L.p2p_ptr[nc];
+  L.p2p_body_pairs = (int64_t)bp;
+  for (int c = 0; c < nc; c++) {
+    if (L.m2l_ptr[c + 1] > L.m2l_ptr[c]) L.m2l_targets.push_back(c);
+    if (L.p2p_ptr[c + 1] > L.p2p_ptr[c]) L.p2p_targets.push_back(c);
+  }
+  for (bool p2p : {false, true}) {
+    const int64_t n = p2p ? L.np2p : L.nm2l;
+    int *d = dst(p2p, n);
+    if (!d) return hipErrorOutOfMemory;
+    if (n)
+      TCHK(hipMemcpyAsync(d, src2.as<int>() + (p2p ? L.nm2l : 0), 4 * (size_t)n, hipMemcpyDeviceToDevice, s));
+  }
+  done = true;
   return hipSuccess;
 }
 
