@@ -250,42 +250,55 @@ __global__ void tile_of_kernel(int nt, const int *__restrict__ cells, int TT, in
   local[cells[i]] = i % TT;
 }
 
-// pair sort keys (tile, class, target in the tile); values the pair index
+// pair sort keys (tile, class, target in the tile), the pair's source with
+// them; the reflections ride in the key above the sorted bits.  A tile's
+// pairs are sorted on as many bits as tiles, classes and targets take: 31 for
+// 12M pairs of a 1M-body tree, four passes of 0.1 ms where fixed fields of 32
+// and 8 bits took seven
+struct TileKey {
+  int lb, cb;  // bits of the target in the tile, of the class
+  __device__ unsigned long long body(unsigned long long k) const { return k & ((1ull << 61) - 1); }
+  __device__ unsigned long long segment(unsigned long long k) const { return body(k) >> lb; }
+  __device__ int local(unsigned long long k) const { return (int)(k & ((1ull << lb) - 1)); }
+  __device__ int rep(unsigned long long k) const { return (int)((k >> lb) & ((1ull << cb) - 1)); }
+  __device__ int tile(unsigned long long k) const { return (int)(body(k) >> (lb + cb)); }
+  __device__ int refl(unsigned long long k) const { return (int)(k >> 61); }
+};
 __global__ void pair_tile_key_kernel(int64_t np, const int *__restrict__ ptgt, const int *__restrict__ slot,
                                      const int *__restrict__ slot2grp, const int *__restrict__ gcanon,
-                                     const int *__restrict__ tile_of, const int *__restrict__ local,
-                                     unsigned long long *__restrict__ key, int *__restrict__ val) {
+                                     const unsigned char *__restrict__ grefl, const int *__restrict__ tile_of,
+                                     const int *__restrict__ local, TileKey K, unsigned long long *__restrict__ key) {
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= np) return;
   const int c = ptgt[p], g = slot2grp[slot[p]];
-  key[p] = ((unsigned long long)tile_of[c] << 40) | ((unsigned long long)gcanon[g] << 8) | (unsigned)local[c];
-  val[p] = (int)p;
+  key[p] = (unsigned long long)grefl[g] << 61 | (unsigned long long)tile_of[c] << (K.lb + K.cb) |
+           (unsigned long long)gcanon[g] << K.lb | (unsigned)local[c];
 }
 
 // sorted position i: flags of run starts (segment = (tile, class), run = target)
-__global__ void seg_flags_kernel(int64_t np, const unsigned long long *__restrict__ key, int *__restrict__ segf,
+__global__ void seg_flags_kernel(int64_t np, TileKey K, const unsigned long long *__restrict__ key, int *__restrict__ segf,
                                  int *__restrict__ runs) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= np) return;
-  const bool segb = i == 0 || (key[i] >> 8) != (key[i - 1] >> 8);
-  const bool runb = i == 0 || key[i] != key[i - 1];
+  const bool segb = i == 0 || K.segment(key[i]) != K.segment(key[i - 1]);
+  const bool runb = i == 0 || K.body(key[i]) != K.body(key[i - 1]);
   segf[i] = segb ? 1 : 0;
   runs[i] = runb ? (int)i : 0;  // max-scanned into the run start
 }
 
 // per segment: start, length and the longest run of one target
-__global__ void seg_stats_kernel(int64_t np, const unsigned long long *__restrict__ key,
+__global__ void seg_stats_kernel(int64_t np, TileKey K, const unsigned long long *__restrict__ key,
                                  const int *__restrict__ segid, const int *__restrict__ runstart,
                                  int *__restrict__ sstart, int *__restrict__ slen, int *__restrict__ smost) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= np) return;
   const int sg = segid[i] - 1;
-  if (i == 0 || (key[i] >> 8) != (key[i - 1] >> 8)) sstart[sg] = (int)i;
-  if (i + 1 == np || (key[i + 1] >> 8) != (key[i] >> 8)) slen[sg] = (int)(i + 1);  // end, made a length below
+  if (i == 0 || K.segment(key[i]) != K.segment(key[i - 1])) sstart[sg] = (int)i;
+  if (i + 1 == np || K.segment(key[i + 1]) != K.segment(key[i])) slen[sg] = (int)(i + 1);  // end, made a length below
   // the longest run of one target; runs of one pair cannot raise the slice
   // count max(ceil(m / SW), longest run) above ceil(m / SW) >= 1, so only
   // longer runs (a target's several reflections of one class) take an atomic
-  if (i + 1 == np || key[i + 1] != key[i]) {
+  if (i + 1 == np || K.body(key[i + 1]) != K.body(key[i])) {
     const int len = (int)(i - runstart[i] + 1);
     if (len > 1) atomicMax(&smost[sg], len);
   }
@@ -302,31 +315,29 @@ __global__ void seg_slices_kernel(int nseg, const int *__restrict__ sstart, int 
 }
 
 // deal every sorted pair into its slice: the tile's source and (target | reflection << 8)
-__global__ void deal_kernel(int64_t np, const unsigned long long *__restrict__ key, const int *__restrict__ val,
-                            const int *__restrict__ segid, const int *__restrict__ sstart, const int *__restrict__ slen,
-                            const int *__restrict__ nsl, const int *__restrict__ psrc, const int *__restrict__ slot,
-                            const int *__restrict__ slot2grp, const unsigned char *__restrict__ grefl,
+__global__ void deal_kernel(int64_t np, TileKey K, const unsigned long long *__restrict__ key,
+                            const int *__restrict__ src, const int *__restrict__ segid,
+                            const int *__restrict__ sstart, const int *__restrict__ slen, const int *__restrict__ nsl,
                             int *__restrict__ tsrc, unsigned short *__restrict__ tlt) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= np) return;
   const int sg = segid[i] - 1, s0 = sstart[sg], m = slen[sg], S = nsl[sg];
   const int r = (int)(i - s0), j = r % S, q = r / S;
   const int out = s0 + j * (m / S) + min(j, m % S) + q;
-  const int p = val[i];
-  tsrc[out] = psrc[p];
-  tlt[out] = (unsigned short)((key[i] & 255) | ((unsigned)grefl[slot2grp[slot[p]]] << 8));
+  tsrc[out] = src[i];
+  tlt[out] = (unsigned short)(K.local(key[i]) | K.refl(key[i]) << 8);
 }
 
 // the slice descriptors of every segment, and each tile's first slice
-__global__ void slice_desc_kernel(int nseg, const unsigned long long *__restrict__ key, const int *__restrict__ sstart,
+__global__ void slice_desc_kernel(int nseg, TileKey K, const unsigned long long *__restrict__ key, const int *__restrict__ sstart,
                                   const int *__restrict__ slen, const int *__restrict__ nsl,
                                   const int *__restrict__ sbase, int *__restrict__ slice, int *__restrict__ tptr) {
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= nseg) return;
   const int s0 = sstart[g], m = slen[g], S = nsl[g];
   const unsigned long long k = key[s0];
-  const int rep = (int)((k >> 8) & 0xffffffffull), tile = (int)(k >> 40);
-  if (g == 0 || (key[sstart[g - 1]] >> 40) != (k >> 40)) tptr[tile] = sbase[g];
+  const int rep = K.rep(k), tile = K.tile(k);
+  if (g == 0 || K.tile(key[sstart[g - 1]]) != tile) tptr[tile] = sbase[g];
   for (int j = 0; j < S; j++) {
     int *o = slice + 4 * (size_t)(sbase[g] + j);
     o[0] = rep;
@@ -414,21 +425,21 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, int TT, 
   for (DBufT *d : {&dgi, &dgi2, &dcf, &dcid}) TCHK(d->need(4 * (size_t)ng));
   for (DBufT *d : {&dadx, &dcdx}) TCHK(d->need(24 * (size_t)ng));
   constexpr int kKeyBits = 3 * kKBits + kImgBits + 6;
-  auto sort_u64 = [&](const DBufT &k, const DBufT &ko, const DBufT &v, const DBufT &vo, int n, int bits) -> hipError_t {
+  auto sort_u64 = [&](const DBufT &k, const DBufT &ko, const int *v, const DBufT &vo, int n, int bits) -> hipError_t {
     size_t bytes = 0;
     TCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, k.as<unsigned long long>(), ko.as<unsigned long long>(),
-                                            v.as<int>(), vo.as<int>(), n, 0, bits, s));
+                                            v, vo.as<int>(), n, 0, bits, s));
     TCHK(tmp.need(bytes));
     return hipcub::DeviceRadixSort::SortPairs(tmp.p, bytes, k.as<unsigned long long>(), ko.as<unsigned long long>(),
-                                              v.as<int>(), vo.as<int>(), n, 0, bits, s);
+                                              v, vo.as<int>(), n, 0, bits, s);
   };
-  TCHK(sort_u64(dfk, dgk, dfs, dgs, ng, kKeyBits));
+  TCHK(sort_u64(dfk, dgk, dfs.as<int>(), dgs, ng, kKeyBits));
   group_class_kernel<<<nbg, 256, 0, s>>>(ng, dgk.as<unsigned long long>(), dgs.as<int>(), R0,
                                          cycle ? make_double3(cycle[0], cycle[1], cycle[2]) : make_double3(0, 0, 0),
                                          cycle ? 1 : 0, ds2g.as<int>(), dgr.as<unsigned char>(),
                                          dck.as<unsigned long long>(), dgi.as<int>(), dadx.as<double>());
   TCHK(hipGetLastError());
-  TCHK(sort_u64(dck, dck2, dgi, dgi2, ng, kKeyBits));
+  TCHK(sort_u64(dck, dck2, dgi.as<int>(), dgi2, ng, kKeyBits));
   class_flag_kernel<<<nbg, 256, 0, s>>>(ng, dck2.as<unsigned long long>(), dcf.as<int>());
   TCHK(hipGetLastError());
   size_t tbc = 0;
@@ -454,7 +465,7 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, int TT, 
   target_key_kernel<<<nbc, 256, 0, s>>>(nc, dptr.as<int>(), dlev.as<int>(), dtk.as<unsigned long long>(),
                                         dtc.as<int>());
   TCHK(hipGetLastError());
-  TCHK(sort_u64(dtk, dtk2, dtc, dtc2, nc, 40));
+  TCHK(sort_u64(dtk, dtk2, dtc.as<int>(), dtc2, nc, 40));
   tile_of_kernel<<<(unsigned)((ntg + 255) / 256), 256, 0, s>>>(ntg, dtc2.as<int>(), TT, dtof.as<int>(),
                                                                 dloc.as<int>());
   TCHK(hipGetLastError());
@@ -463,25 +474,30 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, int TT, 
   T.ntile = (ntg + TT - 1) / TT;
   T.tgt.assign((size_t)T.ntile * TT, -1);
   // pairs sorted by (tile, class, target)
-  DBufT dpk(s), dpk2(s), dpv(s), dpv2(s);
+  DBufT dpk(s), dpk2(s), dpv2(s);
   TCHK(dpk.need(8 * (size_t)np));
   TCHK(dpk2.need(8 * (size_t)np));
-  TCHK(dpv.need(4 * (size_t)np));
   TCHK(dpv2.need(4 * (size_t)np));
+  auto bits = [](int64_t n) {  // of 0 .. n - 1
+    int b = 1;
+    while ((1ll << b) < n) b++;
+    return b;
+  };
+  const TileKey K{bits(TT), bits(ng)};
+  const int kbits = K.lb + K.cb + bits(T.ntile);
+  if (kbits > 61) return hipSuccess;
   pair_tile_key_kernel<<<nbp, 256, 0, s>>>(np, dtgt.as<int>(), dslot.as<int>(), ds2g.as<int>(), dgc.as<int>(),
-                                           dtof.as<int>(), dloc.as<int>(), dpk.as<unsigned long long>(),
-                                           dpv.as<int>());
+                                           dgr.as<unsigned char>(), dtof.as<int>(), dloc.as<int>(), K,
+                                           dpk.as<unsigned long long>());
   TCHK(hipGetLastError());
-  int tbits = 1;
-  while ((1 << tbits) < T.ntile) tbits++;
-  TCHK(sort_u64(dpk, dpk2, dpv, dpv2, (int)np, 40 + tbits));
+  TCHK(sort_u64(dpk, dpk2, psrc, dpv2, (int)np, kbits));
   // segments (tile, class) and runs (target)
   DBufT dsegf(s), dsegid(s), druns(s), drs(s);
   TCHK(dsegf.need(4 * (size_t)np));
   TCHK(dsegid.need(4 * (size_t)np));
   TCHK(druns.need(4 * (size_t)np));
   TCHK(drs.need(4 * (size_t)np));
-  seg_flags_kernel<<<nbp, 256, 0, s>>>(np, dpk2.as<unsigned long long>(), dsegf.as<int>(), druns.as<int>());
+  seg_flags_kernel<<<nbp, 256, 0, s>>>(np, K, dpk2.as<unsigned long long>(), dsegf.as<int>(), druns.as<int>());
   TCHK(hipGetLastError());
   size_t ts1 = 0, ts2 = 0;
   TCHK(hipcub::DeviceScan::InclusiveSum(nullptr, ts1, dsegf.as<int>(), dsegid.as<int>(), (int)np, s));
@@ -496,7 +512,7 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, int TT, 
   DBufT dss(s), dsl(s), dsm(s), dns(s), dsb(s);
   for (DBufT *b : {&dss, &dsl, &dsm, &dns, &dsb}) TCHK(b->need(4 * ((size_t)nseg + 1)));
   TCHK(hipMemsetAsync(dsm.p, 0, 4 * (size_t)nseg, s));
-  seg_stats_kernel<<<nbp, 256, 0, s>>>(np, dpk2.as<unsigned long long>(), dsegid.as<int>(), drs.as<int>(),
+  seg_stats_kernel<<<nbp, 256, 0, s>>>(np, K, dpk2.as<unsigned long long>(), dsegid.as<int>(), drs.as<int>(),
                                        dss.as<int>(), dsl.as<int>(), dsm.as<int>());
   TCHK(hipGetLastError());
   const unsigned nbs = (unsigned)((nseg + 255) / 256);
@@ -533,11 +549,10 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, int TT, 
     osd = dsd.as<int>();
   }
   TCHK(dtp.need(4 * ((size_t)T.ntile + 1)));
-  deal_kernel<<<nbp, 256, 0, s>>>(np, dpk2.as<unsigned long long>(), dpv2.as<int>(), dsegid.as<int>(), dss.as<int>(),
-                                  dsl.as<int>(), dns.as<int>(), psrc, dslot.as<int>(), ds2g.as<int>(),
-                                  dgr.as<unsigned char>(), osrc, olt);
+  deal_kernel<<<nbp, 256, 0, s>>>(np, K, dpk2.as<unsigned long long>(), dpv2.as<int>(), dsegid.as<int>(),
+                                  dss.as<int>(), dsl.as<int>(), dns.as<int>(), osrc, olt);
   TCHK(hipGetLastError());
-  slice_desc_kernel<<<nbs, 256, 0, s>>>(nseg, dpk2.as<unsigned long long>(), dss.as<int>(), dsl.as<int>(),
+  slice_desc_kernel<<<nbs, 256, 0, s>>>(nseg, K, dpk2.as<unsigned long long>(), dss.as<int>(), dsl.as<int>(),
                                         dns.as<int>(), dsb.as<int>(), osd, dtp.as<int>());
   TCHK(hipGetLastError());
   G.cdx.resize(3 * (size_t)G.ncanon);

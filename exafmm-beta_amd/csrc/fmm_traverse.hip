@@ -142,14 +142,14 @@ __global__ __launch_bounds__(256) void trav_round_kernel(const int2 *__restrict_
 // sort keys (target, source) and the per-target counts; a wavefront's lanes
 // holding one target in a row (the traversal emits a target's pairs
 // together) add their count with one atomic
-__global__ void pair_keys_kernel(const int2 *__restrict__ pr, size_t n, unsigned long long *__restrict__ key,
-                                 int *__restrict__ count) {
+__global__ void pair_keys_kernel(const int2 *__restrict__ pr, size_t n, int bits,
+                                 unsigned long long *__restrict__ key, int *__restrict__ count) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int lane = threadIdx.x & 63;
   int t = -1;
   if (i < n) {
     const int2 p = pr[i];
-    key[i] = ((unsigned long long)(unsigned)p.x << 32) | (unsigned)p.y;
+    key[i] = ((unsigned long long)(unsigned)p.x << bits) | (unsigned)p.y;
     t = p.x;
   }
   const int prev = __shfl_up(t, 1, 64);
@@ -162,9 +162,10 @@ __global__ void pair_keys_kernel(const int2 *__restrict__ pr, size_t n, unsigned
   }
 }
 
-__global__ void key_src_kernel(const unsigned long long *__restrict__ key, size_t n, int *__restrict__ src) {
+__global__ void key_src_kernel(const unsigned long long *__restrict__ key, size_t n, int bits,
+                               int *__restrict__ src) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) src[i] = (int)(unsigned)(key[i] & 0xffffffffull);
+  if (i < n) src[i] = (int)(key[i] & ((1ull << bits) - 1));
 }
 
 // grid-stride over the pairs, one atomic per block (256 threads)
@@ -227,19 +228,16 @@ hipError_t pairs_to_csr(const int2 *pr, size_t n, int ncell, std::vector<int> &p
   if (n > 0) {
     TCHK(keys.need(8 * n));
     TCHK(keys2.need(8 * n));
-    pair_keys_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(pr, n, keys.as<unsigned long long>(), cnt.as<int>());
+    int bits = 1;  // the cell indices' bits: the sort takes a pass for every 8 of the two
+    while ((1ll << bits) < (long long)ncell) bits++;
+    pair_keys_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(pr, n, bits, keys.as<unsigned long long>(),
+                                                                 cnt.as<int>());
     TCHK(hipGetLastError());
-    int hi_bit = 64;  // sort on the bits the cell indices use
-    {
-      int b = 0;
-      while ((1ll << b) < (long long)ncell) b++;
-      hi_bit = 32 + b;
-    }
     hipcub::DoubleBuffer<unsigned long long> db(keys.as<unsigned long long>(), keys2.as<unsigned long long>());
     size_t tb = 0;
-    TCHK(hipcub::DeviceRadixSort::SortKeys(nullptr, tb, db, (int)n, 0, hi_bit, s));
+    TCHK(hipcub::DeviceRadixSort::SortKeys(nullptr, tb, db, (int)n, 0, 2 * bits, s));
     TCHK(tmp.need(tb));
-    TCHK(hipcub::DeviceRadixSort::SortKeys(tmp.p, tb, db, (int)n, 0, hi_bit, s));
+    TCHK(hipcub::DeviceRadixSort::SortKeys(tmp.p, tb, db, (int)n, 0, 2 * bits, s));
     int *dst;
     if (keep) {
       int dev = 0;
@@ -250,7 +248,7 @@ hipError_t pairs_to_csr(const int2 *pr, size_t n, int ncell, std::vector<int> &p
       TCHK(out.need(sizeof(int) * n));
       dst = out.as<int>();
     }
-    key_src_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(db.Current(), n, dst);
+    key_src_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(db.Current(), n, bits, dst);
     TCHK(hipGetLastError());
     if (!keep) TCHK(hipMemcpyAsync(src.data(), out.p, sizeof(int) * n, hipMemcpyDeviceToHost, s));
   } else if (keep) {
