@@ -280,12 +280,23 @@ int download_staged(fmm_ctx *c, void *dst, const void *src, size_t bytes) {
 
 // a device array taken over by a context buffer (both hipMalloc'd)
 void adopt(DBuf &b, fmmdev::DevArray &a) {
+  if (!a.p) return;
   if (b.p) (void)hipFree(b.p);
   b.p = a.p;
-  b.cap = a.bytes;
+  b.cap = a.cap;
   a.p = nullptr;
-  a.bytes = 0;
+  a.bytes = a.cap = 0;
   a.device = -1;
+}
+// and the other way: the buffer's allocation for a builder to fill (hipMalloc
+// and hipFree of the pair arrays took 1.2 ms of a 1M-body step)
+void lend(fmmdev::DevArray &a, DBuf &b, int device) {
+  a.p = b.p;
+  a.cap = b.cap;
+  a.bytes = 0;
+  a.device = b.p ? device : -1;
+  b.p = nullptr;
+  b.cap = 0;
 }
 
 // the host copies of a device-built plan's lists and tiles, for host-side
@@ -512,6 +523,8 @@ void plan_stats(const fmm_plan *pl, fmm_stats &s) {
 // lists_on_device: the lists' source columns are already in c->m2l_src, c->p2p_src
 int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, bool x_on_device = false,
                 bool lists_on_device = false);
+int plan_build_device(fmm_ctx *c, fmm_plan **out, int n, const double *x, int ncrit, double theta, int nspawn,
+                      bool for_upload);
 }  // namespace
 
 int fmm_make_bodies(int n, const char *dist, int seed, double *x, double *q) {
@@ -538,6 +551,14 @@ int fmm_plan_build(fmm_plan **out, int n, const double *x, int ncrit, double the
 // fmm_plan_build with the lists from the device traversal (fmm_traverse.hip)
 int fmm_plan_build_device(fmm_ctx *c, fmm_plan **out, int n, const double *x, int ncrit, double theta,
                           int nspawn) {
+  return plan_build_device(c, out, n, x, ncrit, theta, nspawn, false);
+}
+}  // extern "C"
+
+namespace {
+// for_upload: the plan goes into c next and fills c's own pair arrays
+int plan_build_device(fmm_ctx *c, fmm_plan **out, int n, const double *x, int ncrit, double theta, int nspawn,
+                      bool for_upload) {
   if (!c || !out) return FMM_ERR_ARG;
   *out = nullptr;
   if (n < 0 || (n > 0 && !x) || ncrit < 1 || !(theta > 0) || nspawn < 1)
@@ -579,6 +600,15 @@ int fmm_plan_build_device(fmm_ctx *c, fmm_plan **out, int n, const double *x, in
     const double xper[3] = {0, 0, 0};
     // the source columns stay on the device with the plan (pl->dev)
     pl->dev = std::make_shared<fmmdev::PlanArrays>();
+    if (for_upload) {
+      c->have_bodies = false;
+      graph_reset(c);
+      lend(pl->dev->m2l_src, c->m2l_src, c->p.device);
+      lend(pl->dev->p2p_src, c->p2p_src, c->p.device);
+      lend(pl->dev->t_slice, c->t_slice, c->p.device);
+      lend(pl->dev->t_src, c->t_src, c->p.device);
+      lend(pl->dev->t_lt, c->t_lt, c->p.device);
+    }
     HIPCHK(fmmdev::device_lists(t.ncell, t.X.data(), t.R.data(), t.nchild.data(), t.ichild.data(), t.nbody.data(),
                                 theta, nspawn, xper, 0, 0, L.m2l_ptr, L.m2l_src, L.p2p_ptr, L.p2p_src,
                                 L.p2p_body_pairs, c->st, pl->dev.get()));
@@ -615,6 +645,9 @@ int fmm_plan_build_device(fmm_ctx *c, fmm_plan **out, int n, const double *x, in
   *out = pl.release();
   return FMM_OK;
 }
+}  // namespace
+
+extern "C" {
 
 void fmm_plan_destroy(fmm_plan *pl) { delete pl; }
 
@@ -879,7 +912,7 @@ int fmm_set_bodies_device(fmm_ctx *c, int n, const double *x, const double *q) {
   if (!c->st) FMM_FAIL(FMM_ERR_STATE, "context was not created successfully");
   if (c->p.images != 0) FMM_FAIL(FMM_ERR_UNSUPPORTED, "fmm_set_bodies_device: free space only (images = 0)");
   fmm_plan *pl = nullptr;
-  int rc = fmm_plan_build_device(c, &pl, n, x, c->p.ncrit, c->p.theta, c->p.nspawn);
+  int rc = plan_build_device(c, &pl, n, x, c->p.ncrit, c->p.theta, c->p.nspawn, true);
   if (rc != FMM_OK) return rc;
   // the plan's contents move into the context (no copy of the tree or
   // lists); the bodies are still in c->xin from the tree build
@@ -909,6 +942,7 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
   // device, else from host copies
   const bool on_dev = pl.dev && (pl.dev->lists || pl.dev->tiles) && pl.dev->device == c->p.device;
   if (pl.dev && !on_dev) HIPCHK(plan_to_host(&pl));
+  const bool own = on_dev && pl.dev.use_count() == 1;  // arrays nobody else holds become the context's
   std::shared_ptr<fmmdev::PlanArrays> pdev = on_dev ? pl.dev : nullptr;
   const bool dev_lists = pdev && pdev->lists, dev_tiles = pdev && pdev->tiles;
   const int n = pl.n;
@@ -975,7 +1009,11 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
   HIPCHK(fmmdev::launch_body_leaf((int)t.leaves.size(), c->leaves.as<int>(), c->ibody.as<int>(), c->nbody.as<int>(),
                                   c->body_leaf.as<int>(), c->st));
   UP(m2l_ptr, L.m2l_ptr) UP(m2l_tgt, L.m2l_targets)
-  if (dev_lists) {
+  if (dev_lists && own) {
+    adopt(c->m2l_src, pdev->m2l_src);
+    adopt(c->p2p_src, pdev->p2p_src);
+    lists_on_device = true;
+  } else if (dev_lists) {
     DC(m2l_src, pdev->m2l_src) DC(p2p_src, pdev->p2p_src)
   } else if (!lists_on_device) {
     UP(m2l_src, L.m2l_src) UP(p2p_src, L.p2p_src)
@@ -1051,6 +1089,9 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
         // the lists just uploaded (the host build's groups, classes, tiles
         // and slices), their pair arrays left there; irregular trees and
         // offsets out of the key's range fall back to the host build
+        lend(loc.t_slice, c->t_slice, c->p.device);
+        lend(loc.t_src, c->t_src, c->p.device);
+        lend(loc.t_lt, c->t_lt, c->p.device);
         const hipError_t e = fmmdev::device_groups_tiles(t, L, fmmdev::m2l_tile_targets(c->p.P),
                                                          fmmdev::kM2LSlicePairs, 0, c->groups, tiles, done, c->st,
                                                          &loc, c->m2l_src.as<int>(),
@@ -1065,7 +1106,7 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
         }
       }
       if (!done) {
-        if (dev_lists) {  // host grouping reads them
+        if (dev_lists && !lists_on_device) {  // host grouping reads them
           const hipError_t e = fmmdev::fetch_lists(*pdev, c->lists, c->st);
           if (e != hipSuccess) {
             (void)hipStreamSynchronize(c->st);
@@ -1098,14 +1139,19 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
         tiles = fmm::build_m2l_tiles(t, G, fmmdev::m2l_tile_targets(c->p.P), fmmdev::kM2LSlicePairs, 0);
       c->ntile = (int)(tiles.item.size() / 4);  // work items
       UP(t_tgt, tiles.tgt) UP(t_ptr, tiles.item)
-      if (dt) {
+      if (dt && own) {
+        adopt(c->t_slice, pdev->t_slice);
+        adopt(c->t_src, pdev->t_src);
+        adopt(c->t_lt, pdev->t_lt);
+      } else if (dt) {
         DC(t_slice, pdev->t_slice) DC(t_src, pdev->t_src) DC(t_lt, pdev->t_lt)
-      } else if (loc.tiles) {  // built here on the device
+      } else {
         adopt(c->t_slice, loc.t_slice);
         adopt(c->t_src, loc.t_src);
         adopt(c->t_lt, loc.t_lt);
-      } else {
-        UP(t_slice, tiles.slice) UP(t_src, tiles.src) UP(t_lt, tiles.lt)
+        if (!loc.tiles) {  // not built here on the device
+          UP(t_slice, tiles.slice) UP(t_src, tiles.src) UP(t_lt, tiles.lt)
+        }
       }
       UP(c_dx, G.cdx)
     } else {

@@ -156,13 +156,14 @@ void plan_scratch_release(hipStream_t s);
 // its owner goes; move-only.
 struct DevArray {
   void *p = nullptr;
-  size_t bytes = 0;
+  size_t bytes = 0;  // in use
+  size_t cap = 0;    // allocated
   int device = -1;
   DevArray() = default;
   DevArray(const DevArray &) = delete;
   DevArray &operator=(const DevArray &) = delete;
   ~DevArray() { reset(); }
-  hipError_t alloc(size_t b, int dev);  // the device must be current
+  hipError_t alloc(size_t b, int dev);  // keeps an allocation that is large enough; the device must be current
   void reset();
   template <class T> T *as() const { return static_cast<T *>(p); }
 };

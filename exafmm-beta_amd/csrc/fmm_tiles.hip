@@ -355,9 +355,9 @@ hipError_t device_groups_tiles(const fmm::Tree &t, const fmm::Lists &L, int TT, 
   done = false;
   if (keep) {
     keep->tiles = false;
-    keep->t_slice.reset();
-    keep->t_src.reset();
-    keep->t_lt.reset();
+    keep->t_slice.bytes = 0;
+    keep->t_src.bytes = 0;
+    keep->t_lt.bytes = 0;
     keep->nslice = 0;
   }
   const int nc = t.ncell;

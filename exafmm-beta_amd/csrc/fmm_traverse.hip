@@ -252,7 +252,7 @@ hipError_t pairs_to_csr(const int2 *pr, size_t n, int ncell, std::vector<int> &p
     TCHK(hipGetLastError());
     if (!keep) TCHK(hipMemcpyAsync(src.data(), out.p, sizeof(int) * n, hipMemcpyDeviceToHost, s));
   } else if (keep) {
-    keep->reset();
+    keep->bytes = 0;
   }
   std::vector<int> c((size_t)ncell + 1);
   TCHK(hipMemcpyAsync(c.data(), cnt.p, sizeof(int) * ((size_t)ncell + 1), hipMemcpyDeviceToHost, s));
@@ -474,8 +474,8 @@ hipError_t device_lists(int ncell, const double *X, const double *R, const int *
                         std::vector<int> &p2p_src, int64_t &body_pairs, hipStream_t s, PlanArrays *keep) {
   if (keep) {
     keep->lists = false;
-    keep->m2l_src.reset();
-    keep->p2p_src.reset();
+    keep->m2l_src.bytes = 0;
+    keep->p2p_src.bytes = 0;
     TCHK(hipGetDevice(&keep->device));
   }
   m2l_ptr.assign((size_t)ncell + 1, 0);
@@ -918,14 +918,22 @@ void plan_scratch_release(hipStream_t s) {
 }
 
 hipError_t DevArray::alloc(size_t b, int dev) {
+  if (p && device == dev && cap >= b) {
+    bytes = b;
+    return hipSuccess;
+  }
+  // a context's array that was too small grows by a quarter more, as its other
+  // buffers do
+  const size_t want = cap ? b + b / 4 : b;
   reset();
   if (b == 0) return hipSuccess;
-  hipError_t e = hipMalloc(&p, b);
+  hipError_t e = hipMalloc(&p, want);
   if (e != hipSuccess) {
     p = nullptr;
     return e;
   }
   bytes = b;
+  cap = want;
   device = dev;
   return hipSuccess;
 }
@@ -939,7 +947,7 @@ void DevArray::reset() {
     if (!same && cur >= 0) (void)hipSetDevice(cur);
   }
   p = nullptr;
-  bytes = 0;
+  bytes = cap = 0;
   device = -1;
 }
 
