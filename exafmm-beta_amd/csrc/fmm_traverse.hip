@@ -29,19 +29,6 @@ namespace fmmdev {
 
 namespace {
 
-// this lane's exclusive prefix of v over the wavefront, and the total
-__device__ __forceinline__ int wave_excl(int v, int &total) {
-  const int l = threadIdx.x & 63;
-  int x = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_up(x, o, 64);
-    if (l >= o) x += y;
-  }
-  total = __shfl(x, 63, 64);
-  return x - v;
-}
-
 struct TravCells {
   const double *X;  // 3 per cell
   const double *R;
@@ -88,78 +75,112 @@ __device__ __forceinline__ void classify(const TravCells &t, int Ci, int Cj, dou
 }
 
 // count (write = false) or emit (write = true) one round; cnt[0..2]: M2L,
-// P2P and next-frontier totals (running offsets while writing)
+// P2P and next-frontier totals (running offsets while writing).  The count
+// leaves what every pair becomes for the emission (0 M2L, 1 P2P, 1 + its
+// children if split), which tests only the split ones again.  Bound by the
+// blocks' additions to the three counters, some 3 ns each: a thread takes
+// kTravPairs pairs and a block adds once for 2048 of them (the
+// largest round of a 1M-body tree: 232 us counting and 237 emitting with an
+// addition for 256 pairs, 51 and 92 now).
+constexpr int kTravPairs = 8;
 template <bool WRITE>
 __global__ __launch_bounds__(256) void trav_round_kernel(const int2 *__restrict__ F, int nf, TravCells t, double theta,
                                                          double xp0, double xp1, double xp2, int nspawn,
+                                                         unsigned char *__restrict__ kinds,
                                                          unsigned long long *__restrict__ cnt, int2 *__restrict__ m2l,
                                                          int2 *__restrict__ p2p, int2 *__restrict__ next) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  int kind = -1, na = 0, nb = 0, sa = 0, sb = 0;
-  if (i < nf) {
-    const int2 pr = F[i];
-    classify(t, pr.x, pr.y, theta, xp0, xp1, xp2, nspawn, kind, na, nb, sa, sb);
+  const int i0 = blockIdx.x * (256 * kTravPairs) + threadIdx.x;
+  int na, nb, sa, sb, cm = 0, cp = 0, cn = 0, kd[kTravPairs];
+#pragma unroll
+  for (int k = 0; k < kTravPairs; k++) {
+    const int i = i0 + 256 * k;
+    kd[k] = -1;
+    if (i < nf) {
+      if (WRITE) {
+        kd[k] = kinds[i];
+      } else {
+        const int2 pr = F[i];
+        classify(t, pr.x, pr.y, theta, xp0, xp1, xp2, nspawn, kd[k], na, nb, sa, sb);
+        if (kd[k] == kNext) kd[k] = 1 + na * nb;
+        kinds[i] = (unsigned char)kd[k];
+      }
+    }
+    cm += kd[k] == kM2L;
+    cp += kd[k] == kP2P;
+    cn += kd[k] >= kNext ? kd[k] - 1 : 0;
   }
-  const int cm = kind == kM2L, cp = kind == kP2P, cn = na * nb;
-  // offsets within the wavefront, then within the block (one set of global
-  // atomics per block: per-wavefront atomics on three counters serialised)
-  int tm, tp, tn;
-  const int om = wave_excl(cm, tm), op = wave_excl(cp, tp), on = wave_excl(cn, tn);
-  __shared__ int wtot[3][4];
-  __shared__ unsigned long long bbase[3];
+  // offsets within the wavefront (the three counts packed), then in the block
+  const unsigned long long mine = (unsigned long long)cn << 32 | (unsigned)(cm | cp << 16);
+  unsigned long long off = mine;
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned long long y = __shfl_up(off, o, 64);
+    if (lane >= o) off += y;
+  }
+  __shared__ unsigned long long wtot[4], bbase[3];
   const int wv = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) {
-    wtot[0][wv] = tm;
-    wtot[1][wv] = tp;
-    wtot[2][wv] = tn;
-  }
+  if (lane == 63) wtot[wv] = off;
+  off -= mine;
   __syncthreads();
   if (threadIdx.x < 3) {
-    int tot = 0;
-    for (int k = 0; k < 4; k++) tot += wtot[threadIdx.x][k];
-    bbase[threadIdx.x] = tot ? atomicAdd(&cnt[threadIdx.x], (unsigned long long)tot) : 0ull;
+    const unsigned long long sum = wtot[0] + wtot[1] + wtot[2] + wtot[3];
+    const unsigned long long v =
+        threadIdx.x == 0 ? sum & 0xffff : threadIdx.x == 1 ? sum >> 16 & 0xffff : sum >> 32;
+    bbase[threadIdx.x] = v ? atomicAdd(&cnt[threadIdx.x], v) : 0ull;
   }
-  __syncthreads();
   if (!WRITE) return;
-  int pm = 0, pp = 0, pn = 0;  // the earlier wavefronts' counts
-  for (int k = 0; k < wv; k++) {
-    pm += wtot[0][k];
-    pp += wtot[1][k];
-    pn += wtot[2][k];
-  }
-  const unsigned long long bm = bbase[0] + pm, bp = bbase[1] + pp, bn = bbase[2] + pn;
-  if (i >= nf) return;
-  const int2 pr = F[i];
-  if (cm) m2l[bm + om] = pr;
-  if (cp) p2p[bp + op] = pr;
-  if (cn) {
-    int2 *o = next + bn + on;
-    for (int a = 0; a < na; a++)
-      for (int b = 0; b < nb; b++) o[a * nb + b] = make_int2(sa + a, sb + b);
+  __syncthreads();
+  for (int k = 0; k < wv; k++) off += wtot[k];  // the earlier wavefronts' counts
+  int2 *om = m2l + bbase[0] + (off & 0xffff), *op = p2p + bbase[1] + (off >> 16 & 0xffff),
+       *on = next + bbase[2] + (off >> 32);
+#pragma unroll
+  for (int k = 0; k < kTravPairs; k++) {
+    if (kd[k] < 0) continue;
+    const int2 pr = F[i0 + 256 * k];
+    if (kd[k] == kM2L) {
+      *om++ = pr;
+    } else if (kd[k] == kP2P) {
+      *op++ = pr;
+    } else {
+      int kind;
+      classify(t, pr.x, pr.y, theta, xp0, xp1, xp2, nspawn, kind, na, nb, sa, sb);
+      for (int a = 0; a < na; a++)
+        for (int b = 0; b < nb; b++) *on++ = make_int2(sa + a, sb + b);
+    }
   }
 }
 
-// sort keys (target, source) and the per-target counts; a wavefront's lanes
-// holding one target in a row (the traversal emits a target's pairs
-// together) add their count with one atomic
+// sort keys (target, source)
 __global__ void pair_keys_kernel(const int2 *__restrict__ pr, size_t n, int bits,
-                                 unsigned long long *__restrict__ key, int *__restrict__ count) {
+                                 unsigned long long *__restrict__ key) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int lane = threadIdx.x & 63;
-  int t = -1;
-  if (i < n) {
-    const int2 p = pr[i];
-    key[i] = ((unsigned long long)(unsigned)p.x << bits) | (unsigned)p.y;
-    t = p.x;
+  if (i >= n) return;
+  const int2 p = pr[i];
+  key[i] = ((unsigned long long)(unsigned)p.x << bits) | (unsigned)p.y;
+}
+
+// sorted keys below k
+template <typename K>
+__device__ __forceinline__ int keys_below(const K *__restrict__ key, int n, K k) {
+  int lo = 0, hi = n;
+  while (lo < hi) {
+    const int m = (lo + hi) >> 1;
+    if (key[m] < k)
+      lo = m + 1;
+    else
+      hi = m;
   }
-  const int prev = __shfl_up(t, 1, 64);
-  const bool head = lane == 0 || prev != t;
-  const unsigned long long heads = __ballot(head);
-  if (head && t >= 0) {
-    const unsigned long long above = lane == 63 ? 0ull : heads >> (lane + 1);
-    const int len = above ? __ffsll((long long)above) : 64 - lane;
-    atomicAdd(&count[t], len);
-  }
+  return lo;
+}
+
+// ptr[c] = first pair of target c in the sorted keys, c = 0 .. ncell (counts
+// by atomics while the keys are made took 86 us for 12M pairs in the order of
+// their targets and 478 us otherwise; this takes 8)
+__global__ void pair_ptr_kernel(int ncell, const unsigned long long *__restrict__ key, int n, int bits,
+                                int *__restrict__ ptr) {
+  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c <= ncell) ptr[c] = keys_below(key, n, (unsigned long long)c << bits);
 }
 
 __global__ void key_src_kernel(const unsigned long long *__restrict__ key, size_t n, int bits,
@@ -222,16 +243,13 @@ hipError_t pairs_to_csr(const int2 *pr, size_t n, int ncell, std::vector<int> &p
   ptr.assign((size_t)ncell + 1, 0);
   src.clear();
   if (!keep) src.resize(n);
-  Buf keys(s), keys2(s), cnt(s), tmp(s), out(s);
-  TCHK(cnt.need(sizeof(int) * ((size_t)ncell + 1)));
-  TCHK(hipMemsetAsync(cnt.p, 0, sizeof(int) * ((size_t)ncell + 1), s));
+  Buf keys(s), keys2(s), dptr(s), tmp(s), out(s);
   if (n > 0) {
     TCHK(keys.need(8 * n));
     TCHK(keys2.need(8 * n));
     int bits = 1;  // the cell indices' bits: the sort takes a pass for every 8 of the two
     while ((1ll << bits) < (long long)ncell) bits++;
-    pair_keys_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(pr, n, bits, keys.as<unsigned long long>(),
-                                                                 cnt.as<int>());
+    pair_keys_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(pr, n, bits, keys.as<unsigned long long>());
     TCHK(hipGetLastError());
     hipcub::DoubleBuffer<unsigned long long> db(keys.as<unsigned long long>(), keys2.as<unsigned long long>());
     size_t tb = 0;
@@ -251,21 +269,15 @@ hipError_t pairs_to_csr(const int2 *pr, size_t n, int ncell, std::vector<int> &p
     key_src_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(db.Current(), n, bits, dst);
     TCHK(hipGetLastError());
     if (!keep) TCHK(hipMemcpyAsync(src.data(), out.p, sizeof(int) * n, hipMemcpyDeviceToHost, s));
+    TCHK(dptr.need(sizeof(int) * ((size_t)ncell + 1)));
+    pair_ptr_kernel<<<(unsigned)(ncell / 256 + 1), 256, 0, s>>>(ncell, db.Current(), (int)n, bits, dptr.as<int>());
+    TCHK(hipGetLastError());
+    TCHK(hipMemcpyAsync(ptr.data(), dptr.p, sizeof(int) * ((size_t)ncell + 1), hipMemcpyDeviceToHost, s));
   } else if (keep) {
     keep->bytes = 0;
   }
-  std::vector<int> c((size_t)ncell + 1);
-  TCHK(hipMemcpyAsync(c.data(), cnt.p, sizeof(int) * ((size_t)ncell + 1), hipMemcpyDeviceToHost, s));
-  TCHK(hipStreamSynchronize(s));
-  int64_t a = 0;
-  for (int i = 0; i < ncell; i++) {
-    ptr[i] = (int)a;
-    a += c[i];
-  }
-  ptr[ncell] = (int)a;
-  return hipSuccess;
+  return hipStreamSynchronize(s);
 }
-
 
 // ---- the octree (include/build_tree.h:77-209, as fmm_host.cpp builds it) ----
 //
@@ -484,7 +496,7 @@ hipError_t device_lists(int ncell, const double *X, const double *R, const int *
   p2p_src.clear();
   body_pairs = 0;
   if (ncell == 0) return hipSuccess;
-  Buf dX(s), dR(s), dnc(s), dic(s), dnb(s), cnt(s), F0(s), F1(s), M(s), Pp(s), bp(s);
+  Buf dX(s), dR(s), dnc(s), dic(s), dnb(s), cnt(s), F0(s), F1(s), M(s), Pp(s), bp(s), kinds(s);
   TCHK(dX.need(sizeof(double) * 3 * (size_t)ncell));
   TCHK(dR.need(sizeof(double) * (size_t)ncell));
   TCHK(dnc.need(sizeof(int) * (size_t)ncell));
@@ -509,9 +521,10 @@ hipError_t device_lists(int ncell, const double *X, const double *R, const int *
     if (nf > 0x7fffffff) return hipErrorInvalidValue;  // frontier beyond one launch's index range
     // count: the M2L, P2P and next-frontier pairs of this traversal round
     TCHK(hipMemsetAsync(cnt.p, 0, sizeof(h), s));
-    const unsigned nb = (unsigned)((nf + 255) / 256);
+    const unsigned nb = (unsigned)((nf + 256 * kTravPairs - 1) / (256 * kTravPairs));
+    TCHK(kinds.need(nf));
     trav_round_kernel<false><<<nb, 256, 0, s>>>(F0.as<int2>(), (int)nf, t, theta, xper[0], xper[1], xper[2], nspawn,
-                                                cnt.as<unsigned long long>(), nullptr, nullptr, nullptr);
+                                                kinds.as<unsigned char>(), cnt.as<unsigned long long>(), nullptr, nullptr, nullptr);
     TCHK(hipGetLastError());
     TCHK(hipMemcpyAsync(h, cnt.p, sizeof(h), hipMemcpyDeviceToHost, s));
     TCHK(hipStreamSynchronize(s));
@@ -531,7 +544,7 @@ hipError_t device_lists(int ncell, const double *X, const double *R, const int *
     const unsigned long long base[3] = {nm, np, 0};
     TCHK(hipMemcpyAsync(cnt.p, base, sizeof(base), hipMemcpyHostToDevice, s));
     trav_round_kernel<true><<<nb, 256, 0, s>>>(F0.as<int2>(), (int)nf, t, theta, xper[0], xper[1], xper[2], nspawn,
-                                               cnt.as<unsigned long long>(), M.as<int2>(), Pp.as<int2>(),
+                                               kinds.as<unsigned char>(), cnt.as<unsigned long long>(), M.as<int2>(), Pp.as<int2>(),
                                                F1.as<int2>());
     TCHK(hipGetLastError());
     nm += h[0];
@@ -698,19 +711,9 @@ __global__ void visit_ptr_kernel(int ncell, int n, const unsigned *__restrict__ 
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= 2 * (ncell + 1)) return;
   const bool p2p = i > ncell;
-  auto below = [&](unsigned k) {  // keys < k
-    int lo = 0, hi = n;
-    while (lo < hi) {
-      const int m = (lo + hi) >> 1;
-      if (key[m] < k)
-        lo = m + 1;
-      else
-        hi = m;
-    }
-    return lo;
-  };
   const unsigned list = (unsigned)kP2P << tbits;
-  ptr[i] = p2p ? below(list + (unsigned)(i - ncell - 1)) - below(list) : below((unsigned)i);
+  ptr[i] = p2p ? keys_below(key, n, list + (unsigned)(i - ncell - 1)) - keys_below(key, n, list)
+               : keys_below(key, n, (unsigned)i);
 }
 }  // namespace
 
