@@ -478,9 +478,11 @@ int groups_kind_for(const fmm_params &p) {
   return p.precision != FMM_FP64 && !takes_tiles(p) ? FMM_MIXED : FMM_FP64;
 }
 
-// lists: the interaction lists of pl->tree, if not walked on the host
+// tree, lists: the tree of the bodies and the lists of pl->tree where they are
+// not made on the host (false: they are)
 void plan_fill(fmm_plan *pl, int n, const double *x, int ncrit, double theta, int nspawn, int images = 0,
-               const double *cycle = nullptr, const std::function<bool(fmm_plan &)> &lists = nullptr) {
+               const double *cycle = nullptr, const std::function<bool(fmm_plan &)> &tree = nullptr,
+               const std::function<bool(fmm_plan &)> &lists = nullptr) {
   pl->images = images;
   if (images > 0)
     for (int d = 0; d < 3; d++) pl->cycle[d] = cycle[d];
@@ -488,7 +490,7 @@ void plan_fill(fmm_plan *pl, int n, const double *x, int ncrit, double theta, in
   double t0 = now_ms();
   fmm::get_bounds(n, x, pl->xmin, pl->xmax);
   double t1 = now_ms();
-  pl->tree = fmm::build_tree(n, x, ncrit, pl->xmin, pl->xmax);
+  if (!tree || !tree(*pl)) pl->tree = fmm::build_tree(n, x, ncrit, pl->xmin, pl->xmax);
   double t2 = now_ms();
   const double xper[3] = {0, 0, 0};
   if (!lists || !lists(*pl)) pl->lists = fmm::build_lists(pl->tree, theta, nspawn, xper, images, pl->cycle);
@@ -556,6 +558,32 @@ int fmm_plan_build_device(fmm_ctx *c, fmm_plan **out, int n, const double *x, in
 }  // extern "C"
 
 namespace {
+// the tree of n bodies built on the device (fmm::build_tree's cells and order);
+// the bodies are left in c->xin
+int device_tree_of(fmm_ctx *c, fmm::Tree &t, int n, const double *x, int ncrit, const double *xmin,
+                   const double *xmax) {
+  t = fmm::Tree();
+  t.n = n;
+  if (n == 0) {
+    t.level_ptr.assign(1, 0);
+    return FMM_OK;
+  }
+  double X0[3], R0;
+  fmm::root_box(xmin, xmax, X0, R0);
+  // the bodies go up through the context's pinned staging into its
+  // upload buffer (scratch between uploads)
+  const int rc = upload_staged(c, {{&c->xin, x, sizeof(double) * 3 * (size_t)n}});
+  if (rc) {
+    (void)hipStreamSynchronize(c->st);
+    return rc;
+  }
+  HIPCHK(fmmdev::device_tree(n, x, ncrit, X0, R0, t.perm, t.iparent, t.ichild, t.nchild, t.ibody, t.nbody, t.level,
+                             t.X, t.R, c->st, c->xin.as<double>()));
+  t.ncell = (int)t.nbody.size();
+  fmm::finish_tree(t);
+  return FMM_OK;
+}
+
 // for_upload: the plan goes into c next and fills c's own pair arrays
 int plan_build_device(fmm_ctx *c, fmm_plan **out, int n, const double *x, int ncrit, double theta, int nspawn,
                       bool for_upload) {
@@ -573,26 +601,8 @@ int plan_build_device(fmm_ctx *c, fmm_plan **out, int n, const double *x, int nc
     double t1 = now_ms();
     HIPCHK(hipSetDevice(c->p.device));
     {
-      fmm::Tree &t = pl->tree;
-      t = fmm::Tree();
-      t.n = n;
-      if (n > 0) {
-        double X0[3], R0;
-        fmm::root_box(pl->xmin, pl->xmax, X0, R0);
-        // the bodies go up through the context's pinned staging into its
-        // upload buffer (scratch between uploads)
-        int rc = upload_staged(c, {{&c->xin, x, sizeof(double) * 3 * (size_t)n}});
-        if (rc) {
-          (void)hipStreamSynchronize(c->st);
-          return rc;
-        }
-        HIPCHK(fmmdev::device_tree(n, x, ncrit, X0, R0, t.perm, t.iparent, t.ichild, t.nchild, t.ibody, t.nbody,
-                                   t.level, t.X, t.R, c->st, c->xin.as<double>()));
-        t.ncell = (int)t.nbody.size();
-        fmm::finish_tree(t);
-      } else {
-        t.level_ptr.assign(1, 0);
-      }
+      const int rc = device_tree_of(c, pl->tree, n, x, ncrit, pl->xmin, pl->xmax);
+      if (rc) return rc;
     }
     double t2 = now_ms();
     const fmm::Tree &t = pl->tree;
@@ -878,6 +888,21 @@ int fmm_set_bodies(fmm_ctx *c, int n, const double *x, const double *q) {
   // 97810 cells 43 and 4.0; with periodic images (27 roots) 81 cells 0.18 and
   // 0.39, 585 cells 1.2 and 0.53, 4830 cells 7.6 and 0.95.
   const int least = c->p.images > 0 ? 200 : 600;
+  // The device tree takes 0.7 ms at least (its sorts and level launches): at
+  // 16000 bodies the whole call 2.46 ms against 2.04 with the host's, at 62000
+  // 2.87 and 3.39 (uniform 2.95 and 3.32), at 2^20 11.7 and 20.6, at 2^23 66
+  // and 300.
+  constexpr int least_bodies = 50000;
+  bool x_on_device = false;
+  const auto tree = [&](fmm_plan &p) {
+    if (n < least_bodies) return false;
+    x_on_device = device_tree_of(c, p.tree, n, x, c->p.ncrit, p.xmin, p.xmax) == FMM_OK;
+    if (!x_on_device) {  // no room beside the solve's buffers: the host builds it
+      (void)hipStreamSynchronize(c->st);
+      (void)hipGetLastError();
+    }
+    return x_on_device;
+  };
   const auto lists = [&](fmm_plan &p) {
     if (p.tree.ncell < least) return false;
     c->have_bodies = false;  // the columns of the bodies before are overwritten
@@ -898,12 +923,12 @@ int fmm_set_bodies(fmm_ctx *c, int n, const double *x, const double *q) {
     return on_device || e != hipSuccess;
   };
   try {
-    plan_fill(&pl, n, x, c->p.ncrit, c->p.theta, c->p.nspawn, c->p.images, c->p.cycle, lists);
+    plan_fill(&pl, n, x, c->p.ncrit, c->p.theta, c->p.nspawn, c->p.images, c->p.cycle, tree, lists);
   } catch (const std::bad_alloc &) {
     FMM_FAIL(FMM_ERR_MEMORY, "host allocation failed while building the tree");
   }
   HIPCHK(e);
-  return upload_plan(c, std::move(pl), x, q, false, on_device);
+  return upload_plan(c, std::move(pl), x, q, x_on_device, on_device);
 }
 
 int fmm_set_bodies_device(fmm_ctx *c, int n, const double *x, const double *q) {

@@ -42,3 +42,23 @@ def test_lists_in_the_host_order(dist, n, theta, ncrit, nspawn, images):
             assert f.stats()[k] == h.stats()[k] > 0, k
         for a, b in zip(f.lists(), h.lists()):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("dist,n,ncrit,images", [("cube1", 50000, 64, 0), ("plummer1", 50021, 10, 0),
+                                                 ("line", 60000, 32, 0), ("plummer1", 50000, 64, 1)])
+def test_tree_of_many_bodies(dist, n, ncrit, images):
+    """From 50000 bodies the tree of fmm_set_bodies is built on the device too:
+    the host's cells, numbers and body order, and its lists."""
+    import exafmm_amd as F
+    x, q = _bodies(F, dist, n)
+    x[7] = x[5]
+    kw = dict(images=images, cycle=float(2 * abs(x).max())) if images else {}
+    h = F.Plan(x, ncrit=ncrit, theta=0.5)
+    with F.FMM(P=4, theta=0.5, ncrit=ncrit, **kw) as f:
+        f.set_bodies(x, q)
+        a, b = f.tree(), h.tree()
+        for k in ("perm", "iparent", "ichild", "nchild", "ibody", "nbody", "X", "R"):
+            assert np.array_equal(a[k], b[k]), k
+        if not images:
+            for u, v in zip(f.lists(), h.lists()):
+                assert np.array_equal(u, v)
