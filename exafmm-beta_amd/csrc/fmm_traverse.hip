@@ -176,7 +176,7 @@ __device__ __forceinline__ int keys_below(const K *__restrict__ key, int n, K k)
 
 // ptr[c] = first pair of target c in the sorted keys, c = 0 .. ncell (counts
 // by atomics while the keys are made took 86 us for 12M pairs in the order of
-// their targets and 478 us otherwise; this takes 8)
+// their targets and 478 us otherwise; this takes 10)
 __global__ void pair_ptr_kernel(int ncell, const unsigned long long *__restrict__ key, int n, int bits,
                                 int *__restrict__ ptr) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
@@ -634,29 +634,37 @@ __global__ __launch_bounds__(256) void visit_count_kernel(const int2 *__restrict
   cn[i] = na * nb;
 }
 
-// the next round: the children of every split pair from slot co[i] on, a
-// wavefront's lanes a pair's children
+// the next round: the children of every split pair from slot co[i] on.  A
+// wavefront takes 64 pairs and its lanes their children, each finding its pair
+// by a search in the pairs' slots (pair by pair, a lane a child, the rounds of
+// a 62k-body tree took 16 us each, most of it for pairs of a few children;
+// 8 us now)
 __global__ __launch_bounds__(256) void visit_expand_kernel(const int2 *__restrict__ F, int nf, TravCells t,
                                                            double theta, Shifts sh, int nspawn,
                                                            const unsigned char *__restrict__ kind,
                                                            const int *__restrict__ co, int2 *__restrict__ next,
                                                            int *__restrict__ par) {
-  const int i0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 64, lane = threadIdx.x & 63;
-  int na = 0, nb = 0, sa = 0, sb = 0, at = 0;
-  const int i = i0 + lane;
+  __shared__ int soff[4][65], sa0[4][64], sb0[4][64], snn[4][64];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, i0 = (blockIdx.x * 4 + w) * 64, i = i0 + lane;
+  int *off = soff[w];
+  off[lane] = co[min(i, nf)];
+  if (lane == 63) off[64] = co[min(i0 + 64, nf)];
   if (i < nf && kind[i] == kNext) {
+    int na, nb, sa, sb;
     visit_kind(t, F[i], theta, sh, nspawn, na, nb, sa, sb);
-    sb |= F[i].y & ~fmm::kCellMask;
-    at = co[i];
+    sa0[w][lane] = sa;
+    sb0[w][lane] = sb | (F[i].y & ~fmm::kCellMask);
+    snn[w][lane] = 8 * (na - 1) + nb - 1;
   }
-  for (unsigned long long m = __ballot(na > 0); m; m &= m - 1) {
-    const int l = __ffsll((long long)m) - 1;
-    const int a = __shfl(na, l), b = __shfl(nb, l), ca = __shfl(sa, l), cb = __shfl(sb, l), o = __shfl(at, l);
-    if (lane < a * b) {
-      const int k = kVisit.o[a - 1][b - 1][lane];
-      next[o + lane] = make_int2(ca + (k >> 3), cb + (k & 7));
-      par[o + lane] = i0 + l;
-    }
+  __syncthreads();
+  for (int c = off[0] + lane; c < off[64]; c += 64) {
+    int l = 0;  // the last pair with off[l] <= c: the one that has child c
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1)
+      if (off[l + d] <= c) l += d;
+    const int k = (&kVisit.o[0][0][0])[64 * snn[w][l] + c - off[l]];
+    next[c] = make_int2(sa0[w][l] + (k >> 3), sb0[w][l] + (k & 7));
+    par[c] = i0 + l;
   }
 }
 
