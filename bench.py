@@ -35,7 +35,6 @@ METRIC = "particles/s per FMM solve + p50/p99 latency, mixed vs FP64 at equal L2
 PEAK_FP64_TFLOPS = 78.6   # MI355X FP64 (vector and matrix)
 PEAK_FP32_TFLOPS = 157.3  # MI355X FP32 matrix (MFMA)
 PEAK_FP32_VALU_TFLOPS = 157.3  # MI355X FP32 vector (the packed-FP32 rate)
-PEAK_FP16_TFLOPS = 2500.0  # MI355X FP16 dense MFMA
 PEAK_HBM_GBS = 8000.0
 
 WORKLOADS = {
@@ -201,11 +200,16 @@ def m2l_flops(P, pairs):
     return 8.0 * (P * (P + 1) // 2) * P * P * pairs
 
 
-def m2l_exec_flops(P, pairs):
-    """M2L work as the kernels execute it: one dense real P^2 x P^2 operator
-    applied per pair (2 P^4 flop), without the padding of partly filled
-    slices or chunks."""
-    return 2.0 * P ** 4 * pairs
+def m2l_exec_flops(P, pairs, tiles):
+    """M2L work as the kernels execute it, without the padding of partly filled
+    4 x 4 blocks, slices or chunks.  Target tiles: rotate, shift, rotate back
+    (Re and Im parts: (n+1)^2 and n^2 multiply-adds a degree in each rotation,
+    (P-m)^2 an order in the shift, 4 a term in each rotation about z); chunks
+    and per target: one dense real P^2 x P^2 operator."""
+    if not tiles:
+        return 2.0 * P ** 4 * pairs
+    blocks = sum((n + 1) ** 2 + n ** 2 for n in range(P))
+    return 2.0 * (3 * blocks + 8 * (P * (P + 1) // 2)) * pairs
 
 
 def p2p_flops(body_pairs):
@@ -340,12 +344,11 @@ def solve_and_time(F, w, plan, x, q, precision, steps, warmup, log, m2l_mode=0, 
     f.close()
     m2l_ms, p2p_ms = float(np.mean(km)), float(np.mean(kp))
     fm = m2l_flops(P, st["m2l_pairs"])
-    fe = m2l_exec_flops(P, st["m2l_pairs"])
+    tiles = st["m2l_path"] == F.M2L_TILES
+    fe = m2l_exec_flops(P, st["m2l_pairs"], tiles)
     fp = p2p_flops(st["p2p_body_pairs"])
-    # mixed16: three FP16 products (hi x hi, hi x lo, lo x hi) per dense term
-    peak = {"fp64": PEAK_FP64_TFLOPS, "mixed": PEAK_FP32_TFLOPS, "mixed16": PEAK_FP16_TFLOPS}[precision]
-    if precision == "mixed16":
-        fe = 3 * fe
+    # the tiles' M2L runs in FP64 in every precision, mixed chunks on FP32 operands
+    peak = PEAK_FP64_TFLOPS if tiles or precision == "fp64" else PEAK_FP32_TFLOPS
     return {
         "wall_s": wall, "lat": lat, "dev": dev, "st": st, "trg": trg, "perm": perm,
         "accuracy": {"pot_rel_l2": pot_rel, "acc_rel_l2": acc_rel, "targets": int(w["ntarget"]),
@@ -566,16 +569,17 @@ def main():
     kernels = r["kernels"]
     dom = "m2l" if kernels["m2l"]["avg_ms"] >= kernels["p2p"]["avg_ms"] else "p2p"
     kd = kernels[dom]
-    # M2L runs on MFMA (FP64 MFMA, or FP32 MFMA when mixed); achieved/frac use
-    # the algorithmic count, *_executed the dense real form the MFMAs execute
+    # M2L runs on MFMA; achieved/frac use the algorithmic count, *_executed the
+    # multiply-adds of the form that runs
     roofline = {"bound": "mfma", "kernel": dom, "achieved": kd["tflops"], "peak": kd["peak_tflops"],
                 "unit": "TFLOP/s", "frac": kd["frac"],
                 "traffic": traffic_from_profile(args.workload, dom)}
     if dom == "m2l":
         roofline.update(achieved_executed=kd["exec_tflops"], frac_executed=kd["frac_executed"],
                         count="achieved: 8*NTERM*P^2 flop per M2L pair (the reference's complex "
-                              "NTERM x P^2 product); achieved_executed: 2*P^4 per pair (the dense "
-                              "real operator applied on MFMA, padding not counted)")
+                              "NTERM x P^2 product); achieved_executed: the multiply-adds of the "
+                              "kernel's own form (tiles: rotate, shift, rotate back; padding not "
+                              "counted)")
     host_ms = st["host_bounds_ms"] + st["host_tree_ms"] + st["host_lists_ms"] + st["host_upload_ms"]
     value = n * args.steps / r["wall_s"]
     out = {
@@ -629,7 +633,7 @@ def main():
                          "frac_executed": rm["kernels"]["m2l"]["frac_executed"]}}
         out["mixed_over_fp64"] = vm / value
         out["mixed_vs_fp64_rel_l2"] = dict(zip(("pot", "acc"), rel_l2(r["trg"], rm["trg"])))
-        # the same with the M2L on split-FP16 operands (FMM_MIXED16)
+        # the same as FMM_MIXED16
         rh = solve_and_time(F, w, plan, x, q, "mixed16", args.steps, args.warmup, log, args.m2l_mode)
         vh = n * args.steps / rh["wall_s"]
         out["mixed16_same_system"] = {

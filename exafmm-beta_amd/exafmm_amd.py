@@ -36,8 +36,8 @@ SYMBOLS = [
 
 FMM_FP64 = 0
 FMM_MIXED = 1
-FMM_MIXED16 = 2  # mixed with the M2L on split-FP16 operands (hi + lo halves, FP32 accumulate)
-M2L_AUTO = 0      # offset groups on MFMA in target tiles (P <= 12), else per target
+FMM_MIXED16 = 2  # as FMM_MIXED, on target tiles only
+M2L_AUTO = 0      # target tiles (P <= 12), else per target
 M2L_TARGET = 1    # per-target kernel on vector ALUs, fixed summation order
 M2L_GROUPED = 2   # offset groups on MFMA, one block per group chunk, FP64 atomics
 M2L_TILES = 3     # offset groups on MFMA, one block per target tile, LDS accumulation

@@ -169,7 +169,9 @@ const char *fmm_last_error(const fmm_ctx *c);
 
 /* Replaces BoundBox::getBounds + BuildTree::buildTree (include/bound_box.h:11-25,
  * include/build_tree.h:186-209) and the list part of Traversal::traverse
- * (include/traversal.h:326-352): host bounds, octree and interaction lists,
+ * (include/traversal.h:326-352): bounds, octree and interaction lists on the
+ * host, the octree of 50000 bodies and more and the lists of some hundred
+ * cells and more on the device (the same cells and lists, in the same order),
  * then upload of bodies (in tree order), cells and lists.  x is (n,3) in the
  * caller's order. */
 int fmm_set_bodies(fmm_ctx *c, int n, const double *x, const double *q);
