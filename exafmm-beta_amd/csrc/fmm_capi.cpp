@@ -157,7 +157,14 @@ int ensure(fmm_ctx *c, DBuf &b, size_t bytes) {
   // 25% headroom: a stream of slightly growing systems reallocates rarely
   // (hipMalloc/hipFree synchronise the device)
   size_t sz = bytes ? bytes + bytes / 4 : 16;
-  HIPCHK(hipMalloc(&b.p, sz));
+  hipError_t e = hipMalloc(&b.p, sz);
+  if (e == hipErrorOutOfMemory && c->st) {  // the builders' idle scratch makes room
+    (void)hipGetLastError();
+    fmmdev::plan_scratch_release(c->st);
+    e = hipMalloc(&b.p, sz);
+  }
+  if (e != hipSuccess) b.p = nullptr;
+  HIPCHK(e);
   b.cap = sz;
   return FMM_OK;
 }

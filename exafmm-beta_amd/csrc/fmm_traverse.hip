@@ -892,6 +892,11 @@ hipError_t plan_scratch_get(void **p, size_t *cap, size_t bytes, hipStream_t s) 
     }
   }
   hipError_t e = hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory) {  // blocks of other sizes kept for this stream make room
+    (void)hipGetLastError();
+    plan_scratch_release(s);
+    e = hipMalloc(p, bytes);
+  }
   if (e != hipSuccess) {
     *p = nullptr;
     return e;
