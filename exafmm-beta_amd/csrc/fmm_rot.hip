@@ -535,9 +535,9 @@ template <int P> struct Rot {
 // part's products and by the second wavefront of the SIMD (registers: the
 // record alone takes 108 at P = 12).  Measured on MI355X against one dense
 // operator per class on v_mfma_f64_16x16x4 (same lists), M2L in ms: 8M cube,
-// P = 12: 155 -> 47; 1M Plummer, P = 10: 6.7 -> 2.9; 10^6 cube, P = 8: 3.7 ->
+// P = 12: 155 -> 42.5; 1M Plummer, P = 10: 6.7 -> 3.0; 10^6 cube, P = 8: 3.7 ->
 // 2.1, P = 4: 1.10 -> 0.66; also against FP32 (P = 12 10.4 ms, P = 8 2.65) and
-// split-FP16 (8.4, 2.27) dense operators on that cube (5.2, 2.1 here).
+// split-FP16 (8.4, 2.27) dense operators on that cube (4.6, 2.1 here).
 // TT: what LDS leaves room for with 8 wavefronts a CU (P >= 9), 16 below.
 template <int P, int TT>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void m2l_rot_kernel(

@@ -1,12 +1,13 @@
 // fmm_tiles.hip -- the M2L offset groups and target tiles built on the device.
 //
 // The same partition as fmm::build_m2l_groups and the same tiles, slices and
-// work items as fmm::build_m2l_tiles (fmm_host.cpp), for trees whose cells all have the radius of their level (trees built by
-// fmm::build_tree or fmmdev::device_tree):
+// work items as fmm::build_m2l_tiles (fmm_host.cpp), for trees whose cells all
+// have the radius of their level (trees built by fmm::build_tree or
+// fmmdev::device_tree):
 //
 //  * every M2L pair's offset, in units of its finer cell's size, reduced by
-//    common factors of two (the host's lattice key), packed into one 64-bit key; a hash table on the device gives
-//    each pair its key's slot;
+//    common factors of two (the host's lattice key), packed into one 64-bit
+//    key; a hash table gives each pair its key's slot;
 //  * over the distinct keys only (thousands): group numbers in key order,
 //    reflection classes and their representatives' offsets -- the host's
 //    numbering is first-appearance order, which only permutes the groups and
