@@ -24,6 +24,7 @@
 #include <type_traits>
 
 #include "fmm_device.hpp"
+#include "fmm_p2m_lanes.hpp"
 
 namespace fmmdev {
 
@@ -140,12 +141,14 @@ __device__ void regular_column(double dx, double dy, double dz, int m, double2 *
 template <int P, int S>
 __global__ __launch_bounds__(64) void p2m_kernel(DevBodies B, DevCells C, const int *__restrict__ leaves,
                                                  int nleaf, double2 *__restrict__ M) {
-  constexpr int NT = nterm(P), H = (P + 1) / 2, LW = 64 / (H * S);
+  using Ln = P2MLanes<P, S>;
+  static_assert(Ln::sound(), "a group's sums are read from its own row and leaf");
+  constexpr int NT = nterm(P);
   __shared__ double2 sRed[S > 1 ? 64 * (P + 1) : 1];
   const int lane = threadIdx.x;
-  const int h = lane % H, slot = lane / H % S, lf = lane / (H * S);
-  const int li = blockIdx.x * LW + lf;
-  const bool act = lf < LW && li < nleaf;
+  const int h = Ln::column(lane), slot = Ln::slot(lane);
+  const int li = blockIdx.x * Ln::LW + Ln::leaf(lane);
+  const bool act = Ln::holds(lane) && li < nleaf;
   const int c = act ? leaves[li] : 0;
   const double Xc = C.cx[c], Yc = C.cy[c], Zc = C.cz[c];
   const int b1 = act ? C.ibody[c] + C.nbody[c] : 0;
@@ -215,10 +218,10 @@ __global__ __launch_bounds__(64) void p2m_kernel(DevBodies B, DevCells C, const 
 #pragma unroll
     for (int t = 0; t <= P; t++) sRed[t * 64 + lane] = acc[t];
     __syncthreads();
-    if (slot == 0) {
+    if (Ln::adds(lane)) {
 #pragma unroll
       for (int t = 0; t <= P; t++)
-        for (int k = 1; k < S; k++) acc[t] = cadd(acc[t], sRed[t * 64 + lane + H * k]);
+        for (int k = 1; k < S; k++) acc[t] = cadd(acc[t], sRed[Ln::entry(t, lane, k)]);
     }
   }
   if (!act || slot > 0) return;
@@ -2098,7 +2101,7 @@ static hipError_t dispatch(int P, A... a) {
 
 template <int P> struct RunP2M {
   template <int S> static void go(DevBodies B, DevCells C, const int *leaves, int nleaf, double2 *M, hipStream_t s) {
-    constexpr int LW = 64 / ((P + 1) / 2 * S);
+    constexpr int LW = P2MLanes<P, S>::LW;
     hipLaunchKernelGGL((p2m_kernel<P, S>), dim3((nleaf + LW - 1) / LW), dim3(64), 0, s, B, C, leaves, nleaf, M);
   }
   static hipError_t run(DevBodies B, DevCells C, const int *leaves, int nleaf, double2 *M, hipStream_t s) {
