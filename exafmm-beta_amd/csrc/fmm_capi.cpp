@@ -469,6 +469,16 @@ void fmm_destroy(fmm_ctx *c) {
 const char *fmm_last_error(const fmm_ctx *c) { return c ? c->err.c_str() : "null context"; }
 
 namespace {
+// Supercells of 2 prange + 1 boxes a side, prange = (int)(0.5 / theta + 1), have
+// (2 prange + 1)^6 offsets a level (far_sums_kernel): 1.84e9 at 17, more than
+// an int counts at 18
+int far_prange(const fmm_params &p) { return (int)std::fmin(0.5 / p.theta + 1, fmmdev::kFarMaxRange + 1); }
+int check_far(fmm_ctx *c) {
+  if (c->p.images >= 2 && far_prange(c->p) > fmmdev::kFarMaxRange)
+    FMM_FAIL(FMM_ERR_ARG, "theta too small for far images (images >= 2 needs theta > 0.5 / " +
+                              std::to_string(fmmdev::kFarMaxRange) + ")");
+  return FMM_OK;
+}
 // the M2L of these parameters runs on target tiles (offset groups that do not
 // fix the levels, whatever the precision), else on chunks (MIXED: by level)
 bool takes_tiles(const fmm_params &p) {
@@ -885,6 +895,8 @@ int fmm_set_bodies(fmm_ctx *c, int n, const double *x, const double *q) {
   if (!c) return FMM_ERR_ARG;
   if (n < 0 || (n > 0 && (!x || !q))) FMM_FAIL(FMM_ERR_ARG, "fmm_set_bodies: bad n or NULL array");
   if (!c->st) FMM_FAIL(FMM_ERR_STATE, "context was not created successfully");
+  if (n > 0)
+    if (const int rf = check_far(c)) return rf;
   fmm_plan pl;
   bool on_device = false;  // lists
   hipError_t e = hipSetDevice(c->p.device);
@@ -967,6 +979,8 @@ int fmm_set_bodies_plan(fmm_ctx *c, const fmm_plan *pl, const double *x, const d
 namespace {
 int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, bool x_on_device, bool lists_on_device) {
   HIPCHK(hipSetDevice(c->p.device));
+  if (pl.tree.ncell > 0)
+    if (const int rf = check_far(c)) return rf;
   graph_reset(c);
   c->have_bodies = false;
   const double t3 = now_ms();
@@ -1209,7 +1223,7 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
   c->far = c->p.images >= 2 && nc > 0;
   if (c->far) {  // traversePeriodic (include/traversal.h:233-287) as one operator on the root
     const int P = c->p.P, PP = P * P;
-    const int prange = (int)(0.5 / c->p.theta + 1), nb = 2 * prange + 1;
+    const int prange = far_prange(c->p), nb = 2 * prange + 1;
     const size_t mb = sizeof(double) * PP * PP;
     if ((rc = ensure(c, c->per_F, mb)) || (rc = ensure(c, c->per_T, mb)) || (rc = ensure(c, c->per_S, mb)) ||
         (rc = ensure(c, c->per_cur, mb)) || (rc = ensure(c, c->per_tmp, mb)) ||

@@ -94,7 +94,8 @@ hipError_t launch_m2m_rot(int P, const int *parents, const int *child8, int np, 
 hipError_t launch_l2l_rot(int P, const int2 *kids, int nk, const void *rec, double2 *L, hipStream_t s);
 // periodic far images, one level of supercells of period cyc: T = sum of its
 // M2L operators, S = I + its M2M operators (dense P^2 x P^2, row-major; S may be
-// null); sums: far_sums_bytes(P) of scratch
+// null); prange <= kFarMaxRange; sums: far_sums_bytes(P) of scratch
+constexpr int kFarMaxRange = 17;
 size_t far_sums_bytes(int P);
 hipError_t launch_far_ops(int P, int prange, double3 cyc, void *sums, double *T, double *S, hipStream_t s);
 hipError_t launch_matmul(const double *A, const double *B, double *C, int n, int acc, hipStream_t s);

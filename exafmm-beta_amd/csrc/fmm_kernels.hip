@@ -1358,6 +1358,7 @@ __global__ __launch_bounds__(256) void far_sums_kernel(int prange, double3 cyc, 
   const int ncol = reg ? P : NC, SL = 256 / ncol;
   const int col = tid % ncol, slot = tid / ncol;
   if (slot < SL) {
+    static_assert((2 * kFarMaxRange + 1) <= 35, "side^3 and the last step past it fit an int up to 35^6 + 48 * 256");
     const int side = reg ? nb : nb * nb, half = side / 2;
     const int first = reg ? slot : blockIdx.x * SL + slot, step = reg ? SL : kFarBlocks * SL;
     for (int e = first; e < side * side * side; e += step) {
@@ -2216,6 +2217,7 @@ template <int P> struct RunFarOps {
 };
 size_t far_sums_bytes(int P) { return sizeof(double2) * ((size_t)kFarBlocks * (2 * P - 1) * (2 * P - 1) + P * P); }
 hipError_t launch_far_ops(int P, int prange, double3 cyc, void *sums, double *T, double *S, hipStream_t s) {
+  if (prange < 1 || prange > kFarMaxRange) return hipErrorInvalidValue;
   return dispatch<RunFarOps>(P, prange, cyc, static_cast<double2 *>(sums), T, S, s);
 }
 template <int P> struct RunPeriodicFar {

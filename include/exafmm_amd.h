@@ -64,7 +64,8 @@ typedef struct {
   int nspawn;     /* Traversal nspawn: both-sides split threshold */
   int images;     /* periodic images (Traversal(..., images, ...)): 0 = free space; > 0 = the
                    * 27 neighbouring copies in the lists plus images - 1 levels of far copies
-                   * (include/traversal.h:233-287, 326-352) */
+                   * (include/traversal.h:233-287, 326-352); images >= 2 needs theta > 0.5 / 17
+                   * (bodies are refused with FMM_ERR_ARG below) */
   double theta;   /* multipole acceptance parameter */
   double eps2;    /* softening added to r^2 in P2P */
   int precision;  /* fmm_precision */
