@@ -168,6 +168,15 @@ struct M2LTiles {
 M2LTiles build_m2l_tiles(const Tree &t, const M2LGroups &G, int TT, int SW, int seg = 0);
 void split_m2l_tiles(M2LTiles &T, int seg);
 
+// The rounds of fmmdev::device_visit_lists count their pairs and offsets in 32
+// bits.  A pair splits into at most 64: a round of n pairs whose children may
+// pass an int is added up in 64 bits (visit_sum_wraps), and a walk whose
+// rounds hold more than 2^30 pairs in all is the host's (visit_fits: the
+// pairs before and the next round's).
+constexpr int64_t kVisitMaxPairs = (int64_t)1 << 30;
+constexpr bool visit_sum_wraps(int64_t n) { return 64 * n > INT32_MAX; }
+constexpr bool visit_fits(int64_t before, int64_t next) { return next >= 0 && before + next <= kVisitMaxPairs; }
+
 // (Re)build G.chunk from the groups: chunks of at most chunk_pairs pairs,
 // ordered by first target and dealt round-robin-contiguously to the 8 XCDs.
 void deal_m2l_chunks(M2LGroups &G, int chunk_pairs);

@@ -634,6 +634,19 @@ __global__ __launch_bounds__(256) void visit_count_kernel(const int2 *__restrict
   cn[i] = na * nb;
 }
 
+// *out += cn[0] + ... + cn[n - 1], one atomic per block
+__global__ __launch_bounds__(256) void children_total_kernel(const int *__restrict__ cn, int n,
+                                                             unsigned long long *__restrict__ out) {
+  __shared__ unsigned long long part[4];
+  unsigned long long v = 0;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < (size_t)n; i += (size_t)gridDim.x * 256) v += cn[i];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) atomicAdd(out, part[0] + part[1] + part[2] + part[3]);
+}
+
 // the next round: the children of every split pair from slot co[i] on.  A
 // wavefront takes 64 pairs and its lanes their children, each finding its pair
 // by a search in the pairs' slots (pair by pair, a lane a child, the rounds of
@@ -770,13 +783,11 @@ hipError_t device_visit_lists(const fmm::Tree &t, double theta, int nspawn, int 
   TCHK(R.back().F.need(sizeof(int2) * nimg));
   TCHK(hipMemcpyAsync(R.back().F.p, root, sizeof(int2) * nimg, hipMemcpyHostToDevice, s));
   Buf cn(s);
-  int64_t total = 0;
+  int64_t total = nimg;  // pairs of all rounds
   for (;;) {
     Round &r = R.back();
     const size_t n = (size_t)r.n;
     const unsigned nb = (unsigned)(n / 256 + 1);
-    total += r.n;
-    if (total > 0x3fffffff) return hipSuccess;  // beyond the 32-bit sums: the host walks this tree
     TCHK(r.kind.need(n));
     TCHK(cn.need(4 * (n + 1)));
     TCHK(r.co.need(4 * (n + 1)));
@@ -784,14 +795,27 @@ hipError_t device_visit_lists(const fmm::Tree &t, double theta, int nspawn, int 
                                           cn.as<int>());
     TCHK(hipGetLastError());
     TCHK(scan(cn, r.co, r.n + 1));
-    int nn = 0;
-    TCHK(hipMemcpyAsync(&nn, r.co.as<int>() + n, 4, hipMemcpyDeviceToHost, s));
-    TCHK(hipStreamSynchronize(s));
-    if (nn < 0) return hipSuccess;
+    int n32 = 0;
+    int64_t nn = 0;
+    if (fmm::visit_sum_wraps(r.n)) {  // the sum in 32 bits may have wrapped: added up in 64
+      TCHK(dbp.need(8));
+      TCHK(hipMemsetAsync(dbp.p, 0, 8, s));
+      children_total_kernel<<<(unsigned)std::min<size_t>(nb, 2048), 256, 0, s>>>(cn.as<int>(), r.n,
+                                                                              dbp.as<unsigned long long>());
+      TCHK(hipGetLastError());
+      TCHK(hipMemcpyAsync(&nn, dbp.p, 8, hipMemcpyDeviceToHost, s));
+      TCHK(hipStreamSynchronize(s));
+    } else {
+      TCHK(hipMemcpyAsync(&n32, r.co.as<int>() + n, 4, hipMemcpyDeviceToHost, s));
+      TCHK(hipStreamSynchronize(s));
+      nn = n32;
+    }
+    if (!fmm::visit_fits(total, nn)) return hipSuccess;  // beyond the 32-bit sums: the host walks this tree
     if (nn == 0) break;
     R.emplace_back(s);
     Round &q = R.back();
-    q.n = nn;
+    q.n = (int)nn;
+    total += nn;
     TCHK(q.F.need(sizeof(int2) * (size_t)nn));
     TCHK(q.par.need(4 * (size_t)nn));
     visit_expand_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(
