@@ -157,14 +157,7 @@ int ensure(fmm_ctx *c, DBuf &b, size_t bytes) {
   // 25% headroom: a stream of slightly growing systems reallocates rarely
   // (hipMalloc/hipFree synchronise the device)
   size_t sz = bytes ? bytes + bytes / 4 : 16;
-  hipError_t e = hipMalloc(&b.p, sz);
-  if (e == hipErrorOutOfMemory && c->st) {  // the builders' idle scratch makes room
-    (void)hipGetLastError();
-    fmmdev::plan_scratch_release(c->st);
-    e = hipMalloc(&b.p, sz);
-  }
-  if (e != hipSuccess) b.p = nullptr;
-  HIPCHK(e);
+  HIPCHK(fmmdev::device_alloc(&b.p, sz));
   b.cap = sz;
   return FMM_OK;
 }
@@ -1144,7 +1137,8 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
                                                          c->p.images > 0 ? c->p.cycle : nullptr);
         if (e != hipSuccess) {
           (void)hipStreamSynchronize(c->st);
-          HIPCHK(e);
+          if (e != hipErrorOutOfMemory) HIPCHK(e);
+          done = false;  // no room beside the solve's buffers: the host groups
         }
         if (!done) {
           c->groups = fmm::M2LGroups();

@@ -153,6 +153,9 @@ hipError_t init_scratch(int device);
 hipError_t plan_scratch_get(void **p, size_t *cap, size_t bytes, hipStream_t s);
 void plan_scratch_put(void *p, size_t cap, hipStream_t s);
 void plan_scratch_release(hipStream_t s);
+// hipMalloc on the current device; out of memory, the blocks cached for any
+// stream are given back and it is tried once more (*p null after a failure)
+hipError_t device_alloc(void **p, size_t bytes);
 // One device allocation (hipMalloc on `device`), freed on that device when
 // its owner goes; move-only.
 struct DevArray {

@@ -915,16 +915,8 @@ hipError_t plan_scratch_get(void **p, size_t *cap, size_t bytes, hipStream_t s) 
       }
     }
   }
-  hipError_t e = hipMalloc(p, bytes);
-  if (e == hipErrorOutOfMemory) {  // blocks of other sizes kept for this stream make room
-    (void)hipGetLastError();
-    plan_scratch_release(s);
-    e = hipMalloc(p, bytes);
-  }
-  if (e != hipSuccess) {
-    *p = nullptr;
-    return e;
-  }
+  const hipError_t e = device_alloc(p, bytes);
+  if (e != hipSuccess) return e;
   *cap = bytes;
   return hipSuccess;
 }
@@ -957,21 +949,44 @@ void plan_scratch_release(hipStream_t s) {
   for (auto &b : c.blocks) (void)hipFree(b.second);
 }
 
+// every stream's idle blocks
+static bool plan_scratch_release_all() {
+  std::vector<void *> idle;
+  {
+    std::lock_guard<std::mutex> lk(g_scratch_mu);
+    for (auto &c : g_scratch) {
+      for (auto &b : c.second.blocks) idle.push_back(b.second);
+      c.second = ScratchCache();
+    }
+  }
+  for (void *p : idle) (void)hipFree(p);  // waits for the device's work
+  return !idle.empty();
+}
+
+hipError_t device_alloc(void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    if (plan_scratch_release_all()) e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) (void)hipGetLastError();
+  }
+  if (e != hipSuccess) *p = nullptr;
+  return e;
+}
+
 hipError_t DevArray::alloc(size_t b, int dev) {
   if (p && device == dev && cap >= b) {
     bytes = b;
     return hipSuccess;
   }
   // a context's array that was too small grows by a quarter more, as its other
-  // buffers do
-  const size_t want = cap ? b + b / 4 : b;
+  // buffers do, where there is room
+  size_t want = cap ? b + b / 4 : b;
   reset();
   if (b == 0) return hipSuccess;
-  hipError_t e = hipMalloc(&p, want);
-  if (e != hipSuccess) {
-    p = nullptr;
-    return e;
-  }
+  hipError_t e = device_alloc(&p, want);
+  if (e == hipErrorOutOfMemory && want > b) e = device_alloc(&p, want = b);
+  if (e != hipSuccess) return e;
   bytes = b;
   cap = want;
   device = dev;
