@@ -477,13 +477,14 @@ int check_far(fmm_ctx *c) {
 bool takes_tiles(const fmm_params &p) {
   return (p.m2l_mode == FMM_M2L_TILES || p.m2l_mode == FMM_M2L_AUTO) && fmmdev::rot_supported(p.P);
 }
-bool uniform_levels(const fmm::Tree &t) {  // every radius R0 / 2^level
-  for (int k = 0; k < t.ncell; k++)
-    if (t.R[k] != t.R[0] / (1 << t.level[k])) return false;
+bool uniform_levels(const fmm::Tree &t) {  // every radius its root's / 2^level (a forest's roots start their systems)
+  double R0 = 0.0;
+  for (int k = 0; k < t.ncell; k++) {
+    if (t.level[k] == 0) R0 = t.R[k];
+    if (t.R[k] != R0 / (1 << t.level[k])) return false;
+  }
   return true;
 }
-// groups built on the device hold no pair arrays (grp_ptr is {0})
-bool holds_pairs(const fmm::M2LGroups &g) { return g.grp_ptr.size() == (size_t)g.ngroup + 1; }
 int groups_kind_for(const fmm_params &p) {
   return p.precision != FMM_FP64 && !takes_tiles(p) ? FMM_MIXED : FMM_FP64;
 }
@@ -762,7 +763,7 @@ int fmm_plan_prepare(fmm_plan *pl, const fmm_params *p) {
   try {
     const int TT = fmmdev::m2l_tile_targets(p->P);
     const bool fit_tiles = takes_tiles(*p) && pl->tiles.TT == TT;
-    if (pl->groups_kind != kind || !(fit_tiles || holds_pairs(pl->groups))) {
+    if (pl->groups_kind != kind || !(fit_tiles || fmm::holds_pairs(pl->groups))) {
       if (plan_to_host(pl) != hipSuccess) return FMM_ERR_DEVICE;
       pl->dev.reset();  // lists on the host now, other tiles than the device's below
       pl->groups = fmm::build_m2l_groups(pl->tree, pl->lists, fmmdev::kM2LChunkPairs, kind == FMM_MIXED,
@@ -791,19 +792,19 @@ int fmm_plan_merge(fmm_plan **out, int k, const fmm_plan *const *plans) {
     parts.push_back({&plans[i]->tree, &plans[i]->lists, &plans[i]->groups, &plans[i]->tiles});
   }
   if (n > INT32_MAX) return FMM_ERR_ARG;
-  // groups built with the plan on the device hold no pair arrays (grp_ptr is
-  // {0}): a merge with them takes no groups, the upload builds its own
-  bool same_kind = true;
-  for (int i = 0; i < k; i++)
-    same_kind = same_kind && plans[i]->groups_kind == kind &&
-                plans[i]->groups.grp_ptr.size() == (size_t)plans[i]->groups.ngroup + 1;
+  // a merge with groups that hold no pair arrays (built on the device) takes
+  // them where it takes the tiles built beside them
+  bool same_kind = true, held = true, with_tiles = plans[0]->tiles.TT > 0;
+  for (int i = 0; i < k; i++) {
+    same_kind = same_kind && plans[i]->groups_kind == kind;
+    held = held && fmm::holds_pairs(plans[i]->groups);
+    with_tiles = with_tiles && plans[i]->tiles.TT == plans[0]->tiles.TT;
+  }
   fmm_plan *pl = new (std::nothrow) fmm_plan();
   if (!pl) return FMM_ERR_MEMORY;
   try {
-    const bool with_groups = same_kind && kind >= 0;
-    bool with_tiles = with_groups;
-    for (int i = 0; i < k; i++) with_tiles = with_tiles && plans[i]->tiles.TT == plans[0]->tiles.TT;
-    with_tiles = with_tiles && plans[0]->tiles.TT > 0;
+    const bool with_groups = same_kind && kind >= 0 && (held || with_tiles);
+    with_tiles = with_tiles && with_groups;
     fmm::merge_plans(parts, pl->tree, pl->lists, with_groups ? &pl->groups : nullptr, fmmdev::kM2LChunkPairs,
                      with_tiles ? &pl->tiles : nullptr);
     pl->groups_kind = with_groups ? kind : -1;
@@ -1115,7 +1116,7 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
     // groups built with the plan on the device hold no pair arrays: they serve
     // only with the tiles built beside them (of this order's tile size)
     const bool fit_tiles = c->use_tiles && pl.tiles.TT == fmmdev::m2l_tile_targets(c->p.P);
-    if (pl.groups_kind == groups_kind_for(c->p) && (fit_tiles || holds_pairs(pl.groups))) {
+    if (pl.groups_kind == groups_kind_for(c->p) && (fit_tiles || fmm::holds_pairs(pl.groups))) {
       c->groups = std::move(pl.groups);
       if (fit_tiles) {
         tiles = std::move(pl.tiles);
@@ -1165,7 +1166,9 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
           HIPCHK(e != hipSuccess ? e : e2);
         }
         // mixed: on a tree whose levels do not share a radius the pairs of
-        // other radii than their group's run per target, as on chunks
+        // other radii than their group's run per target, as on chunks; the
+        // systems of a forest are looked at one by one (the tiles' FP64
+        // operators carry no radius)
         const bool by_level = c->mixed && (!c->use_tiles || !uniform_levels(t));
         c->groups = fmm::build_m2l_groups(t, L, fmmdev::kM2LChunkPairs, by_level,
                                           c->p.images > 0 ? c->p.cycle : nullptr);

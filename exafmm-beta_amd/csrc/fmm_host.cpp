@@ -931,7 +931,7 @@ M2LGroups build_m2l_groups(const Tree &t, const Lists &L, int chunk_pairs, bool 
   if (!by_level) G.cscale.clear();
   // global group per pair; by_level: a pair whose radii differ from its
   // group's first pair (the chunks' scale) or from its reflection class's
-  // first pair (the tiles' operator scale, one per class) runs per target
+  // first pair runs per target
   // (radius not uniform on its level); counts per (run, group) and per
   // target of the ungrouped rest
   std::vector<std::vector<int>> cnt(T);
@@ -1310,15 +1310,19 @@ void merge_plans(const std::vector<PlanPart> &parts, Tree &T, Lists &L, M2LGroup
   G->rest_ptr.assign(nc + 1, 0);
   co = 0;
   int po = 0;
+  bool held = true;
+  for (const PlanPart &p : parts) held = held && holds_pairs(*p.g);
   for (const PlanPart &p : parts) {
     const M2LGroups &g = *p.g;
-    for (int k = 0; k < g.ngroup; k++) G->grp_ptr.push_back(g.grp_ptr[k + 1] + po);
-    for (int v : g.tgt) G->tgt.push_back(v + co);
-    for (int v : g.src) G->src.push_back(v + co);
-    G->dx.insert(G->dx.end(), g.dx.begin(), g.dx.end());
-    G->scale.insert(G->scale.end(), g.scale.begin(), g.scale.end());
-    for (int v : g.canon) G->canon.push_back(v + G->ncanon);
-    G->refl.insert(G->refl.end(), g.refl.begin(), g.refl.end());
+    if (held) {
+      for (int k = 0; k < g.ngroup; k++) G->grp_ptr.push_back(g.grp_ptr[k + 1] + po);
+      for (int v : g.tgt) G->tgt.push_back(v + co);
+      for (int v : g.src) G->src.push_back(v + co);
+      G->dx.insert(G->dx.end(), g.dx.begin(), g.dx.end());
+      G->scale.insert(G->scale.end(), g.scale.begin(), g.scale.end());
+      for (int v : g.canon) G->canon.push_back(v + G->ncanon);
+      G->refl.insert(G->refl.end(), g.refl.begin(), g.refl.end());
+    }
     G->cdx.insert(G->cdx.end(), g.cdx.begin(), g.cdx.end());
     G->cscale.insert(G->cscale.end(), g.cscale.begin(), g.cscale.end());
     G->ncanon += g.ncanon;
@@ -1331,7 +1335,7 @@ void merge_plans(const std::vector<PlanPart> &parts, Tree &T, Lists &L, M2LGroup
     po += (int)g.tgt.size();
   }
   G->nrest = (int64_t)G->rest_src.size();
-  deal_m2l_chunks(*G, chunk_pairs);
+  if (held) deal_m2l_chunks(*G, chunk_pairs);
   if (!tiles) return;
   // tiles concatenated part by part (each part's tile count is a multiple of
   // the XCD count, so every part keeps its XCD dealing)

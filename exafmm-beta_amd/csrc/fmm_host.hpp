@@ -134,6 +134,9 @@ struct M2LGroups {
   std::vector<double> cdx;         // 3 per representative
   std::vector<double> cscale;      // 2 per representative when grouped by level
 };
+// false for groups built on the device: they hold the counts and the
+// representatives' offsets only (grp_ptr is {0}), their pairs are the tiles'
+inline bool holds_pairs(const M2LGroups &g) { return g.grp_ptr.size() == (size_t)g.ngroup + 1; }
 // by_level: a group also fixes the source and target levels (the scaled FP32
 // operator depends on R_s and R_t); pairs whose radii differ from their
 // group's are left ungrouped.
@@ -184,7 +187,8 @@ void deal_m2l_chunks(M2LGroups &G, int chunk_pairs);
 // Several independent systems as one forest (batched evaluation): cell, body
 // and pair indices of part k are offset by the sizes of parts 0..k-1, levels
 // are kept, and no pair joins two systems.  G (optional) merges the parts'
-// M2L groups (every part must carry groups of the same kind).
+// M2L groups (every part must carry groups of the same kind; where a part's
+// hold no pairs neither do the merged ones, which then serve with tiles only).
 struct PlanPart {
   const Tree *t;
   const Lists *l;

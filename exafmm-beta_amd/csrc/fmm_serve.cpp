@@ -108,8 +108,8 @@ void builder_loop(fmm_server *s) {
                 : fmm_plan_build(&pl, r->n, r->x.data(), s->p.ncrit, s->p.theta, s->p.nspawn);
     // M2L groups for the slots' contexts; the tiles of a request that runs
     // alone are left to the upload, which builds them on the device (a batch
-    // of several takes its requests' groups and tiles, so that a request's
-    // M2L is the same alone and in a batch)
+    // of several concatenates its requests' tiles, those of device-built
+    // plans too, so that a request's M2L is the same alone and in a batch)
     if (rc == FMM_OK && !(s->p.m2l_mode == FMM_M2L_TILES && s->cfg.batch_requests == 1))
       rc = fmm_plan_prepare(pl, &s->p);
     fmm_stats st{};
