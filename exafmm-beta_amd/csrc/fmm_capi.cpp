@@ -278,18 +278,21 @@ int download_staged(fmm_ctx *c, void *dst, const void *src, size_t bytes) {
   return FMM_OK;
 }
 
-// a device array taken over by a context buffer (both hipMalloc'd)
+// a device array taken over by a context buffer (both hipMalloc'd); the
+// buffer's own allocation goes where the array's came from
 void adopt(DBuf &b, fmmdev::DevArray &a) {
   if (!a.p) return;
-  if (b.p) (void)hipFree(b.p);
+  if (b.p && a.pool)
+    fmmdev::plan_scratch_put(b.p, b.cap, a.pool);
+  else if (b.p)
+    (void)hipFree(b.p);
   b.p = a.p;
   b.cap = a.cap;
   a.p = nullptr;
   a.bytes = a.cap = 0;
   a.device = -1;
 }
-// and the other way: the buffer's allocation for a builder to fill (hipMalloc
-// and hipFree of the pair arrays took 1.2 ms of a 1M-body step)
+// and the other way: the buffer's allocation for a builder to fill
 void lend(fmmdev::DevArray &a, DBuf &b, int device) {
   a.p = b.p;
   a.cap = b.cap;
@@ -595,7 +598,10 @@ int device_tree_of(fmm_ctx *c, fmm::Tree &t, int n, const double *x, int ncrit, 
   return FMM_OK;
 }
 
-// for_upload: the plan goes into c next and fills c's own pair arrays
+// for_upload: the plan goes into c next, which takes its pair arrays over: they
+// come from c's cached blocks, where those of the system before go in exchange
+// (hipMalloc and hipFree of them took 1.2 ms of a 1M-body step; filling that
+// system's own arrays would lose it where a builder fails)
 int plan_build_device(fmm_ctx *c, fmm_plan **out, int n, const double *x, int ncrit, double theta, int nspawn,
                       bool for_upload) {
   if (!c || !out) return FMM_ERR_ARG;
@@ -621,15 +627,10 @@ int plan_build_device(fmm_ctx *c, fmm_plan **out, int n, const double *x, int nc
     const double xper[3] = {0, 0, 0};
     // the source columns stay on the device with the plan (pl->dev)
     pl->dev = std::make_shared<fmmdev::PlanArrays>();
-    if (for_upload) {
-      c->have_bodies = false;
-      graph_reset(c);
-      lend(pl->dev->m2l_src, c->m2l_src, c->p.device);
-      lend(pl->dev->p2p_src, c->p2p_src, c->p.device);
-      lend(pl->dev->t_slice, c->t_slice, c->p.device);
-      lend(pl->dev->t_src, c->t_src, c->p.device);
-      lend(pl->dev->t_lt, c->t_lt, c->p.device);
-    }
+    if (for_upload)
+      for (fmmdev::DevArray *a : {&pl->dev->m2l_src, &pl->dev->p2p_src, &pl->dev->t_slice, &pl->dev->t_src,
+                                  &pl->dev->t_lt})
+        a->pool = c->st;
     HIPCHK(fmmdev::device_lists(t.ncell, t.X.data(), t.R.data(), t.nchild.data(), t.ichild.data(), t.nbody.data(),
                                 theta, nspawn, xper, 0, 0, L.m2l_ptr, L.m2l_src, L.p2p_ptr, L.p2p_src,
                                 L.p2p_body_pairs, c->st, pl->dev.get()));
@@ -918,11 +919,11 @@ int fmm_set_bodies(fmm_ctx *c, int n, const double *x, const double *q) {
   };
   const auto lists = [&](fmm_plan &p) {
     if (p.tree.ncell < least) return false;
-    c->have_bodies = false;  // the columns of the bodies before are overwritten
-    graph_reset(c);
     e = fmmdev::device_visit_lists(
         p.tree, c->p.theta, c->p.nspawn, c->p.images, c->p.cycle, p.lists,
-        [&](bool p2p, int64_t k) -> int * {
+        [&](bool p2p, int64_t k) -> int * {  // the lists are made: the columns of the bodies before go
+          c->have_bodies = false;
+          graph_reset(c);
           DBuf &b = p2p ? c->p2p_src : c->m2l_src;
           return ensure(c, b, sizeof(int) * (size_t)k) == FMM_OK ? b.as<int>() : nullptr;
         },

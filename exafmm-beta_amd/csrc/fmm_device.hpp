@@ -150,19 +150,22 @@ hipError_t init_scratch(int device);
 // its work (the owner calls it before destroying s).  Replaces a
 // hipMallocAsync / hipFreeAsync pair per buffer, about 0.2 ms of host time
 // each on this runtime.
-hipError_t plan_scratch_get(void **p, size_t *cap, size_t bytes, hipStream_t s);
+// (spare: a new block gets that much more, where there is room)
+hipError_t plan_scratch_get(void **p, size_t *cap, size_t bytes, hipStream_t s, size_t spare = 0);
 void plan_scratch_put(void *p, size_t cap, hipStream_t s);
 void plan_scratch_release(hipStream_t s);
 // hipMalloc on the current device; out of memory, the blocks cached for any
 // stream are given back and it is tried once more (*p null after a failure)
 hipError_t device_alloc(void **p, size_t bytes);
 // One device allocation (hipMalloc on `device`), freed on that device when
-// its owner goes; move-only.
+// its owner goes; move-only.  With a pool it is taken from and given back to
+// that stream's cached blocks.
 struct DevArray {
   void *p = nullptr;
   size_t bytes = 0;  // in use
   size_t cap = 0;    // allocated
   int device = -1;
+  hipStream_t pool = nullptr;
   DevArray() = default;
   DevArray(const DevArray &) = delete;
   DevArray &operator=(const DevArray &) = delete;

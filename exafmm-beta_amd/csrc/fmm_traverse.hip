@@ -897,7 +897,7 @@ std::map<hipStream_t, ScratchCache> g_scratch;
 constexpr size_t kScratchKeep = (size_t)8 << 30;
 }  // namespace
 
-hipError_t plan_scratch_get(void **p, size_t *cap, size_t bytes, hipStream_t s) {
+hipError_t plan_scratch_get(void **p, size_t *cap, size_t bytes, hipStream_t s, size_t spare) {
   *p = nullptr;
   *cap = 0;
   if (bytes == 0) bytes = 1;
@@ -915,9 +915,10 @@ hipError_t plan_scratch_get(void **p, size_t *cap, size_t bytes, hipStream_t s) 
       }
     }
   }
-  const hipError_t e = device_alloc(p, bytes);
+  hipError_t e = device_alloc(p, bytes + spare);
+  if (e == hipErrorOutOfMemory && spare > 0) e = device_alloc(p, bytes), spare = 0;
   if (e != hipSuccess) return e;
-  *cap = bytes;
+  *cap = bytes + spare;
   return hipSuccess;
 }
 
@@ -984,6 +985,13 @@ hipError_t DevArray::alloc(size_t b, int dev) {
   size_t want = cap ? b + b / 4 : b;
   reset();
   if (b == 0) return hipSuccess;
+  if (pool) {
+    const hipError_t e = plan_scratch_get(&p, &cap, b, pool, b / 4);
+    if (e != hipSuccess) return e;
+    bytes = b;
+    device = dev;
+    return hipSuccess;
+  }
   hipError_t e = device_alloc(&p, want);
   if (e == hipErrorOutOfMemory && want > b) e = device_alloc(&p, want = b);
   if (e != hipSuccess) return e;
@@ -994,7 +1002,9 @@ hipError_t DevArray::alloc(size_t b, int dev) {
 }
 
 void DevArray::reset() {
-  if (p) {
+  if (p && pool) {
+    plan_scratch_put(p, cap, pool);
+  } else if (p) {
     int cur = -1;
     const bool same = hipGetDevice(&cur) == hipSuccess && cur == device;
     if (!same) (void)hipSetDevice(device);

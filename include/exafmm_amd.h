@@ -174,7 +174,8 @@ const char *fmm_last_error(const fmm_ctx *c);
  * host, the octree of 50000 bodies and more and the lists of some hundred
  * cells and more on the device (the same cells and lists, in the same order),
  * then upload of bodies (in tree order), cells and lists.  x is (n,3) in the
- * caller's order. */
+ * caller's order.  Where the tree or the lists cannot be made the context keeps
+ * the bodies it has, as fmm_set_bodies_device does; a failing upload loses them. */
 int fmm_set_bodies(fmm_ctx *c, int n, const double *x, const double *q);
 /* Same, with a plan built by fmm_plan_build for these x (the context copies
  * what it needs; the plan stays owned by the caller). */

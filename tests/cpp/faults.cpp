@@ -17,13 +17,14 @@
 namespace {
 std::function<bool(size_t)> refuse;  // a request of this size
 int refused = 0;
+hipError_t refusal = hipErrorOutOfMemory;  // with this
 }  // namespace
 
 extern "C" hipError_t hipMalloc(void **p, size_t n) {
   static const auto real = reinterpret_cast<hipError_t (*)(void **, size_t)>(dlsym(RTLD_NEXT, "hipMalloc"));
   if (refuse && refuse(n)) {
     refused++;
-    return hipErrorOutOfMemory;
+    return refusal;
   }
   return real(p, n);
 }
@@ -85,11 +86,55 @@ void groups() {
     fmm_destroy(d);
   }
 }
+
+// an allocation fails while the next system's tree, lists or groups are made:
+// the context still has the system before, and takes the next one afterwards
+void kept() {
+  const System a(20000, "cube", 1), b(30000, "plummer", 2);
+  for (bool device : {false, true}) {
+    const auto set = [&](fmm_ctx *c, const System &s) {
+      return (device ? fmm_set_bodies_device : fmm_set_bodies)(c, s.n(), s.x.data(), s.q.data());
+    };
+    int total = 0, at = 0;  // allocations of b's plan
+    {
+      fmm_ctx *c = context(8);
+      EXPECT(set(c, a) == FMM_OK);
+      refuse = [&](size_t) { return total++, false; };
+      fmm_plan *p = nullptr;
+      EXPECT(fmm_plan_build_device(c, &p, b.n(), b.x.data(), 64, 0.4, 5000) == FMM_OK);
+      refuse = nullptr;
+      fmm_plan_destroy(p);
+      fmm_destroy(c);
+    }
+    EXPECT(total > 8);
+    // fmm_set_bodies makes the lists alone there: its first allocations
+    for (int k : device ? std::vector<int>{0, total / 4, total / 2, 3 * total / 4} : std::vector<int>{0, 1, 2}) {
+      fmm_ctx *c = context(8), *d = context(8);
+      EXPECT(set(c, a) == FMM_OK);
+      const std::vector<double> ta = solve(c, a.n());
+      refused = at = 0;
+      refusal = hipErrorUnknown;  // no second try, nothing falls back
+      refuse = [&](size_t) { return at++ == k; };
+      const int rc = set(c, b);
+      refuse = nullptr;
+      refusal = hipErrorOutOfMemory;
+      std::printf("%s, allocation %d of %d: %d, refused %d\n", device ? "device" : "host", k, total, rc, refused);
+      EXPECT(refused == 1 && rc == FMM_ERR_DEVICE);
+      EXPECT(rel(solve(c, a.n()), ta) < 1e-12);  // the order of the atomic additions
+      EXPECT(set(c, b) == FMM_OK);
+      EXPECT(set(d, b) == FMM_OK);
+      EXPECT(rel(solve(c, b.n()), solve(d, b.n())) < 1e-12);
+      fmm_destroy(c);
+      fmm_destroy(d);
+    }
+  }
+}
 }  // namespace
 
 int main(int argc, char **argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "groups") groups();
+  else if (what == "kept") kept();
   else bad++;
   std::puts(bad ? "bad" : "ok");
   return bad != 0;

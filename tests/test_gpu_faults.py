@@ -28,3 +28,7 @@ def faults(tmp_path_factory):
 
 def test_groups_on_the_host(faults):
     faults("groups")
+
+
+def test_system_kept_when_the_next_fails(faults):
+    faults("kept")
