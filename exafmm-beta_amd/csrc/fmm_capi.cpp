@@ -88,7 +88,8 @@ struct fmm_ctx {
   // offset-grouped M2L: chunks (GROUPED) or target tiles (AUTO)
   bool use_mfma = false, use_tiles = false;
   int nchunk = 0, ntile = 0;
-  int p2p_nwide = 0;  // P2P targets [0, p2p_nwide) are leaves of >= 16 bodies
+  fmmdev::P2PCounts p2p_n;  // P2P targets by leaf size and system size
+  int p2m_few = 0;          // leaves [0, p2m_few): of small systems
   fmm::M2LGroups groups;
   DBuf g_tgt, g_src, g_dx, g_chunk, r_ptr, r_src, r_tgt;
   DBuf t_tgt, t_ptr, t_slice, t_src, t_lt, g_ops, c_dx;
@@ -999,6 +1000,26 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
     hcy[k] = t.X[3 * (size_t)k + 1];
     hcz[k] = t.X[3 * (size_t)k + 2];
   }
+  // the systems of a forest: their cells follow one another, each from its root
+  int nsystem = 0;
+  for (int k = 0; k < nc; k++) nsystem += t.level[k] == 0;
+  std::vector<int> system(nsystem > 1 ? nc : 0);
+  for (int k = 0, s = -1; k < (int)system.size(); k++) system[k] = s += t.level[k] == 0;
+  // per system: has it less than `fill` of these cells
+  auto fewer = [&](const std::vector<int> &cells, size_t fill) {
+    std::vector<size_t> num(std::max(nsystem, 1), 0);
+    if (nsystem <= 1) num[0] = cells.size();
+    else
+      for (int cell : cells) num[system[cell]]++;
+    std::vector<char> few;
+    for (size_t k : num) few.push_back(k < fill);
+    return few;
+  };
+  using Cells = std::vector<int>;
+  auto few_first = [&](Cells::iterator b, Cells::iterator e, const std::vector<char> &few) {
+    if (few.size() == 1) return few[0] ? e : b;
+    return std::stable_partition(b, e, [&](int cell) { return few[system[cell]] != 0; });
+  };
   // internal cells per level (M2M), body -> leaf map (L2P)
   std::vector<int> internal;
   c->internal_ptr.assign(t.depth + 2, 0);
@@ -1042,7 +1063,9 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
   UP(cx, hcx) UP(cy, hcy) UP(cz, hcz)
   UP(ibody, t.ibody) UP(nbody, t.nbody) UP(ichild, t.ichild) UP(nchild, t.nchild)
   UP(iparent, t.iparent)
-  UP(leaves, t.leaves) UP(internal, internal) UP(level_cells, t.level_cells)
+  Cells leaves(t.leaves);
+  c->p2m_few = (int)(few_first(leaves.begin(), leaves.end(), fewer(t.leaves, fmmdev::kP2MFillLeaves)) - leaves.begin());
+  UP(leaves, leaves) UP(internal, internal) UP(level_cells, t.level_cells)
   if ((rc = ensure(c, c->body_leaf, sizeof(int) * n))) {
     (void)hipStreamSynchronize(c->st);
     return rc;
@@ -1059,12 +1082,17 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
   } else if (!lists_on_device) {
     UP(m2l_src, L.m2l_src) UP(p2p_src, L.p2p_src)
   }
-  // P2P targets, leaves of >= 16 bodies first (the kernel's targets per lane
-  // follow the leaf size, so every leaf is summed the same way in any batch)
-  std::vector<int> p2p_order(L.p2p_targets);
-  c->p2p_nwide = (int)(std::stable_partition(p2p_order.begin(), p2p_order.end(),
-                                             [&](int cell) { return t.nbody[cell] >= fmmdev::kP2PWideLeaf; }) -
-                       p2p_order.begin());
+  // P2P targets, leaves of >= 16 bodies first, small systems before large ones
+  // (the kernel's targets per lane follow the leaf size, its wavefronts a leaf
+  // the system's, so every leaf is summed the same way in any batch)
+  Cells p2p_order(L.p2p_targets);
+  {
+    const auto b = p2p_order.begin(), e = p2p_order.end();
+    const auto w = std::stable_partition(b, e, [&](int cell) { return t.nbody[cell] >= fmmdev::kP2PWideLeaf; });
+    const std::vector<char> few = fewer(L.p2p_targets, fmmdev::kP2PFillLeaves);
+    const auto wf = few_first(b, w, few), nf = few_first(w, e, few);
+    c->p2p_n = {(int)(wf - b), (int)(w - wf), (int)(nf - w), (int)(e - nf)};
+  }
   UP(p2p_ptr, L.p2p_ptr) UP(p2p_tgt, p2p_order)
   // M2M / L2L operators: every level's radius uniform and every child at
   // X_parent + R_child (+-1, +-1, +-1) (up to rounding of the centres)
@@ -1368,8 +1396,8 @@ int fmm_upward(fmm_ctx *c) {
   if (c->tree.ncell == 0) return FMM_OK;
   const int P = c->p.P;
   auto C = dev_cells(c);
-  HIPCHK(fmmdev::launch_p2m(P, dev_bodies(c), C, c->leaves.as<int>(), (int)c->tree.leaves.size(),
-                            c->M.as<double2>(), c->st));
+  HIPCHK(fmmdev::launch_p2m(P, dev_bodies(c), C, c->leaves.as<int>(), c->p2m_few,
+                            (int)c->tree.leaves.size() - c->p2m_few, c->M.as<double2>(), c->st));
   const size_t rb = fmmdev::rot_ops_bytes(P);
   for (int l = c->tree.depth; l >= 0; l--) {
     const int b = c->internal_ptr[l], e = c->internal_ptr[l + 1];
@@ -1390,8 +1418,8 @@ int p2p_on(fmm_ctx *c, hipStream_t s) {
   const double3 xper = c->cyc;  // image shifts of the source codes
   if (c->timing) HIPCHK(hipEventRecord(c->kev[0], s));
   HIPCHK((c->mixed ? fmmdev::launch_p2p32 : fmmdev::launch_p2p)(
-      dev_bodies(c), dev_cells(c), c->p2p_tgt.as<int>(), (int)c->lists.p2p_targets.size(),
-      c->p2p_ptr.as<int>(), c->p2p_src.as<int>(), xper, c->p.eps2, c->tree.adopted ? 1 : 0, c->p2p_nwide, s));
+      dev_bodies(c), dev_cells(c), c->p2p_tgt.as<int>(), c->p2p_n, c->p2p_ptr.as<int>(), c->p2p_src.as<int>(), xper,
+      c->p.eps2, c->tree.adopted ? 1 : 0, s));
   if (c->timing) HIPCHK(hipEventRecord(c->kev[1], s));
   return FMM_OK;
 }
@@ -1971,8 +1999,10 @@ int fmm_kernel_p2p(fmm_ctx *c, int ni, const double *xi, double *trgi, int nj, c
   const double3 cyc = xper ? make_double3(xper[0], xper[1], xper[2]) : make_double3(0, 0, 0);
   OpDev dv;
   if ((rc = op_upload(c, h, dv))) return rc;
-  HIPCHK(fmmdev::launch_p2p(dev_bodies_of(dv, B), dev_cells_of(dv, C), dv.i + tg, 1, dv.i + ptr, dv.i + src, cyc,
-                            c->p.eps2, 1, ni >= fmmdev::kP2PWideLeaf ? 1 : 0, c->st));
+  const bool wide = ni >= fmmdev::kP2PWideLeaf;
+  const fmmdev::P2PCounts one{wide ? 1 : 0, 0, wide ? 0 : 1, 0};
+  HIPCHK(fmmdev::launch_p2p(dev_bodies_of(dv, B), dev_cells_of(dv, C), dv.i + tg, one, dv.i + ptr, dv.i + src, cyc,
+                            c->p.eps2, 1, c->st));
   return op_add_targets(c, dv, B, ni, trgi);
 }
 
@@ -1990,7 +2020,7 @@ int fmm_kernel_p2m(fmm_ctx *c, const double *Xc, int n, const double *x, const d
   const size_t Mo = h.zeros(2 * (size_t)nterm(c));
   OpDev dv;
   if ((rc = op_upload(c, h, dv))) return rc;
-  HIPCHK(fmmdev::launch_p2m(c->p.P, dev_bodies_of(dv, B), dev_cells_of(dv, C), dv.i + leaves, 1,
+  HIPCHK(fmmdev::launch_p2m(c->p.P, dev_bodies_of(dv, B), dev_cells_of(dv, C), dv.i + leaves, 1, 0,
                             reinterpret_cast<double2 *>(dv.d + Mo), c->st));
   return op_add_expansion(c, dv, Mo, c->p.P, false, M);
 }

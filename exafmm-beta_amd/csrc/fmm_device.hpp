@@ -51,7 +51,12 @@ bool order_supported(int P);
 hipError_t init_constants();
 
 // P2M for every leaf in `leaves` (kernels/laplace.h:237-252)
-hipError_t launch_p2m(int P, DevBodies B, DevCells C, const int *leaves, int nleaf, double2 *M,
+// P2M and P2P deal a leaf's bodies or list to more lanes while the leaves do not
+// fill the GPU.  The sums' order follows, so it is decided for each system of a
+// forest by its own leaves: leaves[0, nfew) are of systems of less than
+// kP2MFillLeaves leaves, the other nmany of larger ones
+constexpr int kP2MFillLeaves = 8192, kP2PFillLeaves = 12000;
+hipError_t launch_p2m(int P, DevBodies B, DevCells C, const int *leaves, int nfew, int nmany, double2 *M,
                       hipStream_t s);
 // M2M into every parent listed in `cells` from its children (laplace.h:254-290)
 hipError_t launch_m2m(int P, DevCells C, const int *cells, int ncell, double2 *M, hipStream_t s);
@@ -107,13 +112,17 @@ hipError_t launch_m_to_f32(int P, const double2 *M, const double *R, int ncell, 
 hipError_t launch_m2l_mfma32(int P, const int4 *chunks, int nchunk, const double *gdx, const double2 *gscale,
                              const int *ptgt, const int *psrc, const float2 *M32, double2 *L, hipStream_t s);
 // P2P for every target leaf over its CSR list (laplace.h:150-235); overwrites
-// the targets of each listed leaf.  targets[0, nwide) are leaves of at least kP2PWideLeaf bodies (run with four
-// targets per lane), the rest run with one
+// the targets of each listed leaf.  targets: wide leaves (at least kP2PWideLeaf
+// bodies, run with four targets per lane, the rest with one) of systems with
+// less than kP2PFillLeaves targets, then of larger ones, then the rest likewise
 constexpr int kP2PWideLeaf = 16;
-hipError_t launch_p2p32(DevBodies B, DevCells C, const int *targets, int ntarget, const int *ptr,
-                        const int *src, double3 xper, double eps2, int mask_all, int nwide, hipStream_t s);
-hipError_t launch_p2p(DevBodies B, DevCells C, const int *targets, int ntarget, const int *ptr,
-                      const int *src, double3 xper, double eps2, int mask_all, int nwide, hipStream_t s);
+struct P2PCounts {
+  int wide_few = 0, wide_many = 0, few = 0, many = 0;
+};
+hipError_t launch_p2p32(DevBodies B, DevCells C, const int *targets, P2PCounts n, const int *ptr,
+                        const int *src, double3 xper, double eps2, int mask_all, hipStream_t s);
+hipError_t launch_p2p(DevBodies B, DevCells C, const int *targets, P2PCounts n, const int *ptr,
+                      const int *src, double3 xper, double eps2, int mask_all, hipStream_t s);
 
 // Direct sum (include/traversal.h:355-377) of all n sources at nt targets
 // (SoA txyz); writes tpot/tax/tay/taz.

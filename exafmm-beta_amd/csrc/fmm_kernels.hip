@@ -2105,17 +2105,16 @@ template <int P> struct RunP2M {
     constexpr int LW = P2MLanes<P, S>::LW;
     hipLaunchKernelGGL((p2m_kernel<P, S>), dim3((nleaf + LW - 1) / LW), dim3(64), 0, s, B, C, leaves, nleaf, M);
   }
-  static hipError_t run(DevBodies B, DevCells C, const int *leaves, int nleaf, double2 *M, hipStream_t s) {
+  static hipError_t run(DevBodies B, DevCells C, const int *leaves, int nfew, int nmany, double2 *M, hipStream_t s) {
     constexpr int SM = 64 / ((P + 1) / 2);  // one leaf a wavefront
-    if (nleaf <= 0) return hipSuccess;
     // few leaves: a leaf's bodies over the whole wavefront, else over two groups
     // of lanes.  Upward pass with SM / 2 / 1 groups: 253 leaves, P = 8, 29 / 38 /
     // 46 us; 3229, P = 8, 52 / 55 / 66; 13003, P = 10, 101 / 101 / 116; 56095, P =
     // 10, 244 / 177 / 195; 797144, P = 12, 3032 / 1530 / 1487
-    if (nleaf < 8192)
-      go<SM>(B, C, leaves, nleaf, M, s);
-    else
-      go<2>(B, C, leaves, nleaf, M, s);
+    if (nfew > 0) go<SM>(B, C, leaves, nfew, M, s);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    if (nmany > 0) go<2>(B, C, leaves + nfew, nmany, M, s);
     return hipGetLastError();
   }
 };
@@ -2162,9 +2161,9 @@ template <int P> struct RunM2LMfma {
   }
 };
 
-hipError_t launch_p2m(int P, DevBodies B, DevCells C, const int *leaves, int nleaf, double2 *M,
+hipError_t launch_p2m(int P, DevBodies B, DevCells C, const int *leaves, int nfew, int nmany, double2 *M,
                       hipStream_t s) {
-  return dispatch<RunP2M>(P, B, C, leaves, nleaf, M, s);
+  return dispatch<RunP2M>(P, B, C, leaves, nfew, nmany, M, s);
 }
 hipError_t launch_m2m(int P, DevCells C, const int *cells, int ncell, double2 *M, hipStream_t s) {
   return dispatch<RunM2M>(P, C, cells, ncell, M, s);
@@ -2245,21 +2244,22 @@ hipError_t launch_m2l_mfma32(int P, const int4 *chunks, int nchunk, const double
 // longest lists then set the time.  Solve of 1 / 4 wavefronts a leaf, P = 8:
 // 239 leaves 0.262 / 0.146 ms, 3037 0.705 / 0.550, 4118 (ragged) 2.05 / 0.74,
 // 7229 0.685 / 0.665, 10047 0.854 / 0.826, 13003 1.080 / 1.093, 13248 0.687 /
-// 0.759, 21300 1.611 / 1.697; a mixed-precision solve of 3037 0.526 / 0.420
-template <template <int, int> class F, typename... A> static hipError_t p2p_dispatch(int ntarget, int nwide, A... a) {
-  nwide = std::min(std::max(nwide, 0), ntarget);
-  const bool four = ntarget < 12000;
-  if (nwide > 0) {
-    if (four) F<4, 4>::run(0, nwide, a...);
-    else F<4, 1>::run(0, nwide, a...);
-  }
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  if (ntarget > nwide) {
-    if (four) F<1, 4>::run(nwide, ntarget - nwide, a...);
-    else F<1, 1>::run(nwide, ntarget - nwide, a...);
-  }
-  return hipGetLastError();
+// 0.759, 21300 1.611 / 1.697; a mixed-precision solve of 3037 0.526 / 0.420.
+// The leaves counted are the system's own: see P2PCounts.
+template <template <int, int> class F, typename... A> static hipError_t p2p_dispatch(P2PCounts n, A... a) {
+  int first = 0;
+  hipError_t e = hipSuccess;
+  auto go = [&](auto run, int m) {
+    if (m <= 0 || e != hipSuccess) return;
+    run(first, m, a...);
+    first += m;
+    e = hipGetLastError();
+  };
+  go(F<4, 4>::run, n.wide_few);
+  go(F<4, 1>::run, n.wide_many);
+  go(F<1, 4>::run, n.few);
+  go(F<1, 1>::run, n.many);
+  return e;
 }
 template <int K, int W> struct RunP2P {
   static void run(int first, int n, DevBodies B, DevCells C, const int *targets, const int *ptr, const int *src,
@@ -2275,14 +2275,14 @@ template <int K, int W> struct RunP2P32 {
                        eps2);
   }
 };
-hipError_t launch_p2p32(DevBodies B, DevCells C, const int *targets, int ntarget, const int *ptr,
+hipError_t launch_p2p32(DevBodies B, DevCells C, const int *targets, P2PCounts n, const int *ptr,
                         const int *src, double3 xper, double eps2, int /*mask_all: every pair is masked*/,
-                        int nwide, hipStream_t s) {
-  return p2p_dispatch<RunP2P32>(ntarget, nwide, B, C, targets, ptr, src, xper, eps2, s);
+                        hipStream_t s) {
+  return p2p_dispatch<RunP2P32>(n, B, C, targets, ptr, src, xper, eps2, s);
 }
-hipError_t launch_p2p(DevBodies B, DevCells C, const int *targets, int ntarget, const int *ptr,
-                      const int *src, double3 xper, double eps2, int mask_all, int nwide, hipStream_t s) {
-  return p2p_dispatch<RunP2P>(ntarget, nwide, B, C, targets, ptr, src, xper, eps2, mask_all, s);
+hipError_t launch_p2p(DevBodies B, DevCells C, const int *targets, P2PCounts n, const int *ptr,
+                      const int *src, double3 xper, double eps2, int mask_all, hipStream_t s) {
+  return p2p_dispatch<RunP2P>(n, B, C, targets, ptr, src, xper, eps2, mask_all, s);
 }
 
 }  // namespace fmmdev

@@ -13,9 +13,10 @@
 // Requests arriving while others run are planned at once and join the next
 // batch a slot takes: batches form continuously, and batches of different
 // slots overlap on the device (separate streams, default priority).  A
-// system's arithmetic does not depend on its batch: its cells, lists, M2L
-// tiles and chunks are the same as alone; only the order of FP64 atomic
-// additions into L may differ.
+// system's cells, lists, M2L tiles and chunks are the same as alone, and its
+// leaves are summed in the same order; a batch may change the order of FP64
+// atomic additions into L and, up to order 12, the form of M2M and L2L (by
+// rotation alone, general in a forest), which is rounding.
 #include <algorithm>
 #include <chrono>
 #include <condition_variable>

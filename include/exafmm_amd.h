@@ -354,7 +354,9 @@ int fmm_get_lists(fmm_ctx *c, int *m2l_ptr, int *m2l_src, int *p2p_ptr, int *p2p
  * target tiles: when batches hold one request a slot's upload builds their
  * groups on the device and the builders plan tree and lists only, else the
  * builders build them too.  A system's result does not depend on its batch
- * beyond the order of FP64 atomic additions into its local expansions. */
+ * beyond rounding: the order of the FP64 atomic additions into its local
+ * expansions, and, up to order 12, M2M and L2L, which a batch of several runs in
+ * their general form and not by rotation. */
 typedef struct fmm_server fmm_server;
 
 typedef struct {
