@@ -538,8 +538,9 @@ void plan_stats(const fmm_plan *pl, fmm_stats &s) {
 // x_on_device: x is already in c->xin (fmm_set_bodies_device: the plan was
 // just built from it there)
 // lists_on_device: the lists' source columns are already in c->m2l_src, c->p2p_src
+// kept: tiles that the caller keeps, read in place of pl's
 int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, bool x_on_device = false,
-                bool lists_on_device = false);
+                bool lists_on_device = false, const fmm::M2LTiles *kept = nullptr);
 int plan_build_device(fmm_ctx *c, fmm_plan **out, int n, const double *x, int ncrit, double theta, int nspawn,
                       bool for_upload);
 }  // namespace
@@ -968,12 +969,49 @@ int fmm_set_bodies_plan(fmm_ctx *c, const fmm_plan *pl, const double *x, const d
   if (pl->images != c->p.images ||
       (pl->images > 0 && (pl->cycle[0] != c->p.cycle[0] || pl->cycle[1] != c->p.cycle[1] || pl->cycle[2] != c->p.cycle[2])))
     FMM_FAIL(FMM_ERR_ARG, "fmm_set_bodies_plan: the plan's periodic images differ from the context's");
-  fmm_plan copy = *pl;
-  return upload_plan(c, std::move(copy), x, q);
+  // the plan stays the caller's: what the context keeps is copied.  Its tiles
+  // are read where they are, and of the groups beside them only the classes'
+  // offsets and the pairs without a group are taken
+  const bool fits = pl->groups_kind == groups_kind_for(c->p);
+  const bool tiled = fits && takes_tiles(c->p) && pl->tiles.TT == fmmdev::m2l_tile_targets(c->p.P);
+  fmm_plan copy;
+  try {
+    copy.n = pl->n;
+    copy.tree = pl->tree;
+    copy.lists = pl->lists;
+    copy.images = pl->images;
+    std::copy(pl->cycle, pl->cycle + 3, copy.cycle);
+    std::copy(pl->xmin, pl->xmin + 3, copy.xmin);
+    std::copy(pl->xmax, pl->xmax + 3, copy.xmax);
+    copy.t_bounds = pl->t_bounds;
+    copy.t_tree = pl->t_tree;
+    copy.t_lists = pl->t_lists;
+    copy.t_groups = pl->t_groups;
+    copy.dev = pl->dev;
+    if (fits) {
+      copy.groups_kind = pl->groups_kind;
+      if (!tiled) {
+        copy.groups = pl->groups;
+      } else {
+        fmm::M2LGroups &g = copy.groups;
+        g.ngroup = pl->groups.ngroup;
+        g.ncanon = pl->groups.ncanon;
+        g.cdx = pl->groups.cdx;
+        g.nrest = pl->groups.nrest;
+        g.rest_ptr = pl->groups.rest_ptr;
+        g.rest_src = pl->groups.rest_src;
+        g.rest_targets = pl->groups.rest_targets;
+      }
+    }
+  } catch (const std::bad_alloc &) {
+    FMM_FAIL(FMM_ERR_MEMORY, "fmm_set_bodies_plan: host allocation failed");
+  }
+  return upload_plan(c, std::move(copy), x, q, false, false, tiled ? &pl->tiles : nullptr);
 }
 
 namespace {
-int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, bool x_on_device, bool lists_on_device) {
+int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, bool x_on_device, bool lists_on_device,
+                const fmm::M2LTiles *kept) {
   HIPCHK(hipSetDevice(c->p.device));
   if (pl.tree.ncell > 0)
     if (const int rf = check_far(c)) return rf;
@@ -1139,16 +1177,20 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
   c->nchunk = 0;
   c->ntile = 0;
   fmm::M2LTiles tiles;
+  const fmm::M2LTiles *tl = &tiles;
   fmmdev::PlanArrays loc;  // groups and tiles built on the device by this upload
   bool plan_tiles = false;  // tiles taken from the plan
   if (c->use_mfma) {
     // groups built with the plan on the device hold no pair arrays: they serve
     // only with the tiles built beside them (of this order's tile size)
-    const bool fit_tiles = c->use_tiles && pl.tiles.TT == fmmdev::m2l_tile_targets(c->p.P);
+    const bool fit_tiles = c->use_tiles && (kept || pl.tiles.TT == fmmdev::m2l_tile_targets(c->p.P));
     if (pl.groups_kind == groups_kind_for(c->p) && (fit_tiles || fmm::holds_pairs(pl.groups))) {
       c->groups = std::move(pl.groups);
       if (fit_tiles) {
-        tiles = std::move(pl.tiles);
+        if (kept)
+          tl = kept;
+        else
+          tiles = std::move(pl.tiles);
         plan_tiles = true;
       }
     } else {
@@ -1204,13 +1246,13 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
       }
     }
     const fmm::M2LGroups &G = c->groups;
-    UP(g_dx, G.dx) UP(r_ptr, G.rest_ptr) UP(r_src, G.rest_src) UP(r_tgt, G.rest_targets)
+    UP(r_ptr, G.rest_ptr) UP(r_src, G.rest_src) UP(r_tgt, G.rest_targets)
     if (c->use_tiles) {
       const bool dt = plan_tiles && dev_tiles;  // the plan's tiles, their pair arrays on this device
-      if (tiles.TT == 0)
+      if (tl->TT == 0)
         tiles = fmm::build_m2l_tiles(t, G, fmmdev::m2l_tile_targets(c->p.P), fmmdev::kM2LSlicePairs, 0);
-      c->ntile = (int)(tiles.item.size() / 4);  // work items
-      UP(t_tgt, tiles.tgt) UP(t_ptr, tiles.item)
+      c->ntile = (int)(tl->item.size() / 4);  // work items
+      UP(t_tgt, tl->tgt) UP(t_ptr, tl->item)
       if (dt && own) {
         adopt(c->t_slice, pdev->t_slice);
         adopt(c->t_src, pdev->t_src);
@@ -1222,13 +1264,13 @@ int upload_plan(fmm_ctx *c, fmm_plan &&pl, const double *x, const double *q, boo
         adopt(c->t_src, loc.t_src);
         adopt(c->t_lt, loc.t_lt);
         if (!loc.tiles) {  // not built here on the device
-          UP(t_slice, tiles.slice) UP(t_src, tiles.src) UP(t_lt, tiles.lt)
+          UP(t_slice, tl->slice) UP(t_src, tl->src) UP(t_lt, tl->lt)
         }
       }
       UP(c_dx, G.cdx)
     } else {
       c->nchunk = (int)(G.chunk.size() / 4);
-      UP(g_tgt, G.tgt) UP(g_src, G.src) UP(g_chunk, G.chunk)
+      UP(g_dx, G.dx) UP(g_tgt, G.tgt) UP(g_src, G.src) UP(g_chunk, G.chunk)
     }
     if (c->mixed && !c->use_tiles) {
       UP(g_sc, G.scale) UP(cr, t.R)
