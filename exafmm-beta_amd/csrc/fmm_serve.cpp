@@ -83,11 +83,32 @@ int64_t footprint(const fmm_params &p, const fmm_stats &s) {
   return b;
 }
 
+// On target tiles, batches that form by chance (no batch_delay_ms) hold requests
+// of up to this many bodies; larger ones run alone, their groups and tiles built
+// on the device by the upload.  Preparing, merging and uploading a batch is host
+// threads' work and grows with the pairs.  ms a request of streams at
+// saturation, P = 8, fused / alone: 2^12 bodies 0.26 / 0.46 (2 slots), 0.22 / 0.26
+// (8), 2^13 0.47 / 0.54 and 0.36 / 0.30, 2^14 1.25 / 0.67 and 0.73 / 0.39, 2^16
+// 5.7 / 1.35 and 3.1 / 1.1; mixed sizes with the line at 10000 / at 2^14: 2^10..14
+// 0.30 / 0.27 (2 slots), 2^12..18 1.31 / 1.38 (8; no line 3.5, grouped chunks 2.8).
+constexpr int kFuseBodies = 1 << 14;
+bool runs_alone(const fmm_server *s, int n) {
+  return s->p.m2l_mode == FMM_M2L_TILES &&
+         (s->cfg.batch_requests == 1 || (s->cfg.batch_delay_ms == 0 && n > kFuseBodies));
+}
+
 void builder_loop(fmm_server *s) {
   fmm::set_host_threads(1);  // requests are planned in parallel, each on one thread
   // plan_on_device: this builder's own context (stream) for the tree and lists
   fmm_ctx *bc = nullptr;
-  if (s->cfg.plan_on_device && fmm_create(&bc, &s->p) != FMM_OK) {
+  fmm_params bp = s->p;
+  // requests that a batch may hold get their tiles from fmm_plan_prepare: a
+  // system of some thousand bodies is grouped sooner on the host
+  if (s->cfg.batch_requests > 1 && bp.m2l_mode == FMM_M2L_TILES) {  // tree and lists only
+    bp.m2l_mode = FMM_M2L_TARGET;
+    bp.precision = FMM_FP64;
+  }
+  if (s->cfg.plan_on_device && fmm_create(&bc, &bp) != FMM_OK) {
     fmm_destroy(bc);
     bc = nullptr;  // plan on the host instead
   }
@@ -109,10 +130,9 @@ void builder_loop(fmm_server *s) {
                 : fmm_plan_build(&pl, r->n, r->x.data(), s->p.ncrit, s->p.theta, s->p.nspawn);
     // M2L groups for the slots' contexts; the tiles of a request that runs
     // alone are left to the upload, which builds them on the device (a batch
-    // of several concatenates its requests' tiles, those of device-built
-    // plans too, so that a request's M2L is the same alone and in a batch)
-    if (rc == FMM_OK && !(s->p.m2l_mode == FMM_M2L_TILES && s->cfg.batch_requests == 1))
-      rc = fmm_plan_prepare(pl, &s->p);
+    // of several concatenates its requests' tiles, so that a request's M2L is
+    // the same alone and in a batch)
+    if (rc == FMM_OK && !runs_alone(s, r->n)) rc = fmm_plan_prepare(pl, &s->p);
     fmm_stats st{};
     if (rc == FMM_OK) fmm_plan_stats(pl, &st);
     std::lock_guard<std::mutex> lk(s->mu);
@@ -182,7 +202,12 @@ void slot_loop(fmm_server *s, int slot) {
       for (auto it = s->ready.begin(); it != s->ready.end();) {
         const auto &r = it->second;
         const bool first = batch.empty();
-        if (!first && ((int)batch.size() >= s->cfg.batch_requests || bodies + r->n > s->cfg.batch_bodies ||
+        if (!first && !runs_alone(s, batch[0]->n) && runs_alone(s, r->n)) {  // the first of another batch
+          ++it;
+          continue;
+        }
+        if (!first && ((int)batch.size() >= s->cfg.batch_requests || runs_alone(s, batch[0]->n) ||
+                       bodies + r->n > s->cfg.batch_bodies ||
                        s->inflight_bytes + bytes + r->footprint > s->cfg.device_budget))
           break;
         batch.push_back(r);
@@ -273,7 +298,7 @@ void fmm_server_default_config(fmm_server_config *cfg) {
                    // 16 host cores (builders take the rest; at 10 they fall behind)
   cfg->device_budget = (int64_t)32 << 30;
   cfg->batch_bodies = 1 << 20;
-  cfg->batch_requests = 1;  // a batch of several is merged and grouped on the host: slower
+  cfg->batch_requests = 1;  // a batch of several is grouped and merged on the host: slower from 2^13 bodies on
   cfg->batch_delay_ms = 0.0;
   cfg->plan_on_device = 0;
 }

@@ -349,9 +349,10 @@ int fmm_get_lists(fmm_ctx *c, int *m2l_ptr, int *m2l_src, int *p2p_ptr, int *p2p
  * device_budget beside the batches in flight, and evaluates them as one
  * forest (one launch per phase for the whole batch).  Batches of different
  * slots overlap on the GPU.  By default a batch holds one request: a batch of
- * several is merged, then grouped on the host, which measured slower than
- * more slots working at once.  With m2l_mode AUTO the loop's M2L runs on
- * target tiles: when batches hold one request a slot's upload builds their
+ * several is grouped and merged on the host, which pays below some 10000 bodies
+ * a request only.  On target tiles requests of more than 2^14 bodies run alone
+ * unless batch_delay_ms holds batches open.  With m2l_mode AUTO the loop's M2L runs on
+ * target tiles: for requests that run alone a slot's upload builds their
  * groups on the device and the builders plan tree and lists only, else the
  * builders build them too.  A system's result does not depend on its batch
  * beyond rounding: the order of the FP64 atomic additions into its local
