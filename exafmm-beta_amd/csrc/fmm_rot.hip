@@ -24,7 +24,10 @@
 // and 4 P^2 doubles go through LDS between them (twice a slice).  When the
 // last row of tiles holds only one or two degrees (P = 9, 10, 5, 6) their Re
 // and Im parts share it (b = part, degree), and the orders of the same size
-// likewise: 57 instead of 84 products a slice at P = 10.
+// likewise: 57 instead of 84 products a slice at P = 10.  Of a single degree
+// (P = 5, 9) both blocks of a part hold the values and compute different tiles:
+// 12 instead of 18 products at P = 5, 45 instead of 57 at P = 9 (M2L of the 10^6
+// cube 0.50 -> 0.45 ms and 1.27 -> 1.13).
 //
 // M2M and L2L factor the same way with T_m[j,n] = (-r)^(j-n) / (j-n)! (n <= j)
 // and r^(n-j) / (n-j)! (n >= j); as both sides are in one normalisation, s is
@@ -54,9 +57,13 @@ template <int P> struct RotCfg {
   static constexpr int NL = COMB ? G - 1 : G;   // full rows of tiles
   static constexpr int NF = tri(NL, 0);         // full tiles (of each part)
   static constexpr int NX = COMB ? G : 0;       // tiles of the shared row
+  // one degree in it: its values sit in both blocks of a part, which compute
+  // different tiles (2 p and 2 p + 1); the four blocks of m = 0 (Re) likewise
+  static constexpr bool ONE = COMB && REM == 1;
+  static constexpr int NXO = ONE ? (NX + 1) / 2 : NX, NXS = ONE ? (NX + 3) / 4 : NX;
   // products: rotations of the full rows (Re, Im), of the shared row; shifts
-  static constexpr int NQ = sq_sum(NL), NQX = NX * NX;
-  static constexpr int NFRAG = 3 * NQ + 2 * NQX;
+  static constexpr int NQ = sq_sum(NL), NQX = NXO * NX;
+  static constexpr int NFRAG = 3 * NQ + NQX + NXS * NX;
   static constexpr int QRE = 0, QIM = NQ, QX = 2 * NQ, TF = 2 * NQ + NQX, TX = 3 * NQ + NQX;
   static constexpr int NCS = NF + NX;           // (s cos m phi, s sin m phi) of every tile
   static constexpr int NREC = NFRAG + 2 * NCS;  // doubles a lane of one class's record
@@ -211,7 +218,8 @@ __global__ __launch_bounds__(256) void rot_ops_kernel(int kind, const double *__
       v = rot(4 * i + b, 4 * (h / (i + 1)) + r, 4 * (h % (i + 1)) + k, part);
     } else if (f < C::TF) {  // shared row
       const int h = f - C::QX;
-      v = rot(4 * (C::G - 1) + (b & 1), 4 * (h / C::G) + r, 4 * (h % C::G) + k, b >> 1);
+      const int jo = C::ONE ? 2 * (h / C::G) + (b & 1) : h / C::G;
+      v = rot(C::ONE ? P - 1 : 4 * (C::G - 1) + (b & 1), 4 * jo + r, 4 * (h % C::G) + k, b >> 1);
     } else if (f < C::TX) {  // shift levels
       int h = f - C::TF, lev = 0;
       while (h >= C::tiles(lev) * C::tiles(lev)) {
@@ -221,8 +229,8 @@ __global__ __launch_bounds__(256) void rot_ops_kernel(int kind, const double *__
       const int t = C::tiles(lev), mm = C::m0(lev);
       v = shift(mm + b, mm + 4 * (h / t) + r, mm + 4 * (h % t) + k);
     } else if (f < C::NFRAG) {  // shared orders m < REM
-      const int h = f - C::TX, m = b & 1;
-      v = m < C::REM ? shift(m, 4 * (h / C::G) + r, 4 * (h % C::G) + k) : 0.0;
+      const int h = f - C::TX, m = C::ONE ? 0 : b & 1, jo = C::ONE ? 4 * (h / C::G) + b : h / C::G;
+      v = m < C::REM ? shift(m, 4 * jo + r, 4 * (h % C::G) + k) : 0.0;
     } else if (f < C::NREC) {  // z rotation factors, lane (r = lane / 16, b, c)
       const int h = (f - C::NFRAG) >> 1, sn = (f - C::NFRAG) & 1, rr = lane >> 4;
       int n, m;
@@ -236,7 +244,7 @@ __global__ __launch_bounds__(256) void rot_ops_kernel(int kind, const double *__
         n = 4 * i + b;
         m = 4 * j + rr;
       } else {  // own factor cos, partner factor -sin (Re) or +sin (Im)
-        n = 4 * (C::G - 1) + (b & 1);
+        n = C::ONE ? P - 1 : 4 * (C::G - 1) + (b & 1);
         m = 4 * (h - C::NF) + rr;
         neg = !(b >> 1);
       }
@@ -274,6 +282,7 @@ template <int P> struct Rot {
   using C = RotCfg<P>;
   static constexpr int NT = C::NT, G = C::G, NL = C::NL, NF = C::NF, NX = C::NX, AST = C::AST, PART = C::PART;
   static constexpr int NF1 = NF > 0 ? NF : 1, NX1 = NX > 0 ? NX : 1;
+  static constexpr int NXO = C::NXO, NXO1 = NXO > 0 ? NXO : 1;  // results of the shared row
   int r, b, c;
   int row[G], last;  // term of this lane's element of tile (i, 0), of tile (G-1, G-1)
   int w1, w2, x1, x2, x2l;
@@ -296,8 +305,9 @@ template <int P> struct Rot {
     w1 = b * AST + 4 * r + c;
     w2 = r * AST + 4 * b + c;
     x1 = min(b & 1, C::REM - 1) * AST + (b >> 1) * PART + 4 * r + c;
-    x2 = r * AST + (b >> 1) * PART + 4 * (b & 1) + c;
-    x2l = min(4 * (G - 1) + r, C::ROWS - 1) * AST + (b >> 1) * PART + 4 * (b & 1) + c;
+    const int xo = C::ONE ? c : (b >> 1) * PART + 4 * (b & 1) + c;
+    x2 = r * AST + xo;
+    x2l = min(4 * (G - 1) + r, C::ROWS - 1) * AST + xo;
     sX = buf;
   }
   __device__ __forceinline__ int term(int i, int j) const { return i == G - 1 && j == G - 1 ? last : row[i] + 4 * j; }
@@ -325,6 +335,14 @@ template <int P> struct Rot {
       }
     }
   }
+  // results of the shared row: tile, its term (a stand-in past the order), whether it exists
+  __device__ __forceinline__ int xtile(int p) const { return C::ONE ? 2 * p + (b & 1) : p; }
+  __device__ __forceinline__ int xterm(int p) const {
+    return C::ONE ? min(row[G - 1] + 4 * xtile(p), NT - 1) : term(G - 1, p);
+  }
+  __device__ __forceinline__ bool xvalid(int p) const {
+    return C::ONE ? 4 * xtile(p) + r < P : valid(G - 1, p);
+  }
   // an expansion's terms as this lane holds them
   __device__ __forceinline__ void gather(const double2 *m, double2 (&pf)[NF1], double (&px)[NX1]) const {
 #pragma unroll
@@ -334,14 +352,26 @@ template <int P> struct Rot {
 #pragma unroll
     for (int j = 0; j < NX; j++) px[j] = reinterpret_cast<const double *>(m + term(G - 1, j))[b >> 1];
   }
+  // an expansion that results are added to, as this lane holds those
+  __device__ __forceinline__ void gather_out(const double2 *m, double2 (&av)[NF1], double (&ax)[NXO1]) const {
+#pragma unroll
+    for (int i = 0; i < NL; i++)
+#pragma unroll
+      for (int j = 0; j <= i; j++) av[tri(i, j)] = m[term(i, j)];
+#pragma unroll
+    for (int p = 0; p < NXO; p++) ax[p] = reinterpret_cast<const double *>(m + xterm(p))[b >> 1];
+  }
   // z rotation factors of the class's offset reflected by the bits rf (x, y,
   // z): the operator changes by the sign (-1)^(x m + z (n + m)) on both sides,
   // and phi -> -phi when one of x and y is reflected
   __device__ __forceinline__ void zfactors(int rf, double2 (&z)[C::NCS]) const {
-    const unsigned mc = (unsigned)((rf & r) ^ ((rf >> 2) & (b ^ r))) << 31;
-    const unsigned ms = mc ^ ((unsigned)(rf ^ (rf >> 1)) << 31);
+    const unsigned mc = (unsigned)((rf & r) ^ ((rf >> 2) & (b ^ r))) << 31, sc = (unsigned)(rf ^ (rf >> 1)) << 31;
+    const unsigned mx = C::ONE ? (unsigned)((rf & r) ^ ((rf >> 2) & r)) << 31 : mc;  // n = P - 1 is even
 #pragma unroll
-    for (int t = 0; t < C::NCS; t++) z[t] = make_double2(flip(cs[t].x, mc), flip(cs[t].y, ms));
+    for (int t = 0; t < C::NCS; t++) {
+      const unsigned m = t < NF ? mc : mx;
+      z[t] = make_double2(flip(cs[t].x, m), flip(cs[t].y, m ^ sc));
+    }
   }
   __device__ __forceinline__ void zrot(const double2 (&z)[C::NCS], const double2 (&pf)[NF1], const double (&px)[NX1],
                                        double (&re)[NF1], double (&im)[NF1], double (&xv)[NX1]) const {
@@ -355,17 +385,26 @@ template <int P> struct Rot {
   }
   // z rotation back, added to av, ax
   __device__ __forceinline__ void zback(const double2 (&z)[C::NCS], const double (&re)[NF1], const double (&im)[NF1],
-                                        const double (&xv)[NX1], double2 (&av)[NF1], double (&ax)[NX1]) const {
+                                        const double (&xv)[NXO1], double2 (&av)[NF1], double (&ax)[NXO1]) const {
 #pragma unroll
     for (int t = 0; t < NF; t++) {
       av[t].x = fma(z[t].x, re[t], fma(z[t].y, im[t], av[t].x));
       av[t].y = fma(z[t].x, im[t], fma(-z[t].y, re[t], av[t].y));
     }
 #pragma unroll
-    for (int j = 0; j < NX; j++) ax[j] = fma(z[NF + j].x, xv[j], fma(-z[NF + j].y, partner(xv[j]), ax[j]));
+    for (int p = 0; p < NXO; p++) {
+      const double2 z0 = z[NF + (C::ONE ? 2 * p : p)];
+      double cx = z0.x, cy = z0.y;
+      if constexpr (C::ONE) {
+        const double2 z1 = z[NF + (2 * p + 1 < NX ? 2 * p + 1 : 2 * p)];
+        cx = b & 1 ? z1.x : cx;
+        cy = b & 1 ? z1.y : cy;
+      }
+      ax[p] = fma(cx, xv[p], fma(-cy, partner(xv[p]), ax[p]));
+    }
   }
   // this lane's terms stored into an expansion
-  __device__ __forceinline__ void scatter(double2 *acc, const double2 (&av)[NF1], const double (&ax)[NX1]) const {
+  __device__ __forceinline__ void scatter(double2 *acc, const double2 (&av)[NF1], const double (&ax)[NXO1]) const {
 #pragma unroll
     for (int i = 0; i < NL; i++)
 #pragma unroll
@@ -375,8 +414,8 @@ template <int P> struct Rot {
     for (int i = 0; i < NL; i++)
       if (4 * i + 3 < P ? r <= b : valid(i, i)) acc[row[i] + 4 * i] = av[tri(i, i)];
 #pragma unroll
-    for (int j = 0; j < NX; j++)
-      if (valid(G - 1, j)) reinterpret_cast<double *>(acc + row[G - 1] + 4 * j)[b >> 1] = ax[j];
+    for (int p = 0; p < NXO; p++)
+      if (xvalid(p)) reinterpret_cast<double *>(acc + row[G - 1] + 4 * xtile(p))[b >> 1] = ax[p];
   }
   // products of one part: rotation of the full rows, of the shared row, shift
   __device__ __forceinline__ void rot_part(int q, double (&v)[NF1]) const {
@@ -393,16 +432,14 @@ template <int P> struct Rot {
 #pragma unroll
     for (int t = 0; t < NF; t++) v[t] = o[t];
   }
-  __device__ __forceinline__ void mul_shared(int q, double (&v)[NX1]) const {
-    double o[NX1];
+  template <int NO, int NO1> __device__ __forceinline__ void mul_shared(int q, const double (&v)[NX1],
+                                                                        double (&o)[NO1]) const {
 #pragma unroll
-    for (int t = 0; t < NX; t++) o[t] = 0.0;
+    for (int t = 0; t < NO; t++) o[t] = 0.0;
 #pragma unroll
     for (int ji = 0; ji < NX; ji++)
 #pragma unroll
-      for (int jo = 0; jo < NX; jo++) o[jo] = mm(A[q + jo * G + ji], v[ji], o[jo]);
-#pragma unroll
-    for (int t = 0; t < NX; t++) v[t] = o[t];
+      for (int jo = 0; jo < NO; jo++) o[jo] = mm(A[q + jo * G + ji], v[ji], o[jo]);
   }
   __device__ __forceinline__ void shift_part(double (&v)[NF1]) const {
     double o[NF1];
@@ -446,19 +483,25 @@ template <int P> struct Rot {
       for (int i = 0; i < C::tiles(k); i++)
         v[C::off2(k) + i] = sX[w2 + off + (C::m0(k) + 4 * i) * AST + 4 * C::m0(k)];
   }
-  __device__ __forceinline__ void put1x(const double (&v)[NX1]) const {
+  __device__ __forceinline__ void put1x(const double (&v)[NXO1]) const {
 #pragma unroll
-    for (int j = 0; j < NX; j++)
-      if ((b & 1) < C::REM) sX[x1 + 4 * (G - 1) * AST + 16 * j] = v[j];
+    for (int p = 0; p < NXO; p++)
+      if (C::ONE ? xtile(p) < NX : (b & 1) < C::REM) sX[x1 + 4 * (G - 1) * AST + 16 * xtile(p)] = v[p];
   }
   __device__ __forceinline__ void get1x(double (&v)[NX1]) const {
 #pragma unroll
     for (int j = 0; j < NX; j++) v[j] = sX[x1 + 4 * (G - 1) * AST + 16 * j];
   }
-  __device__ __forceinline__ void put2x(const double (&v)[NX1]) const {
+  static constexpr int NXS1 = C::NXS > 0 ? C::NXS : 1;
+  __device__ __forceinline__ void put2x(const double (&v)[NXS1]) const {
 #pragma unroll
-    for (int i = 0; i < NX; i++)
-      if ((i < G - 1 || 4 * i + r < P) && (b & 1) < C::REM) sX[x2 + 4 * i * AST] = v[i];
+    for (int i = 0; i < C::NXS; i++) {
+      if constexpr (C::ONE) {
+        if (4 * (4 * i + b) + r < P) sX[x2 + 4 * (4 * i + b) * AST] = v[i];
+      } else {
+        if ((i < G - 1 || 4 * i + r < P) && (b & 1) < C::REM) sX[x2 + 4 * i * AST] = v[i];
+      }
+    }
   }
   __device__ __forceinline__ void get2x(double (&v)[NX1]) const {
 #pragma unroll
@@ -468,9 +511,10 @@ template <int P> struct Rot {
   // the other part's products
   __device__ __forceinline__ void turn_shift(double (&re)[NF1], double (&im)[NF1], double (&xv)[NX1]) const {
     if constexpr (C::COMB) {
-      mul_shared(C::QX, xv);
+      double xo[NXO1], xs[NXS1];
+      mul_shared<NXO>(C::QX, xv, xo);
       rot_part(C::QRE, re);
-      put1x(xv);
+      put1x(xo);
       put1(re, 0);
       rot_part(C::QIM, im);
       lds_order();
@@ -482,8 +526,8 @@ template <int P> struct Rot {
       lds_order();
       shift_part(re);
       put2(re, 0);
-      mul_shared(C::TX, xv);
-      put2x(xv);
+      mul_shared<C::NXS>(C::TX, xv, xs);
+      put2x(xs);
       shift_part(im);
       lds_order();
       get1(re, 0);
@@ -515,9 +559,10 @@ template <int P> struct Rot {
       lds_order();
     }
   }
-  __device__ __forceinline__ void turn_back(double (&re)[NF1], double (&im)[NF1], double (&xv)[NX1]) const {
+  __device__ __forceinline__ void turn_back(double (&re)[NF1], double (&im)[NF1], const double (&xv)[NX1],
+                                            double (&xo)[NXO1]) const {
     rot_part(C::QRE, re);
-    if constexpr (C::COMB) mul_shared(C::QX, xv);
+    if constexpr (C::COMB) mul_shared<NXO>(C::QX, xv, xo);
     rot_part(C::QIM, im);
   }
 };
@@ -584,11 +629,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void m2
     // the targets' local expansions are read while the back rotation runs
     double2 *acc = sAcc + (lt & 255) * NT;
     double2 av[R::NF1];
-    double ax[R::NX1];
-    rot.gather(acc, av, ax);
-    rot.turn_back(re, im, xv);
+    double ax[R::NXO1], xo[R::NXO1];
+    rot.gather_out(acc, av, ax);
+    rot.turn_back(re, im, xv, xo);
     if (d1.x != d.x) rot.load(ops, d1.x, l);
-    rot.zback(z, re, im, xv, av, ax);
+    rot.zback(z, re, im, xo, av, ax);
     if (c < d.z) rot.scatter(acc, av, ax);
     lds_order();
     d = d1;
@@ -650,7 +695,7 @@ __global__ __launch_bounds__(512) void m2m_rot_kernel(const int *__restrict__ pa
     const int i = g + rot.c;
     const int ch = i < np ? child8[8 * (size_t)i + w] : -1;
     double2 pf[R::NF1], av[R::NF1];
-    double px[R::NX1], ax[R::NX1];
+    double px[R::NX1], ax[R::NXO1], xo[R::NXO1];
     rot.gather(M + (size_t)max(ch, 0) * NT, pf, px);
 #pragma unroll
     for (int t = 0; t < R::NF1; t++) {
@@ -658,15 +703,15 @@ __global__ __launch_bounds__(512) void m2m_rot_kernel(const int *__restrict__ pa
       av[t] = make_double2(0.0, 0.0);
     }
 #pragma unroll
-    for (int t = 0; t < R::NX1; t++) {
+    for (int t = 0; t < R::NX1; t++)
       if (ch < 0) px[t] = 0.0;
-      ax[t] = 0.0;
-    }
+#pragma unroll
+    for (int t = 0; t < R::NXO1; t++) ax[t] = 0.0;
     double re[R::NF1], im[R::NF1], xv[R::NX1];
     rot.zrot(z, pf, px, re, im, xv);
     rot.turn_shift(re, im, xv);
-    rot.turn_back(re, im, xv);
-    rot.zback(z, re, im, xv, av, ax);
+    rot.turn_back(re, im, xv, xo);
+    rot.zback(z, re, im, xo, av, ax);
     rot.scatter(sO[w] + rot.c * NT, av, ax);
     __syncthreads();
     for (int e = threadIdx.x; e < 4 * NT; e += 512) {
@@ -708,17 +753,17 @@ __global__ __launch_bounds__(64) void l2l_rot_kernel(const int2 *__restrict__ ki
     double2 z[C::NCS];
     rot.zfactors(~(kd.y >> 27) & 7, z);  // X_child - X_parent: negative along d when octant bit d is clear
     double2 pf[R::NF1], av[R::NF1];
-    double px[R::NX1], ax[R::NX1];
+    double px[R::NX1], ax[R::NXO1], xo[R::NXO1];
     rot.gather(L + (size_t)(kd.y & ((1 << 27) - 1)) * NT, pf, px);
     double re[R::NF1], im[R::NF1], xv[R::NX1];
     rot.zrot(z, pf, px, re, im, xv);
     rot.turn_shift(re, im, xv);
     double2 *Lc = L + (size_t)kd.x * NT;
-    rot.gather(Lc, av, ax);
-    rot.turn_back(re, im, xv);
+    rot.gather_out(Lc, av, ax);
+    rot.turn_back(re, im, xv, xo);
 #pragma unroll
     for (int t = 0; t < C::NCS; t++) z[t] = make_double2(flip(z[t].x, odd), flip(z[t].y, odd));
-    rot.zback(z, re, im, xv, av, ax);
+    rot.zback(z, re, im, xo, av, ax);
     if (g + rot.c < nk) rot.scatter(Lc, av, ax);
   }
 }
