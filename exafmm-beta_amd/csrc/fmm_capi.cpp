@@ -396,11 +396,11 @@ int fmm_create(fmm_ctx **out, const fmm_params *p) {
     rc = FMM_ERR_UNSUPPORTED;
   } else if (p->precision == FMM_MIXED16 &&
              (!fmmdev::m2l_mixed_supported(p->P) || p->m2l_mode == FMM_M2L_TARGET || p->m2l_mode == FMM_M2L_GROUPED)) {
-    c->err = "mixed precision with split-FP16 M2L needs 2 <= P <= 12 and m2l_mode AUTO or TILES";
+    c->err = "FMM_MIXED16 needs 2 <= P <= 12 and m2l_mode AUTO or TILES";
     rc = FMM_ERR_UNSUPPORTED;
   } else if (p->precision == FMM_MIXED &&
              (!fmmdev::m2l_mixed_supported(p->P) || p->m2l_mode == FMM_M2L_TARGET)) {
-    c->err = "mixed precision needs 2 <= P <= 12 and m2l_mode AUTO or GROUPED";
+    c->err = "mixed precision needs 2 <= P <= 12 and an m2l_mode other than TARGET";
     rc = FMM_ERR_UNSUPPORTED;
   }
   if (rc == FMM_OK) {

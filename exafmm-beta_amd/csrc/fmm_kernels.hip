@@ -136,8 +136,9 @@ __device__ void regular_column(double dx, double dy, double dz, int m, double2 *
 // sums are added in order through LDS; a wavefront takes 64 / (H S) leaves.
 // Bound: FP64 VALU (about 180 instructions a body and lane) and the serial
 // steps of each body.  A lane per (body slot, m) left half its steps masked off
-// and loaded a constant from memory in every step: 8M cube, P = 12, 4.9 -> 0.6
-// ms beside P2P; 1M Plummer, P = 10, 1.5 -> 0.15 ms.
+// and loaded a constant from memory in every step: alone, 8M cube, P = 12, 1.85 ->
+// 0.67 ms, 1M Plummer, P = 10, 0.17 -> 0.09; in a solve, where P2P runs beside it
+// and has most of the SIMDs, 8.0 -> 5.4 and 1.37 -> 0.86.
 template <int P, int S>
 __global__ __launch_bounds__(64) void p2m_kernel(DevBodies B, DevCells C, const int *__restrict__ leaves,
                                                  int nleaf, double2 *__restrict__ M) {

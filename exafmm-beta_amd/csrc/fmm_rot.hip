@@ -673,8 +673,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void m2
 // Bound: latency of the children's gather and the LDS round trips on the small
 // levels, issue on the large ones.  Measured against a dense P^2 x P^2 operator
 // per octant (16 parents a block, each reading 8 operators of 166 KB at P =
-// 12): 8M cube, P = 12, all 13 levels 10.0 -> 0.90 ms; 1M Plummer, P = 10, 10
-// levels 0.91 -> 0.28 ms; 4096 bodies, P = 8: 13 -> 7 us a level.
+// 12), all levels: alone, 8M cube, P = 12, 1.78 -> 0.36 ms, 1M Plummer, P = 10,
+// 0.32 -> 0.10; in a solve, beside P2P, 4.0 -> 2.4 and 0.83 -> 0.56; 4096 bodies, P
+// = 8: 13 -> 7 us a level.
 template <int P>
 __global__ __launch_bounds__(512) void m2m_rot_kernel(const int *__restrict__ parents, const int *__restrict__ child8,
                                                       int np, const double2 *__restrict__ rec,
