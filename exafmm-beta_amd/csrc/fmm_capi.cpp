@@ -251,7 +251,7 @@ int upload_staged(fmm_ctx *c, std::initializer_list<std::tuple<DBuf *, const voi
 // fresh pages): 7.3 ms; four pageable copies and a host loop took 131 ms.
 int download_staged(fmm_ctx *c, void *dst, const void *src, size_t bytes) {
   // a few MB: one pageable copy (3 MB: 0.26 ms and 128 KB 0.02 ms against 0.20
-  // and 0.04 through the slots, which take 1.2 ms more at their first touch)
+  // and 0.04 through the slots, which take 0.3 ms more at their first touch)
   if (bytes <= (size_t)4 << 20) {
     HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
@@ -587,7 +587,11 @@ int device_tree_of(fmm_ctx *c, fmm::Tree &t, int n, const double *x, int ncrit, 
   double X0[3], R0;
   fmm::root_box(xmin, xmax, X0, R0);
   // the bodies go up through the context's pinned staging into its
-  // upload buffer (scratch between uploads)
+  // upload buffer (scratch between uploads); a new staging has room for the
+  // targets that come down through it (up to 16 MB of 32 n bytes), which
+  // would allocate it again in the first fmm_get_targets
+  if (sizeof(double) * 3 * (size_t)n > c->pin_cap)
+    if (const int rc = pin_at_least(c, std::max(30 * (size_t)n, std::min(40 * (size_t)n, (size_t)20 << 20)))) return rc;
   const int rc = upload_staged(c, {{&c->xin, x, sizeof(double) * 3 * (size_t)n}});
   if (rc) {
     (void)hipStreamSynchronize(c->st);
