@@ -974,10 +974,11 @@ int fmm_set_bodies_plan(fmm_ctx *c, const fmm_plan *pl, const double *x, const d
       (pl->images > 0 && (pl->cycle[0] != c->p.cycle[0] || pl->cycle[1] != c->p.cycle[1] || pl->cycle[2] != c->p.cycle[2])))
     FMM_FAIL(FMM_ERR_ARG, "fmm_set_bodies_plan: the plan's periodic images differ from the context's");
   // the plan stays the caller's: what the context keeps is copied.  Its tiles
-  // are read where they are, and of the groups beside them only the classes'
-  // offsets and the pairs without a group are taken
-  const bool fits = pl->groups_kind == groups_kind_for(c->p);
-  const bool tiled = fits && takes_tiles(c->p) && pl->tiles.TT == fmmdev::m2l_tile_targets(c->p.P);
+  // are read where they are (but on another device, from where the copy's are
+  // fetched), and of the groups beside them only the classes' offsets and the
+  // pairs without a group are taken
+  const bool fits = pl->groups_kind == groups_kind_for(c->p), here = !pl->dev || pl->dev->device == c->p.device;
+  const bool tiled = fits && here && takes_tiles(c->p) && pl->tiles.TT == fmmdev::m2l_tile_targets(c->p.P);
   fmm_plan copy;
   try {
     copy.n = pl->n;
@@ -996,6 +997,7 @@ int fmm_set_bodies_plan(fmm_ctx *c, const fmm_plan *pl, const double *x, const d
       copy.groups_kind = pl->groups_kind;
       if (!tiled) {
         copy.groups = pl->groups;
+        if (!here) copy.tiles = pl->tiles;
       } else {
         fmm::M2LGroups &g = copy.groups;
         g.ngroup = pl->groups.ngroup;
