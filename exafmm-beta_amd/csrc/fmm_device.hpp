@@ -154,8 +154,9 @@ hipError_t init_scratch(int device);
 // stream: a block given back on stream s is handed to a later request on s
 // (the stream's order makes the reuse safe), the smallest cached block that
 // fits and is at most twice the request plus 1 MiB, else a new hipMalloc'd
-// one (current device).  A stream keeps at most 8 GiB cached (a block beyond
-// that is freed); plan_scratch_release(s) frees the stream's blocks after
+// one (current device).  A stream keeps at most 12 GiB cached (a block beyond
+// that is freed: with 8 the 60M M2L pairs of 8M bodies, whose pair arrays change
+// places with cached ones, took 53 ms to set in place of 50); plan_scratch_release(s) frees the stream's blocks after
 // its work (the owner calls it before destroying s).  Replaces a
 // hipMallocAsync / hipFreeAsync pair per buffer, about 0.2 ms of host time
 // each on this runtime.

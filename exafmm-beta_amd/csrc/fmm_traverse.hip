@@ -894,7 +894,7 @@ struct ScratchCache {
 };
 std::mutex g_scratch_mu;
 std::map<hipStream_t, ScratchCache> g_scratch;
-constexpr size_t kScratchKeep = (size_t)8 << 30;
+constexpr size_t kScratchKeep = (size_t)12 << 30;
 }  // namespace
 
 hipError_t plan_scratch_get(void **p, size_t *cap, size_t bytes, hipStream_t s, size_t spare) {
